@@ -9,6 +9,7 @@ namespace gemm {
 
 CPT_GEMM_INST_ALL(CPT_GEMM_DECLARE)
 CPT_NT16_INST_ALL(CPT_NT16_DECLARE)
+CPT_ST16_INST_ALL(CPT_ST16_DECLARE)
 
 // out[m, n] = bf16(alpha * sum_s ws[s][m][n])  (split-K reduction, fixed order)
 __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restrict__ ws,
@@ -182,6 +183,27 @@ int dispatch_gs(int64_t gs, KArgs& A, hipStream_t st) {
   }
 }
 
+// A product on the 16x16x32 loop: 128 x 128 tiles when at most two of them per
+// CU cover the output, else 256 x 256 (bit-identical either way).  With at
+// least 512 small tiles the 256 x 256 ones fill half the chip or more and
+// their loop does 1.2-1.5x the FLOP per CU; below, the small ones win.  One
+// block per CU takes 4 LDS stages, more take 2 (two blocks share a CU).
+// Measured on MI355X, us for 256 x 256 / 2 stages / 4 stages:
+//   512 x 2048, k 5632    (64 small tiles)    94.3 /  62.8 /  37.5
+//   2048 x 2048, k 11264  (256)              189.7 / 134.0 /  87.6
+//   512 x 11264, k 2048   (352)               44.6 /  33.7 /  34.5
+//   2048 x 4096, k 11008  (512)              202.7 / 161.5 / 171.7
+//   2048 x 5632, k 2048   (704)               48.8 /  58.3 /  53.6
+//   333 x 22016, k 4096   (516)               84.1 / 104.2 /  89.7
+template <bool AK, bool BK, int EPI, int CACHE, int LT>
+int launch16(const KArgs& A, hipStream_t st) {
+  const int64_t small = ((A.M + 127) / 128) * ((A.N + 127) / 128);
+  const int cus = num_cus();
+  if (small <= cus) return launch_st16<AK, BK, EPI, CACHE, LT, 4>(A, st);
+  if (small <= 2 * (int64_t)cus) return launch_st16<AK, BK, EPI, CACHE, LT, 2>(A, st);
+  return launch_nt16<AK, BK, EPI, CACHE, EPI == EPI_STORE ? 0 : 64, LT>(A, st);
+}
+
 // Adapter terms of one call (see acc_block).  P_t [M, rank] with rows ldp
 // apart; Q_t [n_q, rank] contiguous (q_kmajor) or [rank, n_q] with rows ldq
 // apart.  rank 0: no terms.
@@ -271,11 +293,11 @@ int gemm_bf16_impl(const void* a, int64_t lda, int a_kmajor, const void* b, int6
     // adapter terms are carried by the layouts that need them: K-major A
     if (!a_kmajor) return kErrShape;
     if (nt16 && terms == 1)
-      return b_kmajor ? launch_nt16<true, true, EPI_STORE, 0, 0, 1>(A, st)
-                      : launch_nt16<true, false, EPI_STORE, 0, 0, 1>(A, st);
+      return b_kmajor ? launch16<true, true, EPI_STORE, 0, 1>(A, st)
+                      : launch16<true, false, EPI_STORE, 0, 1>(A, st);
     if (nt16)
-      return b_kmajor ? launch_nt16<true, true, EPI_STORE, 0, 0, 2>(A, st)
-                      : launch_nt16<true, false, EPI_STORE, 0, 0, 2>(A, st);
+      return b_kmajor ? launch16<true, true, EPI_STORE, 0, 2>(A, st)
+                      : launch16<true, false, EPI_STORE, 0, 2>(A, st);
     // the engine carries adapter ranks up to 16
     if (L.rank > 16) return kErrShape;
     if (terms == 1)
@@ -285,10 +307,10 @@ int gemm_bf16_impl(const void* a, int64_t lda, int a_kmajor, const void* b, int6
                     : launch<true, false, EPI_STORE, 0, 0, 2>(A, st);
   }
   if (nt16) {
-    if (a_kmajor && b_kmajor) return launch_nt16<true, true, EPI_STORE, 0, 0, 0>(A, st);
-    if (a_kmajor && !b_kmajor) return launch_nt16<true, false, EPI_STORE, 0, 0, 0>(A, st);
-    if (!a_kmajor && !b_kmajor) return launch_nt16<false, false, EPI_STORE, 0, 0, 0>(A, st);
-    return launch_nt16<false, true, EPI_STORE, 0, 0, 0>(A, st);
+    if (a_kmajor && b_kmajor) return launch16<true, true, EPI_STORE, 0, 0>(A, st);
+    if (a_kmajor && !b_kmajor) return launch16<true, false, EPI_STORE, 0, 0>(A, st);
+    if (!a_kmajor && !b_kmajor) return launch16<false, false, EPI_STORE, 0, 0>(A, st);
+    return launch16<false, true, EPI_STORE, 0, 0>(A, st);
   }
   if (a_kmajor && b_kmajor) return launch<true, true, EPI_STORE, 0, 0>(A, st);
   if (a_kmajor && !b_kmajor) return launch<true, false, EPI_STORE, 0, 0>(A, st);
@@ -402,8 +424,12 @@ int ffn_gate_up_impl(const void* x, const void* w_gate, const void* w_up, int64_
   (terms ? launch_nt16<true, true, EPI_GLU, CACHE, GS, 2>(A, st) \
          : launch_nt16<true, true, EPI_GLU, CACHE, GS, 0>(A, st))
     switch (cache) {
-      case CACHE_NONE: return CPT_F1_NT16(CACHE_NONE, 64);
-      case CACHE_BF16: return CPT_F1_NT16(CACHE_BF16, 64);
+      case CACHE_NONE:
+        return terms ? launch16<true, true, EPI_GLU, CACHE_NONE, 2>(A, st)
+                     : launch16<true, true, EPI_GLU, CACHE_NONE, 0>(A, st);
+      case CACHE_BF16:
+        return terms ? launch16<true, true, EPI_GLU, CACHE_BF16, 2>(A, st)
+                     : launch16<true, true, EPI_GLU, CACHE_BF16, 0>(A, st);
       case CACHE_INT4:
         return group_size == 32   ? CPT_F1_NT16(CACHE_INT4, 32)
                : group_size == 64 ? CPT_F1_NT16(CACHE_INT4, 64)
@@ -506,7 +532,9 @@ int ffn_down_dgrad_impl(const void* grad_y, const void* w_down, int64_t n_tok, i
   (terms ? launch_nt16<true, false, EPI_DGLU, CACHE, GS, 1>(A, st) \
          : launch_nt16<true, false, EPI_DGLU, CACHE, GS, 0>(A, st))
     switch (cache) {
-      case CACHE_BF16: return CPT_B1_NT16(CACHE_BF16, 64);
+      case CACHE_BF16:
+        return terms ? launch16<true, false, EPI_DGLU, CACHE_BF16, 1>(A, st)
+                     : launch16<true, false, EPI_DGLU, CACHE_BF16, 0>(A, st);
       case CACHE_INT4:
         return group_size == 32   ? CPT_B1_NT16(CACHE_INT4, 32)
                : group_size == 64 ? CPT_B1_NT16(CACHE_INT4, 64)

@@ -36,6 +36,12 @@ int device_cus(int dev) {
 }
 }  // namespace
 
+int num_cus() {
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return 0;
+  return device_cus(dev);
+}
+
 int64_t stream_k_bytes(int cus) {
   // cus partial slots of one tile's fp32 accumulators, then cus flags and
   // one error count

@@ -63,12 +63,17 @@ _FUSED_GROUPS = (32, 64, 128)
 # block's MFMAs idle meanwhile) costs more than K1 at HBM speed; a longer
 # k-loop per tile (larger d_model) and more waves of tiles amortise it.
 _F1_CODEC_MIN_TOKENS = {"int8": 4096, "int4": 8192}
-_F1_CODEC_WIDE_D_MODEL = 4096      # from here on, at any token count
+_F1_CODEC_WIDE_D_MODEL = 4096      # from here on, whenever 256 x 256 tiles run
 
 
-def _f1_codec_fused(cache_mode: str, tokens: int, d_model: int) -> bool:
+def _f1_codec_fused(cache_mode: str, tokens: int, d_model: int, d_ff: int = 0) -> bool:
+    """The codec epilogue exists on 256 x 256 tiles only: below the token
+    thresholds a gate/up product that runs on 128 x 128 tiles (G.small_tiles)
+    takes its bf16 output and K1 (64 tokens, 4096 x 11008: 31 + 4 us against
+    73)."""
     m = _F1_CODEC_MIN_TOKENS.get(cache_mode)
-    return m is not None and (tokens >= m or d_model >= _F1_CODEC_WIDE_D_MODEL)
+    return m is not None and (tokens >= m or (
+        d_model >= _F1_CODEC_WIDE_D_MODEL and not (d_ff and G.small_tiles(tokens, 2 * d_ff))))
 
 
 # Outlier channels (config C3) with a bf16 activation and d_model a multiple
@@ -300,7 +305,7 @@ class FlashFFNv3Function(torch.autograd.Function):
             xa_g, xa_u, lkw = _gate_up_lora(x_2d, a_gate, b_gate, s_gate, a_up, b_up, s_up)
         fused_quant = (quant and use_triton and x.dtype == torch.bfloat16)   # :1424-1426
         if (fusable and fused_quant and k_out == 0 and group_size in _FUSED_GROUPS
-                and _f1_codec_fused(cache_mode, x_2d.shape[0], hidden_dim)):
+                and _f1_codec_fused(cache_mode, x_2d.shape[0], hidden_dim, inter)):
             # dual GEMM + GLU + codec in one kernel (K1 fused into the epilogue)
             h_mid, _, _, c_gate, qs_gate, c_up, qs_up = G.ffn_gate_up(
                 x_2d, w_gate, w_up, _CACHE_CODE[cache_mode], group_size, **lkw)
@@ -882,7 +887,8 @@ class FlashFFNv3AdapterFunction(torch.autograd.Function):
         c_gate = qs_gate = c_up = qs_up = None
         h_gate = h_up = xa_g = xa_u = None
         if (fusable and fused_quant and group_size in _FUSED_GROUPS
-                and _f1_codec_fused(cache_mode, x_2d.shape[0], hidden_dim)):
+                and _f1_codec_fused(cache_mode, x_2d.shape[0], hidden_dim,
+                                    w_gate.shape[0])):
             h_mid, _, _, c_gate, qs_gate, c_up, qs_up = G.ffn_gate_up(
                 x_2d, w_gate, w_up, _CACHE_CODE[cache_mode], group_size)
             _V3_COUNTERS["triton_quant_fwd"] += 1

@@ -386,6 +386,12 @@ def _min_splits(K: int, lda: int, ak: int, ldb: int, bk: int) -> int:
     return (nk + per - 1) // per
 
 
+def small_tiles(m: int, n: int) -> bool:
+    """The 16x16x32 loop covers an [m, n] output with 128 x 128 tiles: at most
+    two per CU (launch16 in csrc/gemm.hip; 256 CUs)."""
+    return ((m + 127) // 128) * ((n + 127) // 128) <= 512
+
+
 def mm(a: torch.Tensor, b: torch.Tensor, name: str = "gemm") -> torch.Tensor:
     """a [M, K] @ b [K, N] -> bf16 [M, N] on the MFMA GEMM loops (16x16x32 when
     K is a multiple of 64 and N of 8, else the 32x32x16 engine).  Tall products
