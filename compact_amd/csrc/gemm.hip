@@ -199,8 +199,8 @@ template <bool AK, bool BK, int EPI, int CACHE, int LT>
 int launch16(const KArgs& A, hipStream_t st) {
   const int64_t small = ((A.M + 127) / 128) * ((A.N + 127) / 128);
   const int cus = num_cus();
-  if (small <= cus) return launch_st16<AK, BK, EPI, CACHE, LT, 4>(A, st);
-  if (small <= 2 * (int64_t)cus) return launch_st16<AK, BK, EPI, CACHE, LT, 2>(A, st);
+  if (small <= cus) return launch_st16<kBF16, AK, BK, EPI, CACHE, LT, 4>(A, st);
+  if (small <= 2 * (int64_t)cus) return launch_st16<kBF16, AK, BK, EPI, CACHE, LT, 2>(A, st);
   return launch_nt16<AK, BK, EPI, CACHE, EPI == EPI_STORE ? 0 : 64, LT>(A, st);
 }
 
@@ -316,6 +316,85 @@ int gemm_bf16_impl(const void* a, int64_t lda, int a_kmajor, const void* b, int6
   if (a_kmajor && !b_kmajor) return launch<true, false, EPI_STORE, 0, 0>(A, st);
   if (!a_kmajor && !b_kmajor) return launch<false, false, EPI_STORE, 0, 0>(A, st);
   return launch<false, true, EPI_STORE, 0, 0>(A, st);
+}
+
+// A 16-bit product on 128 x 128 tiles whatever its size: fp16, or k split into
+// `splits` ranges with fp32 partials in ws [splits][M][N] (dual: [..][2 D]).
+template <int DT, bool AK, bool BK, int EPI, int CACHE, int LT>
+int launch_small(const KArgs& A, hipStream_t st) {
+  const int64_t blocks = ((A.M + 127) / 128) * ((A.N + 127) / 128) * (EPI == EPI_F32 ? A.ksplit : 1);
+  return blocks <= num_cus() ? launch_st16<DT, AK, BK, EPI, CACHE, LT, 4>(A, st)
+                             : launch_st16<DT, AK, BK, EPI, CACHE, LT, 2>(A, st);
+}
+
+// k ranges of whole k-tiles, none empty; true if more than one
+inline bool set_split(KArgs& A, int splits, void* ws) {
+  int nk = (int)((A.K[0] + 63) / 64) + (A.npairs == 2 ? (int)((A.K[1] + 63) / 64) : 0);
+  if (nk < 1) nk = 1;
+  if (splits > nk) splits = nk;
+  A.kt_per_split = (nk + splits - 1) / splits;
+  A.ksplit = (nk + A.kt_per_split - 1) / A.kt_per_split;
+  A.ws = (float*)ws;
+  return A.ksplit > 1;
+}
+
+template <int DT>
+int gemm16_impl(const void* a, int64_t lda, int a_kmajor, const void* b, int64_t ldb, int b_kmajor,
+                const void* a2, int64_t lda2, const void* b2, int64_t ldb2, int64_t K2, void* c,
+                int64_t ldc, int64_t M, int64_t N, int64_t K, const LoraTerms& L, int splits,
+                void* ws, void* stream) {
+  if (M < 0 || N < 0 || K < 0 || K2 < 0 || splits < 1) return kErrShape;
+  if (M == 0 || N == 0) return kOk;
+  const bool two = a2 != nullptr;
+  // whole k-tiles, but for a last partial one of two MN-major operands
+  const bool tail = !a_kmajor && !b_kmajor;
+  if (!nt16_fits(M, N, tail ? (K + 63) / 64 * 64 : K, c, ldc) || ldc < N) return kErrShape;
+  if (two && (K2 <= 0 || K2 > 0x7FFFFFFF || (!tail && K2 % 64))) return kErrShape;
+  if (!operand_ok(a, lda, a_kmajor, M, K) || !operand_ok(b, ldb, b_kmajor, N, K) ||
+      (two && (!operand_ok(a2, lda2, a_kmajor, M, K2) || !operand_ok(b2, ldb2, b_kmajor, N, K2))))
+    return kErrAlign;
+  if (two && (lda2 != lda || ldb2 != ldb)) return kErrShape;
+  const int64_t Kmax = two && K2 > K ? K2 : K;
+  if (!operand_fits(lda, a_kmajor, M, Kmax) || !operand_fits(ldb, b_kmajor, N, Kmax))
+    return kErrTooLarge;
+  KArgs A{};
+  A.a[0] = {(const uint16_t*)a, lda};
+  A.b[0] = {(const uint16_t*)b, ldb};
+  A.K[0] = K;
+  A.npairs = 1;
+  if (two) {
+    A.a[1] = {(const uint16_t*)a2, lda2};
+    A.b[1] = {(const uint16_t*)b2, ldb2};
+    A.K[1] = K2;
+    A.npairs = 2;
+  }
+  A.M = M; A.N = N;
+  A.C = (uint16_t*)c;
+  A.ldc = ldc;
+  int terms = 0;
+  if (const int rc = set_lora(A, L, M, N, terms)) return rc;
+  if (terms && !a_kmajor) return kErrShape;
+  hipStream_t st = (hipStream_t)stream;
+  if (set_split(A, splits, ws)) {
+    if (!ws || !al16(ws)) return kErrAlign;
+    A.ldc = N;
+    int rc;
+    if (a_kmajor && b_kmajor) rc = launch_small<DT, true, true, EPI_F32, CACHE_NONE, 0>(A, st);
+    else if (a_kmajor) rc = launch_small<DT, true, false, EPI_F32, CACHE_NONE, 0>(A, st);
+    else if (b_kmajor) rc = launch_small<DT, false, true, EPI_F32, CACHE_NONE, 0>(A, st);
+    else rc = launch_small<DT, false, false, EPI_F32, CACHE_NONE, 0>(A, st);
+    return rc ? rc : st16_reduce(DT, false, A, terms, ldc, st);
+  }
+  if (terms == 1)
+    return b_kmajor ? launch_small<DT, true, true, EPI_STORE, 0, 1>(A, st)
+                    : launch_small<DT, true, false, EPI_STORE, 0, 1>(A, st);
+  if (terms == 2)
+    return b_kmajor ? launch_small<DT, true, true, EPI_STORE, 0, 2>(A, st)
+                    : launch_small<DT, true, false, EPI_STORE, 0, 2>(A, st);
+  if (a_kmajor && b_kmajor) return launch_small<DT, true, true, EPI_STORE, 0, 0>(A, st);
+  if (a_kmajor) return launch_small<DT, true, false, EPI_STORE, 0, 0>(A, st);
+  if (b_kmajor) return launch_small<DT, false, true, EPI_STORE, 0, 0>(A, st);
+  return launch_small<DT, false, false, EPI_STORE, 0, 0>(A, st);
 }
 
 // F1 on the 16x16x32 loop: d_model a multiple of 64 (d_ff is one of 8 and
@@ -458,6 +537,49 @@ int ffn_gate_up_impl(const void* x, const void* w_gate, const void* w_up, int64_
       return terms ? dispatch_gs<EPI_GLU, CACHE_INT8, 2>(group_size, A, st)
                    : dispatch_gs<EPI_GLU, CACHE_INT8, 0>(group_size, A, st);
   }
+}
+
+// F1 without codec on 128 x 128 tiles: fp16, or split k (partials [splits][n][2 D])
+template <int DT>
+int ffn_gate_up16_impl(const void* x, const void* w_gate, const void* w_up, int64_t n_tok,
+                       int64_t hidden, int64_t inter, void* h_mid, void* h_gate, void* h_up,
+                       const LoraTerms& L, int splits, void* ws, void* stream) {
+  if (n_tok < 0 || hidden < 0 || inter < 0 || splits < 1) return kErrShape;
+  if (!h_gate != !h_up || (!h_mid && !h_gate)) return kErrShape;
+  if (n_tok == 0 || inter == 0) return kOk;
+  if (!ffn_nt16_fits(n_tok, inter, hidden)) return kErrShape;
+  if (!operand_ok(x, hidden, true, n_tok, hidden) ||
+      !operand_ok(w_gate, hidden, true, inter, hidden) ||
+      !operand_ok(w_up, hidden, true, inter, hidden) || (h_mid && !al16(h_mid)) ||
+      (h_gate && (!al16(h_gate) || !al16(h_up))))
+    return kErrAlign;
+  if (!operand_fits(hidden, true, n_tok, hidden)) return kErrTooLarge;
+  KArgs A{};
+  A.a[0] = {(const uint16_t*)x, hidden};
+  A.b[0] = {(const uint16_t*)w_gate, hidden};
+  A.b_up = (const uint16_t*)w_up;
+  A.K[0] = hidden;
+  A.npairs = 1;
+  A.M = n_tok;
+  A.N = 2 * inter;
+  A.D = inter;
+  A.h_mid = (uint16_t*)h_mid;
+  A.h_gate = (uint16_t*)h_gate;
+  A.h_up = (uint16_t*)h_up;
+  int terms = 0;
+  if (const int rc = set_lora(A, L, n_tok, inter, terms)) return rc;
+  hipStream_t st = (hipStream_t)stream;
+  if (set_split(A, splits, ws)) {
+    if (!ws || !al16(ws)) return kErrAlign;
+    A.ldc = 2 * inter;
+    const int rc = launch_small<DT, true, true, EPI_F32, CACHE_BF16, 0>(A, st);
+    return rc ? rc : st16_reduce(DT, true, A, terms, 0, st);
+  }
+  if (h_gate)
+    return terms ? launch_small<DT, true, true, EPI_GLU, CACHE_BF16, 2>(A, st)
+                 : launch_small<DT, true, true, EPI_GLU, CACHE_BF16, 0>(A, st);
+  return terms ? launch_small<DT, true, true, EPI_GLU, CACHE_NONE, 2>(A, st)
+               : launch_small<DT, true, true, EPI_GLU, CACHE_NONE, 0>(A, st);
 }
 
 int ffn_down_dgrad_impl(const void* grad_y, const void* w_down, int64_t n_tok, int64_t hidden,
@@ -646,6 +768,45 @@ int cpt_gemm_bf16_lora(const void* a, int64_t lda, int a_kmajor, const void* b, 
                         K, L, stream);
 }
 
+
+int cpt_gemm16(int dtype, const void* a, int64_t lda, int a_kmajor, const void* b, int64_t ldb,
+               int b_kmajor, const void* a2, int64_t lda2, const void* b2, int64_t ldb2,
+               int64_t K2, void* c, int64_t ldc, int64_t M, int64_t N, int64_t K, int64_t rank,
+               int64_t ldp, int q_kmajor, int64_t ldq, const void* p0, const void* q0,
+               float alpha0, const void* p1, const void* q1, float alpha1, int splits,
+               void* workspace, void* stream) {
+  if (rank < 0) return kErrShape;
+  LoraTerms L;
+  L.rank = (int)rank; L.ldp = ldp; L.q_kmajor = q_kmajor ? 1 : 0; L.ldq = ldq;
+  L.p[0] = p0; L.q[0] = q0; L.alpha[0] = alpha0;
+  L.p[1] = p1; L.q[1] = q1; L.alpha[1] = alpha1;
+  if (dtype == kF16)
+    return gemm16_impl<kF16>(a, lda, a_kmajor, b, ldb, b_kmajor, a2, lda2, b2, ldb2, K2, c, ldc, M,
+                             N, K, L, splits, workspace, stream);
+  if (dtype == kBF16)
+    return gemm16_impl<kBF16>(a, lda, a_kmajor, b, ldb, b_kmajor, a2, lda2, b2, ldb2, K2, c, ldc,
+                              M, N, K, L, splits, workspace, stream);
+  return kErrDType;
+}
+
+int cpt_ffn_gate_up16(int dtype, const void* x, const void* w_gate, const void* w_up,
+                      int64_t n_tok, int64_t hidden, int64_t inter, void* h_mid, void* h_gate,
+                      void* h_up, int64_t rank, int64_t ldp, const void* p_gate,
+                      const void* b_gate, float alpha_gate, const void* p_up, const void* b_up,
+                      float alpha_up, int splits, void* workspace, void* stream) {
+  if (rank < 0) return kErrShape;
+  LoraTerms L;
+  L.rank = (int)rank; L.ldp = ldp; L.q_kmajor = 1;
+  L.p[0] = p_gate; L.q[0] = b_gate; L.alpha[0] = alpha_gate;
+  L.p[1] = p_up; L.q[1] = b_up; L.alpha[1] = alpha_up;
+  if (dtype == kF16)
+    return ffn_gate_up16_impl<kF16>(x, w_gate, w_up, n_tok, hidden, inter, h_mid, h_gate, h_up, L,
+                                    splits, workspace, stream);
+  if (dtype == kBF16)
+    return ffn_gate_up16_impl<kBF16>(x, w_gate, w_up, n_tok, hidden, inter, h_mid, h_gate, h_up,
+                                     L, splits, workspace, stream);
+  return kErrDType;
+}
 
 int cpt_gemm_bf16_ex(const void* a, int64_t lda, int a_kmajor, const void* b, int64_t ldb,
                      int b_kmajor, void* c, int64_t ldc, int64_t M, int64_t N, int64_t K,

@@ -27,6 +27,14 @@
 // the second block's MFMAs cover the first one's barrier, prologue and epilogue
 // (2048 x 4096, k 11008: 161.5 us against 202.7).
 
+//
+// Element types: bf16 and fp16 operands (v_mfma_f32_16x16x32_bf16 / _f16, the
+// same rates), fp32 accumulation.  A split product (EPI_F32, A.ksplit > 1)
+// writes fp32 partials of a k range; st16_reduce sums them in split order and
+// runs the epilogue.  An operand pair that is MN-major on both sides (the
+// weight gradients, k = tokens) may end in a partial k-tile: its buffers then
+// start at that tile, so the rows past K read zero.
+
 #pragma once
 
 #include "gemm16_kernel.h"
@@ -82,6 +90,41 @@ __device__ __forceinline__ void tile_of(int b, int nb, int tiles_m, int tiles_n,
   tn = in / rows;
 }
 
+// Rounding to, packing and widening the 16-bit element types
+template <int DT> __device__ __forceinline__ uint32_t pack16(float a, float b) {
+  if constexpr (DT == kBF16) return pack_bf16x2(a, b);
+  else return (uint32_t)f32_to_f16_bits(a) | ((uint32_t)f32_to_f16_bits(b) << 16);
+}
+template <int DT> __device__ __forceinline__ float wide16(uint32_t w, int hi) {
+  if constexpr (DT == kBF16) return __uint_as_float(hi ? w & 0xFFFF0000u : w << 16);
+  else return f16_bits_to_f32((uint16_t)(hi ? w >> 16 : w & 0xFFFFu));
+}
+template <int DT> __device__ __forceinline__ float round16(float x) {
+  if constexpr (DT == kBF16) return round_bf16(x);
+  else return (float)(_Float16)x;
+}
+template <int DT> __device__ __forceinline__ uint4 pack8(const float (&v)[8]) {
+  return make_uint4(pack16<DT>(v[0], v[1]), pack16<DT>(v[2], v[3]), pack16<DT>(v[4], v[5]),
+                    pack16<DT>(v[6], v[7]));
+}
+template <int DT> __device__ __forceinline__ void wide8(const uint4& w, float (&v)[8]) {
+  const uint32_t a[4] = {w.x, w.y, w.z, w.w};
+#pragma unroll
+  for (int e = 0; e < 8; ++e) v[e] = wide16<DT>(a[e >> 1], e & 1);
+}
+
+template <int DT> __device__ __forceinline__ void mfma32(f32x4& c, const bf16x8& a, const bf16x8& b) {
+  if constexpr (DT == kBF16) nt16::mfma(c, a, b);
+  else asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
+}
+typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
+template <int DT>
+__device__ __forceinline__ f32x4 mfma16(const s16x4& a, const s16x4& b, const f32x4& c) {
+  if constexpr (DT == kBF16) return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, c, 0, 0, 0);
+  else return __builtin_amdgcn_mfma_f32_16x16x16f16(__builtin_bit_cast(f16x4, a),
+                                                    __builtin_bit_cast(f16x4, b), c, 0, 0, 0);
+}
+
 struct Lora {
   s16x4 p[2][4], q[2][4], ph[2][4], qh[2][4];
 };
@@ -121,32 +164,34 @@ __device__ __forceinline__ void lora_load(const KArgs& A, int64_t m0, int64_t n0
   }
 }
 
-template <bool DUAL, int LT>
+template <int DT, bool DUAL, int LT>
 __device__ __forceinline__ f32x4 acc_lora(const KArgs& A, const f32x4& a, const Lora& F, int i,
                                           int j) {
   f32x4 v = a;
 #pragma unroll
   for (int t = 0; t < LT; ++t) {
     if (DUAL && (i >> 1) != t) continue;
-    f32x4 l = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(F.q[t][i], F.p[t][j],
-                                                       f32x4{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
-    if (A.lrank > 16)
-      l = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(F.qh[t][i], F.ph[t][j], l, 0, 0, 0);
+    f32x4 l = mfma16<DT>(F.q[t][i], F.p[t][j], f32x4{0.0f, 0.0f, 0.0f, 0.0f});
+    if (A.lrank > 16) l = mfma16<DT>(F.qh[t][i], F.ph[t][j], l);
 #pragma unroll
     for (int r = 0; r < 4; ++r)
-      v[r] = round_bf16(round_bf16(v[r]) + round_bf16(A.lalpha[t] * round_bf16(l[r])));
+      v[r] = round16<DT>(round16<DT>(v[r]) + round16<DT>(A.lalpha[t] * round16<DT>(l[r])));
   }
   return v;
 }
 
-template <bool AK, bool BK, int EPI, int CACHE, int LT, int S>
+template <int DT, bool AK, bool BK, int EPI, int CACHE, int LT, int S>
 __global__ __launch_bounds__(kThreads, S == 2 ? 2 : 1) void st16_kernel(const KArgs A) {
   static_assert(LT == 0 || AK, "adapter terms ride with a K-major A (P's rows are tokens)");
-  constexpr bool DUAL = EPI == EPI_GLU;
+  // EPI_F32 with CACHE_NONE / CACHE_BF16: partials of a plain / dual product
+  constexpr bool DUAL = EPI == EPI_GLU || (EPI == EPI_F32 && CACHE == CACHE_BF16);
+  constexpr bool TAIL = !AK && !BK;
   static_assert(!DUAL || (AK && BK), "F1's operands are K-major");
   extern __shared__ __attribute__((aligned(16))) uint16_t lds[];
+  const int tiles = A.tiles_m * A.tiles_n;
+  const int split = EPI == EPI_F32 ? blockIdx.x / tiles : 0;
   int tm, tn;
-  tile_of(blockIdx.x, gridDim.x, A.tiles_m, A.tiles_n, tm, tn);
+  tile_of(blockIdx.x - split * tiles, tiles, A.tiles_m, A.tiles_n, tm, tn);
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -180,34 +225,46 @@ __global__ __launch_bounds__(kThreads, S == 2 ? 2 : 1) void st16_kernel(const KA
   }
   const uint32_t stepa = AK ? (uint32_t)(kBK * 2) : (uint32_t)(kBK * lda * 2);
   const uint32_t stepb = BK ? (uint32_t)(kBK * 2) : (uint32_t)(kBK * ldb * 2);
-  // the k-tile being loaded: its pair's buffers, byte deltas, k-tiles left
+  auto ktiles = [&](int pr) { return (int)((A.K[pr] + kBK - 1) / kBK); };
+  const int nk_all = ktiles(0) + (A.npairs == 2 ? ktiles(1) : 0);
+  const int kb = EPI == EPI_F32 ? min(nk_all, split * A.kt_per_split) : 0;
+  const int nk = EPI == EPI_F32 ? min(nk_all - kb, A.kt_per_split) : nk_all;
+  // the k-tile being loaded: its pair's buffers and byte deltas, the k-tiles
+  // left in the pair and in the block's range
   i32x4 ra, rb, rbu;
   uint32_t da, db;
-  int left, pair = 0;
-  auto open = [&](int pr) {
+  int left, rem = nk, pair = 0;
+  auto open = [&](int pr, int lk) {
+    // a partial last k-tile: the buffers start at its first row (TAIL)
+    const int64_t k0 = TAIL && ((int64_t)lk + 1) * kBK > A.K[pr] ? (int64_t)lk * kBK : 0;
     ra = AK ? rsrc_sgpr(A.a[pr].p + m0 * lda, (A.M - m0) * lda * 2)
-            : rsrc_sgpr(A.a[pr].p + m0, (A.K[pr] * lda - m0) * 2);
+            : rsrc_sgpr(A.a[pr].p + k0 * lda + m0, ((A.K[pr] - k0) * lda - m0) * 2);
     rb = BK ? rsrc_sgpr(A.b[pr].p + nb0 * ldb, (nrows - nb0) * ldb * 2)
-            : rsrc_sgpr(A.b[pr].p + n0, (A.K[pr] * ldb - n0) * 2);
+            : rsrc_sgpr(A.b[pr].p + k0 * ldb + n0, ((A.K[pr] - k0) * ldb - n0) * 2);
     rbu = DUAL ? rsrc_sgpr(A.b_up + nb0 * ldb, (nrows - nb0) * ldb * 2) : rb;
-    da = db = 0;
-    left = (int)(A.K[pr] / kBK);
+    da = TAIL && k0 ? 0 : (uint32_t)lk * stepa;
+    db = TAIL && k0 ? 0 : (uint32_t)lk * stepb;
+    left = ktiles(pr) - lk;
   };
-  open(0);
+  if (kb < ktiles(0) || A.npairs != 2) {
+    open(0, kb);
+  } else {
+    pair = 1;
+    open(1, kb - ktiles(0));
+  }
   auto advance = [&]() {
     da += stepa;
     db += stepb;
-    if (--left == 0) {
-      if (++pair < A.npairs) {
-        open(pair);
-      } else {
-        ra[2] = rb[2] = rbu[2] = 0;
-        da = db = 0;
-        left = 0x7FFFFFFF;
-      }
+    --left;
+    if (--rem <= 0) {
+      ra[2] = rb[2] = rbu[2] = 0;
+      da = db = 0;
+    } else if (left == 0) {
+      open(++pair, 0);
+    } else if (TAIL && left == 1) {
+      open(pair, ktiles(pair) - 1);
     }
   };
-  const int nk = (int)(A.K[0] / kBK) + (A.npairs == 2 ? (int)(A.K[1] / kBK) : 0);
   // load p (0..7): even p -> A block p / 2, odd -> B
   auto issue = [&](int p, int st) {
     const int i = p >> 1;
@@ -268,7 +325,7 @@ __global__ __launch_bounds__(kThreads, S == 2 ? 2 : 1) void st16_kernel(const KA
       constexpr int t = decltype(tc)::value;
       if constexpr (t < 16) {
         constexpr int i = ord.i[t], j = ord.j[t];
-        nt16::mfma(acc[i][j], f0[2 * i], f0[2 * j + 1]);
+        mfma32<DT>(acc[i][j], f0[2 * i], f0[2 * j + 1]);
         if constexpr (t < 8) f1[t] = rd(cur, 1, t);
         if constexpr (t >= 3 && (t - 3) % 4 == 0) issue(4 + (t - 3) / 4, prev);
         if constexpr (t == 15) {
@@ -278,7 +335,7 @@ __global__ __launch_bounds__(kThreads, S == 2 ? 2 : 1) void st16_kernel(const KA
         }
       } else {
         constexpr int i = ord.i[t - 16], j = ord.j[t - 16];
-        nt16::mfma(acc[i][j], f1[2 * i], f1[2 * j + 1]);
+        mfma32<DT>(acc[i][j], f1[2 * i], f1[2 * j + 1]);
         if constexpr (t < 24) f0[t - 16] = rd(next, 0, t - 16);
         if constexpr ((t - 19) % 4 == 0 && t >= 19) issue((t - 19) / 4, cur);
       }
@@ -290,9 +347,27 @@ __global__ __launch_bounds__(kThreads, S == 2 ? 2 : 1) void st16_kernel(const KA
   asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
 
   // lane holds tile column 64 wn + 16 i + 4 (lane / 16) + 0..3 of tile row
-  // 64 wm + 16 j + lane % 16 in acc[i][j]
+  // 64 wm + 16 j + lane % 16 in acc[i][j] (DUAL: i < 2 gate column 32 wn + 16 i
+  // + .., i >= 2 the same up column)
   const int etid = epi_tid();
   const int el = etid & 63;
+  if constexpr (EPI == EPI_F32) {
+    // partials [split][M][ldc] fp32; DUAL: up columns start at column D
+    float* const out = A.ws + (int64_t)split * A.M * A.ldc;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int64_t n = (DUAL ? nb0 + wn * 32 + 16 * (i & 1) : n0 + wn * 64 + 16 * i) + 4 * (el >> 4);
+      if (n >= nrows) continue;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int64_t m = m0 + wm * 64 + 16 * j + (el & 15);
+        f32x4 v = acc[i][j];
+        asm volatile("" : "+v"(v));
+        if (m < A.M) *reinterpret_cast<f32x4*>(out + m * A.ldc + (DUAL && i >= 2 ? A.D : 0) + n) = v;
+      }
+    }
+    return;
+  } else {
   Lora F;
   if constexpr (LT > 0) lora_load<DUAL, LT>(A, m0, n0, wm, wn, el, F);
   if constexpr (!DUAL) {
@@ -302,10 +377,10 @@ __global__ __launch_bounds__(kThreads, S == 2 ? 2 : 1) void st16_kernel(const KA
       for (int j = 0; j < 4; ++j) {
         f32x4 base = acc[i][j];
         asm volatile("" : "+v"(base));
-        const f32x4 v = LT > 0 ? acc_lora<false, LT>(A, base, F, i, j) : base;
+        const f32x4 v = LT > 0 ? acc_lora<DT, false, LT>(A, base, F, i, j) : base;
         *reinterpret_cast<uint2*>(lds + (wm * 64 + 16 * j + (el & 15)) * kLdOut + wn * 64 + 16 * i +
                                   4 * (el >> 4)) =
-            make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
+            make_uint2(pack16<DT>(v[0], v[1]), pack16<DT>(v[2], v[3]));
       }
     __syncthreads();
     const int cl = (etid & 15) * 8;
@@ -319,42 +394,31 @@ __global__ __launch_bounds__(kThreads, S == 2 ? 2 : 1) void st16_kernel(const KA
         if (nok && m0 + r < A.M) *reinterpret_cast<uint4*>(A.C + (m0 + r) * A.ldc + n) = w;
       }
     } else {
-      // B1 on a bf16 cache: SwiGLU backward of the staged grad_h_mid.  Every
+      // B1 on a 16-bit cache: SwiGLU backward of the staged grad_h_mid.  Every
       // load of a pass precedes its stores (the outputs may lie over the cache)
-      static_assert(EPI == EPI_DGLU && CACHE == CACHE_BF16, "B1 on a bf16 cache");
+      static_assert(EPI == EPI_DGLU && CACHE == CACHE_BF16, "B1 on a 16-bit cache");
 #pragma unroll 2
       for (int p = 0; p < 8; ++p) {
         const int r = p * 16 + (etid >> 4);
         if (!nok || m0 + r >= A.M) continue;
         const int64_t off = (m0 + r) * A.D + n;
-        const uint4 dh = *reinterpret_cast<const uint4*>(lds + r * kLdOut + cl);
-        const uint4 cg = *reinterpret_cast<const uint4*>(A.h_gate + off);
-        const uint4 cu = *reinterpret_cast<const uint4*>(A.h_up + off);
-        const uint32_t dw[4] = {dh.x, dh.y, dh.z, dh.w};
-        const uint32_t gw[4] = {cg.x, cg.y, cg.z, cg.w}, uw[4] = {cu.x, cu.y, cu.z, cu.w};
-        float og[8], ou[8], oh[8];
+        float dh[8], hg[8], hu[8], og[8], ou[8], oh[8];
+        wide8<DT>(*reinterpret_cast<const uint4*>(lds + r * kLdOut + cl), dh);
+        wide8<DT>(*reinterpret_cast<const uint4*>(A.h_gate + off), hg);
+        wide8<DT>(*reinterpret_cast<const uint4*>(A.h_up + off), hu);
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
-          auto up = [&](const uint32_t (&w)[4]) {
-            return __uint_as_float(e & 1 ? w[e >> 1] & 0xFFFF0000u : w[e >> 1] << 16);
-          };
-          const float hu = up(uw);
           float hact;
-          swiglu_bwd1(up(dw), up(gw), hu, og[e], ou[e], hact);
-          oh[e] = hact * hu;
+          swiglu_bwd1(dh[e], hg[e], hu[e], og[e], ou[e], hact);
+          oh[e] = hact * hu[e];
         }
-        auto pack8 = [](const float (&v)[8]) {
-          return make_uint4(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]),
-                            pack_bf16x2(v[4], v[5]), pack_bf16x2(v[6], v[7]));
-        };
-        *reinterpret_cast<uint4*>(A.grad_gate + off) = pack8(og);
-        *reinterpret_cast<uint4*>(A.grad_up + off) = pack8(ou);
-        if (A.h_mid_hat) *reinterpret_cast<uint4*>(A.h_mid_hat + off) = pack8(oh);
+        *reinterpret_cast<uint4*>(A.grad_gate + off) = pack8<DT>(og);
+        *reinterpret_cast<uint4*>(A.grad_up + off) = pack8<DT>(ou);
+        if (A.h_mid_hat) *reinterpret_cast<uint4*>(A.h_mid_hat + off) = pack8<DT>(oh);
       }
     }
   } else {
-    // F1 with no codec: blocks i < 2 are gate columns 32 wn + 16 i + .., i >= 2 the
-    // same up columns
+    // F1 with no codec
     uint16_t* sg = lds;
     uint16_t* su = lds + kT * kGluLdS;
 #pragma unroll
@@ -363,10 +427,10 @@ __global__ __launch_bounds__(kThreads, S == 2 ? 2 : 1) void st16_kernel(const KA
       for (int j = 0; j < 4; ++j) {
         f32x4 base = acc[i][j];
         asm volatile("" : "+v"(base));
-        const f32x4 v = LT > 0 ? acc_lora<true, LT>(A, base, F, i, j) : base;
+        const f32x4 v = LT > 0 ? acc_lora<DT, true, LT>(A, base, F, i, j) : base;
         *reinterpret_cast<uint2*>((i < 2 ? sg : su) + (wm * 64 + 16 * j + (el & 15)) * kGluLdS +
                                   wn * 32 + 16 * (i & 1) + 4 * (el >> 4)) =
-            make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
+            make_uint2(pack16<DT>(v[0], v[1]), pack16<DT>(v[2], v[3]));
       }
     __syncthreads();
     const int cl = (etid & 7) * 8;
@@ -379,15 +443,12 @@ __global__ __launch_bounds__(kThreads, S == 2 ? 2 : 1) void st16_kernel(const KA
       const uint4 wu = *reinterpret_cast<const uint4*>(su + r * kGluLdS + cl);
       const int64_t off = (m0 + r) * A.D + d;
       if (A.h_mid) {
-        const uint32_t gw[4] = {wg.x, wg.y, wg.z, wg.w}, uw[4] = {wu.x, wu.y, wu.z, wu.w};
-        float h[8];
+        float g[8], u[8], h[8];
+        wide8<DT>(wg, g);
+        wide8<DT>(wu, u);
 #pragma unroll
-        for (int e = 0; e < 8; ++e)
-          h[e] = silu_mul1(__uint_as_float(e & 1 ? gw[e >> 1] & 0xFFFF0000u : gw[e >> 1] << 16),
-                           __uint_as_float(e & 1 ? uw[e >> 1] & 0xFFFF0000u : uw[e >> 1] << 16));
-        *reinterpret_cast<uint4*>(A.h_mid + off) =
-            make_uint4(pack_bf16x2(h[0], h[1]), pack_bf16x2(h[2], h[3]), pack_bf16x2(h[4], h[5]),
-                       pack_bf16x2(h[6], h[7]));
+        for (int e = 0; e < 8; ++e) h[e] = silu_mul1(g[e], u[e]);
+        *reinterpret_cast<uint4*>(A.h_mid + off) = pack8<DT>(h);
       }
       if constexpr (CACHE == CACHE_BF16) {
         *reinterpret_cast<uint4*>(A.h_gate + off) = wg;
@@ -395,15 +456,16 @@ __global__ __launch_bounds__(kThreads, S == 2 ? 2 : 1) void st16_kernel(const KA
       }
     }
   }
+  }
 }
 
 }  // namespace st16
 
 // The same product as launch_nt16's, on 128 x 128 tiles (A.tiles_m / tiles_n
-// are recounted here).
-template <bool AK, bool BK, int EPI, int CACHE, int LT, int S>
+// are recounted here; A.ksplit blocks per tile for EPI_F32).
+template <int DT, bool AK, bool BK, int EPI, int CACHE, int LT, int S>
 int launch_st16(KArgs A, hipStream_t st) {
-  auto kern = st16::st16_kernel<AK, BK, EPI, CACHE, LT, S>;
+  auto kern = st16::st16_kernel<DT, AK, BK, EPI, CACHE, LT, S>;
   static bool attr_set = false;   // per instantiation
   if (!attr_set) {
     if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -413,10 +475,10 @@ int launch_st16(KArgs A, hipStream_t st) {
   }
   A.tiles_m = (int)((A.M + st16::kT - 1) / st16::kT);
   A.tiles_n = (int)((A.N + st16::kT - 1) / st16::kT);
-  const int64_t tiles = (int64_t)A.tiles_m * A.tiles_n;
-  if (tiles <= 0) return kOk;
-  if (tiles > 0x7FFFFFFF) return kErrTooLarge;
-  hipLaunchKernelGGL(kern, dim3((unsigned)tiles), dim3(st16::kThreads), st16::lds_bytes<S>(), st,
+  const int64_t blocks = (int64_t)A.tiles_m * A.tiles_n * (EPI == EPI_F32 ? A.ksplit : 1);
+  if (blocks <= 0) return kOk;
+  if (blocks > 0x7FFFFFFF) return kErrTooLarge;
+  hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(st16::kThreads), st16::lds_bytes<S>(), st,
                      A);
   return hipGetLastError() == hipSuccess ? kOk : kErrLaunch;
 }

@@ -1,0 +1,146 @@
+// Split products on the 128 x 128 tiles of the 16x16x32 loop
+// (gemm16s_kernel.h): the kernels that write fp32 partials, and the kernel
+// that sums them and runs the epilogue.
+
+#include "gemm16s_kernel.h"
+
+namespace cpt {
+namespace gemm {
+
+CPT_ST16_INST_F32(CPT_ST16_DEFINE, kBF16)
+CPT_ST16_INST_F32(CPT_ST16_DEFINE, kF16)
+
+namespace st16 {
+
+// l[e] = sum_k P_t[m][k] Q_t[k][n + e] in fp32 (the products are exact)
+template <int DT>
+__device__ __forceinline__ void lora8(const KArgs& A, int t, int64_t m, int64_t n, bool vec,
+                                      float (&l)[8]) {
+#pragma unroll
+  for (int e = 0; e < 8; ++e) l[e] = 0.0f;
+  const int r = A.lrank;
+  for (int k0 = 0; k0 < r; k0 += 8) {
+    float p[8];
+    wide8<DT>(*reinterpret_cast<const uint4*>(A.lp[t] + m * A.lldp + k0), p);
+    if (A.lq_km) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        float q[8];
+        wide8<DT>(*reinterpret_cast<const uint4*>(A.lq[t] + (n + e) * r + k0), q);
+#pragma unroll
+        for (int k = 0; k < 8; ++k) l[e] += p[k] * q[k];
+      }
+    } else {
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        const uint16_t* row = A.lq[t] + (k0 + k) * A.lldq + n;
+        float q[8];
+        if (vec) {
+          wide8<DT>(*reinterpret_cast<const uint4*>(row), q);
+        } else {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) q[e] = wide16<DT>(row[e], 0);
+        }
+#pragma unroll
+        for (int e = 0; e < 8; ++e) l[e] += p[k] * q[e];
+      }
+    }
+  }
+}
+
+// One thread per 8 columns of one row.  HBM-bound on the partials (they mostly
+// sit in the last-level cache): the loads of 4 splits are in flight together,
+// added in split order.
+__device__ __forceinline__ void sum8(const float* p, int64_t stride, int splits, float (&v)[8]) {
+#pragma unroll
+  for (int e = 0; e < 8; ++e) v[e] = 0.0f;
+  int s = 0;
+  for (; s + 4 <= splits; s += 4) {
+    f32x4 w[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      w[j] = reinterpret_cast<const f32x4*>(p + (s + (j >> 1)) * stride)[j & 1];
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[4 * (j & 1) + e] += w[j][e];
+  }
+  for (; s < splits; ++s)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const f32x4 w = reinterpret_cast<const f32x4*>(p + s * stride)[j];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[4 * j + e] += w[e];
+    }
+}
+
+template <int DT>
+__device__ __forceinline__ void add_term(const KArgs& A, int t, int64_t m, int64_t n, bool vec,
+                                         float (&v)[8]) {
+  if (!A.lp[t]) return;
+  float l[8];
+  lora8<DT>(A, t, m, n, vec, l);
+#pragma unroll
+  for (int e = 0; e < 8; ++e)
+    v[e] = round16<DT>(round16<DT>(v[e]) + round16<DT>(A.lalpha[t] * round16<DT>(l[e])));
+}
+
+template <int DT, bool DUAL>
+__global__ __launch_bounds__(256) void reduce_kernel(const KArgs A, int terms, int64_t ldo,
+                                                     bool vec) {
+  const int64_t cols = (DUAL ? A.D : A.N) / 8;
+  const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (e >= A.M * cols) return;
+  const int64_t m = e / cols, n = (e - m * cols) * 8;
+  const float* p = A.ws + m * A.ldc + n;
+  const int64_t stride = A.M * A.ldc;
+  float v[8];
+  sum8(p, stride, A.ksplit, v);
+  if constexpr (!DUAL) {
+    for (int t = 0; t < terms; ++t) add_term<DT>(A, t, m, n, vec, v);
+    *reinterpret_cast<uint4*>(A.C + m * ldo + n) = pack8<DT>(v);
+  } else {
+    float u[8], h[8];
+    sum8(p + A.D, stride, A.ksplit, u);
+    if (terms > 0) add_term<DT>(A, 0, m, n, vec, v);
+    if (terms > 1) add_term<DT>(A, 1, m, n, vec, u);
+    const uint4 wg = pack8<DT>(v), wu = pack8<DT>(u);
+    const int64_t off = m * A.D + n;
+    if (A.h_mid) {
+      wide8<DT>(wg, v);
+      wide8<DT>(wu, u);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) h[i] = silu_mul1(v[i], u[i]);
+      *reinterpret_cast<uint4*>(A.h_mid + off) = pack8<DT>(h);
+    }
+    if (A.h_gate) {
+      *reinterpret_cast<uint4*>(A.h_gate + off) = wg;
+      *reinterpret_cast<uint4*>(A.h_up + off) = wu;
+    }
+  }
+}
+
+}  // namespace st16
+
+int st16_reduce(int dt, bool dual, const KArgs& A, int terms, int64_t ldo, hipStream_t st) {
+  const int64_t n = A.M * ((dual ? A.D : A.N) / 8);
+  const int64_t blocks = (n + 255) / 256;
+  if (blocks <= 0) return kOk;
+  if (blocks > 0x7FFFFFFF) return kErrTooLarge;
+  // 16-byte reads of Q's rows when they all start on 16 bytes
+  bool vec = (A.lldq & 7) == 0;
+  for (int t = 0; t < terms; ++t) vec = vec && aligned16(A.lq[t]);
+#define CPT_ST16_RED(DT, DUAL)                                                                   \
+  hipLaunchKernelGGL((st16::reduce_kernel<DT, DUAL>), dim3((unsigned)blocks), dim3(256), 0, st, A, \
+                     terms, ldo, vec)
+  if (dt == kBF16) {
+    if (dual) CPT_ST16_RED(kBF16, true); else CPT_ST16_RED(kBF16, false);
+  } else {
+    if (dual) CPT_ST16_RED(kF16, true); else CPT_ST16_RED(kF16, false);
+  }
+#undef CPT_ST16_RED
+  return hipGetLastError() == hipSuccess ? kOk : kErrLaunch;
+}
+
+}  // namespace gemm
+}  // namespace cpt

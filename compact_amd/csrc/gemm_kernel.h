@@ -1302,9 +1302,14 @@ int64_t stream_k_bytes(int cus);
 int num_cus();   // CUs of the current device (0 if unknown)
 template <bool AK, bool BK, int EPI, int CACHE, int GS, int LT>
 int launch_nt16(const KArgs& A, hipStream_t st);
-// The same products on 128 x 128 tiles (gemm16s_kernel.h), bit-identical
-template <bool AK, bool BK, int EPI, int CACHE, int LT, int S>
+// The same products on 128 x 128 tiles (gemm16s_kernel.h; DT kBF16 or kF16),
+// bit-identical; EPI_F32: fp32 partials of A.ksplit k ranges (dual product with
+// CACHE_BF16), which st16_reduce sums and finishes.
+template <int DT, bool AK, bool BK, int EPI, int CACHE, int LT, int S>
 int launch_st16(KArgs A, hipStream_t st);
+// Split sums, adapter terms (`terms` of A's) and epilogue of a split product:
+// plain store to A.C (rows ldo apart) or, dual, the GLU outputs of F1.
+int st16_reduce(int dt, bool dual, const KArgs& A, int terms, int64_t ldo, hipStream_t st);
 
 // ---------------------------------------------------------------------------
 // Instantiations of launch<AK, BKM, EPI, CACHE, GS, LT>.  Each group is
@@ -1353,16 +1358,25 @@ int launch_st16(KArgs A, hipStream_t st);
   X(false, false, EPI_STORE, 0, 0, 0) X(false, true, EPI_STORE, 0, 0, 0)     \
   X(true, true, EPI_STORE, 0, 0, 1) X(true, false, EPI_STORE, 0, 0, 1)       \
   X(true, true, EPI_STORE, 0, 0, 2) X(true, false, EPI_STORE, 0, 0, 2)
-#define CPT_ST16_INST_STORE(X)                                               \
-  X(true, true, EPI_STORE, 0, 0) X(true, false, EPI_STORE, 0, 0)             \
-  X(false, false, EPI_STORE, 0, 0) X(false, true, EPI_STORE, 0, 0)           \
-  X(true, true, EPI_STORE, 0, 1) X(true, false, EPI_STORE, 0, 1)             \
-  X(true, true, EPI_STORE, 0, 2) X(true, false, EPI_STORE, 0, 2)
-#define CPT_ST16_INST_FFN(X)                                                 \
-  X(true, true, EPI_GLU, CACHE_NONE, 0) X(true, true, EPI_GLU, CACHE_NONE, 2) \
-  X(true, true, EPI_GLU, CACHE_BF16, 0) X(true, true, EPI_GLU, CACHE_BF16, 2) \
-  X(true, false, EPI_DGLU, CACHE_BF16, 0) X(true, false, EPI_DGLU, CACHE_BF16, 1)
-#define CPT_ST16_INST_ALL(X) CPT_ST16_INST_STORE(X) CPT_ST16_INST_FFN(X)
+#define CPT_ST16_INST_STORE(X, DT)                                           \
+  X(DT, true, true, EPI_STORE, 0, 0) X(DT, true, false, EPI_STORE, 0, 0)     \
+  X(DT, false, false, EPI_STORE, 0, 0) X(DT, false, true, EPI_STORE, 0, 0)   \
+  X(DT, true, true, EPI_STORE, 0, 1) X(DT, true, false, EPI_STORE, 0, 1)     \
+  X(DT, true, true, EPI_STORE, 0, 2) X(DT, true, false, EPI_STORE, 0, 2)
+#define CPT_ST16_INST_GLU(X, DT)                                             \
+  X(DT, true, true, EPI_GLU, CACHE_NONE, 0) X(DT, true, true, EPI_GLU, CACHE_NONE, 2) \
+  X(DT, true, true, EPI_GLU, CACHE_BF16, 0) X(DT, true, true, EPI_GLU, CACHE_BF16, 2)
+// partials of split products: every layout, and the dual gate/up product
+#define CPT_ST16_INST_F32(X, DT)                                             \
+  X(DT, true, true, EPI_F32, CACHE_NONE, 0) X(DT, true, false, EPI_F32, CACHE_NONE, 0) \
+  X(DT, false, false, EPI_F32, CACHE_NONE, 0) X(DT, false, true, EPI_F32, CACHE_NONE, 0) \
+  X(DT, true, true, EPI_F32, CACHE_BF16, 0)
+#define CPT_ST16_INST_DGLU(X)                                                \
+  X(kBF16, true, false, EPI_DGLU, CACHE_BF16, 0) X(kBF16, true, false, EPI_DGLU, CACHE_BF16, 1)
+#define CPT_ST16_INST_ALL(X)                                                 \
+  CPT_ST16_INST_STORE(X, kBF16) CPT_ST16_INST_STORE(X, kF16) CPT_ST16_INST_GLU(X, kBF16) \
+  CPT_ST16_INST_GLU(X, kF16) CPT_ST16_INST_F32(X, kBF16) CPT_ST16_INST_F32(X, kF16) \
+  CPT_ST16_INST_DGLU(X)
 #define CPT_NT16_INST_GLU_A(X)                                               \
   X(true, true, EPI_GLU, CACHE_NONE, 64, 0) X(true, true, EPI_GLU, CACHE_NONE, 64, 2) \
   X(true, true, EPI_GLU, CACHE_BF16, 64, 0) X(true, true, EPI_GLU, CACHE_BF16, 64, 2)
@@ -1397,12 +1411,12 @@ int launch_st16(KArgs A, hipStream_t st);
   template int launch_nt16<AK, BK, EPI, CACHE, GS, LT>(const KArgs&, hipStream_t);
 #define CPT_NT16_DECLARE(AK, BK, EPI, CACHE, GS, LT) \
   extern template int launch_nt16<AK, BK, EPI, CACHE, GS, LT>(const KArgs&, hipStream_t);
-#define CPT_ST16_DEFINE(AK, BK, EPI, CACHE, LT) \
-  template int launch_st16<AK, BK, EPI, CACHE, LT, 2>(KArgs, hipStream_t); \
-  template int launch_st16<AK, BK, EPI, CACHE, LT, 4>(KArgs, hipStream_t);
-#define CPT_ST16_DECLARE(AK, BK, EPI, CACHE, LT) \
-  extern template int launch_st16<AK, BK, EPI, CACHE, LT, 2>(KArgs, hipStream_t); \
-  extern template int launch_st16<AK, BK, EPI, CACHE, LT, 4>(KArgs, hipStream_t);
+#define CPT_ST16_DEFINE(DT, AK, BK, EPI, CACHE, LT) \
+  template int launch_st16<DT, AK, BK, EPI, CACHE, LT, 2>(KArgs, hipStream_t); \
+  template int launch_st16<DT, AK, BK, EPI, CACHE, LT, 4>(KArgs, hipStream_t);
+#define CPT_ST16_DECLARE(DT, AK, BK, EPI, CACHE, LT) \
+  extern template int launch_st16<DT, AK, BK, EPI, CACHE, LT, 2>(KArgs, hipStream_t); \
+  extern template int launch_st16<DT, AK, BK, EPI, CACHE, LT, 4>(KArgs, hipStream_t);
 #define CPT_GEMM_DEFINE(AK, BKM, EPI, CACHE, GS, LT) \
   template int launch<AK, BKM, EPI, CACHE, GS, LT>(KArgs&, hipStream_t);
 #define CPT_GEMM_DECLARE(AK, BKM, EPI, CACHE, GS, LT) \

@@ -87,6 +87,7 @@ def _check_bf16(*ts):
 
 
 LORA_MAX_RANK = 32
+_NO_TERMS = [(None, None, 0.0)] * 2
 
 
 def lora_fusable(rank: int, *dims) -> bool:
@@ -392,20 +393,46 @@ def small_tiles(m: int, n: int) -> bool:
     return ((m + 127) // 128) * ((n + 127) // 128) <= 512
 
 
+# Split products (cpt_gemm16): k-tiles per range at least, and k-tiles taken off
+# each block at least.  A lone block takes 0.4 us per k-tile; the first tiles'
+# latency is worth about 5, the partials and the second kernel about 20.
+# Measured on MI355X, us unsplit / split (both with their launches):
+#   512 x 2048, k 5632   (64 tiles, 4 ranges)   39.6 / 24.0
+#   512 x 2048, k 11264  (64, 4)                81.3 / 35.8
+#   512 x 4096, k 11008  (128, 2)               73.5 / 53.3
+#   4 x 2048, k 5632     (16, 14)               40.4 / 18.1
+#   1024 x 4096, k 11008 (256, 2 ranges)        83.8 / 100.5   not split
+#   4 x 11264, k 2048    (88, 2 ranges)         25.9 / 27.1    not split
+SPLIT_MIN_KT = 6
+SPLIT_MIN_SAVED = 20
+
+
+def split_plan(m: int, n: int, nk: int) -> int:
+    """k ranges of a product of nk k-tiles on 128 x 128 tiles: where the tiles
+    leave half the CUs (of 256) idle, as many as fill them, 1 where the k-tiles
+    they take off each block do not pay for the partials."""
+    small = ((m + 127) // 128) * ((n + 127) // 128)
+    if small == 0 or small > 128:
+        return 1
+    splits = min(256 // small, nk // SPLIT_MIN_KT)
+    return splits if splits > 1 and nk - nk // splits >= SPLIT_MIN_SAVED else 1
+
+
 def mm(a: torch.Tensor, b: torch.Tensor, name: str = "gemm") -> torch.Tensor:
     """a [M, K] @ b [K, N] -> bf16 [M, N] on the MFMA GEMM loops (16x16x32 when
     K is a multiple of 64 and N of 8, else the 32x32x16 engine).  Tall products
     with N <= 32 (the adapter terms' x A^T, grad_y B, ...) go to the skinny
-    kernel; other products with too few 256x256 output tiles to fill the chip
-    (N or M = rank) split K across blocks instead, as do products whose
-    transposed operands are too long for one block's 32-bit offsets."""
+    kernel; products with too few output tiles to fill the chip split K across
+    blocks instead (split_plan on the 16x16x32 loop, mm_splitk on the engine),
+    as do products whose transposed operands are too long for one block's
+    32-bit offsets."""
     M, K = a.shape
     N = b.shape[1]
     if (N <= SKINNY_MAX_RANK and K >= 256 and K % 8 == 0 and M >= 256
             and a.stride(1) == 1):
         return skinny(a, b.t(), 1.0, name)
     tiles = ((M + 255) // 256) * ((N + 255) // 256)
-    if tiles < 128 and K >= 1024:
+    if tiles < 128 and K >= 1024 and (K % 64 or N % 8):
         return mm_splitk(a, b, 1.0, name=name)
     a, lda, ak = _layout_a(a)
     b, ldb, bk = _layout_b(b)
@@ -491,7 +518,7 @@ def mm2(a, b, a2=None, b2=None, name: str = "gemm", lora=None) -> torch.Tensor:
         p_a2, p_b2 = a2.data_ptr(), b2.data_ptr()
     ldc = (N + 7) // 8 * 8
     c = torch.empty((M, ldc), dtype=torch.bfloat16, device=a.device)
-    _stream_k(a.device)
+    r, ldp, qk, ldq, t = 0, 0, 1, 0, _NO_TERMS
     if lora:
         if ak != 1:
             a = a.contiguous()
@@ -499,14 +526,25 @@ def mm2(a, b, a2=None, b2=None, name: str = "gemm", lora=None) -> torch.Tensor:
             assert a2 is None, "adapter terms with a K-concatenated MN-major A"
         dims = ((K, N),) if a2 is None else ((K, N), (K2, N))
         r, ldp, qk, ldq, t, keep = _lora_args(lora, N, dims)
+    splits = (1 if K % 64 or K2 % 64 or N % 8 or not K
+              else split_plan(M, N, (K + K2) // 64))
+    if splits > 1:
+        ws = torch.empty((splits * M * N,), dtype=torch.float32, device=a.device)
         with _timed(name):
+            rc = _lib.lib().cpt_gemm16(
+                _lib.BF16, a.data_ptr(), lda, ak, b.data_ptr(), ldb, bk, p_a2, lda2, p_b2, ldb2,
+                K2, c.data_ptr(), ldc, M, N, K, r, ldp, qk, ldq, t[0][0], t[0][1], t[0][2],
+                t[1][0], t[1][1], t[1][2], splits, ws.data_ptr(), _stream(a))
+        check(rc, name)
+        return c
+    _stream_k(a.device)
+    with _timed(name):
+        if lora:
             rc = _lib.lib().cpt_gemm_bf16_lora(
                 a.data_ptr(), lda, ak, b.data_ptr(), ldb, bk, p_a2, lda2, p_b2, ldb2, K2,
                 c.data_ptr(), ldc, M, N, K, r, ldp, qk, ldq, t[0][0], t[0][1], t[0][2],
                 t[1][0], t[1][1], t[1][2], _stream(a))
-        del keep
-    else:
-        with _timed(name):
+        else:
             rc = _lib.lib().cpt_gemm_bf16(a.data_ptr(), lda, ak, b.data_ptr(), ldb, bk, p_a2,
                                           lda2, p_b2, ldb2, K2, c.data_ptr(), ldc, M, N, K,
                                           _stream(a))
@@ -579,6 +617,7 @@ def ffn_gate_up(x, w_gate, w_up, cache: int, group_size: int, want_h_mid: bool =
     def p(t):
         return None if t is None else t.data_ptr()
 
+    r, ldp, t = 0, 0, _NO_TERMS
     if lora_gate is not None or lora_up is not None:
         # term 0 on the gate columns, term 1 on the up columns (absent: no-op)
         present = [t for t in (lora_gate, lora_up) if t is not None]
@@ -587,14 +626,22 @@ def ffn_gate_up(x, w_gate, w_up, cache: int, group_size: int, want_h_mid: bool =
         assert qk == 1, "the gate/up adapter B factors go K-major"
         if lora_gate is None:
             t = [(None, None, 0.0), t[0]]
-        with _timed("ffn_gate_up"):
+    splits = (split_plan(n, 2 * d, hdim // 64)
+              if cache in (_lib.CACHE_NONE, _lib.CACHE_BF16) and hdim % 64 == 0 and d % 8 == 0
+              else 1)
+    with _timed("ffn_gate_up"):
+        if splits > 1:
+            ws = torch.empty((splits * n * 2 * d,), dtype=torch.float32, device=dev)
+            rc = _lib.lib().cpt_ffn_gate_up16(
+                _lib.BF16, x.data_ptr(), w_gate.data_ptr(), w_up.data_ptr(), n, hdim, d,
+                p(h_mid), p(hg), p(hu), r, ldp, t[0][0], t[0][1], t[0][2], t[1][0], t[1][1],
+                t[1][2], splits, ws.data_ptr(), _stream(x))
+        elif r:
             rc = _lib.lib().cpt_ffn_gate_up_lora(
                 x.data_ptr(), w_gate.data_ptr(), w_up.data_ptr(), n, hdim, d, cache, group_size,
                 p(h_mid), p(hg), p(hu), p(qg), p(sg), p(qu), p(su), r, ldp, t[0][0], t[0][1],
                 t[0][2], t[1][0], t[1][1], t[1][2], _stream(x))
-        del keep
-    else:
-        with _timed("ffn_gate_up"):
+        else:
             rc = _lib.lib().cpt_ffn_gate_up(x.data_ptr(), w_gate.data_ptr(), w_up.data_ptr(), n,
                                             hdim, d, cache, group_size, p(h_mid), p(hg), p(hu),
                                             p(qg), p(sg), p(qu), p(su), _stream(x))

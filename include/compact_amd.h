@@ -308,6 +308,30 @@ int cpt_gemm_bf16_lora(const void* a, int64_t lda, int a_kmajor, const void* b, 
                        const void* q0, float alpha0, const void* p1, const void* q1,
                        float alpha1, void* stream);
 
+/* cpt_gemm_bf16_lora's product (rank 0: cpt_gemm_bf16's) on 128 x 128 tiles for
+ * bf16 or fp16 operands and results (dtype CPT_BF16 / CPT_F16 codes 2 / 1), K
+ * a multiple of 64 (two MN-major operands: any K), N of 8.  splits > 1 shares
+ * the k-tiles of 64 over that many blocks per tile: fp32 partials go to
+ * workspace (splits * M * N floats, 16-byte aligned), summed in k order by a
+ * second kernel that also applies the adapter terms.  With splits = 1 a bf16
+ * product is bit-identical to cpt_gemm_bf16_lora's on the 16x16x32 loop. */
+int cpt_gemm16(int dtype, const void* a, int64_t lda, int a_kmajor, const void* b, int64_t ldb,
+               int b_kmajor, const void* a2, int64_t lda2, const void* b2, int64_t ldb2,
+               int64_t K2, void* c, int64_t ldc, int64_t M, int64_t N, int64_t K, int64_t rank,
+               int64_t ldp, int q_kmajor, int64_t ldq, const void* p0, const void* q0,
+               float alpha0, const void* p1, const void* q1, float alpha1, int splits,
+               void* workspace, void* stream);
+
+/* cpt_ffn_gate_up_lora without a codec (h_gate and h_up both given or both
+ * NULL, h_mid NULL or given; rank 0: no adapter terms) for bf16 or fp16, hidden
+ * a multiple of 64.  splits as in cpt_gemm16, with splits * n_tok * 2 * inter
+ * floats of workspace. */
+int cpt_ffn_gate_up16(int dtype, const void* x, const void* w_gate, const void* w_up,
+                      int64_t n_tok, int64_t hidden, int64_t inter, void* h_mid, void* h_gate,
+                      void* h_up, int64_t rank, int64_t ldp, const void* p_gate,
+                      const void* b_gate, float alpha_gate, const void* p_up, const void* b_up,
+                      float alpha_up, int splits, void* workspace, void* stream);
+
 /* Cache kinds of the fused FFN kernels. */
 enum { CPT_CACHE_NONE = 0, CPT_CACHE_BF16 = 1, CPT_CACHE_INT4 = 4, CPT_CACHE_INT8 = 8 };
 
