@@ -9,7 +9,7 @@
 // 256 x 256 MFMA tile would waste 15/16 of its work and, with only M/256
 // tiles, leave most CUs idle.  Here each wavefront owns 32 rows and one K
 // range, loads A in whole 128-byte row lines, and passes them through its own
-// piece of LDS into the A slot of v_mfma_f32_16x16x32_bf16 (8 consecutive k
+// piece of LDS into the A slot of v_mfma_f32_16x16x32_bf16 or _f16 (8 consecutive k
 // of one row per lane), with Q's fragments (a few hundred KB, L2 resident,
 // loaded straight into the operand layout) in the B slot.  The last k of a
 // range that do not fill a 64-wide step load straight into the A slot.  K is split across blocks so the grid has enough
@@ -67,6 +67,24 @@ __device__ __forceinline__ void wave_lds_order() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// The element types' MFMA, and their output rounding: bf16 rounds alpha * sum
+// once; fp16 rounds the sum and then alpha times it, as the general-layout
+// kernel does (the two differ where the fp16 sum overflows).
+template <int DT>
+__device__ __forceinline__ f32x4 mfma(const bf16x8& a, const bf16x8& b, const f32x4& c) {
+  if constexpr (DT == kBF16) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+  } else {
+    typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a),
+                                                  __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
+  }
+}
+template <int DT> __device__ __forceinline__ uint16_t scaled(float alpha, float sum) {
+  if constexpr (DT == kBF16) return (uint16_t)f32_to_bf16_bits(alpha * sum);
+  else return f32_to_f16_bits(alpha * f16_bits_to_f32(f32_to_f16_bits(sum)));
+}
+
 __device__ __forceinline__ bf16x8 bload(__amdgpu_buffer_rsrc_t r, uint32_t off) {
   auto v = __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0);
   return __builtin_bit_cast(bf16x8, v);
@@ -77,7 +95,7 @@ __device__ __forceinline__ bf16x8 bload(__amdgpu_buffer_rsrc_t r, uint32_t off) 
 // (ceil(M / kRowsPerBlock), splits); split s covers k in
 // [s * kchunk, min(K, (s + 1) * kchunk)), kchunk % 32 == 0.
 // ws != null: fp32 partials ws[(s * M + m) * R + r]; else C = bf16(alpha * acc).
-template <int NB>
+template <int DT, int NB>
 __global__ __launch_bounds__(256) void skinny_proj_kernel(
     const uint16_t* __restrict__ a, int64_t lda, const uint16_t* __restrict__ q, int64_t ldq,
     int64_t M, int R, int64_t K, int64_t kchunk, float* __restrict__ ws, uint16_t* __restrict__ c,
@@ -150,7 +168,7 @@ __global__ __launch_bounds__(256) void skinny_proj_kernel(
             const bf16x8 av = *reinterpret_cast<const bf16x8*>(buf + rofs[b][h]);
 #pragma unroll
             for (int t = 0; t < NB; ++t)
-              acc[b][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, qv[u][h][t], acc[b][t], 0, 0, 0);
+              acc[b][t] = mfma<DT>(av, qv[u][h][t], acc[b][t]);
           }
         wave_lds_order();   // these reads before the buffer's next stores
       }
@@ -170,7 +188,7 @@ __global__ __launch_bounds__(256) void skinny_proj_kernel(
       const bf16x8 av = bload(ra, ok ? oa[b] + dk : kOOB);
 #pragma unroll
       for (int t = 0; t < NB; ++t)
-        acc[b][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, qv[t], acc[b][t], 0, 0, 0);
+        acc[b][t] = mfma<DT>(av, qv[t], acc[b][t]);
     }
   }
 #pragma unroll
@@ -185,7 +203,7 @@ __global__ __launch_bounds__(256) void skinny_proj_kernel(
         if (ws)
           ws[((int64_t)s * M + row) * R + col] = acc[b][t][i];
         else
-          c[row * ldc + col] = (uint16_t)f32_to_bf16_bits(alpha * acc[b][t][i]);
+          c[row * ldc + col] = scaled<DT>(alpha, acc[b][t][i]);
       }
     }
 }
@@ -209,6 +227,7 @@ __device__ __forceinline__ float sum_splits(const float* __restrict__ p, int64_t
 }
 
 // C[m, r] = bf16(alpha * sum_s ws[s][m][r]), splits summed in order
+template <int DT>
 __global__ __launch_bounds__(256) void skinny_reduce_kernel(const float* __restrict__ ws,
                                                             uint16_t* __restrict__ c, int64_t M,
                                                             int R, int64_t ldc, int splits,
@@ -217,7 +236,7 @@ __global__ __launch_bounds__(256) void skinny_reduce_kernel(const float* __restr
   if (e >= M * R) return;
   const float sum = sum_splits(ws + e, M * R, splits);
   const int64_t m = e / R, r = e - m * R;
-  c[m * ldc + r] = (uint16_t)f32_to_bf16_bits(alpha * sum);
+  c[m * ldc + r] = scaled<DT>(alpha, sum);
 }
 
 // ---------------------------------------------------------------------------
@@ -258,7 +277,7 @@ __device__ __forceinline__ bf16x8 red_frag(const uint16_t* piece, int k0, int co
 
 // Grid: (ceil(N / 64), splits); split s covers tokens [s * tchunk,
 // min(T, (s + 1) * tchunk)), tchunk % 64 == 0.  N % 8 == 0, R % 8 == 0.
-template <int NB>
+template <int DT, int NB>
 __global__ __launch_bounds__(256) void skinny_red_kernel(
     const uint16_t* __restrict__ x, int64_t ldx, const uint16_t* __restrict__ p, int64_t ldp,
     int64_t T, int64_t N, int R, int64_t tchunk, float* __restrict__ ws) {
@@ -316,7 +335,7 @@ __global__ __launch_bounds__(256) void skinny_red_kernel(
 #pragma unroll
       for (int t = 0; t < NB; ++t) {
         const bf16x8 b = red_frag<kRedLdP>(ps[buf], kk, t * 16, lane);
-        acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc[t], 0, 0, 0);
+        acc[t] = mfma<DT>(a, b, acc[t]);
       }
     }
     buf ^= 1;
@@ -337,6 +356,7 @@ __global__ __launch_bounds__(256) void skinny_red_kernel(
 
 // out = bf16(alpha * sum_s ws[s][n][r]) at out[n * ldo + r] or, transposed,
 // out[r * ldo + n]; splits summed in order
+template <int DT>
 __global__ __launch_bounds__(256) void skinny_red_reduce_kernel(const float* __restrict__ ws,
                                                                 uint16_t* __restrict__ out,
                                                                 int64_t N, int R, int64_t ldo,
@@ -350,12 +370,13 @@ __global__ __launch_bounds__(256) void skinny_red_reduce_kernel(const float* __r
   const int64_t n = e / R;
   const int64_t r = e % R;
   const float sum = sum_splits(ws + e, N * R, splits);
-  out[trans ? r * ldo + n : n * ldo + r] = (uint16_t)f32_to_bf16_bits(alpha * sum);
+  out[trans ? r * ldo + n : n * ldo + r] = scaled<DT>(alpha, sum);
 }
 
 // Both split sums of a skinny_dual pass in one launch: elements [0, T R) sum
 // the projection's column-block partials into C, the rest the reduction's
 // token-split partials into Z (each as the two kernels above)
+template <int DT>
 __global__ __launch_bounds__(256) void skinny_dual_reduce_kernel(
     const float* __restrict__ ws_c, uint16_t* __restrict__ c, int64_t T, int64_t ldc,
     int csplits, float alpha_c, const float* __restrict__ ws_z, uint16_t* __restrict__ z,
@@ -364,14 +385,14 @@ __global__ __launch_bounds__(256) void skinny_dual_reduce_kernel(
   if (e < T * R) {
     const float sum = sum_splits(ws_c + e, T * R, csplits);
     const int64_t m = e / R, r = e - m * R;
-    c[m * ldc + r] = (uint16_t)f32_to_bf16_bits(alpha_c * sum);
+    c[m * ldc + r] = scaled<DT>(alpha_c, sum);
     return;
   }
   const int64_t ez = e - T * R;
   if (ez >= N * R) return;
   const int64_t n = ez / R, r = ez % R;
   const float sum = sum_splits(ws_z + ez, N * R, splits);
-  z[z_trans ? r * ldz + n : n * ldz + r] = (uint16_t)f32_to_bf16_bits(alpha_z * sum);
+  z[z_trans ? r * ldz + n : n * ldz + r] = scaled<DT>(alpha_z, sum);
 }
 
 // ---------------------------------------------------------------------------
@@ -403,7 +424,7 @@ constexpr int kDualLd = 520;     // LDS row stride of the X piece (elements)
 constexpr int kDualLdP = 40;     // LDS row stride of the P piece (elements)
 constexpr int kDualQLd = 32;     // LDS row stride of the staged B slice (elements, R <= 32)
 
-template <int NB>
+template <int DT, int NB>
 __global__ __launch_bounds__(256) void skinny_dual_kernel(
     const uint16_t* __restrict__ x, int64_t ldx, const uint16_t* __restrict__ q, int64_t ldq,
     const uint16_t* __restrict__ p, int64_t ldp, int64_t T, int64_t N, int R, int64_t tchunk,
@@ -516,7 +537,7 @@ __global__ __launch_bounds__(256) void skinny_dual_kernel(
           &xs[(16 * wave + (lane & 15)) * kDualLd + st * 32 + 8 * (lane >> 4)]);
 #pragma unroll
       for (int t = 0; t < NB; ++t)
-        ac[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, qf[st][t], ac[t], 0, 0, 0);
+        ac[t] = mfma<DT>(a, qf[st][t], ac[t]);
     }
     // reduction: 8 column blocks of 16 over the piece's 64 tokens
 #pragma unroll
@@ -527,7 +548,7 @@ __global__ __launch_bounds__(256) void skinny_dual_kernel(
 #pragma unroll
         for (int t = 0; t < NB; ++t) {
           const bf16x8 bq = red_frag<kDualLdP>(ps, kk, t * 16, lane);
-          az[c][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bq, az[c][t], 0, 0, 0);
+          az[c][t] = mfma<DT>(a, bq, az[c][t]);
         }
       }
     // lane holds C rows 16 w + 4 (lane / 16) + i, rank t * 16 + lane % 16
@@ -589,7 +610,7 @@ inline int scratch_ptr(void** out) {
   return kOk;
 }
 
-int skinny_t_impl(const void* x, int64_t ldx, const void* p, int64_t ldp, void* out,
+int skinny_t_impl(int dtype, const void* x, int64_t ldx, const void* p, int64_t ldp, void* out,
                   int64_t ldo, int out_trans, int64_t T, int64_t N, int64_t R, float alpha,
                   int splits, void* workspace, int64_t workspace_bytes, void* stream);
 
@@ -601,9 +622,10 @@ using namespace cpt::skinny;
 
 extern "C" {
 
-int cpt_gemm_bf16_skinny(const void* a, int64_t lda, const void* q, int64_t ldq, void* c,
-                         int64_t ldc, int64_t M, int64_t R, int64_t K, float alpha, int splits,
-                         void* workspace, void* stream) {
+int cpt_gemm16_skinny(int dtype, const void* a, int64_t lda, const void* q, int64_t ldq, void* c,
+                      int64_t ldc, int64_t M, int64_t R, int64_t K, float alpha, int splits,
+                      void* workspace, void* stream) {
+  if (dtype != kBF16 && dtype != kF16) return kErrDType;
   if (M < 0 || R < 0 || K < 0 || splits < 1) return kErrShape;
   if (R > 32) return kErrShape;
   if (M == 0 || R == 0) return kOk;
@@ -623,31 +645,45 @@ int cpt_gemm_bf16_skinny(const void* a, int64_t lda, const void* q, int64_t ldq,
   hipStream_t st = (hipStream_t)stream;
   float* ws = splits > 1 ? (float*)workspace : nullptr;
   const dim3 grid((unsigned)blocks, (unsigned)splits);
-  if (R <= 16)
-    hipLaunchKernelGGL(skinny_proj_kernel<1>, grid, dim3(256), 0, st, (const uint16_t*)a, lda,
-                       (const uint16_t*)q, ldq, M, (int)R, K, kchunk, ws, (uint16_t*)c, ldc, alpha);
-  else
-    hipLaunchKernelGGL(skinny_proj_kernel<2>, grid, dim3(256), 0, st, (const uint16_t*)a, lda,
-                       (const uint16_t*)q, ldq, M, (int)R, K, kchunk, ws, (uint16_t*)c, ldc, alpha);
+  const auto kern = dtype == kBF16
+                        ? (R <= 16 ? skinny_proj_kernel<kBF16, 1> : skinny_proj_kernel<kBF16, 2>)
+                        : (R <= 16 ? skinny_proj_kernel<kF16, 1> : skinny_proj_kernel<kF16, 2>);
+  hipLaunchKernelGGL(kern, grid, dim3(256), 0, st, (const uint16_t*)a, lda, (const uint16_t*)q,
+                     ldq, M, (int)R, K, kchunk, ws, (uint16_t*)c, ldc, alpha);
   if (hipGetLastError() != hipSuccess) return kErrLaunch;
   if (splits > 1) {
     const int64_t total = M * R;
-    hipLaunchKernelGGL(skinny_reduce_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0,
+    hipLaunchKernelGGL((dtype == kBF16 ? skinny_reduce_kernel<kBF16> : skinny_reduce_kernel<kF16>),
+                       dim3((unsigned)((total + 255) / 256)), dim3(256), 0,
                        st, (const float*)ws, (uint16_t*)c, M, (int)R, ldc, splits, alpha);
     if (hipGetLastError() != hipSuccess) return kErrLaunch;
   }
   return kOk;
 }
 
+int cpt_gemm_bf16_skinny(const void* a, int64_t lda, const void* q, int64_t ldq, void* c,
+                         int64_t ldc, int64_t M, int64_t R, int64_t K, float alpha, int splits,
+                         void* workspace, void* stream) {
+  return cpt_gemm16_skinny(kBF16, a, lda, q, ldq, c, ldc, M, R, K, alpha, splits, workspace,
+                           stream);
+}
+
 }  // extern "C"
 
 extern "C" {
 
+int cpt_gemm16_skinny_t(int dtype, const void* x, int64_t ldx, const void* p, int64_t ldp,
+                        void* out, int64_t ldo, int out_trans, int64_t T, int64_t N, int64_t R,
+                        float alpha, int splits, void* workspace, void* stream) {
+  return skinny_t_impl(dtype, x, ldx, p, ldp, out, ldo, out_trans, T, N, R, alpha, splits,
+                       workspace, -1, stream);
+}
+
 int cpt_gemm_bf16_skinny_t(const void* x, int64_t ldx, const void* p, int64_t ldp, void* out,
                            int64_t ldo, int out_trans, int64_t T, int64_t N, int64_t R,
                            float alpha, int splits, void* workspace, void* stream) {
-  return skinny_t_impl(x, ldx, p, ldp, out, ldo, out_trans, T, N, R, alpha, splits, workspace, -1,
-                       stream);
+  return skinny_t_impl(kBF16, x, ldx, p, ldp, out, ldo, out_trans, T, N, R, alpha, splits,
+                       workspace, -1, stream);
 }
 
 int cpt_gemm_bf16_skinny_t_noalloc(const void* x, int64_t ldx, const void* p, int64_t ldp,
@@ -657,7 +693,7 @@ int cpt_gemm_bf16_skinny_t_noalloc(const void* x, int64_t ldx, const void* p, in
   if (N == 0 || R == 0) return kOk;
   void* ws = nullptr;
   if (const int rc = scratch_ptr(&ws)) return rc;
-  return skinny_t_impl(x, ldx, p, ldp, out, ldo, out_trans, T, N, R, alpha, splits, ws,
+  return skinny_t_impl(kBF16, x, ldx, p, ldp, out, ldo, out_trans, T, N, R, alpha, splits, ws,
                        kScratchBytes, stream);
 }
 
@@ -669,9 +705,10 @@ namespace skinny {
 // workspace_bytes < 0: the caller's workspace holds splits * N * R floats
 // (cpt_gemm_bf16_skinny_t's contract); otherwise the split partials must fit
 // in workspace_bytes.
-int skinny_t_impl(const void* x, int64_t ldx, const void* p, int64_t ldp, void* out,
+int skinny_t_impl(int dtype, const void* x, int64_t ldx, const void* p, int64_t ldp, void* out,
                   int64_t ldo, int out_trans, int64_t T, int64_t N, int64_t R, float alpha,
                   int splits, void* workspace, int64_t workspace_bytes, void* stream) {
+  if (dtype != kBF16 && dtype != kF16) return kErrDType;
   if (T < 0 || N < 0 || R < 0 || splits < 1) return kErrShape;
   if (R > 32) return kErrShape;
   if (N == 0 || R == 0) return kOk;
@@ -692,16 +729,16 @@ int skinny_t_impl(const void* x, int64_t ldx, const void* p, int64_t ldp, void* 
   if (workspace_bytes >= 0 && (int64_t)splits * N * R * 4 > workspace_bytes) return kErrTooLarge;
   hipStream_t st = (hipStream_t)stream;
   const dim3 grid((unsigned)blocks, (unsigned)splits);
-  if (R <= 16)
-    hipLaunchKernelGGL(skinny_red_kernel<1>, grid, dim3(256), 0, st, (const uint16_t*)x, ldx,
-                       (const uint16_t*)p, ldp, T, N, (int)R, tchunk, (float*)workspace);
-  else
-    hipLaunchKernelGGL(skinny_red_kernel<2>, grid, dim3(256), 0, st, (const uint16_t*)x, ldx,
-                       (const uint16_t*)p, ldp, T, N, (int)R, tchunk, (float*)workspace);
+  const auto kern = dtype == kBF16
+                        ? (R <= 16 ? skinny_red_kernel<kBF16, 1> : skinny_red_kernel<kBF16, 2>)
+                        : (R <= 16 ? skinny_red_kernel<kF16, 1> : skinny_red_kernel<kF16, 2>);
+  hipLaunchKernelGGL(kern, grid, dim3(256), 0, st, (const uint16_t*)x, ldx, (const uint16_t*)p,
+                     ldp, T, N, (int)R, tchunk, (float*)workspace);
   if (hipGetLastError() != hipSuccess) return kErrLaunch;
   const int64_t total = N * R;
-  hipLaunchKernelGGL(skinny_red_reduce_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256),
-                     0, st, (const float*)workspace, (uint16_t*)out, N, (int)R, ldo,
+  hipLaunchKernelGGL((dtype == kBF16 ? skinny_red_reduce_kernel<kBF16>
+                                     : skinny_red_reduce_kernel<kF16>),
+                     dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st, (const float*)workspace, (uint16_t*)out, N, (int)R, ldo,
                      out_trans ? 1 : 0, splits, alpha);
   return hipGetLastError() == hipSuccess ? kOk : kErrLaunch;
 }
@@ -721,6 +758,16 @@ int cpt_gemm_bf16_skinny_dual(const void* x, int64_t ldx, const void* q, int64_t
                               const void* p, int64_t ldp, void* c, int64_t ldc, float alpha_c,
                               void* z, int64_t ldz, int z_trans, float alpha_z, int64_t T,
                               int64_t N, int64_t R, int splits, void* workspace, void* stream) {
+  return cpt_gemm16_skinny_dual(kBF16, x, ldx, q, ldq, q_nr, p, ldp, c, ldc, alpha_c, z, ldz,
+                                z_trans, alpha_z, T, N, R, splits, workspace, stream);
+}
+
+int cpt_gemm16_skinny_dual(int dtype, const void* x, int64_t ldx, const void* q, int64_t ldq,
+                           int q_nr, const void* p, int64_t ldp, void* c, int64_t ldc,
+                           float alpha_c, void* z, int64_t ldz, int z_trans, float alpha_z,
+                           int64_t T, int64_t N, int64_t R, int splits, void* workspace,
+                           void* stream) {
+  if (dtype != kBF16 && dtype != kF16) return kErrDType;
   if (T < 0 || N < 0 || R < 0 || splits < 1 || R > 32) return kErrShape;
   if (N == 0 || R == 0) return kOk;
   if (!x || !q || !p || !c || !z || !workspace || !al16(x) || !al16(q) || !al16(p) ||
@@ -748,14 +795,11 @@ int cpt_gemm_bf16_skinny_dual(const void* x, int64_t ldx, const void* q, int64_t
   // (staged through LDS), 2 B as stored otherwise
   const int qmode = !q_nr ? 0 : ((ldq & 7) == 0 && al16(q) ? 1 : 2);
   if (T > 0) {
-    if (R <= 16)
-      hipLaunchKernelGGL(skinny_dual_kernel<1>, grid, dim3(256), 0, st, (const uint16_t*)x, ldx,
-                         (const uint16_t*)q, ldq, (const uint16_t*)p, ldp, T, N, (int)R, tchunk,
-                         ws_c, ws_z, qmode);
-    else
-      hipLaunchKernelGGL(skinny_dual_kernel<2>, grid, dim3(256), 0, st, (const uint16_t*)x, ldx,
-                         (const uint16_t*)q, ldq, (const uint16_t*)p, ldp, T, N, (int)R, tchunk,
-                         ws_c, ws_z, qmode);
+    const auto kern = dtype == kBF16
+                          ? (R <= 16 ? skinny_dual_kernel<kBF16, 1> : skinny_dual_kernel<kBF16, 2>)
+                          : (R <= 16 ? skinny_dual_kernel<kF16, 1> : skinny_dual_kernel<kF16, 2>);
+    hipLaunchKernelGGL(kern, grid, dim3(256), 0, st, (const uint16_t*)x, ldx, (const uint16_t*)q,
+                       ldq, (const uint16_t*)p, ldp, T, N, (int)R, tchunk, ws_c, ws_z, qmode);
     if (hipGetLastError() != hipSuccess) return kErrLaunch;
   } else {
     // no tokens: C has no rows and Z is the empty sum (zero partials summed)
@@ -763,8 +807,9 @@ int cpt_gemm_bf16_skinny_dual(const void* x, int64_t ldx, const void* q, int64_t
   }
   // both split sums in one launch
   const int64_t total = T * R + N * R;
-  hipLaunchKernelGGL(skinny_dual_reduce_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256),
-                     0, st, (const float*)ws_c, (uint16_t*)c, T, ldc, (int)csplits, alpha_c,
+  hipLaunchKernelGGL((dtype == kBF16 ? skinny_dual_reduce_kernel<kBF16>
+                                     : skinny_dual_reduce_kernel<kF16>),
+                     dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st, (const float*)ws_c, (uint16_t*)c, T, ldc, (int)csplits, alpha_c,
                      (const float*)ws_z, (uint16_t*)z, N, ldz, z_trans ? 1 : 0, splits, alpha_z,
                      (int)R);
   return hipGetLastError() == hipSuccess ? kOk : kErrLaunch;

@@ -134,10 +134,25 @@ def _mfma(*ts) -> bool:
     return True
 
 
+def _fits16(a, b) -> bool:
+    """a @ b on the 16-bit MFMA kernels: bf16 of any aligned layout, or fp16
+    that fits the 128 x 128 tiles."""
+    if a.dtype == torch.float16:
+        return G.f16_fits(a, b)
+    return a.shape[0] > 0 and _mfma(a, b)
+
+
+def _fits16_linear(x, *ws) -> bool:
+    """_fits16 of x @ w^T for every w."""
+    if x.dtype == torch.float16:
+        return all(G.f16_fits(x, w.t()) for w in ws)
+    return x.shape[0] > 0 and _mfma(x, *ws)
+
+
 def _mm(a, b, name):
-    """a @ b: the bf16 MFMA GEMMs, or the general-layout kernel for other
+    """a @ b: the 16-bit MFMA GEMMs, or the general-layout kernel for other
     dtypes and layouts."""
-    if _mfma(a, b) and a.shape[0] > 0:
+    if _fits16(a, b):
         return G.mm(a, b, name)
     return G.mm_any(a, b, name=name)
 
@@ -168,15 +183,17 @@ def _addmm(c, a, b, s, name):
 
 def _mm_scaled(a, b, s, name):
     """s * (a @ b) for the thin adapter gradients, which reduce over all
-    tokens: split-K on the bf16 engine, or the general-layout kernel."""
-    if _mfma(a, b) and a.shape[1] > 0:
+    tokens: the token-reduction kernel, split-K on the bf16 engine, or the
+    general-layout kernel."""
+    if (_mfma(a, b) and a.shape[1] > 0) or (a.dtype == b.dtype == torch.float16
+                                            and G.skinny_t_fits(a, b)):
         return G.mm_splitk(a, b, s, name=name)
     return G.mm_any(a, b, s, G.ANY_SCALE, name=name)
 
 
 def _dual_ok(x, b, p) -> bool:
     """The projection x B and the reduction x^T p of one tensor go through
-    G.skinny_dual (one pass over x): bf16 x [T, N] and B [N, r], p [T, r],
+    G.skinny_dual (one pass over x): bf16 or fp16 x [T, N] and B [N, r], p [T, r],
     rank a multiple of 8 up to 32, N a multiple of 8, at least one 512-column
     block of x (thinner tensors keep the separate kernels), when
     _DUAL_SKINNY is on."""
@@ -188,7 +205,7 @@ def _dual_ok(x, b, p) -> bool:
 def _mm_sum(a, b, a2, b2, name):
     """a @ b + a2 @ b2: one K-concatenated accumulation on the bf16 engine, or
     the reference's two rounded products and their rounded sum."""
-    if _mfma(a, b, a2, b2):
+    if _mfma(a, b, a2, b2) or (G.f16_fits(a, b) and G.f16_fits(a2, b2)):
         return G.mm2(a, b, a2, b2, name)
     out = G.mm_any(a, b, name=name)
     return G.mm_any(a2, b2, 1.0, G.ANY_ADD, out=out, name=name)
@@ -196,13 +213,14 @@ def _mm_sum(a, b, a2, b2, name):
 
 def _lora_ok(*pairs, dims) -> bool:
     """The adapter terms (a, b) present ride in the epilogues of the GEMMs
-    with the (k, n) `dims`: bf16 factors of one shared rank up to 16, or up to
-    32 where those GEMMs run on the 16x16x32 loop (G.lora_fusable; the GEMM
+    with the (k, n) `dims`: bf16 or fp16 factors of one shared rank up to 16, or
+    up to 32 where those GEMMs run on the 16x16x32 loop (G.lora_fusable; the GEMM
     wrapper re-lays and zero-pads them for the kernel's 8-wide k chunks)."""
     ranks = {a.shape[0] for a, b in pairs if a is not None}
+    types = {t.dtype for a, b in pairs if a is not None for t in (a, b)}
     return (len(ranks) <= 1 and all(G.lora_fusable(r, *dims) for r in ranks)
-            and all(t.dtype == torch.bfloat16 and t.dim() == 2
-                    for a, b in pairs if a is not None for t in (a, b)))
+            and (not types or types == {torch.bfloat16} or types == {torch.float16})
+            and all(t.dim() == 2 for a, b in pairs if a is not None for t in (a, b)))
 
 
 def outlier_stat_rows(shape) -> int:
@@ -222,8 +240,8 @@ def outlier_stat_rows(shape) -> int:
 def _proj(x_2d, w, a, b, s, name):
     """out = x W^T (+ s * (x A^T) B^T) in PEFT op order (src/flashffn.py:1410-1420).
     Returns (out, xA | None)."""
-    if (a is not None and _mfma(x_2d, w) and _lora_ok((a, b), dims=((w.shape[1], w.shape[0]),))
-            and x_2d.shape[0] > 0):
+    if (a is not None and _fits16_linear(x_2d, w) and x_2d.dtype == a.dtype
+            and _lora_ok((a, b), dims=((w.shape[1], w.shape[0]),))):
         xa = _mm(x_2d, a.t(), name + "_xa")
         return G.linear_lora(x_2d, w, xa, b, s, name), xa
     h = _linear(x_2d, w, name)
@@ -262,6 +280,10 @@ class FlashFFNv3Function(torch.autograd.Function):
     """LoRA-factored SwiGLU FFN with a quantised GLU-cache backward
     (src/flashffn.py:1376-1602).  a_*/b_* may be None (pass s_*=0.0).
 
+    fp16 with 16-byte aligned rows and a d_model and d_ff that are multiples of
+    64 runs the same products on the 128 x 128 MFMA tiles, with the standalone
+    codec and GLU kernels.
+
     bf16 with 16-byte aligned rows runs the fused MFMA kernels: the forward
     gate/up GEMM carries the LoRA terms, SiLU*mul and the codec in its
     epilogue; the backward runs the dgrad GEMM, then the K2 kernel
@@ -292,9 +314,9 @@ class FlashFFNv3Function(torch.autograd.Function):
         k_out = int(inter * outlier_ratio) if (quant and outlier_ratio > 0) else 0
         assert k_out == 0 or x.dtype == torch.bfloat16, "outlier channels need bf16 activations"
         # the dual gate/up kernel, with the gate/up LoRA terms in its epilogue
-        fusable = (_mfma(x_2d, w_gate, w_up)
+        fusable = (_fits16_linear(x_2d, w_gate, w_up)
                    and _lora_ok((a_gate, b_gate), (a_up, b_up), dims=((hidden_dim, inter),))
-                   and x_2d.shape[0] > 0)
+                   and all(t is None or t.dtype == x.dtype for t in (a_gate, a_up)))
 
         c_gate = qs_gate = c_up = qs_up = None
         o_gate = o_up = slot_gate = slot_up = None
@@ -437,10 +459,10 @@ class FlashFFNv3Function(torch.autograd.Function):
         fusable = _mfma(gy, w_down) and lora_d and gy.shape[0] > 0 and (use_k2 or not outl)
         # F1's recompute (k d_model) and the K-concatenated grad_x product (k d_ff)
         d_ff, d_model = w_gate.shape
-        fusable_gu = (_mfma(x_2d, w_gate, w_up)
+        fusable_gu = (_fits16_linear(x_2d, w_gate, w_up)
                       and _lora_ok((a_gate, b_gate), (a_up, b_up),
                                    dims=((d_model, d_ff), (d_ff, d_model)))
-                      and x_2d.shape[0] > 0)
+                      and all(t is None or t.dtype == x.dtype for t in (a_gate, a_up)))
 
         hg = hu = None
         if need_recon and not use_k2:                                     # :1500-1516
@@ -498,7 +520,8 @@ class FlashFFNv3Function(torch.autograd.Function):
                     lora=dlora, inplace=_private(mode, hg, hu))
                 hg = hu = None
             else:
-                if dlora is not None and _mfma(gy, w_down) and gy.shape[0] > 0:
+                if (dlora is not None and _fits16(gy, w_down)
+                        and gy.dtype == a_down.dtype):
                     grad_h_mid = G.mm2(gy, w_down, name="gemm_dgrad_down", lora=[
                         (gyB_d, a_down, s_down)])
                 else:
@@ -549,7 +572,8 @@ class FlashFFNv3Function(torch.autograd.Function):
             stack = (_stackable(b_gate.t() if b_gate is not None else None,
                                 b_up.t() if b_up is not None else None)
                      and (need_x or need_ag or need_au) and grad_h_gate.shape[0] >= 256
-                     and _mfma(grad_h_gate, b_gate, grad_h_up, b_up)
+                     and (_mfma(grad_h_gate, b_gate, grad_h_up, b_up)
+                          or (G.f16_fits(grad_h_gate, b_gate) and G.f16_fits(grad_h_up, b_up)))
                      and grad_h_gate.shape[1] >= 256)
             if stack:
                 r = b_gate.shape[1]
@@ -584,7 +608,9 @@ class FlashFFNv3Function(torch.autograd.Function):
             if need_x:
                 xl = [(ghgB, a_gate, s_gate) if a_gate is not None else None,
                       (ghuB, a_up, s_up) if a_up is not None else None]
-                if _mfma(grad_h_gate, w_gate, grad_h_up, w_up) and fusable_gu:
+                if fusable_gu and (_mfma(grad_h_gate, w_gate, grad_h_up, w_up)
+                                   or (G.f16_fits(grad_h_gate, w_gate)
+                                       and G.f16_fits(grad_h_up, w_up))):
                     # dg @ W_g + du @ W_u as one K-concatenated GEMM, the gate and up
                     # LoRA terms (:1561-1566) in its epilogue
                     grad_x = G.mm2(grad_h_gate, w_gate, grad_h_up, w_up, "gemm_dgrad_x",

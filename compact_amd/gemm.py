@@ -86,6 +86,46 @@ def _check_bf16(*ts):
         assert t.dim() == 2
 
 
+_DT16 = {torch.bfloat16: _lib.BF16, torch.float16: _lib.F16}
+
+
+def _check_16(*ts):
+    """2-D tensors of one 16-bit type; returns its dtype code."""
+    for t in ts:
+        assert t.dtype in _DT16 and t.dtype == ts[0].dtype, \
+            f"one 16-bit type expected, got {t.dtype} and {ts[0].dtype}"
+        assert t.dim() == 2
+    return _DT16[ts[0].dtype]
+
+
+def f16_fits(a: torch.Tensor, b: torch.Tensor) -> bool:
+    """a [M, K] @ b [K, N] in fp16 runs on the 128 x 128 tiles (cpt_gemm16):
+    16-byte aligned rows, N a multiple of 8, K of 64 unless both operands are
+    MN-major, and an MN-major operand within 32-bit offsets."""
+    if not (a.dtype == b.dtype == torch.float16 and a.dim() == 2 and b.dim() == 2):
+        return False
+    (M, K), N = a.shape, b.shape[1]
+    if not (M > 0 and K > 0 and N > 0 and N % 8 == 0 and a.data_ptr() % 16 == 0
+            and b.data_ptr() % 16 == 0):
+        return False
+    rows = (K + 256) * 2
+    if a.stride(1) == 1 and a.stride(0) % 8 == 0 and a.stride(0) >= K:
+        a_mn = False
+    elif (a.stride(0) == 1 and M % 8 == 0 and a.stride(1) % 8 == 0 and a.stride(1) >= M
+          and rows * a.stride(1) < _SPAN_BYTES):
+        a_mn = True
+    else:
+        return False
+    if b.stride(0) == 1 and b.stride(1) % 8 == 0 and b.stride(1) >= K:
+        b_mn = False
+    elif (b.stride(1) == 1 and b.stride(0) % 8 == 0 and b.stride(0) >= N
+          and rows * b.stride(0) < _SPAN_BYTES):
+        b_mn = True
+    else:
+        return False
+    return K % 64 == 0 or (a_mn and b_mn)
+
+
 LORA_MAX_RANK = 32
 _NO_TERMS = [(None, None, 0.0)] * 2
 
@@ -133,7 +173,7 @@ def _lora_args(terms, n_q, dims):
         terms, r = padded, rp
     keep, ps, qs = [], [], []
     for pm, q, _ in terms:
-        _check_bf16(pm, q)
+        _check_16(pm, q)
         assert pm.shape[1] == r and q.shape[0] == r and q.shape[1] == n_q
         if pm.stride(1) != 1 or pm.stride(0) % 8 or pm.data_ptr() % 16:
             pm = pm.contiguous()
@@ -181,7 +221,7 @@ def skinny(a: torch.Tensor, q: torch.Tensor, alpha: float = 1.0,
     view with unit column stride and 16-byte aligned rows (e.g. the column
     half of a wider buffer) to write into."""
     _require_device(a, q)
-    _check_bf16(a, q)
+    dt = _check_16(a, q)
     M, K = a.shape
     R = q.shape[0]
     assert q.shape[1] == K and R <= SKINNY_MAX_RANK
@@ -194,19 +234,18 @@ def skinny(a: torch.Tensor, q: torch.Tensor, alpha: float = 1.0,
     blocks = (M + 127) // 128
     splits = max(1, min(K // 256, (SKINNY_BLOCKS + blocks - 1) // blocks))
     if out is None:
-        c = torch.empty((M, R), dtype=torch.bfloat16, device=a.device)
+        c = torch.empty((M, R), dtype=a.dtype, device=a.device)
     else:
         c = out
-        assert (tuple(c.shape) == (M, R) and c.dtype == torch.bfloat16 and c.stride(1) == 1
+        assert (tuple(c.shape) == (M, R) and c.dtype == a.dtype and c.stride(1) == 1
                 and c.stride(0) % 8 == 0 and c.data_ptr() % 16 == 0), "skinny out layout"
     ws = (torch.empty((splits * M * R,), dtype=torch.float32, device=a.device)
           if splits > 1 else None)
     with _timed(name):
-        rc = _lib.lib().cpt_gemm_bf16_skinny(a.data_ptr(), a.stride(0), q.data_ptr(),
-                                             q.stride(0), c.data_ptr(), c.stride(0), M, R, K,
-                                             float(alpha),
-                                             splits, None if ws is None else ws.data_ptr(),
-                                             _stream(a))
+        rc = _lib.lib().cpt_gemm16_skinny(dt, a.data_ptr(), a.stride(0), q.data_ptr(),
+                                          q.stride(0), c.data_ptr(), c.stride(0), M, R, K,
+                                          float(alpha), splits,
+                                          None if ws is None else ws.data_ptr(), _stream(a))
     check(rc, name)
     return c
 
@@ -221,7 +260,7 @@ def skinny_t(x: torch.Tensor, p: torch.Tensor, alpha: float = 1.0, trans: bool =
     with trans) for R <= 32: the adapter-factor gradients that reduce over
     the tokens, x and p token-major."""
     _require_device(x, p)
-    _check_bf16(x, p)
+    dt = _check_16(x, p)
     T, N = x.shape
     R = p.shape[1]
     assert p.shape[0] == T and R <= SKINNY_MAX_RANK
@@ -234,13 +273,13 @@ def skinny_t(x: torch.Tensor, p: torch.Tensor, alpha: float = 1.0, trans: bool =
     per = (_SPAN_BYTES // (2 * max(x.stride(0), p.stride(0))) - 129) // 64 * 64
     assert per >= 64, "operand rows too long for 32-bit buffer offsets"
     splits = max(splits, (T + per - 1) // per)
-    out = torch.empty((R, N) if trans else (N, R), dtype=torch.bfloat16, device=x.device)
+    out = torch.empty((R, N) if trans else (N, R), dtype=x.dtype, device=x.device)
     ws = torch.empty((splits * N * R,), dtype=torch.float32, device=x.device)
     with _timed(name):
-        rc = _lib.lib().cpt_gemm_bf16_skinny_t(x.data_ptr(), x.stride(0), p.data_ptr(),
-                                               p.stride(0), out.data_ptr(), out.stride(0),
-                                               1 if trans else 0, T, N, R, float(alpha), splits,
-                                               ws.data_ptr(), _stream(x))
+        rc = _lib.lib().cpt_gemm16_skinny_t(dt, x.data_ptr(), x.stride(0), p.data_ptr(),
+                                            p.stride(0), out.data_ptr(), out.stride(0),
+                                            1 if trans else 0, T, N, R, float(alpha), splits,
+                                            ws.data_ptr(), _stream(x))
     check(rc, name)
     return out
 
@@ -276,11 +315,11 @@ def transpose(x: torch.Tensor, name: str = "transpose") -> torch.Tensor:
 
 
 def skinny_dual_ok(x: torch.Tensor, q: torch.Tensor, p: torch.Tensor) -> bool:
-    """skinny_dual takes bf16 x [T, N] with N a multiple of 8 and a rank
+    """skinny_dual takes bf16 or fp16 x [T, N] with N a multiple of 8 and a rank
     (q [R, N], p [T, R]) that is a multiple of 8 up to 32."""
     T, N = x.shape
     R = q.shape[0]
-    return (x.dtype == q.dtype == p.dtype == torch.bfloat16 and x.is_cuda and N % 8 == 0
+    return (x.dtype == q.dtype == p.dtype and x.dtype in _DT16 and x.is_cuda and N % 8 == 0
             and R % 8 == 0 and 0 < R <= SKINNY_MAX_RANK and q.shape[1] == N
             and tuple(p.shape) == (T, R))
 
@@ -316,17 +355,17 @@ def skinny_dual(x: torch.Tensor, q: torch.Tensor, p: torch.Tensor, alpha_c: floa
     assert per >= 64, "operand rows too long for 32-bit buffer offsets"
     splits = max(splits, (T + per - 1) // per)
     if out_c is None:
-        c = torch.empty((T, R), dtype=torch.bfloat16, device=x.device)
+        c = torch.empty((T, R), dtype=x.dtype, device=x.device)
     else:
         c = out_c
-        assert (tuple(c.shape) == (T, R) and c.dtype == torch.bfloat16 and c.stride(1) == 1
+        assert (tuple(c.shape) == (T, R) and c.dtype == x.dtype and c.stride(1) == 1
                 and c.stride(0) % 8 == 0 and c.data_ptr() % 16 == 0), "skinny_dual out layout"
-    z = torch.empty((N, R), dtype=torch.bfloat16, device=x.device)
+    z = torch.empty((N, R), dtype=x.dtype, device=x.device)
     nbytes = int(_lib.lib().cpt_gemm_bf16_skinny_dual_workspace_bytes(T, N, R, splits))
     ws = torch.empty((max(nbytes, 4) // 4,), dtype=torch.float32, device=x.device)
     with _timed(name):
-        rc = _lib.lib().cpt_gemm_bf16_skinny_dual(
-            x.data_ptr(), x.stride(0), q.data_ptr(), ldq, q_nr, p.data_ptr(), p.stride(0),
+        rc = _lib.lib().cpt_gemm16_skinny_dual(
+            _DT16[x.dtype], x.data_ptr(), x.stride(0), q.data_ptr(), ldq, q_nr, p.data_ptr(), p.stride(0),
             c.data_ptr(), c.stride(0), float(alpha_c), z.data_ptr(), z.stride(0), 0,
             float(alpha_z), T, N, R, splits, ws.data_ptr(), _stream(x))
     check(rc, name)
@@ -431,6 +470,8 @@ def mm(a: torch.Tensor, b: torch.Tensor, name: str = "gemm") -> torch.Tensor:
     if (N <= SKINNY_MAX_RANK and K >= 256 and K % 8 == 0 and M >= 256
             and a.stride(1) == 1):
         return skinny(a, b.t(), 1.0, name)
+    if a.dtype == torch.float16:
+        return mm2(a, b, None, None, name)
     tiles = ((M + 255) // 256) * ((N + 255) // 256)
     if tiles < 128 and K >= 1024 and (K % 64 or N % 8):
         return mm_splitk(a, b, 1.0, name=name)
@@ -486,9 +527,10 @@ def stream_k_errors(dev: torch.device) -> int:
 def mm2(a, b, a2=None, b2=None, name: str = "gemm", lora=None) -> torch.Tensor:
     """a @ b (+ a2 @ b2) in one fp32 accumulation -> bf16 [M, N], then the
     adapter terms `lora` = [(p [M, r], q [r, N], alpha), ...] (at most two),
-    each `out = bf16(out + bf16(alpha * bf16(p @ q)))`."""
+    each `out = bf16(out + bf16(alpha * bf16(p @ q)))`.  fp16 likewise, for
+    operands that fit the 128 x 128 tiles (f16_fits)."""
     _require_device(a, b)
-    _check_bf16(a, b)
+    dt = _check_16(a, b)
     M, K = a.shape
     K_, N = b.shape
     assert K == K_, f"inner dims differ: {tuple(a.shape)} @ {tuple(b.shape)}"
@@ -497,7 +539,7 @@ def mm2(a, b, a2=None, b2=None, name: str = "gemm", lora=None) -> torch.Tensor:
     p_a2 = p_b2 = None
     lda2 = ldb2 = K2 = 0
     if a2 is not None:
-        _check_bf16(a2, b2)
+        _check_16(a, a2, b2)
         assert a2.shape[0] == M and b2.shape[1] == N and a2.shape[1] == b2.shape[0]
         K2 = a2.shape[1]
         a2, lda2, ak2 = _layout_a(a2)
@@ -517,7 +559,7 @@ def mm2(a, b, a2=None, b2=None, name: str = "gemm", lora=None) -> torch.Tensor:
             ldb2 = ldb
         p_a2, p_b2 = a2.data_ptr(), b2.data_ptr()
     ldc = (N + 7) // 8 * 8
-    c = torch.empty((M, ldc), dtype=torch.bfloat16, device=a.device)
+    c = torch.empty((M, ldc), dtype=a.dtype, device=a.device)
     r, ldp, qk, ldq, t = 0, 0, 1, 0, _NO_TERMS
     if lora:
         if ak != 1:
@@ -526,15 +568,18 @@ def mm2(a, b, a2=None, b2=None, name: str = "gemm", lora=None) -> torch.Tensor:
             assert a2 is None, "adapter terms with a K-concatenated MN-major A"
         dims = ((K, N),) if a2 is None else ((K, N), (K2, N))
         r, ldp, qk, ldq, t, keep = _lora_args(lora, N, dims)
-    splits = (1 if K % 64 or K2 % 64 or N % 8 or not K
-              else split_plan(M, N, (K + K2) // 64))
-    if splits > 1:
-        ws = torch.empty((splits * M * N,), dtype=torch.float32, device=a.device)
+    half = dt == _lib.F16
+    splits = (1 if (not half and (K % 64 or K2 % 64)) or N % 8 or not K
+              else split_plan(M, N, (K + 63) // 64 + (K2 + 63) // 64))
+    if splits > 1 or half:
+        ws = (torch.empty((splits * M * N,), dtype=torch.float32, device=a.device)
+              if splits > 1 else None)
         with _timed(name):
             rc = _lib.lib().cpt_gemm16(
-                _lib.BF16, a.data_ptr(), lda, ak, b.data_ptr(), ldb, bk, p_a2, lda2, p_b2, ldb2,
+                dt, a.data_ptr(), lda, ak, b.data_ptr(), ldb, bk, p_a2, lda2, p_b2, ldb2,
                 K2, c.data_ptr(), ldc, M, N, K, r, ldp, qk, ldq, t[0][0], t[0][1], t[0][2],
-                t[1][0], t[1][1], t[1][2], splits, ws.data_ptr(), _stream(a))
+                t[1][0], t[1][1], t[1][2], splits, None if ws is None else ws.data_ptr(),
+                _stream(a))
         check(rc, name)
         return c
     _stream_k(a.device)
@@ -591,20 +636,23 @@ def ffn_gate_up(x, w_gate, w_up, cache: int, group_size: int, want_h_mid: bool =
                 lora_gate=None, lora_up=None):
     """Fused dual GEMM + GLU + codec.  Returns (h_mid | None, h_gate | None,
     h_up | None, q_gate | None, s_gate | None, q_up | None, s_up | None).
+    CACHE_BF16 keeps h_gate / h_up in x's type (bf16, or fp16 without codec).
     lora_gate / lora_up = (xa [n, r], B [inter, r], s): the projection's LoRA
     term, added to h_gate / h_up before the GLU and the codec."""
     _require_device(x, w_gate, w_up)
-    _check_bf16(x, w_gate, w_up)
+    dt = _check_16(x, w_gate, w_up)
+    half = dt == _lib.F16
+    assert not half or cache in (_lib.CACHE_NONE, _lib.CACHE_BF16), "the codec takes bf16"
     n, hdim = x.shape
     d = w_gate.shape[0]
     assert w_gate.shape == (d, hdim) and w_up.shape == (d, hdim)
     x, w_gate, w_up = x.contiguous(), w_gate.contiguous(), w_up.contiguous()
     dev = x.device
-    h_mid = torch.empty((n, d), dtype=torch.bfloat16, device=dev) if want_h_mid else None
+    h_mid = torch.empty((n, d), dtype=x.dtype, device=dev) if want_h_mid else None
     hg = hu = qg = sg = qu = su = None
     if cache == _lib.CACHE_BF16:
-        hg = torch.empty((n, d), dtype=torch.bfloat16, device=dev)
-        hu = torch.empty((n, d), dtype=torch.bfloat16, device=dev)
+        hg = torch.empty((n, d), dtype=x.dtype, device=dev)
+        hu = torch.empty((n, d), dtype=x.dtype, device=dev)
     elif cache in (_lib.CACHE_INT4, _lib.CACHE_INT8):
         g = d // group_size
         shape = (n, d // 2) if cache == _lib.CACHE_INT4 else (n, d)
@@ -630,12 +678,13 @@ def ffn_gate_up(x, w_gate, w_up, cache: int, group_size: int, want_h_mid: bool =
               if cache in (_lib.CACHE_NONE, _lib.CACHE_BF16) and hdim % 64 == 0 and d % 8 == 0
               else 1)
     with _timed("ffn_gate_up"):
-        if splits > 1:
-            ws = torch.empty((splits * n * 2 * d,), dtype=torch.float32, device=dev)
+        if splits > 1 or half:
+            ws = (torch.empty((splits * n * 2 * d,), dtype=torch.float32, device=dev)
+                  if splits > 1 else None)
             rc = _lib.lib().cpt_ffn_gate_up16(
-                _lib.BF16, x.data_ptr(), w_gate.data_ptr(), w_up.data_ptr(), n, hdim, d,
+                dt, x.data_ptr(), w_gate.data_ptr(), w_up.data_ptr(), n, hdim, d,
                 p(h_mid), p(hg), p(hu), r, ldp, t[0][0], t[0][1], t[0][2], t[1][0], t[1][1],
-                t[1][2], splits, ws.data_ptr(), _stream(x))
+                t[1][2], splits, None if ws is None else ws.data_ptr(), _stream(x))
         elif r:
             rc = _lib.lib().cpt_ffn_gate_up_lora(
                 x.data_ptr(), w_gate.data_ptr(), w_up.data_ptr(), n, hdim, d, cache, group_size,
@@ -817,6 +866,16 @@ def addmm_(c: torch.Tensor, a: torch.Tensor, b: torch.Tensor, alpha: float,
     return c
 
 
+def skinny_t_fits(a: torch.Tensor, b: torch.Tensor) -> bool:
+    """a [M, K] @ b [K, N] runs on the token-reduction kernel: both token-major
+    (a's transpose and b row-major with 16-byte rows), K >= 256 tokens, M and N
+    multiples of 8, one of them a rank up to 32."""
+    M, K = a.shape
+    N = b.shape[1]
+    return (_row_major(a.t()) and _row_major(b) and K >= 256 and M % 8 == 0 and N % 8 == 0
+            and (M <= SKINNY_MAX_RANK or N <= SKINNY_MAX_RANK))
+
+
 def mm_splitk(a: torch.Tensor, b: torch.Tensor, alpha: float = 1.0, splits: int | None = None,
               name: str = "gemm_splitk") -> torch.Tensor:
     """bf16(alpha * (a @ b)) with the K reduction split across blocks (fp32
@@ -825,16 +884,15 @@ def mm_splitk(a: torch.Tensor, b: torch.Tensor, alpha: float = 1.0, splits: int 
     32 (the rank: grad_A = s (grad B)^T x, grad_B = s grad_y^T (x A^T)) the
     token-reduction kernel runs instead of 256 x 256 tiles."""
     _require_device(a, b)
-    _check_bf16(a, b)
     M, K = a.shape
     K_, N = b.shape
     assert K == K_
     at = a.t()
-    if splits is None and _row_major(at) and _row_major(b) and K >= 256:
-        if M <= SKINNY_MAX_RANK and M % 8 == 0 and N % 8 == 0:
+    if splits is None and skinny_t_fits(a, b):
+        if M <= SKINNY_MAX_RANK:
             return skinny_t(b, at, alpha, trans=True, name=name)
-        if N <= SKINNY_MAX_RANK and N % 8 == 0 and M % 8 == 0:
-            return skinny_t(at, b, alpha, trans=False, name=name)
+        return skinny_t(at, b, alpha, trans=False, name=name)
+    _check_bf16(a, b)
     a, lda, ak = _layout_a(a)
     b, ldb, bk = _layout_b(b)
     if splits is None:

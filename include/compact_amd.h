@@ -308,6 +308,20 @@ int cpt_gemm_bf16_lora(const void* a, int64_t lda, int a_kmajor, const void* b, 
                        const void* q0, float alpha0, const void* p1, const void* q1,
                        float alpha1, void* stream);
 
+/* cpt_gemm_bf16_skinny, _skinny_t and _skinny_dual for bf16 or fp16 (dtype
+ * codes 2 / 1).  fp16 results round the fp32 sum, then alpha times it. */
+int cpt_gemm16_skinny(int dtype, const void* a, int64_t lda, const void* q, int64_t ldq, void* c,
+                      int64_t ldc, int64_t M, int64_t R, int64_t K, float alpha, int splits,
+                      void* workspace, void* stream);
+int cpt_gemm16_skinny_t(int dtype, const void* x, int64_t ldx, const void* p, int64_t ldp,
+                        void* out, int64_t ldo, int out_trans, int64_t T, int64_t N, int64_t R,
+                        float alpha, int splits, void* workspace, void* stream);
+int cpt_gemm16_skinny_dual(int dtype, const void* x, int64_t ldx, const void* q, int64_t ldq,
+                           int q_nr, const void* p, int64_t ldp, void* c, int64_t ldc,
+                           float alpha_c, void* z, int64_t ldz, int z_trans, float alpha_z,
+                           int64_t T, int64_t N, int64_t R, int splits, void* workspace,
+                           void* stream);
+
 /* cpt_gemm_bf16_lora's product (rank 0: cpt_gemm_bf16's) on 128 x 128 tiles for
  * bf16 or fp16 operands and results (dtype CPT_BF16 / CPT_F16 codes 2 / 1), K
  * a multiple of 64 (two MN-major operands: any K), N of 8.  splits > 1 shares

@@ -101,3 +101,55 @@ def test_function_dual_route_matches_separate(device, mode, group):
         else:
             rel = ((g1[k].float() - g0[k].float()).norm() / g0[k].float().norm()).item()
             assert rel < 1e-2, (k, rel)
+
+
+@pytest.mark.parametrize("T,N,r", [(256, 512, 8), (300, 1032, 16), (1024, 2048, 32)])
+def test_fp16_adapter_products(T, N, r):
+    """fp16 through the projection, the token reduction and the dual pass: one
+    fp16 rounding each (alpha * the rounded sum: two) of the fp32 sum."""
+    from compact_amd import gemm as G
+    g = torch.Generator(device="cuda").manual_seed(0)
+    x, q, p = (torch.randn(s, device="cuda", generator=g).half() for s in
+               ((T, N), (r, N), (T, r)))
+    ref_c, ref_z = x.double() @ q.double().t(), 0.5 * (x.double().t() @ p.double())
+    tol_c = N * 2.0 ** -24 * (x.double().abs() @ q.double().abs().t()) + 2.0 ** -25
+    tol_z = T * 2.0 ** -24 * (x.double().abs().t() @ p.double().abs()) + 2.0 ** -25
+    for c in (G.skinny(x, q), G.skinny_dual(x, q, p, 1.0, 0.5)[0]):
+        assert bool(((c.double() - ref_c).abs() <= 2.0 ** -11 * 1.01 * ref_c.abs() + tol_c).all())
+    for z in (G.skinny_t(x, p, 0.5), G.skinny_t(x, p, 0.5, trans=True).t(),
+              G.skinny_dual(x, q, p, 1.0, 0.5)[1]):
+        assert bool(((z.double() - ref_z).abs() <= 2.0 ** -10 * 1.01 * ref_z.abs() + tol_z).all())
+
+
+@pytest.mark.parametrize("n,h,d", [(1, 64, 128), (65, 192, 320), (259, 256, 512), (300, 200, 336)])
+@pytest.mark.parametrize("mode", ["int4", "int8", "bf16", "recompute"])
+@pytest.mark.parametrize("rank", [0, 8, 12, 32])
+def test_fp16_function_equals_general_layout_kernel(n, h, d, mode, rank, monkeypatch):
+    """The fp16 Function on the MFMA tiles against the general-layout kernel:
+    the routes differ in the order of fp32 sums only, so in single fp16
+    roundings (and codes on a rounding tie)."""
+    from compact_amd import flashffn as FF
+    from compact_amd import gemm as G
+    g = torch.Generator(device="cuda").manual_seed(n + h + rank)
+
+    def rn(*s, std=1.0):
+        return (torch.randn(s, device="cuda", generator=g) * std).half().requires_grad_()
+    x, gy = rn(n, h), torch.randn(n, h, device="cuda", generator=g).half()
+    ws = [rn(d, h, std=0.05), rn(d, h, std=0.05), rn(h, d, std=0.05)]
+    ab = [(rn(rank, w.shape[1], std=0.05), rn(w.shape[0], rank, std=0.05)) if rank else (None, None)
+          for w in ws]
+    leaves = [x] + [t for w, (a, b) in zip(ws, ab) for t in (w, a, b) if t is not None]
+
+    def step():
+        args = [t for w, (a, b) in zip(ws, ab) for t in (w, a, b)]
+        y = FF.FlashFFNv3Function.apply(x, *args, 0.5, 0.5, 0.5, mode, 64 if d % 64 == 0 else 16)
+        return [y] + list(torch.autograd.grad(y, leaves, gy))
+    got = step()
+    monkeypatch.setattr(G, "f16_fits", lambda a, b: False)
+    monkeypatch.setattr(G, "skinny_t_fits", lambda a, b: False)
+    monkeypatch.setattr(G, "skinny_dual_ok", lambda *a: False)
+    for a, b in zip(got, step()):
+        assert a.dtype == torch.float16
+        err = (a.double() - b.double()).norm() / b.double().norm().clamp_min(1e-20)
+        # a chain of some ten fp16 roundings (2^-11 each); int caches may flip codes on ties
+        assert err < (2e-2 if mode == "int4" else 5e-3), err.item()
