@@ -48,6 +48,11 @@ SIGNATURES = {
                    _L, _P, _P, ctypes.c_float, _P, _P, ctypes.c_float, _I, _P, _P],
     "cpt_ffn_gate_up16": [_I, _P, _P, _P, _L, _L, _L, _P, _P, _P, _L, _L, _P, _P, ctypes.c_float,
                           _P, _P, ctypes.c_float, _I, _P, _P],
+    "cpt_split_f32": [_P, _L, _L, _L, _P, _P, _P],
+    "cpt_gemm_f32x3": [_P, _L, _L, _I, _P, _L, _L, _I, _P, _L, _P, _L, _L, _P, _P, _P, _P, _P,
+                       _L, _L, _L, _L, ctypes.c_float, _I, _I, _P, _P],
+    "cpt_gemm_any_if": [_P, _P, _P, _P, _I, _P, _L, _L, _P, _L, _L, _P, _L, _L, _L, _L, _L,
+                        ctypes.c_float, _I, _P],
     "cpt_gemm_any": [_I, _P, _L, _L, _P, _L, _L, _P, _L, _L, _L, _L, _L, ctypes.c_float, _I, _P],
     "cpt_gemm_wgrad_glu": [_P, _L, _I, _L, _P, _P, _P, _P, _P, _L, _L, _L, _L, _P],
     "cpt_ffn_gate_up": [_P, _P, _P, _L, _L, _L, _I, _L, _P, _P, _P, _P, _P, _P, _P, _P],

@@ -280,12 +280,18 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 constexpr int64_t kSkSlot = 256 * 256;            // floats per partial (one tile)
 constexpr int kSkSpin = 1 << 22;
 
-template <bool AK, bool BK, int EPI, int CACHE, int GS, int LT, bool SK, bool HI>
+// X3: an fp32 product from three bf16 planes per operand; the k loop runs over
+// the six plane pairs of each operand pair, the smallest products first (see
+// gemm16s_kernel.h), and the epilogue (EPI_F32) writes fp32 to A.ws, split sk_s
+// of it.
+template <bool AK, bool BK, int EPI, int CACHE, int GS, int LT, bool SK, bool HI, bool X3 = false>
 __device__ __forceinline__ void nt16_tile(const KArgs& A, uint16_t* lds, int tm, int tn, int kb,
                                           int ke, int role, int sk_s) {
   static_assert(LT == 0 || AK, "adapter terms ride with a K-major A (P's rows are tokens)");
-  static_assert(EPI == EPI_STORE || EPI == EPI_GLU || EPI == EPI_DGLU || EPI == EPI_GLUO,
+  static_assert(EPI == EPI_STORE || EPI == EPI_GLU || EPI == EPI_DGLU || EPI == EPI_GLUO ||
+                    EPI == EPI_F32,
                 "epilogues of the 16x16x32 loop");
+  static_assert(X3 == (EPI == EPI_F32), "fp32 products write fp32");
   static_assert(EPI != EPI_DGLU || (AK && !BK), "B1: gy (K-major) . W_d (MN-major)");
   constexpr bool DUAL = EPI == EPI_GLU || EPI == EPI_GLUO;
   static_assert(!DUAL || (AK && BK), "F1's operands are K-major");
@@ -364,6 +370,43 @@ __device__ __forceinline__ void nt16_tile(const KArgs& A, uint16_t* lds, int tm,
     const uint32_t lk = (uint32_t)(kc - (p1 ? nk0 : 0));
     return TileLd{p1 ? ra1 : ra0, p1 ? rb1 : rb0, lk * stepa, lk * stepb};
   };
+  // X3: the next k-tile of the range, from one plane pair to the next; past the
+  // range no records (zeros, no memory read)
+  const int npr = A.npairs;
+  auto x3_nk = [&](int sg) { return npr == 2 && (sg & 1) ? (int)(A.K[1] / kBK) : nk0; };
+  int x3_seg = 0, x3_lk = kb, x3_rem = ke - kb;
+  TileLd x3_t;
+  auto x3_open = [&]() {
+    const int pr = npr == 2 ? x3_seg & 1 : 0;
+    const int t4 = 4 * (npr == 2 ? x3_seg >> 1 : x3_seg);
+    const uint16_t* pa = A.a[pr].p + ((0x010120 >> t4) & 15) * A.plane_a[pr];
+    const uint16_t* pb = A.b[pr].p + ((0x001102 >> t4) & 15) * A.plane_b[pr];
+    x3_t.a = AK ? rsrc_sgpr(pa + m0 * lda, (A.M - m0) * lda * 2)
+                : rsrc_sgpr(pa + m0, (A.K[pr] * lda - m0) * 2);
+    x3_t.b = BK ? rsrc_sgpr(pb + n0 * ldb, (A.N - n0) * ldb * 2)
+                : rsrc_sgpr(pb + n0, (A.K[pr] * ldb - n0) * 2);
+    x3_t.da = (uint32_t)x3_lk * stepa;
+    x3_t.db = (uint32_t)x3_lk * stepb;
+  };
+  if constexpr (X3) {
+    while (x3_lk >= x3_nk(x3_seg)) x3_lk -= x3_nk(x3_seg++);
+    x3_open();
+  }
+  auto x3_next = [&]() {
+    const TileLd t = x3_t;
+    if (--x3_rem <= 0) {
+      x3_t.a[2] = x3_t.b[2] = 0;
+      x3_t.da = x3_t.db = 0;
+    } else if (++x3_lk == x3_nk(x3_seg)) {
+      x3_lk = 0;
+      ++x3_seg;
+      x3_open();
+    } else {
+      x3_t.da += stepa;
+      x3_t.db += stepb;
+    }
+    return t;
+  };
   // load p (0..15) of a tile into stage st: even p -> A block p / 2, odd -> B
   auto issue = [&](int p, int st, const TileLd& T) {
     const int i = p >> 1;
@@ -409,7 +452,7 @@ __device__ __forceinline__ void nt16_tile(const KArgs& A, uint16_t* lds, int tm,
 
   // prologue: k-tile kb -> stage 0, kb + 1 -> stage 1; kb landed; F0 of kb
   {
-    const TileLd T0 = tile(kb), T1 = tile(kb + 1);
+    const TileLd T0 = X3 ? x3_next() : tile(kb), T1 = X3 ? x3_next() : tile(kb + 1);
 #pragma unroll
     for (int p = 0; p < 16; ++p) issue(p, 0, T0);
 #pragma unroll
@@ -427,7 +470,7 @@ __device__ __forceinline__ void nt16_tile(const KArgs& A, uint16_t* lds, int tm,
   constexpr Order ord;
   for (int kt = kb; kt < ke; ++kt) {
     const int stage = (kt - kb) & 1;
-    const TileLd T2 = tile(kt + 2);
+    const TileLd T2 = X3 ? x3_next() : tile(kt + 2);
     static_for<0, 128>([&](auto tc) {
       constexpr int t = decltype(tc)::value;
       if constexpr (t < 64) {
@@ -505,6 +548,23 @@ __device__ __forceinline__ void nt16_tile(const KArgs& A, uint16_t* lds, int tm,
   // live across the main loop.
   const int etid = epi_tid();
   const int elane = etid & 63;
+  if constexpr (EPI == EPI_F32) {
+    float* const out = A.ws + (int64_t)sk_s * A.M * A.ldc;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int64_t n = n0 + wn * 128 + 16 * i + 4 * (elane >> 4);
+      if (n >= A.N) continue;   // N % 8 == 0
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const int64_t m = m0 + wm * 128 + 16 * j + (elane & 15);
+        f32x4 v = acc[i][j];
+        asm volatile("" : "+v"(v));
+        v *= A.alpha;   // 1 for partials
+        if (m < A.M) *reinterpret_cast<f32x4*>(out + m * A.ldc + n) = v;
+      }
+    }
+    return;
+  }
   Lora16<HI> F;
   if constexpr (LT > 0) lora16_load<DUAL, LT, HI>(A, m0, n0, wm, wn, elane, F);
   if constexpr (EPI == EPI_STORE || EPI == EPI_DGLU) {
@@ -552,7 +612,7 @@ __device__ __forceinline__ void nt16_tile(const KArgs& A, uint16_t* lds, int tm,
       const uint4 w = *reinterpret_cast<const uint4*>(lds + r * kLdOut + cl);
       if (nok && m0 + r < A.M) *reinterpret_cast<uint4*>(A.C + (m0 + r) * A.ldc + n0 + cl) = w;
     }
-  } else {
+  } else if constexpr (EPI != EPI_F32) {
     // F1: blocks i < 4 are gate columns d = 64 wn + 16 i + ..., i >= 4 the
     // same up columns; staged as glu_finish's two tiles (rows kGluLd apart:
     // 32 lanes of one 8-byte write cover the 64 banks once)
@@ -618,7 +678,43 @@ __global__ __launch_bounds__(kThreads, 1) void nt16_kernel(const KArgs A) {
   }
 }
 
+// fp32 products of plane pairs: block = split * tiles + tile, split s takes
+// k-tiles [s kt_per_split, ..) of the 6 npairs segments.
+template <bool AK, bool BK>
+__global__ __launch_bounds__(kThreads, 1) void nt16_x3_kernel(const KArgs A) {
+  extern __shared__ __attribute__((aligned(16))) uint16_t lds[];
+  if (any_flag(A.flags)) return;
+  const int tiles = A.tiles_m * A.tiles_n;
+  const int split = blockIdx.x / tiles;
+  const int nk = 6 * (int)(A.K[0] / kBK + (A.npairs == 2 ? A.K[1] / kBK : 0));
+  const int kb = split * A.kt_per_split;
+  int tm, tn;
+  tile_coords_of(blockIdx.x - split * tiles, tiles, A.tiles_m, A.tiles_n, tm, tn);
+  nt16_tile<AK, BK, EPI_F32, 0, 0, 0, false, false, true>(
+      A, lds, tm, tn, kb, min(nk, kb + A.kt_per_split), kRoleWhole, split);
+}
+
 }  // namespace nt16
+
+// fp32 products of plane pairs on 256 x 256 tiles, A.ksplit blocks per tile
+template <bool AK, bool BK>
+int launch_nt16_x3(KArgs A, hipStream_t st) {
+  auto kern = nt16::nt16_x3_kernel<AK, BK>;
+  static bool attr_set = false;   // per instantiation
+  if (!attr_set) {
+    if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
+                            nt16::kMainLds) != hipSuccess)
+      return kErrLaunch;
+    attr_set = true;
+  }
+  A.tiles_m = (int)((A.M + 255) / 256);
+  A.tiles_n = (int)((A.N + 255) / 256);
+  const int64_t blocks = (int64_t)A.tiles_m * A.tiles_n * A.ksplit;
+  if (blocks <= 0) return kOk;
+  if (blocks > 0x7FFFFFFF) return kErrTooLarge;
+  hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(nt16::kThreads), nt16::kMainLds, st, A);
+  return hipGetLastError() == hipSuccess ? kOk : kErrLaunch;
+}
 
 template <bool AK, bool BK, int EPI, int CACHE, int GS, int LT>
 int launch_nt16(const KArgs& A, hipStream_t st) {

@@ -35,6 +35,15 @@
 // weight gradients, k = tokens) may end in a partial k-tile: its buffers then
 // start at that tile, so the rows past K read zero.
 
+//
+// fp32 products (DT = kF32): each operand comes as three bf16 planes that sum
+// to it (split_f32_kernel: 8 + 8 + 8 significant bits), and the k loop runs
+// over six pairs of planes, the smallest products first: h l, l h, m m, h m,
+// m h, h h.  The three left out are below 2^-24 of the product; every partial
+// product is exact in fp32 and the sums are fp32, with one rounding per 32 k
+// where v_mfma_f32_32x32x2_f32 rounds every 2.  The 256 x 256 tiles carry the
+// same loop (nt16_x3_kernel); figures beside x3_gemm_impl in gemm.hip.
+
 #pragma once
 
 #include "gemm16_kernel.h"
@@ -115,6 +124,7 @@ template <int DT> __device__ __forceinline__ void wide8(const uint4& w, float (&
 
 template <int DT> __device__ __forceinline__ void mfma32(f32x4& c, const bf16x8& a, const bf16x8& b) {
   if constexpr (DT == kBF16) nt16::mfma(c, a, b);
+  else if constexpr (DT == kF32) nt16::mfma(c, a, b);   // bf16 planes
   else asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
 }
 typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
@@ -186,6 +196,10 @@ __global__ __launch_bounds__(kThreads, S == 2 ? 2 : 1) void st16_kernel(const KA
   // EPI_F32 with CACHE_NONE / CACHE_BF16: partials of a plain / dual product
   constexpr bool DUAL = EPI == EPI_GLU || (EPI == EPI_F32 && CACHE == CACHE_BF16);
   constexpr bool TAIL = !AK && !BK;
+  constexpr bool X3 = DT == kF32;
+  static_assert(!X3 || EPI == EPI_F32, "fp32 products write fp32");
+  if constexpr (X3)
+    if (any_flag(A.flags)) return;
   static_assert(!DUAL || (AK && BK), "F1's operands are K-major");
   extern __shared__ __attribute__((aligned(16))) uint16_t lds[];
   const int tiles = A.tiles_m * A.tiles_n;
@@ -225,33 +239,44 @@ __global__ __launch_bounds__(kThreads, S == 2 ? 2 : 1) void st16_kernel(const KA
   }
   const uint32_t stepa = AK ? (uint32_t)(kBK * 2) : (uint32_t)(kBK * lda * 2);
   const uint32_t stepb = BK ? (uint32_t)(kBK * 2) : (uint32_t)(kBK * ldb * 2);
-  auto ktiles = [&](int pr) { return (int)((A.K[pr] + kBK - 1) / kBK); };
-  const int nk_all = ktiles(0) + (A.npairs == 2 ? ktiles(1) : 0);
+  // Segments of the k loop: the operand pairs, or (X3) the six plane products
+  // of each pair
+  const int nseg = X3 ? 6 * A.npairs : A.npairs;
+  auto pair_of = [&](int sg) { return X3 ? (A.npairs == 2 ? sg & 1 : 0) : sg; };
+  auto ktiles = [&](int sg) { return (int)((A.K[pair_of(sg)] + kBK - 1) / kBK); };
+  int nk_all = ktiles(0) + (A.npairs == 2 ? ktiles(1) : 0);
+  if (X3) nk_all *= 6;
   const int kb = EPI == EPI_F32 ? min(nk_all, split * A.kt_per_split) : 0;
   const int nk = EPI == EPI_F32 ? min(nk_all - kb, A.kt_per_split) : nk_all;
-  // the k-tile being loaded: its pair's buffers and byte deltas, the k-tiles
-  // left in the pair and in the block's range
+  // the k-tile being loaded: its segment's buffers and byte deltas, the k-tiles
+  // left in the segment and in the block's range
   i32x4 ra, rb, rbu;
   uint32_t da, db;
-  int left, rem = nk, pair = 0;
-  auto open = [&](int pr, int lk) {
+  int left, rem = nk, seg = 0;
+  auto open = [&](int sg, int lk) {
+    const int pr = pair_of(sg);
+    const uint16_t* pa = A.a[pr].p;
+    const uint16_t* pb = A.b[pr].p;
+    if constexpr (X3) {
+      // planes (A, B) of term t: (0,2) (2,0) (1,1) (0,1) (1,0) (0,0)
+      const int t4 = 4 * (A.npairs == 2 ? sg >> 1 : sg);
+      pa += ((0x010120 >> t4) & 15) * A.plane_a[pr];
+      pb += ((0x001102 >> t4) & 15) * A.plane_b[pr];
+    }
     // a partial last k-tile: the buffers start at its first row (TAIL)
     const int64_t k0 = TAIL && ((int64_t)lk + 1) * kBK > A.K[pr] ? (int64_t)lk * kBK : 0;
-    ra = AK ? rsrc_sgpr(A.a[pr].p + m0 * lda, (A.M - m0) * lda * 2)
-            : rsrc_sgpr(A.a[pr].p + k0 * lda + m0, ((A.K[pr] - k0) * lda - m0) * 2);
-    rb = BK ? rsrc_sgpr(A.b[pr].p + nb0 * ldb, (nrows - nb0) * ldb * 2)
-            : rsrc_sgpr(A.b[pr].p + k0 * ldb + n0, ((A.K[pr] - k0) * ldb - n0) * 2);
+    ra = AK ? rsrc_sgpr(pa + m0 * lda, (A.M - m0) * lda * 2)
+            : rsrc_sgpr(pa + k0 * lda + m0, ((A.K[pr] - k0) * lda - m0) * 2);
+    rb = BK ? rsrc_sgpr(pb + nb0 * ldb, (nrows - nb0) * ldb * 2)
+            : rsrc_sgpr(pb + k0 * ldb + n0, ((A.K[pr] - k0) * ldb - n0) * 2);
     rbu = DUAL ? rsrc_sgpr(A.b_up + nb0 * ldb, (nrows - nb0) * ldb * 2) : rb;
     da = TAIL && k0 ? 0 : (uint32_t)lk * stepa;
     db = TAIL && k0 ? 0 : (uint32_t)lk * stepb;
-    left = ktiles(pr) - lk;
+    left = ktiles(sg) - lk;
   };
-  if (kb < ktiles(0) || A.npairs != 2) {
-    open(0, kb);
-  } else {
-    pair = 1;
-    open(1, kb - ktiles(0));
-  }
+  int lk0 = kb;
+  while (seg + 1 < nseg && lk0 >= ktiles(seg)) lk0 -= ktiles(seg++);
+  open(seg, lk0);
   auto advance = [&]() {
     da += stepa;
     db += stepb;
@@ -260,9 +285,9 @@ __global__ __launch_bounds__(kThreads, S == 2 ? 2 : 1) void st16_kernel(const KA
       ra[2] = rb[2] = rbu[2] = 0;
       da = db = 0;
     } else if (left == 0) {
-      open(++pair, 0);
+      open(++seg, 0);
     } else if (TAIL && left == 1) {
-      open(pair, ktiles(pair) - 1);
+      open(seg, ktiles(seg) - 1);
     }
   };
   // load p (0..7): even p -> A block p / 2, odd -> B
@@ -363,6 +388,7 @@ __global__ __launch_bounds__(kThreads, S == 2 ? 2 : 1) void st16_kernel(const KA
         const int64_t m = m0 + wm * 64 + 16 * j + (el & 15);
         f32x4 v = acc[i][j];
         asm volatile("" : "+v"(v));
+        if constexpr (X3) v *= A.alpha;   // 1 for partials
         if (m < A.M) *reinterpret_cast<f32x4*>(out + m * A.ldc + (DUAL && i >= 2 ? A.D : 0) + n) = v;
       }
     }

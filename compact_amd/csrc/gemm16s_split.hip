@@ -120,6 +120,21 @@ __global__ __launch_bounds__(256) void reduce_kernel(const KArgs A, int terms, i
   }
 }
 
+// fp32 outputs of a split fp32 product: c = alpha * sum
+__global__ __launch_bounds__(256) void reduce_f32_kernel(const KArgs A, float* c, int64_t ldo) {
+  const int64_t cols = A.N / 8;
+  const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (e >= A.M * cols) return;
+  const int64_t m = e / cols, n = (e - m * cols) * 8;
+  float v[8];
+  sum8(A.ws + m * A.ldc + n, A.M * A.ldc, A.ksplit, v);
+#pragma unroll
+  for (int j = 0; j < 2; ++j)
+    *reinterpret_cast<f32x4*>(c + m * ldo + n + 4 * j) =
+        f32x4{A.alpha * v[4 * j], A.alpha * v[4 * j + 1], A.alpha * v[4 * j + 2],
+              A.alpha * v[4 * j + 3]};
+}
+
 }  // namespace st16
 
 int st16_reduce(int dt, bool dual, const KArgs& A, int terms, int64_t ldo, hipStream_t st) {
@@ -127,6 +142,11 @@ int st16_reduce(int dt, bool dual, const KArgs& A, int terms, int64_t ldo, hipSt
   const int64_t blocks = (n + 255) / 256;
   if (blocks <= 0) return kOk;
   if (blocks > 0x7FFFFFFF) return kErrTooLarge;
+  if (dt == kF32) {
+    hipLaunchKernelGGL(st16::reduce_f32_kernel, dim3((unsigned)blocks), dim3(256), 0, st, A,
+                       (float*)A.C, ldo);
+    return hipGetLastError() == hipSuccess ? kOk : kErrLaunch;
+  }
   // 16-byte reads of Q's rows when they all start on 16 bytes
   bool vec = (A.lldq & 7) == 0;
   for (int t = 0; t < terms; ++t) vec = vec && aligned16(A.lq[t]);

@@ -50,6 +50,8 @@ struct Args {
   float alpha;
   int a_kfast;   // A's unit-stride dimension is k (else m)
   int b_kfast;   // B's unit-stride dimension is k (else n)
+  // runs only if one of these words is set (all null: always)
+  const int* flags[4];
 };
 
 // One operand tile (rows = the 128-wide m or n side, k = 16) into registers.
@@ -89,6 +91,13 @@ __device__ __forceinline__ float rd(float v) {
 template <int DT, int EPI>
 __global__ __launch_bounds__(NTHR) void gemm_any_kernel(Args A) {
   __shared__ float lds[2 * STAGE];
+  if (A.flags[0]) {
+    int set = 0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (A.flags[i]) set |= *A.flags[i];
+    if (!set) return;
+  }
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6;
   const int wm = wave >> 1, wn = wave & 1;
@@ -198,7 +207,17 @@ extern "C" int cpt_gemm_any(int dtype, const void* a, int64_t sam, int64_t sak, 
                             int64_t sbk, int64_t sbn, void* c, int64_t scm, int64_t scn,
                             int64_t M, int64_t N, int64_t K, float alpha, int mode,
                             void* stream) {
+  return cpt_gemm_any_if(nullptr, nullptr, nullptr, nullptr, dtype, a, sam, sak, b, sbk, sbn, c,
+                         scm, scn, M, N, K, alpha, mode, stream);
+}
+
+extern "C" int cpt_gemm_any_if(const void* flag0, const void* flag1, const void* flag2,
+                               const void* flag3, int dtype, const void* a, int64_t sam,
+                               int64_t sak, const void* b, int64_t sbk, int64_t sbn, void* c,
+                               int64_t scm, int64_t scn, int64_t M, int64_t N, int64_t K,
+                               float alpha, int mode, void* stream) {
   using namespace cpt::gemm_any;
+  if (!flag0 && (flag1 || flag2 || flag3)) return kErrShape;
   if (M < 0 || N < 0 || K < 0) return kErrShape;
   if (mode < EPI_STORE || mode > EPI_SCALE) return kErrShape;
   if (dtype != kF32 && dtype != kF16 && dtype != kBF16) return kErrDType;
@@ -213,6 +232,8 @@ extern "C" int cpt_gemm_any(int dtype, const void* a, int64_t sam, int64_t sak, 
   A.sam = sam; A.sak = sak; A.sbk = sbk; A.sbn = sbn; A.scm = scm; A.scn = scn;
   A.M = M; A.N = N; A.K = K;
   A.alpha = alpha;
+  A.flags[0] = (const int*)flag0; A.flags[1] = (const int*)flag1;
+  A.flags[2] = (const int*)flag2; A.flags[3] = (const int*)flag3;
   // read along the unit-stride dimension (k when both are, or neither is, unit)
   A.a_kfast = (sak == 1 || sam != 1) ? 1 : 0;
   A.b_kfast = (sbk == 1 || sbn != 1) ? 1 : 0;

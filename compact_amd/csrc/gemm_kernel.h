@@ -179,7 +179,21 @@ struct KArgs {
   int sk_q, sk_r;          // iterations per stream-K block: sk_q, +1 for the first sk_r
   float* sk_ws;
   int* sk_flags;
+  // fp32 products from three bf16 planes per operand (gemm16s_kernel.h): the
+  // planes of a[p] / b[p] lie plane_a[p] / plane_b[p] elements apart; the
+  // product is skipped when any of the flags is set
+  int64_t plane_a[2], plane_b[2];
+  const int* flags[4];
 };
+
+// A flag of an operand whose values the planes cannot carry (split_f32_kernel)
+__device__ __forceinline__ bool any_flag(const int* const (&f)[4]) {
+  int v = 0;
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    if (f[i]) v |= *f[i];
+  return v != 0;
+}
 
 // EPI_GLUO: F1 with the outlier channels in its codec (16x16x32 loop only)
 enum Epi { EPI_STORE = 0, EPI_GLU = 1, EPI_DGLU = 2, EPI_ADD = 3, EPI_F32 = 4, EPI_GLUO = 5 };
@@ -1307,8 +1321,12 @@ int launch_nt16(const KArgs& A, hipStream_t st);
 // CACHE_BF16), which st16_reduce sums and finishes.
 template <int DT, bool AK, bool BK, int EPI, int CACHE, int LT, int S>
 int launch_st16(KArgs A, hipStream_t st);
+// fp32 products of bf16 planes on 256 x 256 tiles (gemm16_kernel.h)
+template <bool AK, bool BK>
+int launch_nt16_x3(KArgs A, hipStream_t st);
 // Split sums, adapter terms (`terms` of A's) and epilogue of a split product:
 // plain store to A.C (rows ldo apart) or, dual, the GLU outputs of F1.
+// dt kF32: c = alpha * sum.
 int st16_reduce(int dt, bool dual, const KArgs& A, int terms, int64_t ldo, hipStream_t st);
 
 // ---------------------------------------------------------------------------
@@ -1371,12 +1389,16 @@ int st16_reduce(int dt, bool dual, const KArgs& A, int terms, int64_t ldo, hipSt
   X(DT, true, true, EPI_F32, CACHE_NONE, 0) X(DT, true, false, EPI_F32, CACHE_NONE, 0) \
   X(DT, false, false, EPI_F32, CACHE_NONE, 0) X(DT, false, true, EPI_F32, CACHE_NONE, 0) \
   X(DT, true, true, EPI_F32, CACHE_BF16, 0)
+// fp32 products of three bf16 planes per operand
+#define CPT_ST16_INST_X3(X)                                                  \
+  X(kF32, true, true, EPI_F32, CACHE_NONE, 0) X(kF32, true, false, EPI_F32, CACHE_NONE, 0) \
+  X(kF32, false, false, EPI_F32, CACHE_NONE, 0) X(kF32, false, true, EPI_F32, CACHE_NONE, 0)
 #define CPT_ST16_INST_DGLU(X)                                                \
   X(kBF16, true, false, EPI_DGLU, CACHE_BF16, 0) X(kBF16, true, false, EPI_DGLU, CACHE_BF16, 1)
 #define CPT_ST16_INST_ALL(X)                                                 \
   CPT_ST16_INST_STORE(X, kBF16) CPT_ST16_INST_STORE(X, kF16) CPT_ST16_INST_GLU(X, kBF16) \
   CPT_ST16_INST_GLU(X, kF16) CPT_ST16_INST_F32(X, kBF16) CPT_ST16_INST_F32(X, kF16) \
-  CPT_ST16_INST_DGLU(X)
+  CPT_ST16_INST_DGLU(X) CPT_ST16_INST_X3(X)
 #define CPT_NT16_INST_GLU_A(X)                                               \
   X(true, true, EPI_GLU, CACHE_NONE, 64, 0) X(true, true, EPI_GLU, CACHE_NONE, 64, 2) \
   X(true, true, EPI_GLU, CACHE_BF16, 64, 0) X(true, true, EPI_GLU, CACHE_BF16, 64, 2)

@@ -149,12 +149,17 @@ def _fits16_linear(x, *ws) -> bool:
     return x.shape[0] > 0 and _mfma(x, *ws)
 
 
-def _mm(a, b, name):
-    """a @ b: the 16-bit MFMA GEMMs, or the general-layout kernel for other
-    dtypes and layouts."""
+def _planes(t):
+    """The fp32 operands' planes for one call, None for other types."""
+    return G.Planes() if t.dtype == torch.float32 else None
+
+
+def _mm(a, b, name, planes=None):
+    """a @ b: the 16-bit MFMA GEMMs, fp32 on the bf16 MFMAs (`planes`: those of
+    the call), or the general-layout kernel for other dtypes and layouts."""
     if _fits16(a, b):
         return G.mm(a, b, name)
-    return G.mm_any(a, b, name=name)
+    return G.mm_any(a, b, name=name, planes=planes)
 
 
 # The full fine-tune weight gradients dg^T x and du^T x read x with the token
@@ -169,8 +174,8 @@ def _xt_ok(x, *grads):
             and all(_mfma(g, x) for g in grads))
 
 
-def _linear(x, w, name):
-    return _mm(x, w.t(), name)
+def _linear(x, w, name, planes=None):
+    return _mm(x, w.t(), name, planes)
 
 
 def _addmm(c, a, b, s, name):
@@ -181,14 +186,14 @@ def _addmm(c, a, b, s, name):
     return G.mm_any(a, b, s, G.ANY_ADD, out=c, name=name)
 
 
-def _mm_scaled(a, b, s, name):
+def _mm_scaled(a, b, s, name, planes=None):
     """s * (a @ b) for the thin adapter gradients, which reduce over all
     tokens: the token-reduction kernel, split-K on the bf16 engine, or the
     general-layout kernel."""
     if (_mfma(a, b) and a.shape[1] > 0) or (a.dtype == b.dtype == torch.float16
                                             and G.skinny_t_fits(a, b)):
         return G.mm_splitk(a, b, s, name=name)
-    return G.mm_any(a, b, s, G.ANY_SCALE, name=name)
+    return G.mm_any(a, b, s, G.ANY_SCALE, name=name, planes=planes)
 
 
 def _dual_ok(x, b, p) -> bool:
@@ -202,11 +207,14 @@ def _dual_ok(x, b, p) -> bool:
             and G.skinny_dual_ok(x, b.t(), p))
 
 
-def _mm_sum(a, b, a2, b2, name):
+def _mm_sum(a, b, a2, b2, name, planes=None):
     """a @ b + a2 @ b2: one K-concatenated accumulation on the bf16 engine, or
     the reference's two rounded products and their rounded sum."""
     if _mfma(a, b, a2, b2) or (G.f16_fits(a, b) and G.f16_fits(a2, b2)):
         return G.mm2(a, b, a2, b2, name)
+    if (a.dtype == torch.float32 and G.x3_fits(a, b) and G.x3_fits(a2, b2)
+            and a.stride() == a2.stride() and b.stride() == b2.stride()):
+        return G.mm_x3(a, b, planes or G.Planes(), a2, b2, name=name)
     out = G.mm_any(a, b, name=name)
     return G.mm_any(a2, b2, 1.0, G.ANY_ADD, out=out, name=name)
 
@@ -237,17 +245,17 @@ def outlier_stat_rows(shape) -> int:
     return n
 
 
-def _proj(x_2d, w, a, b, s, name):
+def _proj(x_2d, w, a, b, s, name, planes=None):
     """out = x W^T (+ s * (x A^T) B^T) in PEFT op order (src/flashffn.py:1410-1420).
     Returns (out, xA | None)."""
     if (a is not None and _fits16_linear(x_2d, w) and x_2d.dtype == a.dtype
             and _lora_ok((a, b), dims=((w.shape[1], w.shape[0]),))):
         xa = _mm(x_2d, a.t(), name + "_xa")
         return G.linear_lora(x_2d, w, xa, b, s, name), xa
-    h = _linear(x_2d, w, name)
+    h = _linear(x_2d, w, name, planes)
     xa = None
     if a is not None:
-        xa = _mm(x_2d, a.t(), name + "_xa")
+        xa = _mm(x_2d, a.t(), name + "_xa", planes)
         h = _addmm(h, xa, b.t(), s, name + "_lora")
     return h, xa
 
@@ -309,6 +317,7 @@ class FlashFFNv3Function(torch.autograd.Function):
         x_2d = x.reshape(-1, hidden_dim)
         if not x_2d.is_contiguous():
             x_2d = x_2d.contiguous()
+        planes = _planes(x)
         quant = cache_mode in ("int4", "int8")
         inter = w_gate.shape[0]
         k_out = int(inter * outlier_ratio) if (quant and outlier_ratio > 0) else 0
@@ -378,8 +387,8 @@ class FlashFFNv3Function(torch.autograd.Function):
                 _, h_gate, h_up, *_ = G.ffn_gate_up(x_2d, w_gate, w_up, _lib.CACHE_BF16,
                                                     group_size, want_h_mid=False, **lkw)
             else:
-                h_gate, xa_g = _proj(x_2d, w_gate, a_gate, b_gate, s_gate, "gemm_fwd_gate")
-                h_up, xa_u = _proj(x_2d, w_up, a_up, b_up, s_up, "gemm_fwd_up")
+                h_gate, xa_g = _proj(x_2d, w_gate, a_gate, b_gate, s_gate, "gemm_fwd_gate", planes)
+                h_up, xa_u = _proj(x_2d, w_up, a_up, b_up, s_up, "gemm_fwd_up", planes)
             if k_out > 0:
                 rows = outlier_stat_rows(orig_shape)
                 (slot_gate, _), (slot_up, _) = K.outlier_select_pair(h_gate, h_up, k_out, rows)
@@ -394,7 +403,7 @@ class FlashFFNv3Function(torch.autograd.Function):
             else:
                 h_mid = K.silu_mul(h_gate, h_up)
 
-        y, ha_d = _proj(h_mid, w_down, a_down, b_down, s_down, "gemm_fwd_down")   # :1435-1439
+        y, ha_d = _proj(h_mid, w_down, a_down, b_down, s_down, "gemm_fwd_down", planes)   # :1435-1439
 
         if not fused_quant:                                                # :1442-1451
             if quant and k_out > 0:
@@ -442,6 +451,7 @@ class FlashFFNv3Function(torch.autograd.Function):
         x_2d = x.reshape(-1, hidden_dim)
         if not x_2d.is_contiguous():
             x_2d = x_2d.contiguous()
+        planes = _planes(gy)
 
         need_gate_path = (need_x or need_wg or need_ag or need_bg
                           or need_wu or need_au or need_bu)               # :1488-1489
@@ -474,10 +484,10 @@ class FlashFFNv3Function(torch.autograd.Function):
                     _, hg, hu, *_ = G.ffn_gate_up(x_2d, w_gate, w_up, _lib.CACHE_BF16, gs,
                                                   want_h_mid=False, **lkw)
                 else:
-                    hg = _linear(x_2d, w_gate, "gemm_recompute_gate")
+                    hg = _linear(x_2d, w_gate, "gemm_recompute_gate", planes)
                     if a_gate is not None:
                         hg = _addmm(hg, xa_g, b_gate.t(), s_gate, "gemm_recompute_gate_lora")
-                    hu = _linear(x_2d, w_up, "gemm_recompute_up")
+                    hu = _linear(x_2d, w_up, "gemm_recompute_up", planes)
                     if a_up is not None:
                         hu = _addmm(hu, xa_u, b_up.t(), s_up, "gemm_recompute_up_lora")
             elif mode == "bf16":
@@ -498,7 +508,7 @@ class FlashFFNv3Function(torch.autograd.Function):
                 gyB_d, grad_b_down = G.skinny_dual(gy, b_down.t(), ha_d, 1.0, s_down,
                                                    name="gemm_gyB_grad_b_down")
             else:
-                gyB_d = _mm(gy, b_down, "gemm_gyB_down")                  # :1521
+                gyB_d = _mm(gy, b_down, "gemm_gyB_down", planes)                  # :1521
 
         # the down projection's LoRA term of grad_h_mid (:1527-1529) rides in
         # the dgrad GEMM's epilogue
@@ -525,7 +535,7 @@ class FlashFFNv3Function(torch.autograd.Function):
                     grad_h_mid = G.mm2(gy, w_down, name="gemm_dgrad_down", lora=[
                         (gyB_d, a_down, s_down)])
                 else:
-                    grad_h_mid = _mm(gy, w_down, "gemm_dgrad_down")
+                    grad_h_mid = _mm(gy, w_down, "gemm_dgrad_down", planes)
                     if a_down is not None:
                         grad_h_mid = _addmm(grad_h_mid, gyB_d, a_down, s_down,
                                             "gemm_dgrad_down_lora")
@@ -555,12 +565,12 @@ class FlashFFNv3Function(torch.autograd.Function):
                 grad_w_down = G.wgrad_glu(gy, _CACHE_CODE[mode], gs, c_gate, qs_gate, c_up, qs_up,
                                           name="gemm_wgrad_down")
             elif need_wd:
-                grad_w_down = _mm(gy.t(), h_mid_hat, "gemm_wgrad_down")
+                grad_w_down = _mm(gy.t(), h_mid_hat, "gemm_wgrad_down", planes)
             if need_ad:
-                grad_a_down = _mm_scaled(gyB_d.t(), h_mid_hat, s_down, "gemm_grad_a_down")
+                grad_a_down = _mm_scaled(gyB_d.t(), h_mid_hat, s_down, "gemm_grad_a_down", planes)
             del h_mid_hat
         if need_bd and grad_b_down is None:
-            grad_b_down = _mm_scaled(gy.t(), ha_d, s_down, "gemm_grad_b_down")   # :1545
+            grad_b_down = _mm_scaled(gy.t(), ha_d, s_down, "gemm_grad_b_down", planes)   # :1545
 
         grad_x = None
         grad_w_gate = grad_a_gate = grad_b_gate = None
@@ -598,13 +608,13 @@ class FlashFFNv3Function(torch.autograd.Function):
                         ghgB, grad_b_gate = G.skinny_dual(grad_h_gate, b_gate.t(), xa_g, 1.0,
                                                           s_gate, name="gemm_ghgB_grad_b_gate")
                     else:
-                        ghgB = _mm(grad_h_gate, b_gate, "gemm_ghgB")
+                        ghgB = _mm(grad_h_gate, b_gate, "gemm_ghgB", planes)
                 if a_up is not None and (need_x or need_au):
                     if need_bu and _dual_ok(grad_h_up, b_up, xa_u):
                         ghuB, grad_b_up = G.skinny_dual(grad_h_up, b_up.t(), xa_u, 1.0, s_up,
                                                         name="gemm_ghuB_grad_b_up")
                     else:
-                        ghuB = _mm(grad_h_up, b_up, "gemm_ghuB")
+                        ghuB = _mm(grad_h_up, b_up, "gemm_ghuB", planes)
             if need_x:
                 xl = [(ghgB, a_gate, s_gate) if a_gate is not None else None,
                       (ghuB, a_up, s_up) if a_up is not None else None]
@@ -616,25 +626,25 @@ class FlashFFNv3Function(torch.autograd.Function):
                     grad_x = G.mm2(grad_h_gate, w_gate, grad_h_up, w_up, "gemm_dgrad_x",
                                    lora=[t for t in xl if t is not None] or None)
                 else:
-                    grad_x = _mm_sum(grad_h_gate, w_gate, grad_h_up, w_up, "gemm_dgrad_x")
+                    grad_x = _mm_sum(grad_h_gate, w_gate, grad_h_up, w_up, "gemm_dgrad_x", planes)
                     if a_gate is not None:
                         grad_x = _addmm(grad_x, ghgB, a_gate, s_gate, "gemm_dgrad_x_lora_gate")
                     if a_up is not None:
                         grad_x = _addmm(grad_x, ghuB, a_up, s_up, "gemm_dgrad_x_lora_up")
             if need_bg and grad_b_gate is None:
-                grad_b_gate = _mm_scaled(grad_h_gate.t(), xa_g, s_gate, "gemm_grad_b_gate")
+                grad_b_gate = _mm_scaled(grad_h_gate.t(), xa_g, s_gate, "gemm_grad_b_gate", planes)
             if ghB is not None and need_ag and need_au and s_gate == s_up:
                 # s [dg B_g | du B_u]^T x: its row halves equal the two
                 # reductions bit for bit (same token order per row)
-                ga = _mm_scaled(ghB.t(), x_2d, s_gate, "gemm_grad_a_gate_up")
+                ga = _mm_scaled(ghB.t(), x_2d, s_gate, "gemm_grad_a_gate_up", planes)
                 grad_a_gate, grad_a_up = ga[:ghgB.shape[1]], ga[ghgB.shape[1]:]
             else:
                 if need_ag:
-                    grad_a_gate = _mm_scaled(ghgB.t(), x_2d, s_gate, "gemm_grad_a_gate")
+                    grad_a_gate = _mm_scaled(ghgB.t(), x_2d, s_gate, "gemm_grad_a_gate", planes)
                 if need_au:
-                    grad_a_up = _mm_scaled(ghuB.t(), x_2d, s_up, "gemm_grad_a_up")
+                    grad_a_up = _mm_scaled(ghuB.t(), x_2d, s_up, "gemm_grad_a_up", planes)
             if need_bu and grad_b_up is None:
-                grad_b_up = _mm_scaled(grad_h_up.t(), xa_u, s_up, "gemm_grad_b_up")
+                grad_b_up = _mm_scaled(grad_h_up.t(), xa_u, s_up, "gemm_grad_b_up", planes)
             if need_wg and need_wu and _xt_ok(x_2d, grad_h_gate, grad_h_up):
                 # x^T once, so both products read it K-major (bit-identical)
                 x_t = G.transpose(x_2d, "transpose_x").t()
@@ -643,9 +653,9 @@ class FlashFFNv3Function(torch.autograd.Function):
                 x_t = None
             else:
                 if need_wg:
-                    grad_w_gate = _mm(grad_h_gate.t(), x_2d, "gemm_wgrad_gate")
+                    grad_w_gate = _mm(grad_h_gate.t(), x_2d, "gemm_wgrad_gate", planes)
                 if need_wu:
-                    grad_w_up = _mm(grad_h_up.t(), x_2d, "gemm_wgrad_up")
+                    grad_w_up = _mm(grad_h_up.t(), x_2d, "gemm_wgrad_up", planes)
 
         # frozen weights => no dense [D_out, D_in] gradient was built (:1589-1593)
         if not (need_wg or need_wu or need_wd):
@@ -905,6 +915,7 @@ class FlashFFNv3AdapterFunction(torch.autograd.Function):
         x_2d = x.reshape(-1, hidden_dim)
         if not x_2d.is_contiguous():
             x_2d = x_2d.contiguous()
+        planes = _planes(x)
         quant = cache_mode in ("int4", "int8")
         plain_gu = a_gate is None and a_up is None and m_gate is None and m_up is None
         fusable = plain_gu and _mfma(x_2d, w_gate, w_up) and x_2d.shape[0] > 0
@@ -930,9 +941,9 @@ class FlashFFNv3AdapterFunction(torch.autograd.Function):
             h_mid, h_gate, h_up, *_ = G.ffn_gate_up(
                 x_2d, w_gate, w_up, _lib.CACHE_BF16 if keep else _lib.CACHE_NONE, group_size)
         else:
-            h_gate, xa_g = _proj(x_2d, w_gate, a_gate, b_gate, s_gate, "gemm_fwd_gate")
+            h_gate, xa_g = _proj(x_2d, w_gate, a_gate, b_gate, s_gate, "gemm_fwd_gate", planes)
             h_gate = _scaled(h_gate, m_gate, nu_gate, inplace=True)          # :1967
-            h_up, xa_u = _proj(x_2d, w_up, a_up, b_up, s_up, "gemm_fwd_up")
+            h_up, xa_u = _proj(x_2d, w_up, a_up, b_up, s_up, "gemm_fwd_up", planes)
             h_up = _scaled(h_up, m_up, nu_up, inplace=True)                   # :1975
             if fused_quant:
                 h_mid, c_gate, qs_gate, c_up, qs_up = K.silu_mul_quant(
@@ -941,7 +952,7 @@ class FlashFFNv3AdapterFunction(torch.autograd.Function):
             else:
                 h_mid = K.silu_mul(h_gate, h_up)
 
-        y, ha_d = _proj(h_mid, w_down, a_down, b_down, s_down, "gemm_fwd_down")   # :1990-1994
+        y, ha_d = _proj(h_mid, w_down, a_down, b_down, s_down, "gemm_fwd_down", planes)   # :1990-1994
         y = _scaled(y, m_down, nu_down, inplace=True)                              # :1996
 
         if not fused_quant:                                                         # :1998-2007
@@ -988,6 +999,7 @@ class FlashFFNv3AdapterFunction(torch.autograd.Function):
         x_2d = x.reshape(-1, hidden_dim)
         if not x_2d.is_contiguous():
             x_2d = x_2d.contiguous()
+        planes = _planes(gy)
 
         need_gate_path = (need_x or need_wg or need_ag or need_bg or need_mg
                           or need_wu or need_au or need_bu or need_mu)          # :2047-2048
@@ -1007,11 +1019,11 @@ class FlashFFNv3AdapterFunction(torch.autograd.Function):
                     _, hg, hu, *_ = G.ffn_gate_up(x_2d, w_gate, w_up, _lib.CACHE_BF16, gs,
                                                   want_h_mid=False, **lkw)
                 else:
-                    raw_g = _linear(x_2d, w_gate, "gemm_recompute_gate")
+                    raw_g = _linear(x_2d, w_gate, "gemm_recompute_gate", planes)
                     if a_gate is not None:
                         raw_g = _addmm(raw_g, xa_g, b_gate.t(), s_gate, "gemm_recompute_gate_lora")
                     hg = _scaled(raw_g, m_gate, nu_gate)
-                    raw_u = _linear(x_2d, w_up, "gemm_recompute_up")
+                    raw_u = _linear(x_2d, w_up, "gemm_recompute_up", planes)
                     if a_up is not None:
                         raw_u = _addmm(raw_u, xa_u, b_up.t(), s_up, "gemm_recompute_up_lora")
                     hu = _scaled(raw_u, m_up, nu_up)
@@ -1030,7 +1042,7 @@ class FlashFFNv3AdapterFunction(torch.autograd.Function):
         g_eff_y = _scaled(gy, m_down, nu_down)                                  # :2094
         gyB_d = None
         if a_down is not None and (need_gate_path or need_ad):
-            gyB_d = _mm(g_eff_y, b_down, "gemm_gyB_down")
+            gyB_d = _mm(g_eff_y, b_down, "gemm_gyB_down", planes)
         fusable_d = a_down is None and _mfma(g_eff_y, w_down) and g_eff_y.shape[0] > 0
 
         # the SwiGLU backward may write over h_gate / h_up when they are this
@@ -1050,7 +1062,7 @@ class FlashFFNv3AdapterFunction(torch.autograd.Function):
                     g_eff_y, w_down, _lib.CACHE_BF16, gs, hg, None, hu, None, need_h_mid,
                     inplace=own)
             else:
-                grad_h_mid = _mm(g_eff_y, w_down, "gemm_dgrad_down")
+                grad_h_mid = _mm(g_eff_y, w_down, "gemm_dgrad_down", planes)
                 if a_down is not None:
                     grad_h_mid = _addmm(grad_h_mid, gyB_d, a_down, s_down, "gemm_dgrad_down_lora")
                 if use_k2:
@@ -1068,19 +1080,19 @@ class FlashFFNv3AdapterFunction(torch.autograd.Function):
             if h_mid_hat is None:
                 h_mid_hat = K.silu_mul(hg, hu)
             if need_wd:
-                grad_w_down = _mm(g_eff_y.t(), h_mid_hat, "gemm_wgrad_down")
+                grad_w_down = _mm(g_eff_y.t(), h_mid_hat, "gemm_wgrad_down", planes)
             if need_ad:
-                grad_a_down = _mm_scaled(gyB_d.t(), h_mid_hat, s_down, "gemm_grad_a_down")
+                grad_a_down = _mm_scaled(gyB_d.t(), h_mid_hat, s_down, "gemm_grad_a_down", planes)
             if need_md:
                 # raw_d is never stored: one extra GEMM recomputes it
-                raw_d, _ = _proj(h_mid_hat, w_down, None, None, 0.0, "gemm_recompute_down")
+                raw_d, _ = _proj(h_mid_hat, w_down, None, None, 0.0, "gemm_recompute_down", planes)
                 if a_down is not None:
                     raw_d = _addmm(raw_d, ha_d, b_down.t(), s_down, "gemm_recompute_down_lora")
                 grad_m_down = K.col_dot_div(gy, raw_d, nu_down)
                 del raw_d
             del h_mid_hat
         if need_bd:
-            grad_b_down = _mm_scaled(g_eff_y.t(), ha_d, s_down, "gemm_grad_b_down")
+            grad_b_down = _mm_scaled(g_eff_y.t(), ha_d, s_down, "gemm_grad_b_down", planes)
 
         grad_x = None
         grad_w_gate = grad_a_gate = grad_b_gate = grad_m_gate = None
@@ -1097,28 +1109,28 @@ class FlashFFNv3AdapterFunction(torch.autograd.Function):
             g_eff_u = _scaled(grad_h_up, m_up, nu_up, inplace=True)
             ghgB = None
             if a_gate is not None and (need_x or need_ag):
-                ghgB = _mm(g_eff_g, b_gate, "gemm_ghgB")
+                ghgB = _mm(g_eff_g, b_gate, "gemm_ghgB", planes)
             ghuB = None
             if a_up is not None and (need_x or need_au):
-                ghuB = _mm(g_eff_u, b_up, "gemm_ghuB")
+                ghuB = _mm(g_eff_u, b_up, "gemm_ghuB", planes)
             if need_x:
-                grad_x = _mm_sum(g_eff_g, w_gate, g_eff_u, w_up, "gemm_dgrad_x")
+                grad_x = _mm_sum(g_eff_g, w_gate, g_eff_u, w_up, "gemm_dgrad_x", planes)
                 if a_gate is not None:
                     grad_x = _addmm(grad_x, ghgB, a_gate, s_gate, "gemm_dgrad_x_lora_gate")
                 if a_up is not None:
                     grad_x = _addmm(grad_x, ghuB, a_up, s_up, "gemm_dgrad_x_lora_up")
             if need_bg:
-                grad_b_gate = _mm_scaled(g_eff_g.t(), xa_g, s_gate, "gemm_grad_b_gate")
+                grad_b_gate = _mm_scaled(g_eff_g.t(), xa_g, s_gate, "gemm_grad_b_gate", planes)
             if need_ag:
-                grad_a_gate = _mm_scaled(ghgB.t(), x_2d, s_gate, "gemm_grad_a_gate")
+                grad_a_gate = _mm_scaled(ghgB.t(), x_2d, s_gate, "gemm_grad_a_gate", planes)
             if need_bu:
-                grad_b_up = _mm_scaled(g_eff_u.t(), xa_u, s_up, "gemm_grad_b_up")
+                grad_b_up = _mm_scaled(g_eff_u.t(), xa_u, s_up, "gemm_grad_b_up", planes)
             if need_au:
-                grad_a_up = _mm_scaled(ghuB.t(), x_2d, s_up, "gemm_grad_a_up")
+                grad_a_up = _mm_scaled(ghuB.t(), x_2d, s_up, "gemm_grad_a_up", planes)
             if need_wg:
-                grad_w_gate = _mm(g_eff_g.t(), x_2d, "gemm_wgrad_gate")
+                grad_w_gate = _mm(g_eff_g.t(), x_2d, "gemm_wgrad_gate", planes)
             if need_wu:
-                grad_w_up = _mm(g_eff_u.t(), x_2d, "gemm_wgrad_up")
+                grad_w_up = _mm(g_eff_u.t(), x_2d, "gemm_wgrad_up", planes)
 
         # frozen weights => no dense [D_out, D_in] gradient was built (:2194-2197)
         if not (need_wg or need_wu or need_wd):

@@ -910,16 +910,157 @@ def mm_splitk(a: torch.Tensor, b: torch.Tensor, alpha: float = 1.0, splits: int 
     return c if ldc == N else c[:, :N]
 
 
+# ---------------------------------------------------------------------------
+# fp32 products on the bf16 MFMAs (cpt_split_f32, cpt_gemm_f32x3)
+# ---------------------------------------------------------------------------
+
+class Planes:
+    """The bf16 planes of the fp32 operands of one forward or backward call.
+
+    Each operand is split once, however many of the call's products read it,
+    whatever view of it they take.  An instance lives for one call and holds its
+    operands, so no other tensor can take their memory meanwhile; an operand
+    must not be written between its products."""
+
+    MAX_FLAGS = 32
+
+    def __init__(self):
+        self._made = {}
+        self._flags = None
+
+    def of(self, t: torch.Tensor):
+        """(planes bf16 [3, rows, cols], flag int32 [1]) of row-major fp32 t."""
+        key = (t.data_ptr(), t.shape, t.stride(0))
+        hit = self._made.get(key)
+        if hit is None:
+            if self._flags is None:
+                self._flags = torch.zeros((self.MAX_FLAGS,), dtype=torch.int32, device=t.device)
+            i = len(self._made)
+            assert i < self.MAX_FLAGS
+            flag = self._flags[i:i + 1]
+            planes = torch.empty((3,) + tuple(t.shape), dtype=torch.bfloat16, device=t.device)
+            with _timed("split_f32"):
+                rc = _lib.lib().cpt_split_f32(t.data_ptr(), t.stride(0), t.shape[0], t.shape[1],
+                                              planes.data_ptr(), flag.data_ptr(), _stream(t))
+            check(rc, "split_f32")
+            hit = self._made[key] = (planes, flag, t)
+        return hit[0], hit[1]
+
+
+def _x3_operand(t: torch.Tensor):
+    """(row-major storage of t or of its transpose, whether it is t), or None
+    where the split kernel does not take it."""
+    if t.stride(1) == 1 and t.stride(0) >= t.shape[1]:
+        s, own = t, True
+    elif t.stride(0) == 1 and t.stride(1) >= t.shape[0]:
+        s, own = t.t(), False
+    else:
+        return None
+    if s.stride(0) % 4 or s.shape[1] % 8 or s.data_ptr() % 16:
+        return None
+    return s, own
+
+
+def x3_fits(a: torch.Tensor, b: torch.Tensor) -> bool:
+    """a [M, K] @ b [K, N] in fp32 runs on the bf16 MFMAs (mm_x3): row-major or
+    transposed operands with 16-byte aligned rows of whole 8-element vectors, N a
+    multiple of 8, K of 64 unless both operands are stored k by k."""
+    if not (a.dtype == b.dtype == torch.float32 and a.dim() == 2 and b.dim() == 2 and a.is_cuda):
+        return False
+    (M, K), N = a.shape, b.shape[1]
+    if M == 0 or K == 0 or N == 0 or N % 8:
+        return False
+    oa, ob = _x3_operand(a), _x3_operand(b)
+    if oa is None or ob is None:
+        return False
+    rows = (K + 256) * 2
+    if (not oa[1] and rows * M >= _SPAN_BYTES) or (ob[1] and rows * N >= _SPAN_BYTES):
+        return False
+    return K % 64 == 0 or (not oa[1] and ob[1])
+
+
+def x3_plan(m: int, n: int, nk: int, whole: bool) -> tuple[int, int]:
+    """(tile edge, k ranges) of an fp32 product of nk k-tiles of plane pairs; 256
+    x 256 tiles need whole k-tiles.  Times per k-tile with the chip full: 1.33 us
+    a 256 x 256 tile, 0.57 a 128 x 128 one, so the rounds of blocks decide."""
+    small = split_plan(m, n, nk)
+    t128 = ((m + 127) // 128) * ((n + 127) // 128) * small
+    t256 = ((m + 255) // 256) * ((n + 255) // 256)
+    big = max(1, min(256 // t256, nk // SPLIT_MIN_KT))
+    cost128 = 0.57 * min(-(-t128 // 256), 1.9 * -(-t128 // 512)) * nk / small
+    cost256 = 1.33 * -(-t256 * big // 256) * nk / big
+    return (256, big) if whole and cost256 < cost128 else (128, small)
+
+
+def mm_x3(a, b, planes: Planes, a2=None, b2=None, alpha: float = 1.0,
+          name: str = "gemm_f32") -> torch.Tensor:
+    """alpha * (a @ b (+ a2 @ b2)) in fp32 from the operands' bf16 planes
+    (x3_fits each pair, the pairs in one layout), and, on the device and only if
+    a value lies outside the planes' range, again on the general-layout kernel.
+
+    Three times closer to float64 than the general-layout kernel and about
+    twice as fast, splitting included (x3_gemm_impl in csrc/gemm.hip)."""
+    _require_device(a, b)
+    (M, K), N = a.shape, b.shape[1]
+
+    def operand(t, left):
+        s, own = _x3_operand(t)
+        p, flag = planes.of(s)
+        # [M][K] or [N][K] storage is K-major
+        return p.data_ptr(), s.shape[0] * s.shape[1], s.shape[1], int(own == left), flag.data_ptr()
+    pa, sa, lda, ak, fa = operand(a, True)
+    pb, sb, ldb, bk, fb = operand(b, False)
+    pa2 = pb2 = fa2 = fb2 = None
+    sa2 = sb2 = K2 = 0
+    if a2 is not None:
+        K2 = a2.shape[1]
+        pa2, sa2, lda2, ak2, fa2 = operand(a2, True)
+        pb2, sb2, ldb2, bk2, fb2 = operand(b2, False)
+        assert (lda2, ldb2, ak2, bk2) == (lda, ldb, ak, bk), "the pairs share one layout"
+    c = torch.empty((M, N), dtype=torch.float32, device=a.device)
+    tiles, splits = x3_plan(M, N, 6 * ((K + 63) // 64 + (K2 + 63) // 64),
+                            K % 64 == 0 and K2 % 64 == 0)
+    ws = (torch.empty((splits * M * N,), dtype=torch.float32, device=a.device)
+          if splits > 1 else None)
+    st = _stream(a)
+    L = _lib.lib()
+    with _timed(name):
+        rc = L.cpt_gemm_f32x3(pa, sa, lda, ak, pb, sb, ldb, bk, pa2, sa2, pb2, sb2, K2, fa, fb,
+                              fa2, fb2, c.data_ptr(), N, M, N, K, float(alpha), tiles, splits,
+                              None if ws is None else ws.data_ptr(), st)
+        check(rc, name)
+        for i, (u, v) in enumerate(((a, b), (a2, b2))[:1 if a2 is None else 2]):
+            rc = L.cpt_gemm_any_if(fa, fb, fa2, fb2, _lib.F32, u.data_ptr(), u.stride(0),
+                                   u.stride(1), v.data_ptr(), v.stride(0), v.stride(1),
+                                   c.data_ptr(), N, 1, M, N, u.shape[1], float(alpha),
+                                   ANY_ADD if i else ANY_SCALE, st)
+            check(rc, name)
+    return c
+
+
 # epilogues of the general-layout GEMM (cpt_gemm_any)
 ANY_STORE, ANY_ADD, ANY_SCALE = 0, 1, 2
 _ANY_DT = {torch.float32: _lib.F32, torch.float16: _lib.F16, torch.bfloat16: _lib.BF16}
 
 
 def mm_any(a: torch.Tensor, b: torch.Tensor, alpha: float = 1.0, mode: int = ANY_STORE,
-           out: torch.Tensor | None = None, name: str = "gemm_any") -> torch.Tensor:
+           out: torch.Tensor | None = None, name: str = "gemm_any",
+           planes: Planes | None = None) -> torch.Tensor:
     """a [M, K] @ b [K, N] for float32 / float16 / bfloat16 operands of any
-    strides, on the fp32 MFMA (cpt_gemm_any): the products the bf16 engine
-    does not take (config C1's float32, unaligned views, rank-1 factors).
+    strides, in the modes of mm_any_kernel: the products the bf16 engine does
+    not take (config C1's float32, unaligned views, rank-1 factors).  fp32
+    operands that fit (x3_fits) go to the bf16 MFMAs, sharing the planes that
+    the caller's other products made."""
+    if mode != ANY_ADD and a.dtype == torch.float32 and x3_fits(a, b):
+        return mm_x3(a, b, planes or Planes(), alpha=alpha if mode == ANY_SCALE else 1.0,
+                     name=name)
+    return mm_any_kernel(a, b, alpha, mode, out, name)
+
+
+def mm_any_kernel(a: torch.Tensor, b: torch.Tensor, alpha: float = 1.0, mode: int = ANY_STORE,
+                  out: torch.Tensor | None = None, name: str = "gemm_any") -> torch.Tensor:
+    """a [M, K] @ b [K, N] on the general-layout kernel, the fp32 MFMA
+    (cpt_gemm_any).
     mode ANY_STORE: rd(a @ b); ANY_SCALE: rd(alpha * rd(a @ b)); ANY_ADD: in
     place, out = rd(out + rd(alpha * rd(a @ b))), with rd the rounding to the
     operands' dtype (the reference's eager op order)."""

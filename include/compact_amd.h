@@ -336,6 +336,29 @@ int cpt_gemm16(int dtype, const void* a, int64_t lda, int a_kmajor, const void* 
                float alpha0, const void* p1, const void* q1, float alpha1, int splits,
                void* workspace, void* stream);
 
+/* fp32 products on the bf16 MFMAs.  cpt_split_f32 writes x [rows, cols] (rows ld
+ * apart, cols a multiple of 8, 16-byte aligned) as three bf16 planes
+ * [3][rows][cols] that sum to it to 24 bits, and sets the zeroed int *flag if a
+ * value is outside the range where they do (not finite, above 2^55, below 2^-100
+ * and not 0).  cpt_gemm_f32x3 writes c = alpha * (a . b + a2 . b2) from such
+ * planes (plane_* elements apart, layouts, K and N as in cpt_gemm16, both pairs
+ * with one lda and ldb, a2 NULL for one pair) unless one of the flags is set;
+ * tiles is 128, or 256 where K and K2 are multiples of 64; splits > 1 needs splits * M * N floats of workspace.  cpt_gemm_any_if is
+ * cpt_gemm_any run only if one of its flags is set (all NULL: always): the fp32
+ * product for the operands the planes cannot carry. */
+int cpt_split_f32(const void* x, int64_t ld, int64_t rows, int64_t cols, void* planes, void* flag,
+                  void* stream);
+int cpt_gemm_f32x3(const void* a, int64_t plane_a, int64_t lda, int a_kmajor, const void* b,
+                   int64_t plane_b, int64_t ldb, int b_kmajor, const void* a2, int64_t plane_a2,
+                   const void* b2, int64_t plane_b2, int64_t K2, const void* flag_a,
+                   const void* flag_b, const void* flag_a2, const void* flag_b2, void* c,
+                   int64_t ldc, int64_t M, int64_t N, int64_t K, float alpha, int tiles,
+                   int splits, void* workspace, void* stream);
+int cpt_gemm_any_if(const void* flag0, const void* flag1, const void* flag2, const void* flag3,
+                    int dtype, const void* a, int64_t sam, int64_t sak, const void* b, int64_t sbk,
+                    int64_t sbn, void* c, int64_t scm, int64_t scn, int64_t M, int64_t N,
+                    int64_t K, float alpha, int mode, void* stream);
+
 /* cpt_ffn_gate_up_lora without a codec (h_gate and h_up both given or both
  * NULL, h_mid NULL or given; rank 0: no adapter terms) for bf16 or fp16, hidden
  * a multiple of 64.  splits as in cpt_gemm16, with splits * n_tok * 2 * inter
