@@ -1,4 +1,5 @@
-"""ctypes binding of libcompact_amd.so (the C ABI in include/compact_amd.h).
+"""Bindings of libcompact_amd.so (the C ABI in include/compact_amd.h): ctypes for
+every entry point (lib()), a CPython extension for those a step calls (api()).
 
 The library is built in-tree by `python -m compact_amd.build` into
 compact_amd/_build/libcompact_amd.so.  There is no fallback: if the library is
@@ -8,10 +9,13 @@ missing, `lib()` raises, and so does every operator that needs it.
 from __future__ import annotations
 
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "_build", "libcompact_amd.so")
+CAPI_PATH = os.path.join(_HERE, "_build", "_capi.so")
 
 F32, F16, BF16 = 0, 1, 2
 
@@ -127,6 +131,26 @@ def lib():
     L.cpt_abi_version.restype = ctypes.c_int
     _lib = L
     return _lib
+
+
+_api = None
+
+
+def api():
+    """The same entry points through the CPython binding (_build/_capi.so, built
+    with the library): what every step calls.  Loaded once; raises as lib()."""
+    global _api
+    if _api is None:
+        lib()
+        if not os.path.exists(CAPI_PATH):
+            raise LibraryMissing(f"{CAPI_PATH} not found: build it with "
+                                 "`python -m compact_amd.build`")
+        loader = importlib.machinery.ExtensionFileLoader("_capi", CAPI_PATH)
+        spec = importlib.util.spec_from_file_location("_capi", CAPI_PATH, loader=loader)
+        mod = importlib.util.module_from_spec(spec)
+        loader.exec_module(mod)
+        _api = mod
+    return _api
 
 
 # status codes (include/compact_amd.h)

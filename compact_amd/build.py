@@ -16,12 +16,14 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
 CSRC = os.path.join(HERE, "csrc")
 OUT_DIR = os.path.join(HERE, "_build")
 LIB = os.path.join(OUT_DIR, "libcompact_amd.so")
+CAPI = os.path.join(OUT_DIR, "_capi.so")
 ARCH = os.environ.get("CPT_OFFLOAD_ARCH", "gfx950")
 
 COMMON = [
@@ -53,17 +55,31 @@ def _compile(src: str) -> str:
     return obj
 
 
+def _build_capi() -> None:
+    """The CPython binding (csrc/capi.cpp), linked to the library beside it."""
+    tmp = CAPI + ".tmp"
+    cmd = [shutil.which("g++") or "c++", "-O2", "-std=c++17", "-shared", "-fPIC", "-Wall",
+           f"-I{sysconfig.get_paths()['include']}", f"-I{os.path.join(ROOT, 'include')}",
+           os.path.join(CSRC, "capi.cpp"), "-o", tmp, LIB, "-Wl,-rpath,$ORIGIN"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"binding failed:\n{' '.join(cmd)}\n{r.stdout}\n{r.stderr}")
+    os.replace(tmp, CAPI)
+
+
 def build(verbose: bool = False) -> str:
     os.makedirs(OUT_DIR, exist_ok=True)
     srcs = sorted(os.path.join(CSRC, f) for f in os.listdir(CSRC) if f.endswith(".hip"))
     with cf.ThreadPoolExecutor(max_workers=min(8, len(srcs))) as ex:
         objs = list(ex.map(_compile, srcs))
     tmp = LIB + ".tmp"
-    cmd = [hipcc(), "-shared", "-fPIC", f"--offload-arch={ARCH}", "-o", tmp] + objs
+    cmd = [hipcc(), "-shared", "-fPIC", f"--offload-arch={ARCH}", "-Wl,-soname,libcompact_amd.so",
+           "-o", tmp] + objs
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError(f"link failed:\n{' '.join(cmd)}\n{r.stdout}\n{r.stderr}")
     os.replace(tmp, LIB)
+    _build_capi()
     if verbose:
         print(f"built {LIB}")
     return LIB

@@ -125,10 +125,10 @@ def _mfma(*ts) -> bool:
             continue
         if t.dtype != torch.bfloat16 or t.dim() != 2 or t.data_ptr() % 16:
             return False
-        rows, cols = t.shape
-        if t.stride(1) == 1 and cols % 8 == 0 and t.stride(0) % 8 == 0:
+        (rows, cols), (s0, s1) = t.shape, t.stride()
+        if s1 == 1 and cols % 8 == 0 and s0 % 8 == 0:
             continue
-        if t.stride(0) == 1 and rows % 8 == 0 and t.stride(1) % 8 == 0:
+        if s0 == 1 and rows % 8 == 0 and s1 % 8 == 0:
             continue
         return False
     return True
@@ -685,8 +685,31 @@ _FAMILY_NAME = {"dora": "DoRA", "adalora": "AdaLoRA", "vera": "VeRA", "dylora": 
                 "lora": "LoRA"}
 
 
+def _attr(m, name: str, default=None):
+    """getattr(m, name, default) that looks a Module's own tables up first and
+    raises nothing on a miss (an adapter wrapper is searched for a dozen names
+    on every call, most of them absent)."""
+    d = getattr(m, "__dict__", None)
+    if d is not None and isinstance(m, nn.Module):
+        for table in ("_modules", "_parameters", "_buffers"):
+            t = d.get(table)
+            if t and name in t:
+                return t[name]
+        if name not in d and not hasattr(type(m), name) and \
+                type(m).__getattr__ is nn.Module.__getattr__:
+            return default
+    return getattr(m, name, default)
+
+
+_MISSING = object()
+
+
+def _has(m, name: str) -> bool:
+    return _attr(m, name, _MISSING) is not _MISSING
+
+
 def _holds_entries(proj: nn.Module, attr: str) -> bool:
-    v = getattr(proj, attr, None)
+    v = _attr(proj, attr)
     return v is not None and len(v) > 0
 
 
@@ -695,11 +718,10 @@ _WRAPPER_TESTS = (
     ("adalora", lambda p: _holds_entries(p, "lora_E")),
     ("vera", lambda p: _holds_entries(p, "vera_lambda_d")),
     # DyLoRA keeps its factors as bare Parameters with a rank bound r
-    ("dylora", lambda p: all(isinstance(getattr(p, a, None), nn.Parameter)
-                             for a in ("lora_A", "lora_B"))
-     and hasattr(p, "r") and hasattr(p, "scaling")),
-    ("lora", lambda p: isinstance(getattr(p, "lora_A", None), nn.ModuleDict)
-     and len(p.lora_A) > 0),
+    ("dylora", lambda p: isinstance(_attr(p, "lora_A"), nn.Parameter)
+     and isinstance(_attr(p, "lora_B"), nn.Parameter) and _has(p, "r") and _has(p, "scaling")),
+    ("lora", lambda p: isinstance(_attr(p, "lora_A"), nn.ModuleDict)
+     and len(_attr(p, "lora_A")) > 0),
 )
 
 
@@ -707,8 +729,8 @@ def _v3_proj_kind(proj: nn.Module) -> str:
     """Structural classification of one MLP projection (src/flashffn.py:
     1798-1821): 'dora' | 'adalora' | 'vera' | 'dylora' | 'lora' | 'plain' |
     'unknown'."""
-    if not hasattr(proj, "base_layer"):
-        return "plain" if hasattr(proj, "weight") else "unknown"
+    if not _has(proj, "base_layer"):
+        return "plain" if _has(proj, "weight") else "unknown"
     for kind, test in _WRAPPER_TESTS:
         if test(proj):
             return kind
@@ -723,7 +745,7 @@ def _active_adapter(proj: nn.Module) -> str:
 
 def _warn_dropout(family: str, drop: nn.Module):
     """The fused path applies no adapter dropout: say so when it is on."""
-    p = float(getattr(drop, "p", 0.0))
+    p = float(_attr(drop, "p", 0.0))
     if p > 0.0:
         warnings.warn(f"FlashFFNv3 ignores {family} dropout (p={p}); results differ from the "
                       f"reference forward when training with dropout.")
@@ -732,9 +754,9 @@ def _warn_dropout(family: str, drop: nn.Module):
 def _lora_factors(proj: nn.Module, family: str = "LoRA"):
     """(W, A, B, s) of a PEFT LoRA-style wrapper's active adapter."""
     name = _active_adapter(proj)
-    _warn_dropout(family, proj.lora_dropout[name])
-    return (proj.get_base_layer().weight, proj.lora_A[name].weight, proj.lora_B[name].weight,
-            float(proj.scaling[name]))
+    _warn_dropout(family, _attr(proj, "lora_dropout")[name])
+    return (_attr(proj.get_base_layer(), "weight"), _attr(_attr(proj, "lora_A")[name], "weight"),
+            _attr(_attr(proj, "lora_B")[name], "weight"), float(proj.scaling[name]))
 
 
 def _v3_extract_proj(proj: nn.Module):

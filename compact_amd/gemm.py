@@ -145,6 +145,30 @@ def lora_fusable(rank: int, *dims) -> bool:
                                                 for k, n in dims))
 
 
+def _lora_args_whole(terms, n_q, r):
+    """_lora_args' result where the terms can be used as they are (a rank of
+    whole 8-wide chunks, aligned rows, one layout for both), else None."""
+    if r % 8:
+        return None
+    out = []
+    ldp = ldq = q_km = None
+    for pm, q, al in terms:
+        sp, sq = pm.stride(), q.stride()
+        km = sq[0] == 1 and sq[1] == r
+        if ((ldp is not None and (sp[0] != ldp or km != q_km or (not km and sq[0] != ldq)))
+                or sp[1] != 1 or sp[0] % 8 or pm.dtype not in _DT16 or q.dtype != pm.dtype
+                or pm.shape[1] != r or tuple(q.shape) != (r, n_q)):
+            return None
+        pp, qp = pm.data_ptr(), q.data_ptr()
+        if pp % 16 or (qp % 16 if km else sq[1] != 1):
+            return None
+        ldp, q_km, ldq = sp[0], km, r if km else sq[0]
+        out.append((pp, qp, float(al)))
+    if len(out) == 1:
+        out.append((None, None, 0.0))
+    return r, ldp, int(q_km), ldq, out, terms
+
+
 def _lora_args(terms, n_q, dims):
     """(rank, ldp, q_kmajor, ldq, [(p, q, alpha) x 2], keep) for up to two
     terms (p [M, r], q the logical [r, N] factor, alpha) of a GEMM with the
@@ -156,6 +180,9 @@ def _lora_args(terms, n_q, dims):
     terms = [t for t in terms if t is not None]
     assert 1 <= len(terms) <= 2
     r = terms[0][0].shape[1]
+    fast = _lora_args_whole(terms, n_q, r)
+    if fast is not None and lora_fusable(r, *dims):
+        return fast
     assert lora_fusable(r, *dims), \
         f"adapter rank {r} not carried by a GEMM of (k, n) {tuple(dims)} (lora_fusable)"
     if r % 8:
@@ -242,7 +269,7 @@ def skinny(a: torch.Tensor, q: torch.Tensor, alpha: float = 1.0,
     ws = (torch.empty((splits * M * R,), dtype=torch.float32, device=a.device)
           if splits > 1 else None)
     with _timed(name):
-        rc = _lib.lib().cpt_gemm16_skinny(dt, a.data_ptr(), a.stride(0), q.data_ptr(),
+        rc = _lib.api().cpt_gemm16_skinny(dt, a.data_ptr(), a.stride(0), q.data_ptr(),
                                           q.stride(0), c.data_ptr(), c.stride(0), M, R, K,
                                           float(alpha), splits,
                                           None if ws is None else ws.data_ptr(), _stream(a))
@@ -276,7 +303,7 @@ def skinny_t(x: torch.Tensor, p: torch.Tensor, alpha: float = 1.0, trans: bool =
     out = torch.empty((R, N) if trans else (N, R), dtype=x.dtype, device=x.device)
     ws = torch.empty((splits * N * R,), dtype=torch.float32, device=x.device)
     with _timed(name):
-        rc = _lib.lib().cpt_gemm16_skinny_t(dt, x.data_ptr(), x.stride(0), p.data_ptr(),
+        rc = _lib.api().cpt_gemm16_skinny_t(dt, x.data_ptr(), x.stride(0), p.data_ptr(),
                                             p.stride(0), out.data_ptr(), out.stride(0),
                                             1 if trans else 0, T, N, R, float(alpha), splits,
                                             ws.data_ptr(), _stream(x))
@@ -308,7 +335,7 @@ def transpose(x: torch.Tensor, name: str = "transpose") -> torch.Tensor:
     rows, cols = x.shape
     out = torch.empty((cols, rows), dtype=x.dtype, device=x.device)
     with _timed(name):
-        rc = _lib.lib().cpt_transpose_bf16(x.data_ptr(), x.stride(0), rows, cols, out.data_ptr(),
+        rc = _lib.api().cpt_transpose_bf16(x.data_ptr(), x.stride(0), rows, cols, out.data_ptr(),
                                            out.stride(0), _stream(x))
     check(rc, name)
     return out
@@ -361,10 +388,10 @@ def skinny_dual(x: torch.Tensor, q: torch.Tensor, p: torch.Tensor, alpha_c: floa
         assert (tuple(c.shape) == (T, R) and c.dtype == x.dtype and c.stride(1) == 1
                 and c.stride(0) % 8 == 0 and c.data_ptr() % 16 == 0), "skinny_dual out layout"
     z = torch.empty((N, R), dtype=x.dtype, device=x.device)
-    nbytes = int(_lib.lib().cpt_gemm_bf16_skinny_dual_workspace_bytes(T, N, R, splits))
+    nbytes = _lib.api().cpt_gemm_bf16_skinny_dual_workspace_bytes(T, N, R, splits)
     ws = torch.empty((max(nbytes, 4) // 4,), dtype=torch.float32, device=x.device)
     with _timed(name):
-        rc = _lib.lib().cpt_gemm16_skinny_dual(
+        rc = _lib.api().cpt_gemm16_skinny_dual(
             _DT16[x.dtype], x.data_ptr(), x.stride(0), q.data_ptr(), ldq, q_nr, p.data_ptr(), p.stride(0),
             c.data_ptr(), c.stride(0), float(alpha_c), z.data_ptr(), z.stride(0), 0,
             float(alpha_z), T, N, R, splits, ws.data_ptr(), _stream(x))
@@ -575,7 +602,7 @@ def mm2(a, b, a2=None, b2=None, name: str = "gemm", lora=None) -> torch.Tensor:
         ws = (torch.empty((splits * M * N,), dtype=torch.float32, device=a.device)
               if splits > 1 else None)
         with _timed(name):
-            rc = _lib.lib().cpt_gemm16(
+            rc = _lib.api().cpt_gemm16(
                 dt, a.data_ptr(), lda, ak, b.data_ptr(), ldb, bk, p_a2, lda2, p_b2, ldb2,
                 K2, c.data_ptr(), ldc, M, N, K, r, ldp, qk, ldq, t[0][0], t[0][1], t[0][2],
                 t[1][0], t[1][1], t[1][2], splits, None if ws is None else ws.data_ptr(),
@@ -585,12 +612,12 @@ def mm2(a, b, a2=None, b2=None, name: str = "gemm", lora=None) -> torch.Tensor:
     _stream_k(a.device)
     with _timed(name):
         if lora:
-            rc = _lib.lib().cpt_gemm_bf16_lora(
+            rc = _lib.api().cpt_gemm_bf16_lora(
                 a.data_ptr(), lda, ak, b.data_ptr(), ldb, bk, p_a2, lda2, p_b2, ldb2, K2,
                 c.data_ptr(), ldc, M, N, K, r, ldp, qk, ldq, t[0][0], t[0][1], t[0][2],
                 t[1][0], t[1][1], t[1][2], _stream(a))
         else:
-            rc = _lib.lib().cpt_gemm_bf16(a.data_ptr(), lda, ak, b.data_ptr(), ldb, bk, p_a2,
+            rc = _lib.api().cpt_gemm_bf16(a.data_ptr(), lda, ak, b.data_ptr(), ldb, bk, p_a2,
                                           lda2, p_b2, ldb2, K2, c.data_ptr(), ldc, M, N, K,
                                           _stream(a))
     check(rc, name)
@@ -614,7 +641,7 @@ def mm_engine(a: torch.Tensor, b: torch.Tensor, name: str = "gemm_engine") -> to
     ldc = (N + 7) // 8 * 8
     c = torch.empty((M, ldc), dtype=torch.bfloat16, device=a.device)
     with _timed(name):
-        rc = _lib.lib().cpt_gemm_bf16_ex(a.data_ptr(), lda, ak, b.data_ptr(), ldb, bk, c.data_ptr(),
+        rc = _lib.api().cpt_gemm_bf16_ex(a.data_ptr(), lda, ak, b.data_ptr(), ldb, bk, c.data_ptr(),
                                          ldc, M, N, K, 1.0, 0, 1, None, _stream(a))
     check(rc, name)
     return c if ldc == N else c[:, :N]
@@ -681,17 +708,17 @@ def ffn_gate_up(x, w_gate, w_up, cache: int, group_size: int, want_h_mid: bool =
         if splits > 1 or half:
             ws = (torch.empty((splits * n * 2 * d,), dtype=torch.float32, device=dev)
                   if splits > 1 else None)
-            rc = _lib.lib().cpt_ffn_gate_up16(
+            rc = _lib.api().cpt_ffn_gate_up16(
                 dt, x.data_ptr(), w_gate.data_ptr(), w_up.data_ptr(), n, hdim, d,
                 p(h_mid), p(hg), p(hu), r, ldp, t[0][0], t[0][1], t[0][2], t[1][0], t[1][1],
                 t[1][2], splits, None if ws is None else ws.data_ptr(), _stream(x))
         elif r:
-            rc = _lib.lib().cpt_ffn_gate_up_lora(
+            rc = _lib.api().cpt_ffn_gate_up_lora(
                 x.data_ptr(), w_gate.data_ptr(), w_up.data_ptr(), n, hdim, d, cache, group_size,
                 p(h_mid), p(hg), p(hu), p(qg), p(sg), p(qu), p(su), r, ldp, t[0][0], t[0][1],
                 t[0][2], t[1][0], t[1][1], t[1][2], _stream(x))
         else:
-            rc = _lib.lib().cpt_ffn_gate_up(x.data_ptr(), w_gate.data_ptr(), w_up.data_ptr(), n,
+            rc = _lib.api().cpt_ffn_gate_up(x.data_ptr(), w_gate.data_ptr(), w_up.data_ptr(), n,
                                             hdim, d, cache, group_size, p(h_mid), p(hg), p(hu),
                                             p(qg), p(sg), p(qu), p(su), _stream(x))
     check(rc, "ffn_gate_up")
@@ -804,14 +831,14 @@ def ffn_down_dgrad(grad_y, w_down, cache: int, group_size: int, c_gate, s_gate, 
         r, ldp, qk, ldq, t, keep = _lora_args([(gyb, a_down, s)], d, ((hdim, d),))
         assert qk == 0 and ldq == d
         with _timed("ffn_down_dgrad"):
-            rc = _lib.lib().cpt_ffn_down_dgrad_lora(
+            rc = _lib.api().cpt_ffn_down_dgrad_lora(
                 grad_y.data_ptr(), w_down.data_ptr(), n, hdim, d, cache, group_size, p(c_gate),
                 p(s_gate), p(c_up), p(s_up), dg.data_ptr(), du.data_ptr(), p(hm), r, ldp,
                 t[0][0], t[0][1], t[0][2], _stream(grad_y))
         del keep
     else:
         with _timed("ffn_down_dgrad"):
-            rc = _lib.lib().cpt_ffn_down_dgrad(grad_y.data_ptr(), w_down.data_ptr(), n, hdim, d,
+            rc = _lib.api().cpt_ffn_down_dgrad(grad_y.data_ptr(), w_down.data_ptr(), n, hdim, d,
                                                cache, group_size, p(c_gate), p(s_gate), p(c_up),
                                                p(s_up), dg.data_ptr(), du.data_ptr(), p(hm),
                                                _stream(grad_y))
@@ -860,7 +887,7 @@ def addmm_(c: torch.Tensor, a: torch.Tensor, b: torch.Tensor, alpha: float,
     a, lda, ak = _layout_a(a)
     b, ldb, bk = _layout_b(b)
     with _timed(name):
-        rc = _lib.lib().cpt_gemm_bf16_ex(a.data_ptr(), lda, ak, b.data_ptr(), ldb, bk, c.data_ptr(),
+        rc = _lib.api().cpt_gemm_bf16_ex(a.data_ptr(), lda, ak, b.data_ptr(), ldb, bk, c.data_ptr(),
                                          c.stride(0), M, N, K, float(alpha), 1, 1, None, _stream(a))
     check(rc, name)
     return c
@@ -903,7 +930,7 @@ def mm_splitk(a: torch.Tensor, b: torch.Tensor, alpha: float = 1.0, splits: int 
     c = torch.empty((M, ldc), dtype=torch.bfloat16, device=a.device)
     ws = torch.empty((splits * M * N,), dtype=torch.float32, device=a.device)
     with _timed(name):
-        rc = _lib.lib().cpt_gemm_bf16_ex(a.data_ptr(), lda, ak, b.data_ptr(), ldb, bk, c.data_ptr(),
+        rc = _lib.api().cpt_gemm_bf16_ex(a.data_ptr(), lda, ak, b.data_ptr(), ldb, bk, c.data_ptr(),
                                          ldc, M, N, K, float(alpha), 2, splits, ws.data_ptr(),
                                          _stream(a))
     check(rc, name)
@@ -940,7 +967,7 @@ class Planes:
             flag = self._flags[i:i + 1]
             planes = torch.empty((3,) + tuple(t.shape), dtype=torch.bfloat16, device=t.device)
             with _timed("split_f32"):
-                rc = _lib.lib().cpt_split_f32(t.data_ptr(), t.stride(0), t.shape[0], t.shape[1],
+                rc = _lib.api().cpt_split_f32(t.data_ptr(), t.stride(0), t.shape[0], t.shape[1],
                                               planes.data_ptr(), flag.data_ptr(), _stream(t))
             check(rc, "split_f32")
             hit = self._made[key] = (planes, flag, t)
@@ -1023,7 +1050,7 @@ def mm_x3(a, b, planes: Planes, a2=None, b2=None, alpha: float = 1.0,
     ws = (torch.empty((splits * M * N,), dtype=torch.float32, device=a.device)
           if splits > 1 else None)
     st = _stream(a)
-    L = _lib.lib()
+    L = _lib.api()
     with _timed(name):
         rc = L.cpt_gemm_f32x3(pa, sa, lda, ak, pb, sb, ldb, bk, pa2, sa2, pb2, sb2, K2, fa, fb,
                               fa2, fb2, c.data_ptr(), N, M, N, K, float(alpha), tiles, splits,
@@ -1075,7 +1102,7 @@ def mm_any_kernel(a: torch.Tensor, b: torch.Tensor, alpha: float = 1.0, mode: in
     else:
         out = torch.empty((M, N), dtype=a.dtype, device=a.device)
     with _timed(name):
-        rc = _lib.lib().cpt_gemm_any(_ANY_DT[a.dtype], a.data_ptr(), a.stride(0), a.stride(1),
+        rc = _lib.api().cpt_gemm_any(_ANY_DT[a.dtype], a.data_ptr(), a.stride(0), a.stride(1),
                                      b.data_ptr(), b.stride(0), b.stride(1), out.data_ptr(),
                                      out.stride(0), out.stride(1), M, N, K, float(alpha), mode,
                                      _stream(a))

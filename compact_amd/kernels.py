@@ -32,7 +32,14 @@ def v3_reset_counters():
         _V3_COUNTERS[k] = 0
 
 
+# the raw handle of a device's current stream, without a Stream object around
+# it (0.2 us against 3)
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _stream(t: torch.Tensor):
+    if _raw_stream is not None:
+        return _raw_stream(t.get_device())
     return torch.cuda.current_stream(t.device).cuda_stream
 
 
@@ -62,25 +69,41 @@ class KernelTimer:
         return out
 
 
-class _timed:
+class _Timed:
     __slots__ = ("name", "ev")
 
     def __init__(self, name):
         self.name = name
-        self.ev = None
+        self.ev = torch.cuda.Event(enable_timing=True)
 
     def __enter__(self):
-        if KernelTimer.active is not None:
-            self.ev = torch.cuda.Event(enable_timing=True)
-            self.ev.record(torch.cuda.current_stream())
+        self.ev.record(torch.cuda.current_stream())
         return self
 
     def __exit__(self, *exc):
         kt = KernelTimer.active
-        if self.ev is not None and kt is not None:
+        if kt is not None:
             end = torch.cuda.Event(enable_timing=True)
             end.record(torch.cuda.current_stream())
             kt.events.setdefault(self.name, []).append((self.ev, end))
+
+
+class _Untimed:
+    __slots__ = ()
+
+    def __enter__(self):
+        return self
+
+    def __exit__(self, *exc):
+        return None
+
+
+_UNTIMED = _Untimed()
+
+
+def _timed(name):
+    """Times the launches inside it under `name` while a KernelTimer is active."""
+    return _UNTIMED if KernelTimer.active is None else _Timed(name)
 
 
 def _ptr(t):
@@ -110,7 +133,7 @@ def silu_mul(h_gate: torch.Tensor, h_up: torch.Tensor) -> torch.Tensor:
     assert h_up.shape == h_gate.shape and h_up.dtype == h_gate.dtype
     h_gate, h_up = h_gate.contiguous(), h_up.contiguous()
     out = torch.empty_like(h_gate)
-    check(_lib.lib().cpt_silu_mul(h_gate.data_ptr(), h_up.data_ptr(), out.data_ptr(),
+    check(_lib.api().cpt_silu_mul(h_gate.data_ptr(), h_up.data_ptr(), out.data_ptr(),
                                   h_gate.numel(), _dtype_code(h_gate), _stream(h_gate)),
           "silu_mul")
     return out
@@ -125,7 +148,7 @@ def swiglu_backward(grad_h_mid, h_gate, h_up):
     grad_h_mid, h_gate, h_up = grad_h_mid.contiguous(), h_gate.contiguous(), h_up.contiguous()
     dg = torch.empty_like(h_gate)
     du = torch.empty_like(h_up)
-    check(_lib.lib().cpt_swiglu_backward(grad_h_mid.data_ptr(), h_gate.data_ptr(),
+    check(_lib.api().cpt_swiglu_backward(grad_h_mid.data_ptr(), h_gate.data_ptr(),
                                          h_up.data_ptr(), dg.data_ptr(), du.data_ptr(),
                                          h_gate.numel(), _dtype_code(h_gate), _stream(h_gate)),
           "swiglu_backward")
@@ -150,7 +173,7 @@ def swiglu_backward_glu(grad_h_mid, h_gate, h_up, want_h_mid, inplace=False):
         dg = torch.empty_like(h_gate)
         du = torch.empty_like(h_up)
         hm = torch.empty_like(h_gate) if want_h_mid else None
-    check(_lib.lib().cpt_swiglu_backward_glu(grad_h_mid.data_ptr(), h_gate.data_ptr(),
+    check(_lib.api().cpt_swiglu_backward_glu(grad_h_mid.data_ptr(), h_gate.data_ptr(),
                                              h_up.data_ptr(), dg.data_ptr(), du.data_ptr(),
                                              _ptr(hm), h_gate.numel(), _dtype_code(h_gate),
                                              _stream(h_gate)),
@@ -177,7 +200,7 @@ def v3_quantize_group_absmax(t: torch.Tensor, bits: int, group_size: int = 64):
     else:
         payload = torch.empty((n, d), dtype=torch.int8, device=t.device)
     scales = torch.empty((n, g), dtype=torch.float16, device=t.device)
-    check(_lib.lib().cpt_v3_quantize_group_absmax(t.data_ptr(), _dtype_code(t), n, d, bits,
+    check(_lib.api().cpt_v3_quantize_group_absmax(t.data_ptr(), _dtype_code(t), n, d, bits,
                                                   group_size, payload.data_ptr(),
                                                   scales.data_ptr(), _stream(t)),
           "v3_quantize_group_absmax")
@@ -195,7 +218,7 @@ def v3_dequantize_group_absmax(payload, scales, bits, group_size=64, dtype=torch
     assert tuple(scales.shape) == (n, d // group_size) and scales.dtype == torch.float16
     payload, scales = payload.contiguous(), scales.contiguous()
     out = torch.empty((n, d), dtype=dtype, device=payload.device)
-    check(_lib.lib().cpt_v3_dequantize_group_absmax(payload.data_ptr(), scales.data_ptr(), n, d,
+    check(_lib.api().cpt_v3_dequantize_group_absmax(payload.data_ptr(), scales.data_ptr(), n, d,
                                                     bits, group_size, out.data_ptr(),
                                                     _DT[dtype], _stream(payload)),
           "v3_dequantize_group_absmax")
@@ -232,7 +255,7 @@ def silu_mul_quant(h_gate, h_up, bits, group_size=64):
         q_gate = torch.empty((n, d), dtype=torch.int8, device=dev)
         q_up = torch.empty((n, d), dtype=torch.int8, device=dev)
     with _timed("silu_mul_quant"):
-        rc = _lib.lib().cpt_silu_mul_quant(h_gate.data_ptr(), h_up.data_ptr(), n, d, bits,
+        rc = _lib.api().cpt_silu_mul_quant(h_gate.data_ptr(), h_up.data_ptr(), n, d, bits,
                                            group_size, h_mid.data_ptr(), q_gate.data_ptr(),
                                            s_gate.data_ptr(), q_up.data_ptr(), s_up.data_ptr(),
                                            _stream(h_gate))
@@ -267,7 +290,7 @@ def dequant_swiglu_backward(grad_h_mid, q_gate, s_gate, q_up, s_up, bits, group_
     grad_h_up = torch.empty_like(grad_h_mid)
     h_mid_hat = torch.empty_like(grad_h_mid) if want_h_mid else None
     with _timed("dequant_swiglu_backward"):
-        rc = _lib.lib().cpt_dequant_swiglu_backward(
+        rc = _lib.api().cpt_dequant_swiglu_backward(
             grad_h_mid.data_ptr(), q_gate.data_ptr(), s_gate.data_ptr(), q_up.data_ptr(),
             s_up.data_ptr(), n, d, bits, group_size, grad_h_gate.data_ptr(),
             grad_h_up.data_ptr(), _ptr(h_mid_hat), _stream(grad_h_mid))
@@ -350,7 +373,7 @@ def outlier_select_pair(t0: torch.Tensor, t1: torch.Tensor, k: int, rows: int | 
     sumsq = torch.empty((2, d), dtype=torch.float64, device=dev)
     slot = torch.empty((2, d), dtype=torch.int16, device=dev)
     idx = torch.empty((2, max(k, 1)), dtype=torch.int32, device=dev)
-    check(_lib.lib().cpt_outlier_select_pair(
+    check(_lib.api().cpt_outlier_select_pair(
         t0.data_ptr(), t1.data_ptr(), _dtype_code(t0), n, d, k, partial.data_ptr(),
         sumsq.data_ptr(), slot[0].data_ptr(), idx[0].data_ptr(), slot[1].data_ptr(),
         idx[1].data_ptr(), _stream(t0)), "outlier_select_pair")
@@ -418,7 +441,7 @@ def silu_mul_quant_outlier(h_gate, h_up, bits, group_size, slot_gate, slot_up, k
         su = torch.empty((n, g), dtype=torch.float16, device=dev)
         og, ou = _outlier_buf(n, k, dev), _outlier_buf(n, k, dev)
     with _timed("silu_mul_quant_outlier"):
-        rc = _lib.lib().cpt_silu_mul_quant_outlier(
+        rc = _lib.api().cpt_silu_mul_quant_outlier(
             h_gate.data_ptr(), h_up.data_ptr(), n, d, bits, group_size, slot_gate.data_ptr(),
             slot_up.data_ptr(), k, h_mid.data_ptr(), qg.data_ptr(), sg.data_ptr(), og.data_ptr(),
             qu.data_ptr(), su.data_ptr(), ou.data_ptr(), _stream(h_gate))
@@ -440,7 +463,7 @@ def dequant_swiglu_backward_outlier(grad_h_mid, q_gate, s_gate, o_gate, slot_gat
     hm = torch.empty_like(grad_h_mid) if want_h_mid else None
     k = o_gate.shape[1]
     with _timed("dequant_swiglu_backward_outlier"):
-        rc = _lib.lib().cpt_dequant_swiglu_backward_outlier(
+        rc = _lib.api().cpt_dequant_swiglu_backward_outlier(
             grad_h_mid.data_ptr(), q_gate.data_ptr(), s_gate.data_ptr(), slot_gate.data_ptr(),
             o_gate.data_ptr(), q_up.data_ptr(), s_up.data_ptr(), slot_up.data_ptr(),
             o_up.data_ptr(), k, n, d, bits, group_size, dg.data_ptr(), du.data_ptr(), _ptr(hm),
@@ -468,7 +491,7 @@ def dora_scale(x: torch.Tensor, m: torch.Tensor, nu: torch.Tensor, out=None) -> 
     assert out.is_contiguous() and out.shape == x.shape and out.dtype == x.dtype
     n, d = x.shape
     with _timed("dora_scale"):
-        rc = _lib.lib().cpt_dora_scale(x.data_ptr(), m.data_ptr(), nu.data_ptr(), n, d,
+        rc = _lib.api().cpt_dora_scale(x.data_ptr(), m.data_ptr(), nu.data_ptr(), n, d,
                                        _dtype_code(x), out.data_ptr(), _stream(x))
     check(rc, "dora_scale")
     return out
@@ -482,7 +505,7 @@ def col_dot_div(a: torch.Tensor, b: torch.Tensor, den: torch.Tensor) -> torch.Te
     assert a.dtype == b.dtype == den.dtype, "col_dot_div: one dtype expected"
     a, b, den = a.contiguous(), b.contiguous(), den.contiguous()
     n, d = a.shape
-    L = _lib.lib()
+    L = _lib.api()
     ws = torch.empty((max(1, L.cpt_col_dot_workspace_bytes(n, d)) + 3) // 4,
                      dtype=torch.float32, device=a.device)
     out = torch.empty((d,), dtype=a.dtype, device=a.device)
@@ -506,7 +529,7 @@ def dora_col_norm(w: torch.Tensor, a: torch.Tensor, b: torch.Tensor, s: float,
         f"dora_col_norm: w {tuple(w.shape)}, a {tuple(a.shape)}, b {tuple(b.shape)}"
     assert w.dtype == a.dtype == b.dtype, "dora_col_norm: one dtype expected"
     w, a, b = w.contiguous(), a.contiguous(), b.contiguous()
-    L = _lib.lib()
+    L = _lib.api()
     ws = torch.empty((L.cpt_dora_col_norm_workspace_bytes(rows, r) + 3) // 4 + 1,
                      dtype=torch.float32, device=w.device)
     nu = torch.empty((rows,), dtype=out_dtype, device=w.device)
@@ -535,7 +558,7 @@ def topk_abs(t: torch.Tensor, k: int):
     values = torch.empty((n, k), dtype=t.dtype, device=t.device)
     indices = torch.empty((n, k), dtype=torch.int16, device=t.device)
     with _timed("topk_abs"):
-        rc = _lib.lib().cpt_topk_abs(t.data_ptr(), _dtype_code(t), n, d, k, values.data_ptr(),
+        rc = _lib.api().cpt_topk_abs(t.data_ptr(), _dtype_code(t), n, d, k, values.data_ptr(),
                                      indices.data_ptr(), _stream(t))
     check(rc, "topk_abs")
     return values, indices
@@ -550,7 +573,7 @@ def topk_scatter(values: torch.Tensor, indices: torch.Tensor, d: int) -> torch.T
     n, k = values.shape
     out = torch.empty((n, d), dtype=values.dtype, device=values.device)
     with _timed("topk_scatter"):
-        rc = _lib.lib().cpt_topk_scatter(values.data_ptr(), indices.data_ptr(),
+        rc = _lib.api().cpt_topk_scatter(values.data_ptr(), indices.data_ptr(),
                                          _dtype_code(values), n, d, k, out.data_ptr(),
                                          _stream(values))
     check(rc, "topk_scatter")
