@@ -79,6 +79,8 @@ SIGNATURES = {
                                    _L, _P, _P, _P, _L, _L, _P, _P, ctypes.c_float, _P],
     "cpt_dora_scale": [_P, _P, _P, _L, _L, _I, _P, _P],
     "cpt_col_dot_div": [_P, _P, _P, _L, _L, _I, _P, _P, _P],
+    "cpt_col_dot_div_rows": [_P, _P, _P, _L, _L, _L, _I, _P, _P, _P],
+    "cpt_dora_col_norm16": [_P, _P, _P, _L, _L, _L, ctypes.c_double, _I, _P, _P, _I, _P],
     "cpt_dora_col_norm": [_P, _P, _P, _L, _L, _L, ctypes.c_double, _I, _P, _P, _I, _P],
     "cpt_topk_abs": [_P, _I, _L, _L, _L, _P, _P, _P],
     "cpt_topk_scatter": [_P, _P, _I, _L, _L, _L, _P, _P],
@@ -92,6 +94,7 @@ SIGNATURES = {
 SIZE_QUERIES = {
     "cpt_col_dot_workspace_bytes": [_L, _L],
     "cpt_dora_col_norm_workspace_bytes": [_L, _L],
+    "cpt_dora_col_norm16_workspace_bytes": [_L, _L, _L],
     "cpt_gemm_stream_k_bytes": [],
     "cpt_gemm_bf16_skinny_dual_workspace_bytes": [_L, _L, _L, _I],
 }

@@ -84,10 +84,11 @@ PyMethodDef methods[] = {
     CPT_ENTRY(cpt_ffn_down_dgrad_lora),
     CPT_ENTRY(cpt_transpose_bf16),
     CPT_ENTRY(cpt_dora_scale),
-    CPT_ENTRY(cpt_col_dot_div),
-    CPT_ENTRY(cpt_col_dot_workspace_bytes),
+    CPT_ENTRY(cpt_col_dot_div_rows),
     CPT_ENTRY(cpt_dora_col_norm),
     CPT_ENTRY(cpt_dora_col_norm_workspace_bytes),
+    CPT_ENTRY(cpt_dora_col_norm16),
+    CPT_ENTRY(cpt_dora_col_norm16_workspace_bytes),
     CPT_ENTRY(cpt_topk_abs),
     CPT_ENTRY(cpt_topk_scatter),
     {nullptr, nullptr, 0, nullptr}};

@@ -279,9 +279,94 @@ def _gate_up_lora(x_2d, a_gate, b_gate, s_gate, a_up, b_up, s_up):
     else:
         xa_g = _mm(x_2d, a_gate.t(), "gemm_fwd_gate_xa") if a_gate is not None else None
         xa_u = _mm(x_2d, a_up.t(), "gemm_fwd_up_xa") if a_up is not None else None
-    kw = dict(lora_gate=None if a_gate is None else (xa_g, b_gate, s_gate),
-              lora_up=None if a_up is None else (xa_u, b_up, s_up))
-    return xa_g, xa_u, kw
+    return xa_g, xa_u, _gate_up_terms(a_gate, b_gate, s_gate, xa_g, a_up, b_up, s_up, xa_u)
+
+
+def _gate_up_terms(a_gate, b_gate, s_gate, xa_g, a_up, b_up, s_up, xa_u):
+    """G.ffn_gate_up's keyword terms; a B factor goes in as rows of its ranks."""
+    def rows(b):
+        return b if b.stride(1) == 1 else b.contiguous()
+    return dict(lora_gate=None if a_gate is None else (xa_g, rows(b_gate), s_gate),
+                lora_up=None if a_up is None else (xa_u, rows(b_up), s_up))
+
+
+def _gate_up_ok(x_2d, w_gate, a_gate, b_gate, w_up, a_up, b_up, dims) -> bool:
+    """The gate and up products run as one dual product on the 16-bit kernels,
+    the adapter terms in its epilogue."""
+    return (_fits16_linear(x_2d, w_gate, w_up)
+            and _lora_ok((a_gate, b_gate), (a_up, b_up), dims=dims)
+            and all(t is None or t.dtype == x_2d.dtype for t in (a_gate, a_up)))
+
+
+def _thin_backward(grad_h_gate, b_gate, xa_g, s_gate, grad_h_up, b_up, xa_u, s_up, need_g, need_u,
+                   need_bg, need_bu, planes):
+    """The rank-sized products of the gate / up gradients: dg B_g where `need_g`
+    (the gate adapter is there and grad_x or grad A_g is asked for), du B_u where
+    `need_u`, and with them in one pass the B gradients (:1556-1557 with
+    :1575-1582) where the dual kernel takes them.  Returns (ghgB | None, ghuB |
+    None, both side by side [N, r_g + r_u] | None, grad_b_gate | None,
+    grad_b_up | None)."""
+    grad_b_gate = grad_b_up = None
+    ghgB = ghuB = ghB = None
+    # dg B_g and du B_u side by side in one [N, r_g + r_u] buffer, so
+    # one token reduction over x gives both A gradients below
+    stack = (_stackable(b_gate.t() if b_gate is not None else None,
+                        b_up.t() if b_up is not None else None)
+             and (need_g or need_u) and grad_h_gate.shape[0] >= 256
+             and (_mfma(grad_h_gate, b_gate, grad_h_up, b_up)
+                  or (G.f16_fits(grad_h_gate, b_gate) and G.f16_fits(grad_h_up, b_up)))
+             and grad_h_gate.shape[1] >= 256)
+    if stack:
+        r = b_gate.shape[1]
+        ghB = torch.empty((grad_h_gate.shape[0], r + b_up.shape[1]),
+                          dtype=grad_h_gate.dtype, device=grad_h_gate.device)
+        # with the B gradient, both products of grad_h in one pass
+        # (:1556-1557 with :1575-1582)
+        if need_bg and _dual_ok(grad_h_gate, b_gate, xa_g):
+            _, grad_b_gate = G.skinny_dual(grad_h_gate, b_gate.t(), xa_g, 1.0, s_gate,
+                                           out_c=ghB[:, :r], name="gemm_ghgB_grad_b_gate")
+        else:
+            G.skinny(grad_h_gate, b_gate.t(), 1.0, "gemm_ghgB", out=ghB[:, :r])
+        if need_bu and _dual_ok(grad_h_up, b_up, xa_u):
+            _, grad_b_up = G.skinny_dual(grad_h_up, b_up.t(), xa_u, 1.0, s_up,
+                                         out_c=ghB[:, r:], name="gemm_ghuB_grad_b_up")
+        else:
+            G.skinny(grad_h_up, b_up.t(), 1.0, "gemm_ghuB", out=ghB[:, r:])
+        ghgB, ghuB = ghB[:, :r], ghB[:, r:]
+    else:
+        if need_g:
+            if need_bg and _dual_ok(grad_h_gate, b_gate, xa_g):
+                ghgB, grad_b_gate = G.skinny_dual(grad_h_gate, b_gate.t(), xa_g, 1.0,
+                                                  s_gate, name="gemm_ghgB_grad_b_gate")
+            else:
+                ghgB = _mm(grad_h_gate, b_gate, "gemm_ghgB", planes)
+        if need_u:
+            if need_bu and _dual_ok(grad_h_up, b_up, xa_u):
+                ghuB, grad_b_up = G.skinny_dual(grad_h_up, b_up.t(), xa_u, 1.0, s_up,
+                                                name="gemm_ghuB_grad_b_up")
+            else:
+                ghuB = _mm(grad_h_up, b_up, "gemm_ghuB", planes)
+    return ghgB, ghuB, ghB, grad_b_gate, grad_b_up
+
+
+def _grad_x(grad_h_gate, w_gate, a_gate, s_gate, ghgB, grad_h_up, w_up, a_up, s_up, ghuB, fusable,
+            planes):
+    """dg W_g + du W_u, then the adapter terms (:1558-1566)."""
+    xl = [(ghgB, a_gate, s_gate) if a_gate is not None else None,
+          (ghuB, a_up, s_up) if a_up is not None else None]
+    if fusable and (_mfma(grad_h_gate, w_gate, grad_h_up, w_up)
+                    or (G.f16_fits(grad_h_gate, w_gate) and G.f16_fits(grad_h_up, w_up))):
+        # dg @ W_g + du @ W_u as one K-concatenated GEMM, the gate and up
+        # LoRA terms (:1561-1566) in its epilogue
+        grad_x = G.mm2(grad_h_gate, w_gate, grad_h_up, w_up, "gemm_dgrad_x",
+                       lora=[t for t in xl if t is not None] or None)
+    else:
+        grad_x = _mm_sum(grad_h_gate, w_gate, grad_h_up, w_up, "gemm_dgrad_x", planes)
+        if a_gate is not None:
+            grad_x = _addmm(grad_x, ghgB, a_gate, s_gate, "gemm_dgrad_x_lora_gate")
+        if a_up is not None:
+            grad_x = _addmm(grad_x, ghuB, a_up, s_up, "gemm_dgrad_x_lora_up")
+    return grad_x
 
 
 class FlashFFNv3Function(torch.autograd.Function):
@@ -323,9 +408,8 @@ class FlashFFNv3Function(torch.autograd.Function):
         k_out = int(inter * outlier_ratio) if (quant and outlier_ratio > 0) else 0
         assert k_out == 0 or x.dtype == torch.bfloat16, "outlier channels need bf16 activations"
         # the dual gate/up kernel, with the gate/up LoRA terms in its epilogue
-        fusable = (_fits16_linear(x_2d, w_gate, w_up)
-                   and _lora_ok((a_gate, b_gate), (a_up, b_up), dims=((hidden_dim, inter),))
-                   and all(t is None or t.dtype == x.dtype for t in (a_gate, a_up)))
+        fusable = _gate_up_ok(x_2d, w_gate, a_gate, b_gate, w_up, a_up, b_up,
+                              ((hidden_dim, inter),))
 
         c_gate = qs_gate = c_up = qs_up = None
         o_gate = o_up = slot_gate = slot_up = None
@@ -469,18 +553,15 @@ class FlashFFNv3Function(torch.autograd.Function):
         fusable = _mfma(gy, w_down) and lora_d and gy.shape[0] > 0 and (use_k2 or not outl)
         # F1's recompute (k d_model) and the K-concatenated grad_x product (k d_ff)
         d_ff, d_model = w_gate.shape
-        fusable_gu = (_fits16_linear(x_2d, w_gate, w_up)
-                      and _lora_ok((a_gate, b_gate), (a_up, b_up),
-                                   dims=((d_model, d_ff), (d_ff, d_model)))
-                      and all(t is None or t.dtype == x.dtype for t in (a_gate, a_up)))
+        fusable_gu = _gate_up_ok(x_2d, w_gate, a_gate, b_gate, w_up, a_up, b_up,
+                                 ((d_model, d_ff), (d_ff, d_model)))
 
         hg = hu = None
         if need_recon and not use_k2:                                     # :1500-1516
             if mode == "recompute":
                 if fusable_gu:
                     # the forward's kernel and terms on the same inputs: bitwise equal
-                    lkw = dict(lora_gate=None if a_gate is None else (xa_g, b_gate, s_gate),
-                               lora_up=None if a_up is None else (xa_u, b_up, s_up))
+                    lkw = _gate_up_terms(a_gate, b_gate, s_gate, xa_g, a_up, b_up, s_up, xa_u)
                     _, hg, hu, *_ = G.ffn_gate_up(x_2d, w_gate, w_up, _lib.CACHE_BF16, gs,
                                                   want_h_mid=False, **lkw)
                 else:
@@ -576,61 +657,13 @@ class FlashFFNv3Function(torch.autograd.Function):
         grad_w_gate = grad_a_gate = grad_b_gate = None
         grad_w_up = grad_a_up = grad_b_up = None
         if need_gate_path:                                                # :1551-1587
-            ghgB = ghuB = ghB = None
-            # dg B_g and du B_u side by side in one [N, r_g + r_u] buffer, so
-            # one token reduction over x gives both A gradients below
-            stack = (_stackable(b_gate.t() if b_gate is not None else None,
-                                b_up.t() if b_up is not None else None)
-                     and (need_x or need_ag or need_au) and grad_h_gate.shape[0] >= 256
-                     and (_mfma(grad_h_gate, b_gate, grad_h_up, b_up)
-                          or (G.f16_fits(grad_h_gate, b_gate) and G.f16_fits(grad_h_up, b_up)))
-                     and grad_h_gate.shape[1] >= 256)
-            if stack:
-                r = b_gate.shape[1]
-                ghB = torch.empty((grad_h_gate.shape[0], r + b_up.shape[1]),
-                                  dtype=grad_h_gate.dtype, device=grad_h_gate.device)
-                # with the B gradient, both products of grad_h in one pass
-                # (:1556-1557 with :1575-1582)
-                if need_bg and _dual_ok(grad_h_gate, b_gate, xa_g):
-                    _, grad_b_gate = G.skinny_dual(grad_h_gate, b_gate.t(), xa_g, 1.0, s_gate,
-                                                   out_c=ghB[:, :r], name="gemm_ghgB_grad_b_gate")
-                else:
-                    G.skinny(grad_h_gate, b_gate.t(), 1.0, "gemm_ghgB", out=ghB[:, :r])
-                if need_bu and _dual_ok(grad_h_up, b_up, xa_u):
-                    _, grad_b_up = G.skinny_dual(grad_h_up, b_up.t(), xa_u, 1.0, s_up,
-                                                 out_c=ghB[:, r:], name="gemm_ghuB_grad_b_up")
-                else:
-                    G.skinny(grad_h_up, b_up.t(), 1.0, "gemm_ghuB", out=ghB[:, r:])
-                ghgB, ghuB = ghB[:, :r], ghB[:, r:]
-            else:
-                if a_gate is not None and (need_x or need_ag):
-                    if need_bg and _dual_ok(grad_h_gate, b_gate, xa_g):
-                        ghgB, grad_b_gate = G.skinny_dual(grad_h_gate, b_gate.t(), xa_g, 1.0,
-                                                          s_gate, name="gemm_ghgB_grad_b_gate")
-                    else:
-                        ghgB = _mm(grad_h_gate, b_gate, "gemm_ghgB", planes)
-                if a_up is not None and (need_x or need_au):
-                    if need_bu and _dual_ok(grad_h_up, b_up, xa_u):
-                        ghuB, grad_b_up = G.skinny_dual(grad_h_up, b_up.t(), xa_u, 1.0, s_up,
-                                                        name="gemm_ghuB_grad_b_up")
-                    else:
-                        ghuB = _mm(grad_h_up, b_up, "gemm_ghuB", planes)
+            ghgB, ghuB, ghB, grad_b_gate, grad_b_up = _thin_backward(
+                grad_h_gate, b_gate, xa_g, s_gate, grad_h_up, b_up, xa_u, s_up,
+                a_gate is not None and (need_x or need_ag),
+                a_up is not None and (need_x or need_au), need_bg, need_bu, planes)
             if need_x:
-                xl = [(ghgB, a_gate, s_gate) if a_gate is not None else None,
-                      (ghuB, a_up, s_up) if a_up is not None else None]
-                if fusable_gu and (_mfma(grad_h_gate, w_gate, grad_h_up, w_up)
-                                   or (G.f16_fits(grad_h_gate, w_gate)
-                                       and G.f16_fits(grad_h_up, w_up))):
-                    # dg @ W_g + du @ W_u as one K-concatenated GEMM, the gate and up
-                    # LoRA terms (:1561-1566) in its epilogue
-                    grad_x = G.mm2(grad_h_gate, w_gate, grad_h_up, w_up, "gemm_dgrad_x",
-                                   lora=[t for t in xl if t is not None] or None)
-                else:
-                    grad_x = _mm_sum(grad_h_gate, w_gate, grad_h_up, w_up, "gemm_dgrad_x", planes)
-                    if a_gate is not None:
-                        grad_x = _addmm(grad_x, ghgB, a_gate, s_gate, "gemm_dgrad_x_lora_gate")
-                    if a_up is not None:
-                        grad_x = _addmm(grad_x, ghuB, a_up, s_up, "gemm_dgrad_x_lora_up")
+                grad_x = _grad_x(grad_h_gate, w_gate, a_gate, s_gate, ghgB, grad_h_up, w_up, a_up,
+                                 s_up, ghuB, fusable_gu, planes)
             if need_bg and grad_b_gate is None:
                 grad_b_gate = _mm_scaled(grad_h_gate.t(), xa_g, s_gate, "gemm_grad_b_gate", planes)
             if ghB is not None and need_ag and need_au and s_gate == s_up:
@@ -939,33 +972,37 @@ class FlashFFNv3AdapterFunction(torch.autograd.Function):
             x_2d = x_2d.contiguous()
         planes = _planes(x)
         quant = cache_mode in ("int4", "int8")
-        plain_gu = a_gate is None and a_up is None and m_gate is None and m_up is None
-        fusable = plain_gu and _mfma(x_2d, w_gate, w_up) and x_2d.shape[0] > 0
+        fusable = _gate_up_ok(x_2d, w_gate, a_gate, b_gate, w_up, a_up, b_up,
+                              ((hidden_dim, w_gate.shape[0]),))
+        plain = fusable and m_gate is None and m_up is None
         fused_quant = quant and use_triton and x.dtype == torch.bfloat16   # :1979-1981
 
         c_gate = qs_gate = c_up = qs_up = None
         h_gate = h_up = xa_g = xa_u = None
-        if (fusable and fused_quant and group_size in _FUSED_GROUPS
+        lkw = {}
+        if fusable:
+            xa_g, xa_u, lkw = _gate_up_lora(x_2d, a_gate, b_gate, s_gate, a_up, b_up, s_up)
+        if (plain and fused_quant and group_size in _FUSED_GROUPS
                 and _f1_codec_fused(cache_mode, x_2d.shape[0], hidden_dim,
                                     w_gate.shape[0])):
             h_mid, _, _, c_gate, qs_gate, c_up, qs_up = G.ffn_gate_up(
-                x_2d, w_gate, w_up, _CACHE_CODE[cache_mode], group_size)
+                x_2d, w_gate, w_up, _CACHE_CODE[cache_mode], group_size, **lkw)
             _V3_COUNTERS["triton_quant_fwd"] += 1
-        elif fusable and fused_quant:
-            # the dual GEMM with a bf16 epilogue, then the standalone K1
-            _, h_gate, h_up, *_ = G.ffn_gate_up(x_2d, w_gate, w_up, _lib.CACHE_BF16, group_size,
-                                                want_h_mid=False)
-            h_mid, c_gate, qs_gate, c_up, qs_up = K.silu_mul_quant(
-                h_gate, h_up, _bits(cache_mode), group_size)
-            h_gate = h_up = None
-        elif fusable and not fused_quant:
+        elif plain and not fused_quant:
             keep = cache_mode != "recompute"
             h_mid, h_gate, h_up, *_ = G.ffn_gate_up(
-                x_2d, w_gate, w_up, _lib.CACHE_BF16 if keep else _lib.CACHE_NONE, group_size)
+                x_2d, w_gate, w_up, _lib.CACHE_BF16 if keep else _lib.CACHE_NONE, group_size,
+                **lkw)
         else:
-            h_gate, xa_g = _proj(x_2d, w_gate, a_gate, b_gate, s_gate, "gemm_fwd_gate", planes)
+            if fusable:
+                # the dual GEMM with a 16-bit epilogue, then DoRA's scale and K1
+                _, h_gate, h_up, *_ = G.ffn_gate_up(x_2d, w_gate, w_up, _lib.CACHE_BF16,
+                                                    group_size, want_h_mid=False, **lkw)
+            else:
+                h_gate, xa_g = _proj(x_2d, w_gate, a_gate, b_gate, s_gate, "gemm_fwd_gate",
+                                     planes)
+                h_up, xa_u = _proj(x_2d, w_up, a_up, b_up, s_up, "gemm_fwd_up", planes)
             h_gate = _scaled(h_gate, m_gate, nu_gate, inplace=True)          # :1967
-            h_up, xa_u = _proj(x_2d, w_up, a_up, b_up, s_up, "gemm_fwd_up", planes)
             h_up = _scaled(h_up, m_up, nu_up, inplace=True)                   # :1975
             if fused_quant:
                 h_mid, c_gate, qs_gate, c_up, qs_up = K.silu_mul_quant(
@@ -1028,27 +1065,31 @@ class FlashFFNv3AdapterFunction(torch.autograd.Function):
         need_h_mid = need_wd or need_md or (a_down is not None and need_ad)
         need_recon = need_gate_path or need_h_mid
         use_k2 = mode in ("int4", "int8") and ctx.use_triton and need_gate_path
-        plain_gu = a_gate is None and a_up is None and m_gate is None and m_up is None
-        fusable_gu = plain_gu and _mfma(x_2d, w_gate, w_up) and x_2d.shape[0] > 0
+        d_ff, d_model = w_gate.shape
+        # the forward's dual product (recomputed bit for bit), and with it the
+        # K-concatenated grad_x product's adapter terms
+        fusable_fwd = _gate_up_ok(x_2d, w_gate, a_gate, b_gate, w_up, a_up, b_up,
+                                  ((d_model, d_ff),))
+        fusable_gu = fusable_fwd and _lora_ok((a_gate, b_gate), (a_up, b_up),
+                                              dims=((d_ff, d_model),))
 
         hg = hu = raw_g = raw_u = None
         if need_recon and not use_k2:                                           # :2055-2078
             if mode == "recompute":
-                if fusable_gu:
+                if fusable_fwd:
                     # the forward's kernel and terms on the same inputs: bitwise equal
-                    lkw = dict(lora_gate=None if a_gate is None else (xa_g, b_gate, s_gate),
-                               lora_up=None if a_up is None else (xa_u, b_up, s_up))
-                    _, hg, hu, *_ = G.ffn_gate_up(x_2d, w_gate, w_up, _lib.CACHE_BF16, gs,
-                                                  want_h_mid=False, **lkw)
+                    lkw = _gate_up_terms(a_gate, b_gate, s_gate, xa_g, a_up, b_up, s_up, xa_u)
+                    _, raw_g, raw_u, *_ = G.ffn_gate_up(x_2d, w_gate, w_up, _lib.CACHE_BF16, gs,
+                                                        want_h_mid=False, **lkw)
                 else:
                     raw_g = _linear(x_2d, w_gate, "gemm_recompute_gate", planes)
                     if a_gate is not None:
                         raw_g = _addmm(raw_g, xa_g, b_gate.t(), s_gate, "gemm_recompute_gate_lora")
-                    hg = _scaled(raw_g, m_gate, nu_gate)
                     raw_u = _linear(x_2d, w_up, "gemm_recompute_up", planes)
                     if a_up is not None:
                         raw_u = _addmm(raw_u, xa_u, b_up.t(), s_up, "gemm_recompute_up_lora")
-                    hu = _scaled(raw_u, m_up, nu_up)
+                hg = _scaled(raw_g, m_gate, nu_gate)
+                hu = _scaled(raw_u, m_up, nu_up)
             elif mode == "bf16":
                 hg, hu = cq_gate, cq_up
             else:
@@ -1062,10 +1103,18 @@ class FlashFFNv3AdapterFunction(torch.autograd.Function):
                 hu = K.v3_dequantize_group_absmax(cq_up, qs_up, _bits(mode), gs, ctx.in_dtype)
 
         g_eff_y = _scaled(gy, m_down, nu_down)                                  # :2094
+        grad_w_down = grad_a_down = grad_b_down = grad_m_down = None
         gyB_d = None
         if a_down is not None and (need_gate_path or need_ad):
-            gyB_d = _mm(g_eff_y, b_down, "gemm_gyB_down", planes)
-        fusable_d = a_down is None and _mfma(g_eff_y, w_down) and g_eff_y.shape[0] > 0
+            if need_bd and _dual_ok(g_eff_y, b_down, ha_d):
+                gyB_d, grad_b_down = G.skinny_dual(g_eff_y, b_down.t(), ha_d, 1.0, s_down,
+                                                   name="gemm_gyB_grad_b_down")
+            else:
+                gyB_d = _mm(g_eff_y, b_down, "gemm_gyB_down", planes)
+        # the down adapter's term of grad_h_mid rides in the dgrad GEMM's epilogue
+        lora_d = _lora_ok((a_down, b_down), dims=((w_down.shape[0], w_down.shape[1]),))
+        dlora = (gyB_d, a_down, s_down) if (a_down is not None and lora_d) else None
+        fusable_d = _mfma(g_eff_y, w_down) and lora_d and g_eff_y.shape[0] > 0
 
         # the SwiGLU backward may write over h_gate / h_up when they are this
         # backward's own and no magnitude gradient reads them afterwards
@@ -1076,17 +1125,22 @@ class FlashFFNv3AdapterFunction(torch.autograd.Function):
             if use_k2 and fusable_d and gs in _FUSED_DGRAD_GROUPS:              # :2101-2110
                 grad_h_gate, grad_h_up, h_mid_hat = G.ffn_down_dgrad(
                     g_eff_y, w_down, _CACHE_CODE[mode], gs, cq_gate, qs_gate, cq_up, qs_up,
-                    need_h_mid)
+                    need_h_mid, lora=dlora)
                 _V3_COUNTERS["triton_dequant_bwd"] += 1
             elif (not use_k2) and fusable_d and hg is not None and hu is not None \
                     and _mfma(hg, hu):
                 grad_h_gate, grad_h_up, h_mid_hat = G.ffn_down_dgrad(
                     g_eff_y, w_down, _lib.CACHE_BF16, gs, hg, None, hu, None, need_h_mid,
-                    inplace=own)
+                    lora=dlora, inplace=own)
             else:
-                grad_h_mid = _mm(g_eff_y, w_down, "gemm_dgrad_down", planes)
-                if a_down is not None:
-                    grad_h_mid = _addmm(grad_h_mid, gyB_d, a_down, s_down, "gemm_dgrad_down_lora")
+                if (dlora is not None and _fits16(g_eff_y, w_down)
+                        and g_eff_y.dtype == a_down.dtype):
+                    grad_h_mid = G.mm2(g_eff_y, w_down, name="gemm_dgrad_down", lora=[dlora])
+                else:
+                    grad_h_mid = _mm(g_eff_y, w_down, "gemm_dgrad_down", planes)
+                    if a_down is not None:
+                        grad_h_mid = _addmm(grad_h_mid, gyB_d, a_down, s_down,
+                                            "gemm_dgrad_down_lora")
                 if use_k2:
                     grad_h_gate, grad_h_up, h_mid_hat = K.dequant_swiglu_backward(
                         grad_h_mid, cq_gate, qs_gate, cq_up, qs_up, _bits(mode), gs,
@@ -1097,7 +1151,6 @@ class FlashFFNv3AdapterFunction(torch.autograd.Function):
                         inplace=own and grad_h_mid.is_contiguous())
                 del grad_h_mid
 
-        grad_w_down = grad_a_down = grad_b_down = grad_m_down = None
         if need_h_mid:                                                          # :2112-2131
             if h_mid_hat is None:
                 h_mid_hat = K.silu_mul(hg, hu)
@@ -1107,13 +1160,19 @@ class FlashFFNv3AdapterFunction(torch.autograd.Function):
                 grad_a_down = _mm_scaled(gyB_d.t(), h_mid_hat, s_down, "gemm_grad_a_down", planes)
             if need_md:
                 # raw_d is never stored: one extra GEMM recomputes it
-                raw_d, _ = _proj(h_mid_hat, w_down, None, None, 0.0, "gemm_recompute_down", planes)
-                if a_down is not None:
-                    raw_d = _addmm(raw_d, ha_d, b_down.t(), s_down, "gemm_recompute_down_lora")
+                if (a_down is not None and _fits16_linear(h_mid_hat, w_down)
+                        and h_mid_hat.dtype == b_down.dtype
+                        and _lora_ok((a_down, b_down), dims=((w_down.shape[1], w_down.shape[0]),))):
+                    raw_d = G.linear_lora(h_mid_hat, w_down, ha_d, b_down, s_down,
+                                          "gemm_recompute_down")
+                else:
+                    raw_d = _linear(h_mid_hat, w_down, "gemm_recompute_down", planes)
+                    if a_down is not None:
+                        raw_d = _addmm(raw_d, ha_d, b_down.t(), s_down, "gemm_recompute_down_lora")
                 grad_m_down = K.col_dot_div(gy, raw_d, nu_down)
                 del raw_d
             del h_mid_hat
-        if need_bd:
+        if need_bd and grad_b_down is None:
             grad_b_down = _mm_scaled(g_eff_y.t(), ha_d, s_down, "gemm_grad_b_down", planes)
 
         grad_x = None
@@ -1129,26 +1188,26 @@ class FlashFFNv3AdapterFunction(torch.autograd.Function):
             # h = c * raw  =>  dL/draw = grad_h * c (grad_h is private here)
             g_eff_g = _scaled(grad_h_gate, m_gate, nu_gate, inplace=True)
             g_eff_u = _scaled(grad_h_up, m_up, nu_up, inplace=True)
-            ghgB = None
-            if a_gate is not None and (need_x or need_ag):
-                ghgB = _mm(g_eff_g, b_gate, "gemm_ghgB", planes)
-            ghuB = None
-            if a_up is not None and (need_x or need_au):
-                ghuB = _mm(g_eff_u, b_up, "gemm_ghuB", planes)
+            ghgB, ghuB, ghB, grad_b_gate, grad_b_up = _thin_backward(
+                g_eff_g, b_gate, xa_g, s_gate, g_eff_u, b_up, xa_u, s_up,
+                a_gate is not None and (need_x or need_ag),
+                a_up is not None and (need_x or need_au), need_bg, need_bu, planes)
             if need_x:
-                grad_x = _mm_sum(g_eff_g, w_gate, g_eff_u, w_up, "gemm_dgrad_x", planes)
-                if a_gate is not None:
-                    grad_x = _addmm(grad_x, ghgB, a_gate, s_gate, "gemm_dgrad_x_lora_gate")
-                if a_up is not None:
-                    grad_x = _addmm(grad_x, ghuB, a_up, s_up, "gemm_dgrad_x_lora_up")
-            if need_bg:
+                grad_x = _grad_x(g_eff_g, w_gate, a_gate, s_gate, ghgB, g_eff_u, w_up, a_up, s_up,
+                                 ghuB, fusable_gu, planes)
+            if need_bg and grad_b_gate is None:
                 grad_b_gate = _mm_scaled(g_eff_g.t(), xa_g, s_gate, "gemm_grad_b_gate", planes)
-            if need_ag:
-                grad_a_gate = _mm_scaled(ghgB.t(), x_2d, s_gate, "gemm_grad_a_gate", planes)
-            if need_bu:
+            if need_bu and grad_b_up is None:
                 grad_b_up = _mm_scaled(g_eff_u.t(), xa_u, s_up, "gemm_grad_b_up", planes)
-            if need_au:
-                grad_a_up = _mm_scaled(ghuB.t(), x_2d, s_up, "gemm_grad_a_up", planes)
+            if ghB is not None and need_ag and need_au and s_gate == s_up:
+                # its row halves equal the two reductions bit for bit
+                ga = _mm_scaled(ghB.t(), x_2d, s_gate, "gemm_grad_a_gate_up", planes)
+                grad_a_gate, grad_a_up = ga[:ghgB.shape[1]], ga[ghgB.shape[1]:]
+            else:
+                if need_ag:
+                    grad_a_gate = _mm_scaled(ghgB.t(), x_2d, s_gate, "gemm_grad_a_gate", planes)
+                if need_au:
+                    grad_a_up = _mm_scaled(ghuB.t(), x_2d, s_up, "gemm_grad_a_up", planes)
             if need_wg:
                 grad_w_gate = _mm(g_eff_g.t(), x_2d, "gemm_wgrad_gate", planes)
             if need_wu:

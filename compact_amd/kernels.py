@@ -505,13 +505,14 @@ def col_dot_div(a: torch.Tensor, b: torch.Tensor, den: torch.Tensor) -> torch.Te
     assert a.dtype == b.dtype == den.dtype, "col_dot_div: one dtype expected"
     a, b, den = a.contiguous(), b.contiguous(), den.contiguous()
     n, d = a.shape
-    L = _lib.api()
-    ws = torch.empty((max(1, L.cpt_col_dot_workspace_bytes(n, d)) + 3) // 4,
-                     dtype=torch.float32, device=a.device)
+    # partials of at least 32 rows, at most 64 of them
+    rows = max(32, (n + 63) // 64)
+    ws = torch.empty((max(1, (n + rows - 1) // rows), d), dtype=torch.float32, device=a.device)
     out = torch.empty((d,), dtype=a.dtype, device=a.device)
     with _timed("col_dot_div"):
-        rc = L.cpt_col_dot_div(a.data_ptr(), b.data_ptr(), den.data_ptr(), n, d, _dtype_code(a),
-                               ws.data_ptr(), out.data_ptr(), _stream(a))
+        rc = _lib.api().cpt_col_dot_div_rows(a.data_ptr(), b.data_ptr(), den.data_ptr(), n, d,
+                                             rows, _dtype_code(a), ws.data_ptr(), out.data_ptr(),
+                                             _stream(a))
     check(rc, "col_dot_div")
     return out
 
@@ -530,13 +531,17 @@ def dora_col_norm(w: torch.Tensor, a: torch.Tensor, b: torch.Tensor, s: float,
     assert w.dtype == a.dtype == b.dtype, "dora_col_norm: one dtype expected"
     w, a, b = w.contiguous(), a.contiguous(), b.contiguous()
     L = _lib.api()
-    ws = torch.empty((L.cpt_dora_col_norm_workspace_bytes(rows, r) + 3) // 4 + 1,
-                     dtype=torch.float32, device=w.device)
+    # 16-bit weights with a rank of whole 8s: one pass on the matrix cores
+    mfma = (w.dtype != torch.float32 and 0 < r <= 32 and r % 8 == 0 and cols % 8 == 0 and cols > 0
+            and w.data_ptr() % 16 == 0 and a.data_ptr() % 16 == 0)
+    nbytes = (L.cpt_dora_col_norm16_workspace_bytes(rows, cols, r) if mfma
+              else L.cpt_dora_col_norm_workspace_bytes(rows, r))
+    ws = torch.empty((nbytes + 3) // 4 + 1, dtype=torch.float32, device=w.device)
     nu = torch.empty((rows,), dtype=out_dtype, device=w.device)
     with _timed("dora_col_norm"):
-        rc = L.cpt_dora_col_norm(w.data_ptr(), a.data_ptr(), b.data_ptr(), rows, cols, r,
-                                 float(s), _dtype_code(w), ws.data_ptr(), nu.data_ptr(),
-                                 _DT[out_dtype], _stream(w))
+        norm = L.cpt_dora_col_norm16 if mfma else L.cpt_dora_col_norm
+        rc = norm(w.data_ptr(), a.data_ptr(), b.data_ptr(), rows, cols, r, float(s),
+                  _dtype_code(w), ws.data_ptr(), nu.data_ptr(), _DT[out_dtype], _stream(w))
     check(rc, "dora_col_norm")
     return nu
 

@@ -492,6 +492,18 @@ int64_t cpt_col_dot_workspace_bytes(int64_t n, int64_t d);
 int cpt_col_dot_div(const void* a, const void* b, const void* den, int64_t n, int64_t d,
                     int dtype, void* workspace, void* out, void* stream);
 
+/* cpt_col_dot_div with partial sums over `rows` rows each (workspace:
+ * ceil(n / rows) * d floats, at least one). */
+int cpt_col_dot_div_rows(const void* a, const void* b, const void* den, int64_t n, int64_t d,
+                         int64_t rows, int dtype, void* workspace, void* out, void* stream);
+
+/* cpt_dora_col_norm for bf16 or fp16 with r a multiple of 8 up to 32, cols of 8,
+ * w and a 16-byte aligned: one pass over w on the matrix cores. */
+int64_t cpt_dora_col_norm16_workspace_bytes(int64_t rows, int64_t cols, int64_t r);
+int cpt_dora_col_norm16(const void* w, const void* a, const void* b, int64_t rows, int64_t cols,
+                        int64_t r, double s, int dtype, void* workspace, void* nu, int nu_dtype,
+                        void* stream);
+
 /* Bytes of fp32 workspace cpt_dora_col_norm needs. */
 int64_t cpt_dora_col_norm_workspace_bytes(int64_t rows, int64_t r);
 

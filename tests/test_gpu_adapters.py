@@ -280,3 +280,35 @@ def test_dylora_rank_sampling_matches_module(device):
             y = fwd(x).float()
         tol = max(2e-2, 4 * 2.0 ** -8 * float(y_mod.detach().abs().max()))
         assert float((y - y_mod).abs().max()) <= tol
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows,cols,r", [(1, 8, 8), (16, 128, 16), (17, 136, 24), (100, 264, 32),
+                                         (1040, 4096, 16), (64, 11008, 8)])
+def test_dora_col_norm_one_pass(dt, rows, cols, r):
+    """The one-pass 16-bit norm: partial row groups and k ranges, ranks 8 to 32,
+    against float64 (products exact in fp32, so the sums' few 2^-24 only)."""
+    g = torch.Generator(device="cuda").manual_seed(rows + cols + r)
+
+    def rn(*s, std=1.0):
+        return (torch.randn(s, device="cuda", generator=g) * std).to(dt)
+    from compact_amd import kernels as K
+    w, a, b = rn(rows, cols, std=0.05), rn(r, cols, std=0.05), rn(rows, r, std=0.3)
+    ref = (w.double() + 1.5 * b.double() @ a.double()).norm(dim=1)
+    got = K.dora_col_norm(w, a, b, 1.5)
+    assert ((got.double() - ref).abs() / ref).max().item() < 2e-6
+    assert torch.equal(got, K.dora_col_norm(w, a, b, 1.5))
+
+
+@pytest.mark.parametrize("n", [0, 1, 31, 33, 2048, 4100])
+def test_col_dot_div_row_chunks(n):
+    """Chunk edges of the partial sums: n products of one rounding each, summed in
+    fp32 (n 2^-24 of their magnitudes), one output rounding."""
+    from compact_amd import kernels as K
+    g = torch.Generator(device="cuda").manual_seed(n)
+    a, b = (torch.randn(n, 72, device="cuda", generator=g).bfloat16() for _ in range(2))
+    den = torch.rand(72, device="cuda", generator=g).bfloat16() + 0.5
+    prod = (a * b).double()
+    ref, size = prod.sum(0) / den.double(), prod.abs().sum(0) / den.double()
+    err = (K.col_dot_div(a, b, den).double() - ref).abs()
+    assert bool((err <= 2.0 ** -8 * 1.01 * ref.abs() + (n + 2) * 2.0 ** -24 * size).all())
