@@ -10,10 +10,14 @@ namespace gemm {
 CPT_GEMM_INST_ALL(CPT_GEMM_DECLARE)
 CPT_NT16_INST_ALL(CPT_NT16_DECLARE)
 CPT_ST16_INST_ALL(CPT_ST16_DECLARE)
-extern template int launch_nt16_x3<true, true>(KArgs, hipStream_t);
-extern template int launch_nt16_x3<true, false>(KArgs, hipStream_t);
-extern template int launch_nt16_x3<false, false>(KArgs, hipStream_t);
-extern template int launch_nt16_x3<false, true>(KArgs, hipStream_t);
+extern template int launch_nt16_f32<true, true, false>(KArgs, hipStream_t);
+extern template int launch_nt16_f32<true, false, false>(KArgs, hipStream_t);
+extern template int launch_nt16_f32<false, false, false>(KArgs, hipStream_t);
+extern template int launch_nt16_f32<false, true, false>(KArgs, hipStream_t);
+extern template int launch_nt16_f32<true, true, true>(KArgs, hipStream_t);
+extern template int launch_nt16_f32<true, false, true>(KArgs, hipStream_t);
+extern template int launch_nt16_f32<false, false, true>(KArgs, hipStream_t);
+extern template int launch_nt16_f32<false, true, true>(KArgs, hipStream_t);
 
 // out[m, n] = bf16(alpha * sum_s ws[s][m][n])  (split-K reduction, fixed order)
 __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restrict__ ws,
@@ -351,8 +355,11 @@ inline bool set_split(KArgs& A, int splits, void* ws) {
 template <int DT>
 int gemm16_impl(const void* a, int64_t lda, int a_kmajor, const void* b, int64_t ldb, int b_kmajor,
                 const void* a2, int64_t lda2, const void* b2, int64_t ldb2, int64_t K2, void* c,
-                int64_t ldc, int64_t M, int64_t N, int64_t K, const LoraTerms& L, int splits,
-                void* ws, void* stream) {
+                int64_t ldc, int64_t M, int64_t N, int64_t K, const LoraTerms& L, int tiles,
+                int splits, void* ws, void* stream) {
+  const bool big = tiles == 256;
+  if (tiles != 128 && !(big && DT == kBF16 && splits > 1 && K % 64 == 0 && K2 % 64 == 0))
+    return kErrShape;
   if (M < 0 || N < 0 || K < 0 || K2 < 0 || splits < 1) return kErrShape;
   if (M == 0 || N == 0) return kOk;
   const bool two = a2 != nullptr;
@@ -389,7 +396,13 @@ int gemm16_impl(const void* a, int64_t lda, int a_kmajor, const void* b, int64_t
     if (!ws || !al16(ws)) return kErrAlign;
     A.ldc = N;
     int rc;
-    if (a_kmajor && b_kmajor) rc = launch_small<DT, true, true, EPI_F32, CACHE_NONE, 0>(A, st);
+    if (big)
+      rc = a_kmajor ? (b_kmajor ? launch_nt16_f32<true, true, false>(A, st)
+                                : launch_nt16_f32<true, false, false>(A, st))
+                    : (b_kmajor ? launch_nt16_f32<false, true, false>(A, st)
+                                : launch_nt16_f32<false, false, false>(A, st));
+    else if (a_kmajor && b_kmajor)
+      rc = launch_small<DT, true, true, EPI_F32, CACHE_NONE, 0>(A, st);
     else if (a_kmajor) rc = launch_small<DT, true, false, EPI_F32, CACHE_NONE, 0>(A, st);
     else if (b_kmajor) rc = launch_small<DT, false, true, EPI_F32, CACHE_NONE, 0>(A, st);
     else rc = launch_small<DT, false, false, EPI_F32, CACHE_NONE, 0>(A, st);
@@ -462,10 +475,10 @@ int x3_gemm_impl(const void* a, int64_t plane_a, int64_t lda, int a_kmajor, cons
   hipStream_t st = (hipStream_t)stream;
   int rc;
   if (big)
-    rc = a_kmajor ? (b_kmajor ? launch_nt16_x3<true, true>(A, st)
-                              : launch_nt16_x3<true, false>(A, st))
-                  : (b_kmajor ? launch_nt16_x3<false, true>(A, st)
-                              : launch_nt16_x3<false, false>(A, st));
+    rc = a_kmajor ? (b_kmajor ? launch_nt16_f32<true, true, true>(A, st)
+                              : launch_nt16_f32<true, false, true>(A, st))
+                  : (b_kmajor ? launch_nt16_f32<false, true, true>(A, st)
+                              : launch_nt16_f32<false, false, true>(A, st));
   else if (a_kmajor && b_kmajor) rc = launch_small<kF32, true, true, EPI_F32, CACHE_NONE, 0>(A, st);
   else if (a_kmajor) rc = launch_small<kF32, true, false, EPI_F32, CACHE_NONE, 0>(A, st);
   else if (b_kmajor) rc = launch_small<kF32, false, true, EPI_F32, CACHE_NONE, 0>(A, st);
@@ -852,8 +865,8 @@ int cpt_gemm16(int dtype, const void* a, int64_t lda, int a_kmajor, const void* 
                int b_kmajor, const void* a2, int64_t lda2, const void* b2, int64_t ldb2,
                int64_t K2, void* c, int64_t ldc, int64_t M, int64_t N, int64_t K, int64_t rank,
                int64_t ldp, int q_kmajor, int64_t ldq, const void* p0, const void* q0,
-               float alpha0, const void* p1, const void* q1, float alpha1, int splits,
-               void* workspace, void* stream) {
+               float alpha0, const void* p1, const void* q1, float alpha1, int tiles,
+               int splits, void* workspace, void* stream) {
   if (rank < 0) return kErrShape;
   LoraTerms L;
   L.rank = (int)rank; L.ldp = ldp; L.q_kmajor = q_kmajor ? 1 : 0; L.ldq = ldq;
@@ -861,10 +874,10 @@ int cpt_gemm16(int dtype, const void* a, int64_t lda, int a_kmajor, const void* 
   L.p[1] = p1; L.q[1] = q1; L.alpha[1] = alpha1;
   if (dtype == kF16)
     return gemm16_impl<kF16>(a, lda, a_kmajor, b, ldb, b_kmajor, a2, lda2, b2, ldb2, K2, c, ldc, M,
-                             N, K, L, splits, workspace, stream);
+                             N, K, L, tiles, splits, workspace, stream);
   if (dtype == kBF16)
     return gemm16_impl<kBF16>(a, lda, a_kmajor, b, ldb, b_kmajor, a2, lda2, b2, ldb2, K2, c, ldc,
-                              M, N, K, L, splits, workspace, stream);
+                              M, N, K, L, tiles, splits, workspace, stream);
   return kErrDType;
 }
 

@@ -291,7 +291,7 @@ __device__ __forceinline__ void nt16_tile(const KArgs& A, uint16_t* lds, int tm,
   static_assert(EPI == EPI_STORE || EPI == EPI_GLU || EPI == EPI_DGLU || EPI == EPI_GLUO ||
                     EPI == EPI_F32,
                 "epilogues of the 16x16x32 loop");
-  static_assert(X3 == (EPI == EPI_F32), "fp32 products write fp32");
+  static_assert(!X3 || EPI == EPI_F32, "fp32 products write fp32");
   static_assert(EPI != EPI_DGLU || (AK && !BK), "B1: gy (K-major) . W_d (MN-major)");
   constexpr bool DUAL = EPI == EPI_GLU || EPI == EPI_GLUO;
   static_assert(!DUAL || (AK && BK), "F1's operands are K-major");
@@ -559,7 +559,7 @@ __device__ __forceinline__ void nt16_tile(const KArgs& A, uint16_t* lds, int tm,
         const int64_t m = m0 + wm * 128 + 16 * j + (elane & 15);
         f32x4 v = acc[i][j];
         asm volatile("" : "+v"(v));
-        v *= A.alpha;   // 1 for partials
+        if constexpr (X3) v *= A.alpha;   // 1 for partials
         if (m < A.M) *reinterpret_cast<f32x4*>(out + m * A.ldc + n) = v;
       }
     }
@@ -678,28 +678,31 @@ __global__ __launch_bounds__(kThreads, 1) void nt16_kernel(const KArgs A) {
   }
 }
 
-// fp32 products of plane pairs: block = split * tiles + tile, split s takes
-// k-tiles [s kt_per_split, ..) of the 6 npairs segments.
-template <bool AK, bool BK>
-__global__ __launch_bounds__(kThreads, 1) void nt16_x3_kernel(const KArgs A) {
+// Split products and (X3) fp32 ones of plane pairs: block = split * tiles +
+// tile, split s takes k-tiles [s kt_per_split, ..) of the pairs (X3: of the 6
+// npairs segments) and writes fp32.
+template <bool AK, bool BK, bool X3>
+__global__ __launch_bounds__(kThreads, 1) void nt16_f32_kernel(const KArgs A) {
   extern __shared__ __attribute__((aligned(16))) uint16_t lds[];
-  if (any_flag(A.flags)) return;
+  if constexpr (X3)
+    if (any_flag(A.flags)) return;
   const int tiles = A.tiles_m * A.tiles_n;
   const int split = blockIdx.x / tiles;
-  const int nk = 6 * (int)(A.K[0] / kBK + (A.npairs == 2 ? A.K[1] / kBK : 0));
+  const int nk = (X3 ? 6 : 1) * (int)(A.K[0] / kBK + (A.npairs == 2 ? A.K[1] / kBK : 0));
   const int kb = split * A.kt_per_split;
   int tm, tn;
   tile_coords_of(blockIdx.x - split * tiles, tiles, A.tiles_m, A.tiles_n, tm, tn);
-  nt16_tile<AK, BK, EPI_F32, 0, 0, 0, false, false, true>(
+  nt16_tile<AK, BK, EPI_F32, 0, 0, 0, false, false, X3>(
       A, lds, tm, tn, kb, min(nk, kb + A.kt_per_split), kRoleWhole, split);
 }
 
 }  // namespace nt16
 
-// fp32 products of plane pairs on 256 x 256 tiles, A.ksplit blocks per tile
-template <bool AK, bool BK>
-int launch_nt16_x3(KArgs A, hipStream_t st) {
-  auto kern = nt16::nt16_x3_kernel<AK, BK>;
+// Split products of bf16 operands, or fp32 ones of plane pairs (X3), on 256 x 256
+// tiles, A.ksplit blocks per tile
+template <bool AK, bool BK, bool X3>
+int launch_nt16_f32(KArgs A, hipStream_t st) {
+  auto kern = nt16::nt16_f32_kernel<AK, BK, X3>;
   static bool attr_set = false;   // per instantiation
   if (!attr_set) {
     if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize,

@@ -42,7 +42,7 @@
 // m h, h h.  The three left out are below 2^-24 of the product; every partial
 // product is exact in fp32 and the sums are fp32, with one rounding per 32 k
 // where v_mfma_f32_32x32x2_f32 rounds every 2.  The 256 x 256 tiles carry the
-// same loop (nt16_x3_kernel); figures beside x3_gemm_impl in gemm.hip.
+// same loop (nt16_f32_kernel); figures beside x3_gemm_impl in gemm.hip.
 
 #pragma once
 

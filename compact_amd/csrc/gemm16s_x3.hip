@@ -1,5 +1,6 @@
-// fp32 products on the bf16 MFMAs (gemm16s_kernel.h): the kernels over three
-// bf16 planes per operand, and the kernel that makes the planes.
+// Products that write fp32 (gemm16_kernel.h, gemm16s_kernel.h): split ones on 256
+// x 256 tiles, fp32 ones over three bf16 planes per operand, and the kernel that
+// makes the planes.
 
 #include "gemm16s_kernel.h"
 
@@ -7,10 +8,14 @@ namespace cpt {
 namespace gemm {
 
 CPT_ST16_INST_X3(CPT_ST16_DEFINE)
-template int launch_nt16_x3<true, true>(KArgs, hipStream_t);
-template int launch_nt16_x3<true, false>(KArgs, hipStream_t);
-template int launch_nt16_x3<false, false>(KArgs, hipStream_t);
-template int launch_nt16_x3<false, true>(KArgs, hipStream_t);
+template int launch_nt16_f32<true, true, false>(KArgs, hipStream_t);
+template int launch_nt16_f32<true, false, false>(KArgs, hipStream_t);
+template int launch_nt16_f32<false, false, false>(KArgs, hipStream_t);
+template int launch_nt16_f32<false, true, false>(KArgs, hipStream_t);
+template int launch_nt16_f32<true, true, true>(KArgs, hipStream_t);
+template int launch_nt16_f32<true, false, true>(KArgs, hipStream_t);
+template int launch_nt16_f32<false, false, true>(KArgs, hipStream_t);
+template int launch_nt16_f32<false, true, true>(KArgs, hipStream_t);
 
 // planes[0..2] = bf16 h, m, l with h = bf16(x), m = bf16(x - h), l = bf16(x - h
 // - m): round-to-nearest each, both differences exact, so x = h + m + l to 24

@@ -1321,9 +1321,9 @@ int launch_nt16(const KArgs& A, hipStream_t st);
 // CACHE_BF16), which st16_reduce sums and finishes.
 template <int DT, bool AK, bool BK, int EPI, int CACHE, int LT, int S>
 int launch_st16(KArgs A, hipStream_t st);
-// fp32 products of bf16 planes on 256 x 256 tiles (gemm16_kernel.h)
-template <bool AK, bool BK>
-int launch_nt16_x3(KArgs A, hipStream_t st);
+// Split products, and fp32 ones of bf16 planes (X3), on 256 x 256 tiles
+template <bool AK, bool BK, bool X3>
+int launch_nt16_f32(KArgs A, hipStream_t st);
 // Split sums, adapter terms (`terms` of A's) and epilogue of a split product:
 // plain store to A.C (rows ldo apart) or, dual, the GLU outputs of F1.
 // dt kF32: c = alpha * sum.

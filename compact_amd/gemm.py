@@ -27,6 +27,8 @@ These replace the cuBLAS GEMMs the reference issues through F.linear / @
 
 from __future__ import annotations
 
+import functools
+
 import torch
 
 from . import _lib
@@ -484,6 +486,46 @@ def split_plan(m: int, n: int, nk: int) -> int:
     return splits if splits > 1 and nk - nk // splits >= SPLIT_MIN_SAVED else 1
 
 
+@functools.lru_cache(maxsize=4096)
+def tile_plan(m: int, n: int, nk: int, half: bool = False) -> tuple[int, int]:
+    """(tile edge, k ranges) of a 16-bit product of nk k-tiles: the unsplit
+    product (one range: launch16 picks its tiles), 128 x 128 tiles split as
+    split_plan has it, or, bf16 only, 256 x 256 tiles with k split to fill the
+    CUs, whichever the measured rates make cheapest.
+
+    Rates on MI355X, us per k-tile: 0.55 for 128 x 128 tiles alone on a CU, 1.0
+    for two sharing it, 1.0 to 1.45 for a 256 x 256 tile as the chip fills up;
+    8 for a block's ends; a split adds 8 and 1.1 per million partials.  Measured,
+    us unsplit (128 x 128 tiles) / split 256 x 256 ones:
+      2048 x 4096, k 22016 (128 large tiles, 2 ranges)  382 / 277
+      2048 x 4096, k 11008 (128, 2)                     160 / 146
+      3000 x 2048, k 11264 (96, 2)                      162 / 127
+      1500 x 4096, k 11008 (96, 2)                      161 / 128
+      1024 x 4096, k 11008 (64, 4)                       91 / 95     kept unsplit
+      4096 x 2048, k 5632  (128, 2)                      87 / 90     kept unsplit"""
+    t128 = ((m + 127) // 128) * ((n + 127) // 128)
+    t256 = ((m + 255) // 256) * ((n + 255) // 256)
+    if t128 == 0:
+        return 128, 1
+    small = split_plan(m, n, nk)
+    if small > 1:
+        cost = 0.55 * nk / small + 12 + 1.1e-6 * small * m * n
+    elif t128 <= 256:
+        cost = 0.55 * nk + 4
+    elif t128 <= 512:
+        cost = 1.0 * nk + 4
+    else:
+        return 128, 1
+    best = (128, small)
+    for s in range(2, min(8, 256 // t256) + 1) if not half else ():
+        if nk // s < SPLIT_MIN_KT:
+            break
+        c = (1.0 + 0.45 * t256 * s / 256) * nk / s + 16 + 1.1e-6 * s * m * n
+        if c < 0.95 * cost:
+            best, cost = (256, s), c / 0.95
+    return best
+
+
 def mm(a: torch.Tensor, b: torch.Tensor, name: str = "gemm") -> torch.Tensor:
     """a [M, K] @ b [K, N] -> bf16 [M, N] on the MFMA GEMM loops (16x16x32 when
     K is a multiple of 64 and N of 8, else the 32x32x16 engine).  Tall products
@@ -596,8 +638,8 @@ def mm2(a, b, a2=None, b2=None, name: str = "gemm", lora=None) -> torch.Tensor:
         dims = ((K, N),) if a2 is None else ((K, N), (K2, N))
         r, ldp, qk, ldq, t, keep = _lora_args(lora, N, dims)
     half = dt == _lib.F16
-    splits = (1 if (not half and (K % 64 or K2 % 64)) or N % 8 or not K
-              else split_plan(M, N, (K + 63) // 64 + (K2 + 63) // 64))
+    tiles, splits = ((128, 1) if (not half and (K % 64 or K2 % 64)) or N % 8 or not K
+                     else tile_plan(M, N, (K + 63) // 64 + (K2 + 63) // 64, half))
     if splits > 1 or half:
         ws = (torch.empty((splits * M * N,), dtype=torch.float32, device=a.device)
               if splits > 1 else None)
@@ -605,8 +647,8 @@ def mm2(a, b, a2=None, b2=None, name: str = "gemm", lora=None) -> torch.Tensor:
             rc = _lib.api().cpt_gemm16(
                 dt, a.data_ptr(), lda, ak, b.data_ptr(), ldb, bk, p_a2, lda2, p_b2, ldb2,
                 K2, c.data_ptr(), ldc, M, N, K, r, ldp, qk, ldq, t[0][0], t[0][1], t[0][2],
-                t[1][0], t[1][1], t[1][2], splits, None if ws is None else ws.data_ptr(),
-                _stream(a))
+                t[1][0], t[1][1], t[1][2], tiles, splits,
+                None if ws is None else ws.data_ptr(), _stream(a))
         check(rc, name)
         return c
     _stream_k(a.device)

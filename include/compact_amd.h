@@ -327,14 +327,15 @@ int cpt_gemm16_skinny_dual(int dtype, const void* x, int64_t ldx, const void* q,
  * a multiple of 64 (two MN-major operands: any K), N of 8.  splits > 1 shares
  * the k-tiles of 64 over that many blocks per tile: fp32 partials go to
  * workspace (splits * M * N floats, 16-byte aligned), summed in k order by a
- * second kernel that also applies the adapter terms.  With splits = 1 a bf16
+ * second kernel that also applies the adapter terms.  tiles is 128, or 256 for
+ * a split bf16 product on 256 x 256 tiles.  With splits = 1 a bf16
  * product is bit-identical to cpt_gemm_bf16_lora's on the 16x16x32 loop. */
 int cpt_gemm16(int dtype, const void* a, int64_t lda, int a_kmajor, const void* b, int64_t ldb,
                int b_kmajor, const void* a2, int64_t lda2, const void* b2, int64_t ldb2,
                int64_t K2, void* c, int64_t ldc, int64_t M, int64_t N, int64_t K, int64_t rank,
                int64_t ldp, int q_kmajor, int64_t ldq, const void* p0, const void* q0,
-               float alpha0, const void* p1, const void* q1, float alpha1, int splits,
-               void* workspace, void* stream);
+               float alpha0, const void* p1, const void* q1, float alpha1, int tiles,
+               int splits, void* workspace, void* stream);
 
 /* fp32 products on the bf16 MFMAs.  cpt_split_f32 writes x [rows, cols] (rows ld
  * apart, cols a multiple of 8, 16-byte aligned) as three bf16 planes

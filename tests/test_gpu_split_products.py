@@ -15,7 +15,7 @@ def _rand(*shape, dtype, seed=0, scale=1.0):
     return (torch.randn(shape, device="cuda", generator=g) * scale).to(dtype)
 
 
-def _gemm16(dt, a, b, a2=None, b2=None, lora=(), splits=1):
+def _gemm16(dt, a, b, a2=None, b2=None, lora=(), splits=1, tiles=128):
     """a [M, K] @ b [K, N] (+ a2 @ b2, + adapter terms) through cpt_gemm16."""
     from compact_amd import _lib
     from compact_amd import gemm as G
@@ -36,7 +36,7 @@ def _gemm16(dt, a, b, a2=None, b2=None, lora=(), splits=1):
     check(_lib.lib().cpt_gemm16(
         _lib.F16 if dt == "fp16" else _lib.BF16, a.data_ptr(), lda, ak, b.data_ptr(), ldb, bk,
         *pair, c.data_ptr(), N, M, N, K, r, r, km, lora[0][1].stride(0) if lora else 0, *t[0],
-        *t[1], splits, ws.data_ptr(), torch.cuda.current_stream().cuda_stream), "gemm16")
+        *t[1], tiles, splits, ws.data_ptr(), torch.cuda.current_stream().cuda_stream), "gemm16")
     return c
 
 
@@ -88,6 +88,27 @@ def test_two_pairs_split_across_the_boundary(dt, splits):
     bound = 640 * 2.0 ** -24 * (a.double().abs() @ b.double().abs()
                                 + a2.double().abs() @ b2.double().abs())
     _close(_gemm16(dt, a, b, a2, b2, splits=splits), ref, dt, bound)
+
+
+@pytest.mark.parametrize("layout", ["nt", "nn", "tn", "tt"])
+@pytest.mark.parametrize("m,n,k,splits", [(1, 8, 128, 2), (260, 264, 448, 3), (520, 136, 1024, 8),
+                                          (2048, 4096, 11008, 2)])
+def test_split_product_on_large_tiles(layout, m, n, k, splits):
+    if layout[0] == "t" and m % 8:
+        m = (m + 7) // 8 * 8
+    d = DT["bf16"]
+    a = _rand(m, k, dtype=d, seed=1) if layout[0] == "n" else _rand(k, m, dtype=d, seed=1).t()
+    b = _rand(n, k, dtype=d, seed=2).t() if layout[1] == "t" else _rand(k, n, dtype=d, seed=2)
+    ref = a.double() @ b.double()
+    bound = k * 2.0 ** -24 * (a.double().abs() @ b.double().abs())
+    got = _gemm16("bf16", a, b, splits=splits, tiles=256)
+    _close(got, ref, "bf16", bound)
+    if layout == "nn":   # two pairs, a range across their boundary, and an adapter term
+        p, q = _rand(m, 16, dtype=d, seed=3), _rand(16, n, dtype=d, seed=4)
+        got = _gemm16("bf16", a, b, a, b, lora=[(p, q, 0.5)], splits=splits, tiles=256)
+        term = 0.5 * (p.double() @ q.double())
+        size = 2 * ref.abs() + (2 * ref + term).abs() + 2 * term.abs()
+        _close(got, 2 * ref + term, "bf16", 2 * bound + EPS["bf16"] * 1.1 * size)
 
 
 @pytest.mark.parametrize("dt", ["bf16", "fp16"])
@@ -165,3 +186,7 @@ def test_split_plan_fills_the_chip_without_empty_ranges():
                 s = G.split_plan(m, n, nk)
                 tiles = -(-m // 128) * -(-n // 128)
                 assert 1 <= s <= nk and (s == 1 or (s * tiles <= 256 and nk // s >= 6))
+                edge, s = G.tile_plan(m, n, nk)
+                tiles = -(-m // edge) * -(-n // edge)
+                assert s == 1 or (s * tiles <= 256 and nk // s >= 6)
+                assert G.tile_plan(m, n, nk, True)[0] == 128
