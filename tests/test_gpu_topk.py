@@ -116,3 +116,24 @@ def test_flashffn_module_vs_standard(device):
     assert R.rel_frob(y_f.float().cpu(), y_s.cpu()) < 1e-2
     y_f.float().pow(2).mean().backward()
     assert all(p.grad is not None for p in fl.parameters())
+
+
+@pytest.mark.parametrize("d", [8, 2048, 4096, 4104, 6144, 6152, 12288, 12296, 16384, 16392, 32760])
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+def test_topk_register_rows_and_their_edges(d, dt):
+    """16-bit rows at the edges of the register-held kernel's chunk counts and
+    past them: magnitudes, their columns and the lowest-column tie rule, with ties,
+    zeros, infinities and NaN in the row."""
+    g = torch.Generator(device="cuda").manual_seed(d)
+    x = torch.randn(5, d, device="cuda", generator=g).to(dt)
+    x[1] = x[1].sign() * 0.5                       # all tied
+    x[2, ::3] = 0
+    x[3, d // 2], x[3, 0] = float("inf"), float("nan")
+    x[4] = 0
+    from compact_amd import kernels as K
+    for k in {1, max(1, d // 3), d}:
+        v, i = K.topk_abs(x, k)
+        key = x.view(torch.int16).int() & 0x7FFF
+        order = key.sort(dim=-1, descending=True, stable=True).indices[:, :k].sort(dim=-1).values
+        assert torch.equal(i.long(), order)
+        assert torch.equal(v.view(torch.int16), x.gather(1, order).view(torch.int16))
