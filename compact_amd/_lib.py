@@ -44,6 +44,8 @@ SIGNATURES = {
     "cpt_gemm_bf16": [_P, _L, _I, _P, _L, _I, _P, _L, _P, _L, _L, _P, _L, _L, _L, _L, _P],
     "cpt_gemm_bf16_ex": [_P, _L, _I, _P, _L, _I, _P, _L, _L, _L, _L, ctypes.c_float, _I, _I, _P, _P],
     "cpt_gemm16_skinny": [_I, _P, _L, _P, _L, _P, _L, _L, _L, _L, ctypes.c_float, _I, _P, _P],
+    "cpt_gemm16_skinny_small": [_I, _P, _L, _P, _L, _L, _P, _L, _L, _P, _L, _L, _L,
+                                ctypes.c_float, _P],
     "cpt_gemm16_skinny_t": [_I, _P, _L, _P, _L, _P, _L, _I, _L, _L, _L, ctypes.c_float, _I, _P,
                             _P],
     "cpt_gemm16_skinny_dual": [_I, _P, _L, _P, _L, _I, _P, _L, _P, _L, ctypes.c_float, _P, _L, _I,

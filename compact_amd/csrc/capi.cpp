@@ -70,6 +70,7 @@ PyMethodDef methods[] = {
     CPT_ENTRY(cpt_gemm_bf16_ex),
     CPT_ENTRY(cpt_gemm16),
     CPT_ENTRY(cpt_gemm16_skinny),
+    CPT_ENTRY(cpt_gemm16_skinny_small),
     CPT_ENTRY(cpt_gemm16_skinny_t),
     CPT_ENTRY(cpt_gemm16_skinny_dual),
     CPT_ENTRY(cpt_gemm_bf16_skinny_dual_workspace_bytes),

@@ -239,6 +239,74 @@ __global__ __launch_bounds__(256) void skinny_reduce_kernel(const float* __restr
   c[m * ldc + r] = scaled<DT>(alpha, sum);
 }
 
+// Few tokens: C[M, r0 + r1] = alpha * A . [Q0; Q1]^T in one launch, the two
+// factors (x A_g^T and x A_u^T) read where they lie.  A block owns 16 rows and
+// its 16 wavefronts a sixteenth of K each (kchunk, a multiple of 32), loaded
+// straight into the MFMA operand layout; their partials are added in K order
+// through LDS.  Bound by latency: 4 x 2048 rows take about the loads of one
+// wavefront in sequence (3.2 us, both factors 3.9), where splitting K over
+// blocks takes two launches per factor and stacking the factors a copy (1808
+// tokens, both factors: 12.4 us in three launches, here 5.3).
+constexpr int kSmallWaves = 16;
+
+template <int DT, int NB>
+__global__ __launch_bounds__(64 * kSmallWaves) void skinny_small_kernel(
+    const uint16_t* __restrict__ a, int64_t lda, const uint16_t* __restrict__ q0, int64_t ldq0,
+    int r0, const uint16_t* __restrict__ q1, int64_t ldq1, int r1, int64_t M, int64_t K,
+    int64_t kchunk, uint16_t* __restrict__ c, int64_t ldc, float alpha) {
+  constexpr int U = 4;   // k-32 steps in flight
+  __shared__ float part[kSmallWaves][NB][16][17];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t m0 = (int64_t)blockIdx.x * 16;
+  const int64_t k_begin = wave * kchunk;
+  const int64_t k_end = min(K, k_begin + kchunk);
+  const int kq = 8 * (lane >> 4);
+  const int64_t row = m0 + (lane & 15);
+  const bool rok = row < M;
+  const uint16_t* pa = a + (rok ? row : 0) * lda + kq;
+  const uint16_t* pq[NB];
+  bool qok[NB];
+#pragma unroll
+  for (int t = 0; t < NB; ++t) {
+    const int r = t * 16 + (lane & 15);
+    qok[t] = r < r0 + r1;
+    pq[t] = (r < r0 ? q0 + r * ldq0 : q1 + (qok[t] ? r - r0 : 0) * ldq1) + kq;
+  }
+  f32x4 acc[NB];
+#pragma unroll
+  for (int t = 0; t < NB; ++t) acc[t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  const bf16x8 zero = __builtin_bit_cast(bf16x8, make_uint4(0, 0, 0, 0));
+  for (int64_t k = k_begin; k < k_end; k += 32 * U) {
+    bf16x8 av[U], qv[U][NB];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      // K % 8 == 0: a lane's 8 k are all in or all out
+      const bool ok = k + 32 * u + kq < k_end;
+      av[u] = ok && rok ? *reinterpret_cast<const bf16x8*>(pa + k + 32 * u) : zero;
+#pragma unroll
+      for (int t = 0; t < NB; ++t)
+        qv[u][t] = ok && qok[t] ? *reinterpret_cast<const bf16x8*>(pq[t] + k + 32 * u) : zero;
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int t = 0; t < NB; ++t) acc[t] = mfma<DT>(av[u], qv[u][t], acc[t]);
+  }
+#pragma unroll
+  for (int t = 0; t < NB; ++t)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) part[wave][t][4 * (lane >> 4) + i][lane & 15] = acc[t][i];
+  __syncthreads();
+  for (int e = threadIdx.x; e < NB * 256; e += 64 * kSmallWaves) {
+    const int t = e >> 8, i = (e >> 4) & 15, col = e & 15;
+    float sum = 0.0f;
+#pragma unroll
+    for (int w = 0; w < kSmallWaves; ++w) sum += part[w][t][i][col];
+    if (m0 + i < M && t * 16 + col < r0 + r1)
+      c[(m0 + i) * ldc + t * 16 + col] = scaled<DT>(alpha, sum);
+  }
+}
+
 // ---------------------------------------------------------------------------
 // Token reductions of the adapter gradients: Z[N, R] = alpha * X^T . P with
 // X [T, N] and P [T, R] token-major (rows t), R <= 32: grad_B = s * grad_y^T
@@ -659,6 +727,30 @@ int cpt_gemm16_skinny(int dtype, const void* a, int64_t lda, const void* q, int6
     if (hipGetLastError() != hipSuccess) return kErrLaunch;
   }
   return kOk;
+}
+
+int cpt_gemm16_skinny_small(int dtype, const void* a, int64_t lda, const void* q0, int64_t ldq0,
+                            int64_t r0, const void* q1, int64_t ldq1, int64_t r1, void* c,
+                            int64_t ldc, int64_t M, int64_t K, float alpha, void* stream) {
+  if (dtype != kBF16 && dtype != kF16) return kErrDType;
+  if (M < 0 || K < 0 || r0 < 0 || r1 < 0 || r0 + r1 > 32) return kErrShape;
+  if (M == 0 || r0 + r1 == 0) return kOk;
+  if (!a || !c || (r0 && !q0) || (r1 && !q1) || !al16(a) || (r0 && (!al16(q0) || (ldq0 & 7))) ||
+      (r1 && (!al16(q1) || (ldq1 & 7))) || (lda & 7) || (K & 7) || lda < K ||
+      (r0 && ldq0 < K) || (r1 && ldq1 < K) || ldc < r0 + r1)
+    return kErrAlign;
+  const int64_t blocks = (M + 15) / 16;
+  if (blocks > 0x7FFFFFFF) return kErrTooLarge;
+  const int64_t kchunk = ((K + kSmallWaves - 1) / kSmallWaves + 31) / 32 * 32;
+  const auto kern = dtype == kBF16
+                        ? (r0 + r1 <= 16 ? skinny_small_kernel<kBF16, 1>
+                                         : skinny_small_kernel<kBF16, 2>)
+                        : (r0 + r1 <= 16 ? skinny_small_kernel<kF16, 1>
+                                         : skinny_small_kernel<kF16, 2>);
+  hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(64 * kSmallWaves), 0, (hipStream_t)stream,
+                     (const uint16_t*)a, lda, (const uint16_t*)q0, ldq0, (int)r0,
+                     (const uint16_t*)q1, ldq1, (int)r1, M, K, kchunk, (uint16_t*)c, ldc, alpha);
+  return hipGetLastError() == hipSuccess ? kOk : kErrLaunch;
 }
 
 int cpt_gemm_bf16_skinny(const void* a, int64_t lda, const void* q, int64_t ldq, void* c,

@@ -272,9 +272,14 @@ def _gate_up_lora(x_2d, a_gate, b_gate, s_gate, a_up, b_up, s_up):
     """(xa_g | None, xa_u | None, ffn_gate_up keyword terms) for the fused
     gate/up GEMM.  With both adapters, x [A_g; A_u]^T is one pass over x: its
     column halves equal the two products bit for bit."""
-    if _stackable(a_gate, a_up) and x_2d.shape[0] >= 256 and x_2d.shape[1] >= 256:
+    n, h = x_2d.shape
+    small = G.skinny_small_pays(n, h)
+    if _stackable(a_gate, a_up) and h >= 256 and h % 8 == 0 and (small or n >= 256):
         r = a_gate.shape[0]
-        xa = _mm(x_2d, torch.cat([a_gate, a_up]).t(), "gemm_fwd_gate_up_xa")
+        if small:
+            xa = G.skinny_small(x_2d, a_gate, a_up, name="gemm_fwd_gate_up_xa")
+        else:
+            xa = _mm(x_2d, torch.cat([a_gate, a_up]).t(), "gemm_fwd_gate_up_xa")
         xa_g, xa_u = xa[:, :r], xa[:, r:]
     else:
         xa_g = _mm(x_2d, a_gate.t(), "gemm_fwd_gate_xa") if a_gate is not None else None

@@ -258,6 +258,8 @@ def skinny(a: torch.Tensor, q: torch.Tensor, alpha: float = 1.0,
         a = a.contiguous()
     if q.stride(1) != 1 or q.stride(0) % 8 or q.stride(0) < K or q.data_ptr() % 16:
         q = q.contiguous()
+    if out is None and skinny_small_pays(M, K):
+        return skinny_small(a, q, None, alpha, name)
     # K ranges for ~SKINNY_BLOCKS blocks of 128 rows (each range >= 256 of
     # K): more ranges cost more partials than they gain in parallelism
     blocks = (M + 127) // 128
@@ -275,6 +277,53 @@ def skinny(a: torch.Tensor, q: torch.Tensor, alpha: float = 1.0,
                                           q.stride(0), c.data_ptr(), c.stride(0), M, R, K,
                                           float(alpha), splits,
                                           None if ws is None else ws.data_ptr(), _stream(a))
+    check(rc, name)
+    return c
+
+
+# Where the projection is one launch of 16-row blocks whose 16 wavefronts split K
+# (skinny_small).  Kernel time on MI355X, us, one factor (two, stacked by a copy
+# for the two-launch kernel) against the two-launch kernel's:
+#   4 x 2048, rank 8       3.2 (3.9)   /  7.5 (11.1)
+#   1808 x 2048, rank 8    4.9 (5.3)   /  7.8 (12.4)
+#   4096 x 4096, rank 16   9.3 (13.7)  / 10.4 (17.7)
+#   512 x 5632, rank 8     9.7 (11.4)  /  8.1 (13.5)   and a launch fewer
+#   512 x 11008, rank 16  20.6 (30.3)  /  8.3 (14.3)
+#   8192 x 4096, rank 16  17.1 (26.0)  / 16.0 (23.4)
+SKINNY_SMALL_ROWS = 4096
+SKINNY_SMALL_K = 6144
+
+
+def skinny_small_pays(m: int, k: int) -> bool:
+    return m <= SKINNY_SMALL_ROWS and k <= SKINNY_SMALL_K
+
+
+def skinny_small(a: torch.Tensor, q0: torch.Tensor, q1: torch.Tensor | None = None,
+                 alpha: float = 1.0, name: str = "gemm_skinny") -> torch.Tensor:
+    """a [M, K] @ [q0; q1].T for 16-bit factors of r0 + r1 <= 32 rows, rounded as
+    skinny's, one launch; every column's sum runs in the same order whatever
+    the ranks are."""
+    _require_device(a, q0, q1)
+    dt = _check_16(a, q0)
+    M, K = a.shape
+
+    def rows(t):
+        ok = t.stride(1) == 1 and t.stride(0) % 8 == 0 and t.stride(0) >= K \
+            and t.data_ptr() % 16 == 0
+        return t if ok else t.contiguous()
+    a, q0 = rows(a), rows(q0)
+    r0, r1 = q0.shape[0], 0
+    assert q0.shape[1] == K
+    if q1 is not None:
+        q1 = rows(q1)
+        r1 = q1.shape[0]
+        assert q1.dtype == a.dtype and q1.shape[1] == K
+    c = torch.empty((M, r0 + r1), dtype=a.dtype, device=a.device)
+    with _timed(name):
+        rc = _lib.api().cpt_gemm16_skinny_small(
+            dt, a.data_ptr(), a.stride(0), q0.data_ptr(), q0.stride(0), r0,
+            None if q1 is None else q1.data_ptr(), 0 if q1 is None else q1.stride(0), r1,
+            c.data_ptr(), r0 + r1, M, K, alpha, _stream(a))
     check(rc, name)
     return c
 
@@ -320,6 +369,10 @@ def skinny_t(x: torch.Tensor, p: torch.Tensor, alpha: float = 1.0, trans: bool =
 # blocks were no better).  Fewer, longer token splits also cut the Z partials
 # by a third.
 SKINNY_DUAL_BLOCKS = 176
+# tokens per split at least: one piece.  At 1808 tokens 64 against 256: 12.8 /
+# 16.9 us over d_ff 5632, 12.1 / 16.2 over d_model 2048 (rank 8); level from 4096
+# tokens on, where the blocks bind.
+SKINNY_DUAL_TOKENS = 64
 
 
 def transpose_ok(x: torch.Tensor) -> bool:
@@ -379,7 +432,8 @@ def skinny_dual(x: torch.Tensor, q: torch.Tensor, p: torch.Tensor, alpha_c: floa
         p = p.contiguous()
     # blocks of 512 columns x T / splits tokens: ~SKINNY_DUAL_BLOCKS of them
     csplits = (N + 511) // 512
-    splits = max(1, min(max(T // 256, 1), (SKINNY_DUAL_BLOCKS + csplits - 1) // csplits))
+    splits = max(1, min(max(T // SKINNY_DUAL_TOKENS, 1),
+                        (SKINNY_DUAL_BLOCKS + csplits - 1) // csplits))
     per = (_SPAN_BYTES // (2 * max(x.stride(0), p.stride(0))) - 129) // 64 * 64
     assert per >= 64, "operand rows too long for 32-bit buffer offsets"
     splits = max(splits, (T + per - 1) // per)
@@ -536,8 +590,7 @@ def mm(a: torch.Tensor, b: torch.Tensor, name: str = "gemm") -> torch.Tensor:
     32-bit offsets."""
     M, K = a.shape
     N = b.shape[1]
-    if (N <= SKINNY_MAX_RANK and K >= 256 and K % 8 == 0 and M >= 256
-            and a.stride(1) == 1):
+    if N <= SKINNY_MAX_RANK and K >= 256 and K % 8 == 0 and a.stride(1) == 1:
         return skinny(a, b.t(), 1.0, name)
     if a.dtype == torch.float16:
         return mm2(a, b, None, None, name)

@@ -313,6 +313,11 @@ int cpt_gemm_bf16_lora(const void* a, int64_t lda, int a_kmajor, const void* b, 
 int cpt_gemm16_skinny(int dtype, const void* a, int64_t lda, const void* q, int64_t ldq, void* c,
                       int64_t ldc, int64_t M, int64_t R, int64_t K, float alpha, int splits,
                       void* workspace, void* stream);
+/* ... the projection for few tokens in one launch: C[M, r0 + r1] = alpha * A .
+ * [Q0; Q1]^T, Q0 [r0, K] and Q1 [r1, K] (either rank may be 0), r0 + r1 <= 32. */
+int cpt_gemm16_skinny_small(int dtype, const void* a, int64_t lda, const void* q0, int64_t ldq0,
+                            int64_t r0, const void* q1, int64_t ldq1, int64_t r1, void* c,
+                            int64_t ldc, int64_t M, int64_t K, float alpha, void* stream);
 int cpt_gemm16_skinny_t(int dtype, const void* x, int64_t ldx, const void* p, int64_t ldp,
                         void* out, int64_t ldo, int out_trans, int64_t T, int64_t N, int64_t R,
                         float alpha, int splits, void* workspace, void* stream);

@@ -153,3 +153,23 @@ def test_fp16_function_equals_general_layout_kernel(n, h, d, mode, rank, monkeyp
         err = (a.double() - b.double()).norm() / b.double().norm().clamp_min(1e-20)
         # a chain of some ten fp16 roundings (2^-11 each); int caches may flip codes on ties
         assert err < (2e-2 if mode == "int4" else 5e-3), err.item()
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,K", [(1, 8), (15, 264), (17, 512), (300, 1032), (64, 5632)])
+@pytest.mark.parametrize("r0,r1", [(8, 0), (1, 0), (8, 8), (16, 16), (24, 3)])
+def test_few_token_projection(dt, M, K, r0, r1):
+    """The one-launch projection: ragged tokens, K ranges that do not fill the 16
+    wavefronts, one and two factors; each factor's columns equal its own call's."""
+    from compact_amd import gemm as G
+    g = torch.Generator(device="cuda").manual_seed(M + K + r0)
+    x, a0, a1 = (torch.randn(s, device="cuda", generator=g).to(dt) for s in
+                 ((M, K), (r0, K), (max(r1, 1), K)))
+    got = G.skinny_small(x, a0, a1 if r1 else None, 0.5)
+    q = torch.cat([a0, a1]) if r1 else a0
+    ref = 0.5 * (x.double() @ q.double().t())
+    # one rounding (fp16: of the sum and of its half, exact), K 2^-24 |A| |Q|
+    half_ulp = 2.0 ** -8 if dt == torch.bfloat16 else 2.0 ** -11
+    bound = 0.5 * K * 2.0 ** -24 * (x.double().abs() @ q.double().abs().t()) + 2.0 ** -24
+    assert bool(((got.double() - ref).abs() <= 1.01 * half_ulp * ref.abs() + bound).all())
+    assert torch.equal(got[:, :r0], G.skinny_small(x, a0, None, 0.5))
