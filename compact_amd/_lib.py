@@ -50,6 +50,9 @@ SIGNATURES = {
                             _P],
     "cpt_gemm16_skinny_dual": [_I, _P, _L, _P, _L, _I, _P, _L, _P, _L, ctypes.c_float, _P, _L, _I,
                                ctypes.c_float, _L, _L, _L, _I, _P, _P],
+    "cpt_gemm16_skinny_dual2": [_I, _P, _P, _L, _P, _P, _L, _I, _P, _P, _L, _P, _P, _L,
+                                ctypes.c_float, _P, _P, _L, _I, ctypes.c_float, ctypes.c_float,
+                                _L, _L, _L, _I, _P, _P],
     "cpt_gemm16": [_I, _P, _L, _I, _P, _L, _I, _P, _L, _P, _L, _L, _P, _L, _L, _L, _L, _L, _L, _I,
                    _L, _P, _P, ctypes.c_float, _P, _P, ctypes.c_float, _I, _I, _P, _P],
     "cpt_ffn_gate_up16": [_I, _P, _P, _P, _L, _L, _L, _P, _P, _P, _L, _L, _P, _P, ctypes.c_float,

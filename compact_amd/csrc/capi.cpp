@@ -73,6 +73,7 @@ PyMethodDef methods[] = {
     CPT_ENTRY(cpt_gemm16_skinny_small),
     CPT_ENTRY(cpt_gemm16_skinny_t),
     CPT_ENTRY(cpt_gemm16_skinny_dual),
+    CPT_ENTRY(cpt_gemm16_skinny_dual2),
     CPT_ENTRY(cpt_gemm_bf16_skinny_dual_workspace_bytes),
     CPT_ENTRY(cpt_gemm_any),
     CPT_ENTRY(cpt_gemm_any_if),

@@ -441,26 +441,49 @@ __global__ __launch_bounds__(256) void skinny_red_reduce_kernel(const float* __r
   out[trans ? r * ldo + n : n * ldo + r] = scaled<DT>(alpha, sum);
 }
 
+// The dual pass of one tensor: see skinny_dual_kernel
+struct DualJob {
+  const uint16_t* x;
+  const uint16_t* q;
+  const uint16_t* p;
+  uint16_t* c;
+  uint16_t* z;
+  float* ws_c;
+  float* ws_z;
+  float alpha_c, alpha_z;
+};
+// One or two tensors of one shape and layout in one launch (the gate and up
+// gradients): blockIdx.z is the job.  A pass at few tokens is bound by its two
+// launches and by too few blocks, so two in one cost hardly more than one: d_ff
+// 5632, rank 8, two calls against one of both, with their sums: 21.5 / 10.9 us at
+// 128 tokens, 30.6 / 19.7 at 1808, 49.7 / 40.4 at 8192; d_ff 11008, rank 16, 8192
+// tokens (at the bandwidth): 102.5 / 94.6.
+struct DualJobs {
+  DualJob j[2];
+  int64_t ldx, ldq, ldp, ldc, ldz, T, N, tchunk;
+  int R, qmode, csplits, splits, z_trans;
+};
+
 // Both split sums of a skinny_dual pass in one launch: elements [0, T R) sum
 // the projection's column-block partials into C, the rest the reduction's
 // token-split partials into Z (each as the two kernels above)
 template <int DT>
-__global__ __launch_bounds__(256) void skinny_dual_reduce_kernel(
-    const float* __restrict__ ws_c, uint16_t* __restrict__ c, int64_t T, int64_t ldc,
-    int csplits, float alpha_c, const float* __restrict__ ws_z, uint16_t* __restrict__ z,
-    int64_t N, int64_t ldz, int z_trans, int splits, float alpha_z, int R) {
+__global__ __launch_bounds__(256) void skinny_dual_reduce_kernel(const DualJobs D) {
+  const DualJob& J = D.j[blockIdx.y];
+  const int64_t T = D.T, N = D.N;
+  const int R = D.R;
   const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (e < T * R) {
-    const float sum = sum_splits(ws_c + e, T * R, csplits);
+    const float sum = sum_splits(J.ws_c + e, T * R, D.csplits);
     const int64_t m = e / R, r = e - m * R;
-    c[m * ldc + r] = scaled<DT>(alpha_c, sum);
+    J.c[m * D.ldc + r] = scaled<DT>(J.alpha_c, sum);
     return;
   }
   const int64_t ez = e - T * R;
   if (ez >= N * R) return;
   const int64_t n = ez / R, r = ez % R;
-  const float sum = sum_splits(ws_z + ez, N * R, splits);
-  z[z_trans ? r * ldz + n : n * ldz + r] = scaled<DT>(alpha_z, sum);
+  const float sum = sum_splits(J.ws_z + ez, N * R, D.splits);
+  J.z[D.z_trans ? r * D.ldz + n : n * D.ldz + r] = scaled<DT>(J.alpha_z, sum);
 }
 
 // ---------------------------------------------------------------------------
@@ -493,10 +516,15 @@ constexpr int kDualLdP = 40;     // LDS row stride of the P piece (elements)
 constexpr int kDualQLd = 32;     // LDS row stride of the staged B slice (elements, R <= 32)
 
 template <int DT, int NB>
-__global__ __launch_bounds__(256) void skinny_dual_kernel(
-    const uint16_t* __restrict__ x, int64_t ldx, const uint16_t* __restrict__ q, int64_t ldq,
-    const uint16_t* __restrict__ p, int64_t ldp, int64_t T, int64_t N, int R, int64_t tchunk,
-    float* __restrict__ ws_c, float* __restrict__ ws_z, int qmode) {
+__global__ __launch_bounds__(256) void skinny_dual_kernel(const DualJobs D) {
+  const DualJob& J = D.j[blockIdx.z];
+  const uint16_t* const x = J.x;
+  const uint16_t* const q = J.q;
+  const uint16_t* const p = J.p;
+  float* const ws_c = J.ws_c;
+  float* const ws_z = J.ws_z;
+  const int64_t ldx = D.ldx, ldq = D.ldq, ldp = D.ldp, T = D.T, N = D.N, tchunk = D.tchunk;
+  const int R = D.R, qmode = D.qmode;
   __shared__ __attribute__((aligned(16))) uint16_t xs[kDualTok * kDualLd];
   __shared__ __attribute__((aligned(16))) uint16_t ps[kDualTok * kDualLdP];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -859,13 +887,34 @@ int cpt_gemm16_skinny_dual(int dtype, const void* x, int64_t ldx, const void* q,
                            float alpha_c, void* z, int64_t ldz, int z_trans, float alpha_z,
                            int64_t T, int64_t N, int64_t R, int splits, void* workspace,
                            void* stream) {
+  return cpt_gemm16_skinny_dual2(dtype, x, nullptr, ldx, q, nullptr, ldq, q_nr, p, nullptr, ldp, c,
+                                 nullptr, ldc, alpha_c, z, nullptr, ldz, z_trans, alpha_z, 0.0f, T,
+                                 N, R, splits, workspace, stream);
+}
+
+int cpt_gemm16_skinny_dual2(int dtype, const void* x0, const void* x1, int64_t ldx, const void* q0,
+                            const void* q1, int64_t ldq, int q_nr, const void* p0, const void* p1,
+                            int64_t ldp, void* c0, void* c1, int64_t ldc, float alpha_c, void* z0,
+                            void* z1, int64_t ldz, int z_trans, float alpha_z0, float alpha_z1,
+                            int64_t T, int64_t N, int64_t R, int splits, void* workspace,
+                            void* stream) {
   if (dtype != kBF16 && dtype != kF16) return kErrDType;
   if (T < 0 || N < 0 || R < 0 || splits < 1 || R > 32) return kErrShape;
   if (N == 0 || R == 0) return kOk;
-  if (!x || !q || !p || !c || !z || !workspace || !al16(x) || !al16(q) || !al16(p) ||
-      (ldx & 7) || (ldp & 7) || (N & 7) || (R & 7) || ldx < N || ldq < (q_nr ? R : N) ||
-      (!q_nr && (ldq & 7)) || ldp < R || ldc < R || ldz < (z_trans ? N : R) ||
-      ((uintptr_t)workspace & 3))
+  const void* const xs[2] = {x0, x1};
+  const void* const qs[2] = {q0, q1};
+  const void* const ps[2] = {p0, p1};
+  void* const cs[2] = {c0, c1};
+  void* const zs[2] = {z0, z1};
+  const int njobs = x1 ? 2 : 1;
+  for (int i = 0; i < njobs; ++i) {
+    if (!xs[i] || !qs[i] || !ps[i] || !cs[i] || !zs[i] || !al16(xs[i]) || !al16(qs[i]) ||
+        !al16(ps[i]))
+      return kErrAlign;
+  }
+  if (!workspace || (ldx & 7) || (ldp & 7) || (N & 7) || (R & 7) || ldx < N ||
+      ldq < (q_nr ? R : N) || (!q_nr && (ldq & 7)) || ldp < R || ldc < R ||
+      ldz < (z_trans ? N : R) || ((uintptr_t)workspace & 3))
     return kErrAlign;
   if ((q_nr ? N : 32) * ldq * 2 >= ((int64_t)1 << 31)) return kErrTooLarge;
   const int64_t tchunk =
@@ -879,31 +928,40 @@ int cpt_gemm16_skinny_dual(int dtype, const void* x, int64_t ldx, const void* q,
     return kErrTooLarge;
   const int64_t csplits = (N + kDualCols - 1) / kDualCols;
   if (csplits > 0x7FFFFFFF || splits > 65535) return kErrTooLarge;
-  float* ws_c = (float*)workspace;
-  float* ws_z = ws_c + csplits * T * R;
-  hipStream_t st = (hipStream_t)stream;
-  const dim3 grid((unsigned)csplits, (unsigned)splits);
+  DualJobs D{};
+  const int64_t per = csplits * T * R + (int64_t)splits * N * R;
+  for (int i = 0; i < njobs; ++i) {
+    float* const ws_c = (float*)workspace + i * per;
+    D.j[i] = DualJob{(const uint16_t*)xs[i], (const uint16_t*)qs[i], (const uint16_t*)ps[i],
+                     (uint16_t*)cs[i], (uint16_t*)zs[i], ws_c, ws_c + csplits * T * R, alpha_c,
+                     i ? alpha_z1 : alpha_z0};
+  }
+  D.ldx = ldx; D.ldq = ldq; D.ldp = ldp; D.ldc = ldc; D.ldz = ldz;
+  D.T = T; D.N = N; D.tchunk = tchunk;
+  D.R = (int)R;
+  D.csplits = (int)csplits;
+  D.splits = splits;
+  D.z_trans = z_trans ? 1 : 0;
   // Q's form in the kernel: 0 rank rows, 1 B as stored with 16-byte rows
   // (staged through LDS), 2 B as stored otherwise
-  const int qmode = !q_nr ? 0 : ((ldq & 7) == 0 && al16(q) ? 1 : 2);
+  D.qmode = !q_nr ? 0 : ((ldq & 7) == 0 ? 1 : 2);
+  hipStream_t st = (hipStream_t)stream;
   if (T > 0) {
+    const dim3 grid((unsigned)csplits, (unsigned)splits, (unsigned)njobs);
     const auto kern = dtype == kBF16
                           ? (R <= 16 ? skinny_dual_kernel<kBF16, 1> : skinny_dual_kernel<kBF16, 2>)
                           : (R <= 16 ? skinny_dual_kernel<kF16, 1> : skinny_dual_kernel<kF16, 2>);
-    hipLaunchKernelGGL(kern, grid, dim3(256), 0, st, (const uint16_t*)x, ldx, (const uint16_t*)q,
-                       ldq, (const uint16_t*)p, ldp, T, N, (int)R, tchunk, ws_c, ws_z, qmode);
+    hipLaunchKernelGGL(kern, grid, dim3(256), 0, st, D);
     if (hipGetLastError() != hipSuccess) return kErrLaunch;
   } else {
     // no tokens: C has no rows and Z is the empty sum (zero partials summed)
-    splits = 0;
+    D.splits = 0;
   }
   // both split sums in one launch
   const int64_t total = T * R + N * R;
   hipLaunchKernelGGL((dtype == kBF16 ? skinny_dual_reduce_kernel<kBF16>
                                      : skinny_dual_reduce_kernel<kF16>),
-                     dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st, (const float*)ws_c, (uint16_t*)c, T, ldc, (int)csplits, alpha_c,
-                     (const float*)ws_z, (uint16_t*)z, N, ldz, z_trans ? 1 : 0, splits, alpha_z,
-                     (int)R);
+                     dim3((unsigned)((total + 255) / 256), (unsigned)njobs), dim3(256), 0, st, D);
   return hipGetLastError() == hipSuccess ? kOk : kErrLaunch;
 }
 

@@ -321,7 +321,17 @@ def _thin_backward(grad_h_gate, b_gate, xa_g, s_gate, grad_h_up, b_up, xa_u, s_u
              and (_mfma(grad_h_gate, b_gate, grad_h_up, b_up)
                   or (G.f16_fits(grad_h_gate, b_gate) and G.f16_fits(grad_h_up, b_up)))
              and grad_h_gate.shape[1] >= 256)
-    if stack:
+    pair = None
+    if (stack and need_bg and need_bu and b_gate.shape == b_up.shape
+            and _dual_ok(grad_h_gate, b_gate, xa_g) and _dual_ok(grad_h_up, b_up, xa_u)):
+        # all four products in one launch, the same values
+        pair = G.skinny_dual_pair(grad_h_gate, b_gate.t(), xa_g, s_gate,
+                                  grad_h_up, b_up.t(), xa_u, s_up, "gemm_ghB_grad_b_gate_up")
+    if pair is not None:
+        r = b_gate.shape[1]
+        ghB, grad_b_gate, grad_b_up = pair
+        ghgB, ghuB = ghB[:, :r], ghB[:, r:]
+    elif stack:
         r = b_gate.shape[1]
         ghB = torch.empty((grad_h_gate.shape[0], r + b_up.shape[1]),
                           dtype=grad_h_gate.dtype, device=grad_h_gate.device)

@@ -406,6 +406,29 @@ def skinny_dual_ok(x: torch.Tensor, q: torch.Tensor, p: torch.Tensor) -> bool:
             and tuple(p.shape) == (T, R))
 
 
+def _dual_q(q: torch.Tensor):
+    """(q, q_nr, ldq): Q as rank rows [R][ld], or its transpose B [N][ld] as
+    stored (no copy)."""
+    R, N = q.shape
+    if q.stride(1) == 1 and q.stride(0) % 8 == 0 and q.stride(0) >= N and q.data_ptr() % 16 == 0:
+        return q, 0, q.stride(0)
+    if q.stride(0) == 1 and q.stride(1) >= R and q.data_ptr() % 16 == 0:
+        return q, 1, q.stride(1)
+    q = q.contiguous()
+    return q, 0, q.stride(0)
+
+
+def _dual_splits(T: int, N: int, ld: int) -> int:
+    """Token splits: blocks of 512 columns x T / splits tokens, about
+    SKINNY_DUAL_BLOCKS of them, each within 32-bit offsets."""
+    csplits = (N + 511) // 512
+    splits = max(1, min(max(T // SKINNY_DUAL_TOKENS, 1),
+                        (SKINNY_DUAL_BLOCKS + csplits - 1) // csplits))
+    per = (_SPAN_BYTES // (2 * ld) - 129) // 64 * 64
+    assert per >= 64, "operand rows too long for 32-bit buffer offsets"
+    return max(splits, (T + per - 1) // per)
+
+
 def skinny_dual(x: torch.Tensor, q: torch.Tensor, p: torch.Tensor, alpha_c: float = 1.0,
                 alpha_z: float = 1.0, out_c: torch.Tensor | None = None,
                 name: str = "gemm_skinny_dual"):
@@ -420,23 +443,10 @@ def skinny_dual(x: torch.Tensor, q: torch.Tensor, p: torch.Tensor, alpha_c: floa
     R = q.shape[0]
     if not _row_major(x) or x.stride(0) < N:
         x = x.contiguous()
-    # Q as rank rows [R][ld], or its transpose B [N][ld] as stored (no copy)
-    if q.stride(1) == 1 and q.stride(0) % 8 == 0 and q.stride(0) >= N and q.data_ptr() % 16 == 0:
-        q_nr, ldq = 0, q.stride(0)
-    elif q.stride(0) == 1 and q.stride(1) >= R and q.data_ptr() % 16 == 0:
-        q_nr, ldq = 1, q.stride(1)
-    else:
-        q = q.contiguous()
-        q_nr, ldq = 0, q.stride(0)
+    q, q_nr, ldq = _dual_q(q)
     if not _row_major(p) or p.stride(0) < R:
         p = p.contiguous()
-    # blocks of 512 columns x T / splits tokens: ~SKINNY_DUAL_BLOCKS of them
-    csplits = (N + 511) // 512
-    splits = max(1, min(max(T // SKINNY_DUAL_TOKENS, 1),
-                        (SKINNY_DUAL_BLOCKS + csplits - 1) // csplits))
-    per = (_SPAN_BYTES // (2 * max(x.stride(0), p.stride(0))) - 129) // 64 * 64
-    assert per >= 64, "operand rows too long for 32-bit buffer offsets"
-    splits = max(splits, (T + per - 1) // per)
+    splits = _dual_splits(T, N, max(x.stride(0), p.stride(0)))
     if out_c is None:
         c = torch.empty((T, R), dtype=x.dtype, device=x.device)
     else:
@@ -453,6 +463,38 @@ def skinny_dual(x: torch.Tensor, q: torch.Tensor, p: torch.Tensor, alpha_c: floa
             float(alpha_z), T, N, R, splits, ws.data_ptr(), _stream(x))
     check(rc, name)
     return c, z
+
+
+def skinny_dual_pair(x0: torch.Tensor, q0: torch.Tensor, p0: torch.Tensor, alpha0: float,
+                     x1: torch.Tensor, q1: torch.Tensor, p1: torch.Tensor, alpha1: float,
+                     name: str = "gemm_skinny_dual_pair"):
+    """skinny_dual of two tensors of one shape, both passes in one launch and
+    their split sums in another (bit for bit the two calls' results): returns
+    ([x0 q0^T | x1 q1^T] side by side [T, 2 R], alpha0 x0^T p0 [N, R],
+    alpha1 x1^T p1 [N, R]), or None where the two do not share a layout."""
+    T, N = x0.shape
+    R = q0.shape[0]
+    q0, q_nr, ldq = _dual_q(q0)
+    q1, *lay1 = _dual_q(q1)
+    if (lay1 != [q_nr, ldq] or x0.stride() != x1.stride() or p0.stride() != p1.stride()
+            or not _row_major(x0) or not _row_major(x1) or x0.stride(0) < N
+            or not _row_major(p0) or not _row_major(p1) or p0.stride(0) < R):
+        return None
+    _require_device(x0, q0, p0, x1, q1, p1)
+    splits = _dual_splits(T, N, max(x0.stride(0), p0.stride(0)))
+    c = torch.empty((T, 2 * R), dtype=x0.dtype, device=x0.device)
+    z0 = torch.empty((N, R), dtype=x0.dtype, device=x0.device)
+    z1 = torch.empty((N, R), dtype=x0.dtype, device=x0.device)
+    nbytes = _lib.api().cpt_gemm_bf16_skinny_dual_workspace_bytes(T, N, R, splits)
+    ws = torch.empty((max(nbytes, 4) // 2,), dtype=torch.float32, device=x0.device)
+    with _timed(name):
+        rc = _lib.api().cpt_gemm16_skinny_dual2(
+            _DT16[x0.dtype], x0.data_ptr(), x1.data_ptr(), x0.stride(0), q0.data_ptr(),
+            q1.data_ptr(), ldq, q_nr, p0.data_ptr(), p1.data_ptr(), p0.stride(0), c.data_ptr(),
+            c.data_ptr() + 2 * R, 2 * R, 1.0, z0.data_ptr(), z1.data_ptr(), R, 0, float(alpha0),
+            float(alpha1), T, N, R, splits, ws.data_ptr(), _stream(x0))
+    check(rc, name)
+    return c, z0, z1
 
 
 def skinny_t_splits(T: int, N: int) -> int:

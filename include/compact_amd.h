@@ -327,6 +327,15 @@ int cpt_gemm16_skinny_dual(int dtype, const void* x, int64_t ldx, const void* q,
                            int64_t T, int64_t N, int64_t R, int splits, void* workspace,
                            void* stream);
 
+/* ... the dual pass of two tensors of one shape and layout (x1 NULL: of one) in
+ * one launch; the workspace holds that of the one tensor for each. */
+int cpt_gemm16_skinny_dual2(int dtype, const void* x0, const void* x1, int64_t ldx, const void* q0,
+                            const void* q1, int64_t ldq, int q_nr, const void* p0, const void* p1,
+                            int64_t ldp, void* c0, void* c1, int64_t ldc, float alpha_c, void* z0,
+                            void* z1, int64_t ldz, int z_trans, float alpha_z0, float alpha_z1,
+                            int64_t T, int64_t N, int64_t R, int splits, void* workspace,
+                            void* stream);
+
 /* cpt_gemm_bf16_lora's product (rank 0: cpt_gemm_bf16's) on 128 x 128 tiles for
  * bf16 or fp16 operands and results (dtype CPT_BF16 / CPT_F16 codes 2 / 1), K
  * a multiple of 64 (two MN-major operands: any K), N of 8.  splits > 1 shares

@@ -173,3 +173,28 @@ def test_few_token_projection(dt, M, K, r0, r1):
     bound = 0.5 * K * 2.0 ** -24 * (x.double().abs() @ q.double().abs().t()) + 2.0 ** -24
     assert bool(((got.double() - ref).abs() <= 1.01 * half_ulp * ref.abs() + bound).all())
     assert torch.equal(got[:, :r0], G.skinny_small(x, a0, None, 0.5))
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("b_form", ["rank_rows", "b", "b_ragged"])
+@pytest.mark.parametrize("T,N,R", [(1, 512, 8), (65, 520, 16), (300, 1032, 8), (1000, 5632, 16)])
+def test_dual_pair_equals_two_calls(device, dt, b_form, T, N, R):
+    """Both gradients' dual passes in one launch: the two calls' bits, with Q as
+    rank rows and as B with rows that are and are not 16-byte multiples; layouts
+    that differ are left to two calls."""
+    G = _G()
+    xs = [rnd((T, N), s, device).to(dt) for s in (1, 2)]
+    qs = [rnd((R, N), s, device, 0.05).to(dt) for s in (3, 4)]
+    if b_form == "b":
+        qs = [q.t().contiguous().t() for q in qs]
+    elif b_form == "b_ragged":
+        qs = [torch.empty(N, R + 3, dtype=dt, device=device)[:, :R].copy_(q.t()).t() for q in qs]
+    ps = rnd((T, 2 * R), 5, device).to(dt)
+    ps = [ps[:, :R], ps[:, R:]]
+    c, z0, z1 = G.skinny_dual_pair(xs[0], qs[0], ps[0], 0.5, xs[1], qs[1], ps[1], 2.0)
+    for x, q, p, a, half, z in zip(xs, qs, ps, (0.5, 2.0), (c[:, :R], c[:, R:]), (z0, z1)):
+        c_alone, z_alone = G.skinny_dual(x, q, p, 1.0, a)
+        assert torch.equal(half, c_alone) and torch.equal(z, z_alone)
+    wide = torch.zeros(T, N + 8, dtype=dt, device=device)[:, :N].copy_(xs[1])
+    if T > 1:
+        assert G.skinny_dual_pair(xs[0], qs[0], ps[0], 0.5, wide, qs[1], ps[1], 2.0) is None
