@@ -10,14 +10,18 @@ namespace gemm {
 CPT_GEMM_INST_ALL(CPT_GEMM_DECLARE)
 CPT_NT16_INST_ALL(CPT_NT16_DECLARE)
 CPT_ST16_INST_ALL(CPT_ST16_DECLARE)
-extern template int launch_nt16_f32<true, true, false>(KArgs, hipStream_t);
-extern template int launch_nt16_f32<true, false, false>(KArgs, hipStream_t);
-extern template int launch_nt16_f32<false, false, false>(KArgs, hipStream_t);
-extern template int launch_nt16_f32<false, true, false>(KArgs, hipStream_t);
-extern template int launch_nt16_f32<true, true, true>(KArgs, hipStream_t);
-extern template int launch_nt16_f32<true, false, true>(KArgs, hipStream_t);
-extern template int launch_nt16_f32<false, false, true>(KArgs, hipStream_t);
-extern template int launch_nt16_f32<false, true, true>(KArgs, hipStream_t);
+extern template int launch_nt16_f32<true, true, false, 8>(KArgs, hipStream_t);
+extern template int launch_nt16_f32<true, false, false, 8>(KArgs, hipStream_t);
+extern template int launch_nt16_f32<false, false, false, 8>(KArgs, hipStream_t);
+extern template int launch_nt16_f32<false, true, false, 8>(KArgs, hipStream_t);
+extern template int launch_nt16_f32<true, true, true, 8>(KArgs, hipStream_t);
+extern template int launch_nt16_f32<true, false, true, 8>(KArgs, hipStream_t);
+extern template int launch_nt16_f32<false, false, true, 8>(KArgs, hipStream_t);
+extern template int launch_nt16_f32<false, true, true, 8>(KArgs, hipStream_t);
+extern template int launch_nt16_f32<true, true, true, 6>(KArgs, hipStream_t);
+extern template int launch_nt16_f32<true, false, true, 6>(KArgs, hipStream_t);
+extern template int launch_nt16_f32<false, false, true, 6>(KArgs, hipStream_t);
+extern template int launch_nt16_f32<false, true, true, 6>(KArgs, hipStream_t);
 
 // out[m, n] = bf16(alpha * sum_s ws[s][m][n])  (split-K reduction, fixed order)
 __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restrict__ ws,
@@ -397,10 +401,10 @@ int gemm16_impl(const void* a, int64_t lda, int a_kmajor, const void* b, int64_t
     A.ldc = N;
     int rc;
     if (big)
-      rc = a_kmajor ? (b_kmajor ? launch_nt16_f32<true, true, false>(A, st)
-                                : launch_nt16_f32<true, false, false>(A, st))
-                    : (b_kmajor ? launch_nt16_f32<false, true, false>(A, st)
-                                : launch_nt16_f32<false, false, false>(A, st));
+      rc = a_kmajor ? (b_kmajor ? launch_nt16_f32<true, true, false, 8>(A, st)
+                                : launch_nt16_f32<true, false, false, 8>(A, st))
+                    : (b_kmajor ? launch_nt16_f32<false, true, false, 8>(A, st)
+                                : launch_nt16_f32<false, false, false, 8>(A, st));
     else if (a_kmajor && b_kmajor)
       rc = launch_small<DT, true, true, EPI_F32, CACHE_NONE, 0>(A, st);
     else if (a_kmajor) rc = launch_small<DT, true, false, EPI_F32, CACHE_NONE, 0>(A, st);
@@ -463,7 +467,8 @@ int x3_gemm_impl(const void* a, int64_t plane_a, int64_t lda, int a_kmajor, cons
   // the six plane products of every k-tile, split together
   const int nk = 6 * (int)((K + 63) / 64 + (two ? (K2 + 63) / 64 : 0));
   if (splits > nk) splits = nk;
-  const bool big = tiles == 256;
+  // 192: tiles of 256 rows and 192 columns
+  const bool big = tiles == 256 || tiles == 192;
   if (tiles != 128 && !big) return kErrShape;
   if (big && (K % 64 || K2 % 64)) return kErrShape;
   A.kt_per_split = (nk + splits - 1) / splits;
@@ -474,11 +479,15 @@ int x3_gemm_impl(const void* a, int64_t plane_a, int64_t lda, int a_kmajor, cons
   A.alpha = A.ksplit > 1 ? 1.0f : alpha;
   hipStream_t st = (hipStream_t)stream;
   int rc;
-  if (big)
-    rc = a_kmajor ? (b_kmajor ? launch_nt16_f32<true, true, true>(A, st)
-                              : launch_nt16_f32<true, false, true>(A, st))
-                  : (b_kmajor ? launch_nt16_f32<false, true, true>(A, st)
-                              : launch_nt16_f32<false, false, true>(A, st));
+  const auto on_256 = [&](auto ni) {
+    constexpr int NI = decltype(ni)::value;
+    return a_kmajor ? (b_kmajor ? launch_nt16_f32<true, true, true, NI>(A, st)
+                                : launch_nt16_f32<true, false, true, NI>(A, st))
+                    : (b_kmajor ? launch_nt16_f32<false, true, true, NI>(A, st)
+                                : launch_nt16_f32<false, false, true, NI>(A, st));
+  };
+  if (tiles == 192) rc = on_256(std::integral_constant<int, 6>{});
+  else if (big) rc = on_256(std::integral_constant<int, 8>{});
   else if (a_kmajor && b_kmajor) rc = launch_small<kF32, true, true, EPI_F32, CACHE_NONE, 0>(A, st);
   else if (a_kmajor) rc = launch_small<kF32, true, false, EPI_F32, CACHE_NONE, 0>(A, st);
   else if (b_kmajor) rc = launch_small<kF32, false, true, EPI_F32, CACHE_NONE, 0>(A, st);

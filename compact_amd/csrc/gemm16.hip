@@ -67,6 +67,27 @@ bool stream_k_plan(int64_t tiles, int nk, StreamK& sk) {
   return true;
 }
 
+// 256 x 192 tiles: a block takes 0.84 of the time of a 256 x 256 one (0.75 of its
+// products, but 7/8 of its operand loads and LDS reads), so they pay where they
+// need no more rounds of one block per CU, which is where the wide tiles leave a
+// quarter or more of the last round empty.  Measured (256 CUs), us on 256 / 192
+// columns, the same bits:
+//   2048 x 5632, k 8192   (176 / 240 blocks)   172.3 / 144.7
+//   5632 x 2048, k 8192   (176 / 242)          184.8 / 161.6
+//   2048 x 5632, k 2048   (176 / 240)           44.9 /  39.4
+//   5632 x 4096, k 4096   (352 / 484)          171.7 / 148.3
+// With a round more than the wide tiles they are level at best (4 of 192 against
+// 3 of 256).
+bool use_192(const KArgs& A, bool a_kmajor) {
+  const int cus = num_cus();
+  if (cus <= 0) return false;
+  const int64_t wide = (int64_t)A.tiles_m * A.tiles_n;
+  // a K-major A's part-empty last round past the first is shared by stream-K
+  if (a_kmajor && wide > cus) return false;
+  const int64_t narrow = (int64_t)A.tiles_m * ((A.N + 191) / 192);
+  return (narrow + cus - 1) / cus <= (wide + cus - 1) / cus;
+}
+
 CPT_NT16_INST_STORE(CPT_NT16_DEFINE)
 
 }  // namespace gemm

@@ -24,7 +24,10 @@
 //
 // Block: 256 threads (4 waves, one per SIMD), a 256 x 256 output tile, k
 // steps of 64; wave w owns C rows 128 (w / 2) .. +127 and columns
-// 128 (w % 2) .. +127 as 8 x 8 MFMA blocks of 16 x 16.
+// 128 (w % 2) .. +127 as 8 x 8 MFMA blocks of 16 x 16.  Plain stores and fp32
+// products also have 256 x 192 tiles (NI = 6 column blocks per wave; the same
+// stages and swizzles, 96 slots a k-tile), for outputs whose 256 x 256 tiles
+// leave CUs idle; the products of an element and their order are the same.
 //
 // LDS: 2 stages x 2 operands x [256 rows][64 k] bf16, unpadded, 128 KiB.
 // Row r keeps its 8 chunks of 8 k-values at chunk position c ^ (r & 6): a
@@ -35,7 +38,8 @@
 // load fetches row 8 q + l / 8, chunk (l % 8) ^ (row & 6) into LDS row
 // 8 q + l / 8, chunk position l % 8.
 //
-// Schedule of one k-tile kt (stage s = kt & 1) over its 128 MFMA slots t:
+// Schedule of one k-tile kt (stage s = kt & 1) over its 128 MFMA slots t (256
+// columns; Sched has both):
 //   t < 64   sub-step 0 (k 0..31) on fragment set F0, in triangular (i, j)
 //            order so the first MFMAs need only the first fragments read;
 //   t >= 64  sub-step 1 (k 32..63) on F1;
@@ -74,27 +78,44 @@ constexpr int kMax2 = kMainLds > kOutLds ? kMainLds : kOutLds;
 constexpr int kLds = kMax2 > kGluLdsBytes ? kMax2 : kGluLdsBytes;
 static_assert(kLds <= 160 * 1024, "LDS per block");
 
-constexpr int kBarA = 34;                         // first slot after barrier A
-constexpr int kLdEvery = 6;                       // slots between loads of one tile
-constexpr int kBarB = 96;                         // first slot after barrier B
-constexpr int kLoadsBeforeB = (kBarB - 1 - kBarA) / kLdEvery + 1;
-static_assert(kBarA - 1 > 2 * 15, "barrier A follows the last F1 read");
-static_assert(kBarA + kLdEvery * 15 < 128, "every load of a tile inside the tile");
-static_assert(kBarB + 2 * 15 < 128, "F0 reads inside the tile");
-static_assert(kLoadsBeforeB <= 16, "vmcnt of barrier B");
+// A tile is 32 NI columns wide: NI = 8 column blocks per wave for 256, 6 for 192
+// (see use_192).  Sched: the slots of a k-tile's schedule.
+template <int NI, bool BK>
+struct Sched {
+  static constexpr int kSub = NI * 8;                     // slots of a sub-step
+  static constexpr int kSlots = 2 * kSub;
+  static constexpr int kFrags = NI + 8;                   // fragments of a sub-step
+  // loads of B: a row block each (K-major), or all 8 of a 256-column stage whose
+  // columns past the tile read nothing (MN-major)
+  static constexpr int kLoadsB = BK ? NI : 8;
+  static constexpr int kLoads = 8 + kLoadsB;
+  static constexpr int kBarA = 2 * kFrags + 2;            // first slot after barrier A
+  static constexpr int kLdEvery = NI == 8 ? 6 : 4;        // slots between loads of one tile
+  static constexpr int kBarB = kSlots - 2 * kFrags;       // first slot after barrier B
+  static constexpr int kLoadsBeforeB = (kBarB - 1 - kBarA) / kLdEvery + 1;
+  static_assert(kBarA - 1 > 2 * (kFrags - 1), "barrier A follows the last F1 read");
+  static_assert(kBarA + kLdEvery * (kLoads - 1) < kSlots, "every load of a tile inside the tile");
+  static_assert(kBarB >= kSub, "F0 is read again once sub-step 0 is done");
+  static_assert(kBarB + 2 * (kFrags - 1) < kSlots, "F0 reads inside the tile");
+  static_assert(kLoadsBeforeB <= kLoads, "vmcnt of barrier B");
+};
 
-// sub-step 0 order: (i, j) over 8 x 8 blocks, block n = max(i, j) ascending
+// sub-step 0 order: (i, j) over NI x 8 blocks, block n = max(i, j) ascending
+template <int NI>
 struct Order {
-  uint8_t i[64], j[64];
+  uint8_t i[NI * 8], j[NI * 8];
   constexpr Order() : i(), j() {
     int t = 0;
     for (int n = 0; n < 8; ++n) {
-      for (int q = 0; q < n; ++q) { i[t] = n; j[t] = q; ++t; }
-      for (int q = 0; q < n; ++q) { i[t] = q; j[t] = n; ++t; }
-      i[t] = n; j[t] = n; ++t;
+      for (int q = 0; q < n && n < NI; ++q) { i[t] = n; j[t] = q; ++t; }
+      for (int q = 0; q < n && q < NI; ++q) { i[t] = q; j[t] = n; ++t; }
+      if (n < NI) { i[t] = n; j[t] = n; ++t; }
     }
   }
 };
+// Fragment (and load) p of a sequence that alternates B and A while there is a B
+// block left: 2 x block + (0: B, 1: A)
+constexpr int alternate(int p, int nb) { return p < 2 * nb ? p : 2 * (p - nb) + 1; }
 
 __device__ __forceinline__ int lds_off(int row, int chunk) {
   return row * kBK + ((chunk ^ (row & 6)) << 3);
@@ -284,13 +305,18 @@ constexpr int kSkSpin = 1 << 22;
 // the six plane pairs of each operand pair, the smallest products first (see
 // gemm16s_kernel.h), and the epilogue (EPI_F32) writes fp32 to A.ws, split sk_s
 // of it.
-template <bool AK, bool BK, int EPI, int CACHE, int GS, int LT, bool SK, bool HI, bool X3 = false>
+template <bool AK, bool BK, int EPI, int CACHE, int GS, int LT, bool SK, bool HI, bool X3 = false,
+          int NI = 8>
 __device__ __forceinline__ void nt16_tile(const KArgs& A, uint16_t* lds, int tm, int tn, int kb,
                                           int ke, int role, int sk_s) {
   static_assert(LT == 0 || AK, "adapter terms ride with a K-major A (P's rows are tokens)");
   static_assert(EPI == EPI_STORE || EPI == EPI_GLU || EPI == EPI_DGLU || EPI == EPI_GLUO ||
                     EPI == EPI_F32,
                 "epilogues of the 16x16x32 loop");
+  static_assert(NI == 8 || (LT == 0 && !SK && (EPI == EPI_STORE || X3)),
+                "192 columns: plain stores and fp32 products");
+  using S = Sched<NI, BK>;
+  constexpr int kTileN = 32 * NI;
   static_assert(!X3 || EPI == EPI_F32, "fp32 products write fp32");
   static_assert(EPI != EPI_DGLU || (AK && !BK), "B1: gy (K-major) . W_d (MN-major)");
   constexpr bool DUAL = EPI == EPI_GLU || EPI == EPI_GLUO;
@@ -301,7 +327,7 @@ __device__ __forceinline__ void nt16_tile(const KArgs& A, uint16_t* lds, int tm,
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wn = wave & 1, wm = wave >> 1;
-  const int64_t m0 = (int64_t)tm * 256, n0 = (int64_t)tn * 256;
+  const int64_t m0 = (int64_t)tm * 256, n0 = (int64_t)tn * kTileN;
   // k-tiles [kb, ke) of the tile; [0, nk0) come from pair 0, the rest from
   // pair 1 (K-concatenated)
   const int nk0 = (int)(A.K[0] / kBK);
@@ -348,7 +374,9 @@ __device__ __forceinline__ void nt16_tile(const KArgs& A, uint16_t* lds, int tm,
     oa[i] = AK ? (uint32_t)(((int64_t)r * lda + ck * 8) * 2)
                : m0 + cm * 8 < A.M ? (uint32_t)(((int64_t)kr * lda + cm * 8) * 2) : kOOB;
     ob[i] = BK ? (uint32_t)(((int64_t)rw * ldb + ck * 8) * 2)
-               : n0 + cm * 8 < A.N ? (uint32_t)(((int64_t)kr * ldb + cm * 8) * 2) : kOOB;
+               : cm * 8 < kTileN && n0 + cm * 8 < A.N
+                   ? (uint32_t)(((int64_t)kr * ldb + cm * 8) * 2)
+                   : kOOB;
   }
   // per k-tile: the pair's buffers and each operand's byte delta (k0 * 2 for a
   // K-major operand, k0 * ld * 2 for an MN-major one), passed as soffset.  The
@@ -407,17 +435,18 @@ __device__ __forceinline__ void nt16_tile(const KArgs& A, uint16_t* lds, int tm,
     }
     return t;
   };
-  // load p (0..15) of a tile into stage st: even p -> A block p / 2, odd -> B
+  // load p of a tile into stage st: A and B in turn, then what is left of A
   auto issue = [&](int p, int st, const TileLd& T) {
-    const int i = p >> 1;
-    uint16_t* dst = lds + (st * 2 + (p & 1)) * kStage + (4 * i + wave) * 512;
-    if (p & 1) load_lds(DUAL && ((i >> 1) & 1) ? rbu : T.b, dst, ob[i], T.db);
+    const bool bside = p < 2 * S::kLoadsB && (p & 1);
+    const int i = alternate(p, S::kLoadsB) >> 1;
+    uint16_t* dst = lds + (st * 2 + (bside ? 1 : 0)) * kStage + (4 * i + wave) * 512;
+    if (bside) load_lds(DUAL && ((i >> 1) & 1) ? rbu : T.b, dst, ob[i], T.db);
     else load_lds(T.a, dst, oa[i], T.da);
   };
 
-  f32x4 acc[8][8];
+  f32x4 acc[NI][8];
 #pragma unroll
-  for (int i = 0; i < 8; ++i)
+  for (int i = 0; i < NI; ++i)
 #pragma unroll
     for (int j = 0; j < 8; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 
@@ -429,9 +458,9 @@ __device__ __forceinline__ void nt16_tile(const KArgs& A, uint16_t* lds, int tm,
   //     reads k-row 8 (l / 16) + (l' % 16) / 4 (+ 4), columns 4 (l' % 4) .. + 3 of
   //     the block; the chunk position is 16 w + 2 (block ^ f') + (l % 4) / 2 with
   //     f' = mn_swz(k-row) / 2, the same for both reads and both sub-steps.
-  const int nofs0 = lds_off(wn * 128 + (lane & 15), lane >> 4);
+  const int nofs0 = lds_off(wn * (kTileN / 2) + (lane & 15), lane >> 4);
   const int mofs0 = lds_off(wm * 128 + (lane & 15), lane >> 4);
-  const int nofs1 = lds_off(wn * 128 + (lane & 15), (lane >> 4) + 4);
+  const int nofs1 = lds_off(wn * (kTileN / 2) + (lane & 15), (lane >> 4) + 4);
   const int mofs1 = lds_off(wm * 128 + (lane & 15), (lane >> 4) + 4);
   const int mn_lane = (8 * (lane >> 4) + ((lane & 15) >> 2)) * 256 + ((lane & 3) >> 1) * 8 + (lane & 1) * 4;
   const int mn_fx = 8 * mn_swz(8 * (lane >> 4) + ((lane & 15) >> 2));   // 16 f'
@@ -443,8 +472,10 @@ __device__ __forceinline__ void nt16_tile(const KArgs& A, uint16_t* lds, int tm,
       const int o = bside ? kStage + (s ? nofs1 : nofs0) : (s ? mofs1 : mofs0);
       return *reinterpret_cast<const bf16x8*>(base + o + (q >> 1) * 16 * kBK);
     }
-    const uint16_t* p = base + (bside ? kStage + 128 * wn : 128 * wm) + mn_lane + s * 32 * 256 +
-                        ((16 * (q >> 1)) ^ mn_fx);
+    // the swizzle moves a block within 8 of them: 128 columns apart it commutes
+    const int blk = bside && NI != 8 ? NI * wn + (q >> 1) : q >> 1;
+    const uint16_t* p = base + (!bside ? 128 * wm : NI == 8 ? kStage + 128 * wn : kStage) + mn_lane +
+                        s * 32 * 256 + ((16 * blk) ^ mn_fx);
     const i16x4 lo = lds_read_tr(p);
     const i16x4 hi = lds_read_tr(p + 4 * 256);
     return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
@@ -454,40 +485,48 @@ __device__ __forceinline__ void nt16_tile(const KArgs& A, uint16_t* lds, int tm,
   {
     const TileLd T0 = X3 ? x3_next() : tile(kb), T1 = X3 ? x3_next() : tile(kb + 1);
 #pragma unroll
-    for (int p = 0; p < 16; ++p) issue(p, 0, T0);
+    for (int p = 0; p < S::kLoads; ++p) issue(p, 0, T0);
 #pragma unroll
-    for (int p = 0; p < 16; ++p) issue(p, 1, T1);
+    for (int p = 0; p < S::kLoads; ++p) issue(p, 1, T1);
   }
-  asm volatile("s_waitcnt vmcnt(16)\n\ts_barrier" ::: "memory");
+  asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(S::kLoads) : "memory");
   __builtin_amdgcn_sched_barrier(0);
   // read order pinned so the loop header's merged waits stay counts, not lgkmcnt(0)
 #pragma unroll
-  for (int q = 0; q < 16; ++q) {
+  for (int n = 0; n < S::kFrags; ++n) {
+    const int q = alternate(n, NI);
     f0[q] = rd(0, 0, q);
     __builtin_amdgcn_sched_barrier(0);
   }
 
-  constexpr Order ord;
+  constexpr Order<NI> ord;
   for (int kt = kb; kt < ke; ++kt) {
     const int stage = (kt - kb) & 1;
     const TileLd T2 = X3 ? x3_next() : tile(kt + 2);
-    static_for<0, 128>([&](auto tc) {
+    static_for<0, S::kSlots>([&](auto tc) {
       constexpr int t = decltype(tc)::value;
-      if constexpr (t < 64) {
+      if constexpr (t < S::kSub) {
         constexpr int i = ord.i[t], j = ord.j[t];
         mfma(acc[i][j], f0[2 * i], f0[2 * j + 1]);
       } else {
-        constexpr int i = (t - 64) >> 3, j = (t - 64) & 7;
+        constexpr int i = (t - S::kSub) >> 3, j = (t - S::kSub) & 7;
         mfma(acc[i][j], f1[2 * i], f1[2 * j + 1]);
       }
-      if constexpr (t % 2 == 0 && t / 2 < 16) f1[t / 2] = rd(stage, 1, t / 2);
-      if constexpr (t == kBarA - 1) asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-      if constexpr (t >= kBarA && (t - kBarA) % kLdEvery == 0 && (t - kBarA) / kLdEvery < 16)
-        issue((t - kBarA) / kLdEvery, stage, T2);
-      if constexpr (t == kBarB - 1)
-        asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(kLoadsBeforeB) : "memory");
-      if constexpr (t >= kBarB && (t - kBarB) % 2 == 0 && (t - kBarB) / 2 < 16)
-        f0[(t - kBarB) / 2] = rd(stage ^ 1, 0, (t - kBarB) / 2);
+      if constexpr (t % 2 == 0 && t / 2 < S::kFrags) {
+        constexpr int q = alternate(t / 2, NI);
+        f1[q] = rd(stage, 1, q);
+      }
+      if constexpr (t == S::kBarA - 1)
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+      if constexpr (t >= S::kBarA && (t - S::kBarA) % S::kLdEvery == 0 &&
+                    (t - S::kBarA) / S::kLdEvery < S::kLoads)
+        issue((t - S::kBarA) / S::kLdEvery, stage, T2);
+      if constexpr (t == S::kBarB - 1)
+        asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(S::kLoadsBeforeB) : "memory");
+      if constexpr (t >= S::kBarB && (t - S::kBarB) % 2 == 0 && (t - S::kBarB) / 2 < S::kFrags) {
+        constexpr int q = alternate((t - S::kBarB) / 2, NI);
+        f0[q] = rd(stage ^ 1, 0, q);
+      }
       __builtin_amdgcn_sched_barrier(0);
     });
   }
@@ -551,8 +590,8 @@ __device__ __forceinline__ void nt16_tile(const KArgs& A, uint16_t* lds, int tm,
   if constexpr (EPI == EPI_F32) {
     float* const out = A.ws + (int64_t)sk_s * A.M * A.ldc;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int64_t n = n0 + wn * 128 + 16 * i + 4 * (elane >> 4);
+    for (int i = 0; i < NI; ++i) {
+      const int64_t n = n0 + wn * (kTileN / 2) + 16 * i + 4 * (elane >> 4);
       if (n >= A.N) continue;   // N % 8 == 0
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
@@ -574,7 +613,7 @@ __device__ __forceinline__ void nt16_tile(const KArgs& A, uint16_t* lds, int tm,
     // on it row by row.
     static_assert(kLdOut == kDgluLd, "B1's staged tile layout");
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
+    for (int i = 0; i < NI; ++i) {
       // a stream-K finisher adds the other block's partial, 8 blocks at a time
       f32x4 pv[8];
       if (part) {
@@ -586,7 +625,7 @@ __device__ __forceinline__ void nt16_tile(const KArgs& A, uint16_t* lds, int tm,
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
         const int ml = wm * 128 + 16 * j + (elane & 15);
-        const int nl = wn * 128 + 16 * i + 4 * (elane >> 4);
+        const int nl = wn * (kTileN / 2) + 16 * i + 4 * (elane >> 4);
         f32x4 base = acc[i][j];
         // one block's accumulators at a time: read all at once, the 256
         // accumulator copies spilled the values that live across the loop
@@ -605,7 +644,7 @@ __device__ __forceinline__ void nt16_tile(const KArgs& A, uint16_t* lds, int tm,
     // ragged M and N: rows past M and 8-column pieces past N (N % 8 == 0) stay
     // unwritten; the operand loads read zeros or discarded values there
     const int cl = (etid & 31) * 8;
-    const bool nok = n0 + cl < A.N;
+    const bool nok = cl < kTileN && n0 + cl < A.N;
 #pragma unroll 4
     for (int p = 0; p < 32; ++p) {
       const int r = p * 8 + (etid >> 5);
@@ -638,7 +677,7 @@ __device__ __forceinline__ void nt16_tile(const KArgs& A, uint16_t* lds, int tm,
 // one whole tile per block.  Two kernels, so the one-tile-per-block kernel
 // keeps its own register allocation.  HI: adapter ranks 17..32 (a third
 // kernel, one tile per block).
-template <bool AK, bool BK, int EPI, int CACHE, int GS, int LT, bool SK, bool HI = false>
+template <bool AK, bool BK, int EPI, int CACHE, int GS, int LT, bool SK, bool HI = false, int NI = 8>
 __global__ __launch_bounds__(kThreads, 1) void nt16_kernel(const KArgs A) {
   static_assert(!SK || (EPI == EPI_STORE && AK), "stream-K: plain store, K-major A");
   static_assert(!HI || (LT > 0 && !SK), "ranks above 16: adapter kernels, one tile per block");
@@ -648,7 +687,7 @@ __global__ __launch_bounds__(kThreads, 1) void nt16_kernel(const KArgs A) {
   if constexpr (!SK) {
     int tm, tn;
     tile_coords_of(b, gridDim.x, A.tiles_m, A.tiles_n, tm, tn);
-    nt16_tile<AK, BK, EPI, CACHE, GS, LT, SK, HI>(A, lds, tm, tn, 0, nk, kRoleWhole, 0);
+    nt16_tile<AK, BK, EPI, CACHE, GS, LT, SK, HI, false, NI>(A, lds, tm, tn, 0, nk, kRoleWhole, 0);
     return;
   }
   // A data-parallel block (b < sk_dp) has one item, its whole tile.  Stream-K
@@ -681,7 +720,7 @@ __global__ __launch_bounds__(kThreads, 1) void nt16_kernel(const KArgs A) {
 // Split products and (X3) fp32 ones of plane pairs: block = split * tiles +
 // tile, split s takes k-tiles [s kt_per_split, ..) of the pairs (X3: of the 6
 // npairs segments) and writes fp32.
-template <bool AK, bool BK, bool X3>
+template <bool AK, bool BK, bool X3, int NI>
 __global__ __launch_bounds__(kThreads, 1) void nt16_f32_kernel(const KArgs A) {
   extern __shared__ __attribute__((aligned(16))) uint16_t lds[];
   if constexpr (X3)
@@ -692,17 +731,36 @@ __global__ __launch_bounds__(kThreads, 1) void nt16_f32_kernel(const KArgs A) {
   const int kb = split * A.kt_per_split;
   int tm, tn;
   tile_coords_of(blockIdx.x - split * tiles, tiles, A.tiles_m, A.tiles_n, tm, tn);
-  nt16_tile<AK, BK, EPI_F32, 0, 0, 0, false, false, X3>(
+  nt16_tile<AK, BK, EPI_F32, 0, 0, 0, false, false, X3, NI>(
       A, lds, tm, tn, kb, min(nk, kb + A.kt_per_split), kRoleWhole, split);
+}
+
+// A plain store of tiles 192 columns wide, where those fill the chip's rounds of
+// blocks better: see use_192
+template <bool AK, bool BK>
+int launch_192(KArgs A, hipStream_t st) {
+  auto kern = nt16_kernel<AK, BK, EPI_STORE, 0, 0, 0, false, false, 6>;
+  static bool attr_set = false;   // per instantiation
+  if (!attr_set) {
+    if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, kLds) !=
+        hipSuccess)
+      return kErrLaunch;
+    attr_set = true;
+  }
+  A.tiles_n = (int)((A.N + 191) / 192);
+  const int64_t blocks = (int64_t)A.tiles_m * A.tiles_n;
+  if (blocks > 0x7FFFFFFF) return kErrTooLarge;
+  hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(kThreads), kLds, st, A);
+  return hipGetLastError() == hipSuccess ? kOk : kErrLaunch;
 }
 
 }  // namespace nt16
 
-// Split products of bf16 operands, or fp32 ones of plane pairs (X3), on 256 x 256
-// tiles, A.ksplit blocks per tile
-template <bool AK, bool BK, bool X3>
+// Split products of bf16 operands, or fp32 ones of plane pairs (X3), on tiles of
+// 256 x 32 NI, A.ksplit blocks per tile
+template <bool AK, bool BK, bool X3, int NI>
 int launch_nt16_f32(KArgs A, hipStream_t st) {
-  auto kern = nt16::nt16_f32_kernel<AK, BK, X3>;
+  auto kern = nt16::nt16_f32_kernel<AK, BK, X3, NI>;
   static bool attr_set = false;   // per instantiation
   if (!attr_set) {
     if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -711,7 +769,7 @@ int launch_nt16_f32(KArgs A, hipStream_t st) {
     attr_set = true;
   }
   A.tiles_m = (int)((A.M + 255) / 256);
-  A.tiles_n = (int)((A.N + 255) / 256);
+  A.tiles_n = (int)((A.N + 32 * NI - 1) / (32 * NI));
   const int64_t blocks = (int64_t)A.tiles_m * A.tiles_n * A.ksplit;
   if (blocks <= 0) return kOk;
   if (blocks > 0x7FFFFFFF) return kErrTooLarge;
@@ -744,6 +802,8 @@ int launch_nt16(const KArgs& A, hipStream_t st) {
   const int64_t tiles = (int64_t)A.tiles_m * A.tiles_n;
   if (tiles <= 0) return kOk;
   if (tiles > 0x7FFFFFFF) return kErrTooLarge;
+  if constexpr (EPI == EPI_STORE && LT == 0)
+    if (use_192(A, AK)) return nt16::launch_192<AK, BK>(A, st);
   KArgs B = A;
   B.sk_dp = (int)tiles;
   B.sk_blocks = 0;

@@ -8,14 +8,18 @@ namespace cpt {
 namespace gemm {
 
 CPT_ST16_INST_X3(CPT_ST16_DEFINE)
-template int launch_nt16_f32<true, true, false>(KArgs, hipStream_t);
-template int launch_nt16_f32<true, false, false>(KArgs, hipStream_t);
-template int launch_nt16_f32<false, false, false>(KArgs, hipStream_t);
-template int launch_nt16_f32<false, true, false>(KArgs, hipStream_t);
-template int launch_nt16_f32<true, true, true>(KArgs, hipStream_t);
-template int launch_nt16_f32<true, false, true>(KArgs, hipStream_t);
-template int launch_nt16_f32<false, false, true>(KArgs, hipStream_t);
-template int launch_nt16_f32<false, true, true>(KArgs, hipStream_t);
+template int launch_nt16_f32<true, true, false, 8>(KArgs, hipStream_t);
+template int launch_nt16_f32<true, false, false, 8>(KArgs, hipStream_t);
+template int launch_nt16_f32<false, false, false, 8>(KArgs, hipStream_t);
+template int launch_nt16_f32<false, true, false, 8>(KArgs, hipStream_t);
+template int launch_nt16_f32<true, true, true, 8>(KArgs, hipStream_t);
+template int launch_nt16_f32<true, false, true, 8>(KArgs, hipStream_t);
+template int launch_nt16_f32<false, false, true, 8>(KArgs, hipStream_t);
+template int launch_nt16_f32<false, true, true, 8>(KArgs, hipStream_t);
+template int launch_nt16_f32<true, true, true, 6>(KArgs, hipStream_t);
+template int launch_nt16_f32<true, false, true, 6>(KArgs, hipStream_t);
+template int launch_nt16_f32<false, false, true, 6>(KArgs, hipStream_t);
+template int launch_nt16_f32<false, true, true, 6>(KArgs, hipStream_t);
 
 // planes[0..2] = bf16 h, m, l with h = bf16(x), m = bf16(x - h), l = bf16(x - h
 // - m): round-to-nearest each, both differences exact, so x = h + m + l to 24

@@ -1144,16 +1144,24 @@ def x3_fits(a: torch.Tensor, b: torch.Tensor) -> bool:
 
 
 def x3_plan(m: int, n: int, nk: int, whole: bool) -> tuple[int, int]:
-    """(tile edge, k ranges) of an fp32 product of nk k-tiles of plane pairs; 256
-    x 256 tiles need whole k-tiles.  Times per k-tile with the chip full: 1.33 us
-    a 256 x 256 tile, 0.57 a 128 x 128 one, so the rounds of blocks decide."""
+    """(tile width, k ranges) of an fp32 product of nk k-tiles of plane pairs; 256
+    x 256 and 256 x 192 tiles need whole k-tiles.  Times per k-tile with the chip
+    full: 1.33 us a 256 x 256 tile, 1.12 a 256 x 192 one, 0.57 a 128 x 128 one, so
+    the rounds of blocks decide.  Measured, us on 256 / 192 columns: 2048 x 5632,
+    k 2048 (176 / 240 blocks) 269 / 226; 2048 x 2048, k 5632 (4 / 2 ranges) 212 /
+    284."""
     small = split_plan(m, n, nk)
     t128 = ((m + 127) // 128) * ((n + 127) // 128) * small
     t256 = ((m + 255) // 256) * ((n + 255) // 256)
     big = max(1, min(256 // t256, nk // SPLIT_MIN_KT))
     cost128 = 0.57 * min(-(-t128 // 256), 1.9 * -(-t128 // 512)) * nk / small
+    t192 = ((m + 255) // 256) * ((n + 191) // 192)
+    narrow = max(1, min(256 // t192, nk // SPLIT_MIN_KT))
     cost256 = 1.33 * -(-t256 * big // 256) * nk / big
-    return (256, big) if whole and cost256 < cost128 else (128, small)
+    cost192 = 1.12 * -(-t192 * narrow // 256) * nk / narrow
+    if not whole or cost128 <= min(cost256, cost192):
+        return 128, small
+    return (192, narrow) if cost192 < cost256 else (256, big)
 
 
 def mm_x3(a, b, planes: Planes, a2=None, b2=None, alpha: float = 1.0,

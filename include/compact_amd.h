@@ -358,9 +358,10 @@ int cpt_gemm16(int dtype, const void* a, int64_t lda, int a_kmajor, const void* 
  * and not 0).  cpt_gemm_f32x3 writes c = alpha * (a . b + a2 . b2) from such
  * planes (plane_* elements apart, layouts, K and N as in cpt_gemm16, both pairs
  * with one lda and ldb, a2 NULL for one pair) unless one of the flags is set;
- * tiles is 128, or 256 where K and K2 are multiples of 64; splits > 1 needs splits * M * N floats of workspace.  cpt_gemm_any_if is
- * cpt_gemm_any run only if one of its flags is set (all NULL: always): the fp32
- * product for the operands the planes cannot carry. */
+ * tiles is 128, or 256 or 192 (256 rows by 256 or 192 columns) where K and K2 are
+ * multiples of 64; splits > 1 needs splits * M * N floats of workspace.
+ * cpt_gemm_any_if is cpt_gemm_any run only if one of its flags is set (all NULL:
+ * always): the fp32 product for the operands the planes cannot carry. */
 int cpt_split_f32(const void* x, int64_t ld, int64_t rows, int64_t cols, void* planes, void* flag,
                   void* stream);
 int cpt_gemm_f32x3(const void* a, int64_t plane_a, int64_t lda, int a_kmajor, const void* b,

@@ -111,3 +111,19 @@ def test_other_views_keep_the_general_kernel(bad):
     a, b = _operands("nn", 64, 128, 129)
     v = bad(a)
     assert not G.x3_fits(v, b[:v.shape[1]])
+
+
+@pytest.mark.parametrize("layout", ["nt", "nn", "tn", "tt"])
+@pytest.mark.parametrize("m,n,k", [(8, 8, 64), (264, 200, 128), (520, 384, 448), (256, 1000, 1024)])
+@pytest.mark.parametrize("ranges", [1, 2])
+def test_192_column_tiles_equal_256(layout, m, n, k, ranges, monkeypatch):
+    """The same plane products in the same order, whatever the width of a tile."""
+    from compact_amd import gemm as G
+    a, b = _operands(layout, m, n, k)
+    a2, b2 = _operands(layout, m, n, k, seed=5)
+    got = []
+    for tiles in (192, 256):
+        monkeypatch.setattr(G, "x3_plan", lambda *_: (tiles, ranges))
+        got.append((G.mm_x3(a, b, G.Planes()), G.mm_x3(a, b, G.Planes(), a2, b2)))
+    assert all(torch.equal(u, v) for u, v in zip(*got))
+    assert _errors(got[0][0], a, b)[1] < 2.0 ** -22

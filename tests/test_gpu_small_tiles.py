@@ -120,3 +120,36 @@ def test_ffn_kernels_equal_large_tiles(m, d, rank):
     dg, du, _ = G.ffn_down_dgrad(gy[:m], wd, _lib.CACHE_BF16, 64, cg, None, cu, None, False,
                                  lora=dl, inplace=True)
     assert torch.equal(dg, got_b[0]) and torch.equal(du, got_b[1])
+
+
+@pytest.mark.parametrize("layout", ["nt", "nn", "tn", "tt"])
+@pytest.mark.parametrize("m,n", [(5512, 1928), (5128, 2112), (5128, 2104), (1800, 5384),
+                                 (11016, 1920)])
+@pytest.mark.parametrize("k,k2", [(64, 0), (128, 64), (1088, 128)])
+def test_192_column_tiles(layout, m, n, k, k2):
+    """Products whose 256 x 256 tiles leave a quarter of a round empty run on 192
+    columns: ragged last row and column (8, 184 and 192 columns of the last tile),
+    one and two pairs, one round and (11016 rows, MN-major A) two.  The k order is
+    that of the 128 x 128 tiles, which take the same columns a part at a time."""
+    from compact_amd import gemm as G
+
+    def pair(kk, seed):
+        # the pairs share leading dimensions: views of one width
+        w = max(k, k2)
+        a = (_rand(m, w, seed=seed)[:, :kk] if layout[0] == "n" else _rand(kk, m, seed=seed).t())
+        b = (_rand(n, w, seed=seed + 1)[:, :kk].t() if layout[1] == "t"
+             else _rand(kk, n, seed=seed + 1))
+        return a, b
+    args = pair(k, 1) + (pair(k2, 3) if k2 else ())
+    wide, narrow = ((m + 255) // 256) * ((n + 255) // 256), ((m + 255) // 256) * ((n + 191) // 192)
+    assert not _is_small(m, n) and -(-narrow // 256) <= -(-wide // 256)
+    if layout[0] == "n" and wide > 256:
+        pytest.skip("K-major A past one round: stream-K shares its tiles (its own k order)")
+    got = G.mm2(*args) if k2 else G.mm(*args)
+    for r0 in range(0, m, 2048):
+        for c0 in range(0, n, 2048):
+            part = [t[r0:r0 + 2048] if i % 2 == 0 else t[:, c0:c0 + 2048]
+                    for i, t in enumerate(args)]
+            assert _is_small(part[0].shape[0], part[1].shape[1])
+            ref = G.mm2(*part) if k2 else G.mm2(*part, None, None)
+            assert torch.equal(got[r0:r0 + 2048, c0:c0 + 2048], ref)
