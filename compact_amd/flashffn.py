@@ -734,18 +734,20 @@ _FAMILY_NAME = {"dora": "DoRA", "adalora": "AdaLoRA", "vera": "VeRA", "dylora": 
 
 
 def _attr(m, name: str, default=None):
-    """getattr(m, name, default) that looks a Module's own tables up first and
-    raises nothing on a miss (an adapter wrapper is searched for a dozen names
-    on every call, most of them absent)."""
-    d = getattr(m, "__dict__", None)
-    if d is not None and isinstance(m, nn.Module):
-        for table in ("_modules", "_parameters", "_buffers"):
-            t = d.get(table)
+    """getattr(m, name, default) that reads a Module's own tables and raises
+    nothing on a miss (an adapter wrapper is searched for a dozen names on every
+    call, most of them absent).  What comes before the tables in a Module's
+    look-up goes through getattr: instance and class attributes (properties among
+    them), a __getattr__ or __getattribute__ of its own."""
+    cls = type(m)
+    if (isinstance(m, nn.Module) and name not in m.__dict__ and not hasattr(cls, name)
+            and cls.__getattr__ is nn.Module.__getattr__
+            and cls.__getattribute__ is object.__getattribute__):
+        for table in ("_parameters", "_buffers", "_modules"):
+            t = m.__dict__.get(table)
             if t and name in t:
                 return t[name]
-        if name not in d and not hasattr(type(m), name) and \
-                type(m).__getattr__ is nn.Module.__getattr__:
-            return default
+        return default
     return getattr(m, name, default)
 
 

@@ -115,3 +115,27 @@ def test_lora_fusable_rule():
     a16 = torch.zeros(16, 256, dtype=bf)
     assert not _lora_ok((a16, torch.zeros(768, 16, dtype=bf)), (a24, b24), dims=((256, 768),))
     assert _lora_ok((None, None), dims=((136, 12),))
+
+
+def test_attribute_lookup_is_getattrs():
+    """The wrapper search's attribute look-up finds what getattr finds: tables,
+    class properties and instance attributes before them, own __getattr__."""
+    from compact_amd.flashffn import _attr
+
+    class Prop(nn.Module):
+        weight = property(lambda self: "property")
+
+    class Own(nn.Module):
+        def __getattr__(self, name):
+            return "own" if name == "weight" else super().__getattr__(name)
+
+    shadowed = nn.Linear(2, 2)
+    shadowed.__dict__["weight"] = "instance"
+    prop = Prop()
+    prop._parameters["weight"] = nn.Parameter(torch.zeros(1))
+    own = Own()
+    own._parameters["weight"] = nn.Parameter(torch.zeros(1))
+    for m in (nn.Linear(2, 2), nn.Linear(2, 2, bias=False), shadowed, prop, own,
+              nn.ModuleDict({"weight": nn.Linear(2, 2)}), object(), nn.BatchNorm1d(2)):
+        for name in ("weight", "bias", "running_mean", "base_layer", "training"):
+            assert _attr(m, name, "absent") is getattr(m, name, "absent")
