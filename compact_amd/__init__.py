@@ -2,7 +2,7 @@
 
 A LLaMA-style SwiGLU FFN whose backward cache is int4/int8 per-group absmax
 codes of h_gate/h_up, computed by hand-written gfx950 HIP kernels behind the C
-ABI in include/compact_amd.h (libcompact_amd.so, loaded with ctypes).  The
+ABI in include/compact_amd.h (libcompact_amd.so).  The
 Python API mirrors the reference's src/flashffn.py.
 """
 

@@ -428,8 +428,8 @@ int gemm16_impl(const void* a, int64_t lda, int a_kmajor, const void* b, int64_t
 // plane_* elements apart), written unless one of the flags is set.  Bound: the
 // bf16 MFMAs at the board's power, six passes.  Measured on MI355X against the
 // general-layout kernel (v_mfma_f32_32x32x2_f32), planes made beforehand:
-//   2048 x 5632, k 2048 (176 tiles of 256 x 256)     280 us against 560
-//   2048 x 2048, k 5632 (64 tiles, 4 k ranges)       226 us against 600
+//   2048 x 5632, k 2048 (240 tiles of 256 x 192)     226 us against 560
+//   2048 x 2048, k 5632 (64 of 256 x 256, 4 ranges)  212 us against 600
 //   4 x 5632, k 2048 (44 tiles of 128 x 128, 4)       29 us against 214
 // Error against float64 (relative Frobenius, N(0, 1) operands): 2.7e-7 against
 // 8.1e-7 at k 2048, 4.7e-7 against 1.3e-6 at k 5632.
