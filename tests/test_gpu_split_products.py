@@ -164,6 +164,35 @@ def test_gate_up(dt, m, dff, rank, splits):
 
 
 @pytest.mark.parametrize("dt", ["bf16", "fp16"])
+@pytest.mark.parametrize("m,n,rank", [(2049, 520, 8), (2017, 264, 16), (1340, 264, 24),
+                                      (1027, 264, 32)])
+@pytest.mark.parametrize("q_kmajor", [True, False])
+@pytest.mark.parametrize("splits", [2, 5])
+def test_adapter_terms_of_larger_outputs(dt, m, n, rank, q_kmajor, splits):
+    """The split sums with the terms on the MFMAs (M N rank above 2^23), ragged in
+    rows and columns: test_adapter_terms' bound."""
+    d, k = DT[dt], 512
+    a, b = _rand(m, k, dtype=d, seed=1), _rand(n, k, dtype=d, seed=2).t()
+    lora, ref = [], a.double() @ b.double()
+    size = ref.abs()
+    for t in range(2):
+        p = _rand(m, rank, dtype=d, seed=3 + t)
+        q = _rand(n, rank, dtype=d, seed=5 + t).t() if q_kmajor else _rand(rank, n, dtype=d,
+                                                                            seed=5 + t)
+        term = (0.5 + t) * (p.double() @ q.double())
+        lora.append((p, q, 0.5 + t))
+        ref, size = ref + term, size + 2 * term.abs() + ref.abs() + term.abs()
+    got = _gemm16(dt, a, b, lora=lora, splits=splits)
+    bound = EPS[dt] * 1.1 * size + k * 2.0 ** -24 * (a.double().abs() @ b.double().abs())
+    _close(got, ref, dt, bound)
+
+
+@pytest.mark.parametrize("dt", ["bf16", "fp16"])
+def test_gate_up_of_larger_outputs(dt):
+    test_gate_up(dt, 2049, 520, 8, 3)
+
+
+@pytest.mark.parametrize("dt", ["bf16", "fp16"])
 def test_non_finite_and_subnormal_values(dt):
     """Infinities and NaN travel as in a sum; subnormals of the type count."""
     d = DT[dt]
