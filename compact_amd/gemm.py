@@ -1172,8 +1172,14 @@ def mm_x3(a, b, planes: Planes, a2=None, b2=None, alpha: float = 1.0,
 
     Three times closer to float64 than the general-layout kernel and about
     twice as fast, splitting included (x3_gemm_impl in csrc/gemm.hip)."""
-    _require_device(a, b)
+    _require_device(a, b, a2, b2)
+    ops = (a, b) if a2 is None else (a, b, a2, b2)
+    assert all(t.dtype == torch.float32 and t.dim() == 2 for t in ops), \
+        f"2-D float32 operands expected, got {[t.dtype for t in ops]}"
     (M, K), N = a.shape, b.shape[1]
+    assert b.shape[0] == K, f"inner dims differ: {tuple(a.shape)} @ {tuple(b.shape)}"
+    assert a2 is None or (a2.shape[0] == M and tuple(b2.shape) == (a2.shape[1], N)), \
+        f"second pair {tuple(a2.shape)} @ {tuple(b2.shape)} of an [{M}, {N}] product"
 
     def operand(t, left):
         s, own = _x3_operand(t)

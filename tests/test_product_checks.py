@@ -1,0 +1,80 @@
+"""What the product wrappers refuse and how they repair operands, on the CPU:
+tensors are taken for device ones and every library call is recorded and
+answered with success, so what runs is the host code in front of the launches."""
+
+import pytest
+import torch
+
+from compact_amd import _lib, flashffn as F, gemm as G, kernels as K
+
+
+class _Library:
+    """The entry points by name; calls: (name, arguments)."""
+
+    def __init__(self):
+        self.calls = []
+
+    def __getattr__(self, name):
+        def call(*args):
+            self.calls.append((name, args))
+            return 1024 if name.endswith("_bytes") else 0
+        return call
+
+
+@pytest.fixture
+def library(monkeypatch):
+    lib = _Library()
+    monkeypatch.setattr(_lib, "api", lambda: lib)
+    monkeypatch.setattr(_lib, "lib", lambda: lib)
+    monkeypatch.setattr(torch.Tensor, "is_cuda", True, raising=False)
+    for mod in (G, K):
+        monkeypatch.setattr(mod, "_stream", lambda t: 0)
+    monkeypatch.setattr(G, "_stream_k", lambda dev: None)
+    return lib
+
+
+# weights (gate, up, down) that do not fit x [64, 256] or each other
+MISFITS = {
+    "wide_gate_up": ((128, 512), (128, 512), (256, 128)),
+    "narrow_gate_up": ((128, 192), (128, 192), (256, 128)),
+    "wide_up": ((128, 256), (128, 512), (256, 128)),
+    "wide_down": ((128, 256), (128, 256), (256, 192)),
+    "narrow_down": ((128, 256), (128, 256), (256, 64)),
+}
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("misfit", MISFITS)
+@pytest.mark.parametrize("function", ["v3", "adapter", "topk"])
+def test_functions_refuse_weights_that_do_not_fit(library, function, misfit, dtype):
+    """Whatever the type's route, a product whose inner dimensions differ is an
+    AssertionError and never a launch over part (or past the end) of an operand."""
+    x = torch.zeros(64, 256, dtype=dtype)
+    wg, wu, wd = (torch.zeros(s, dtype=dtype, requires_grad=True) for s in MISFITS[misfit])
+    with pytest.raises(AssertionError):
+        if function == "v3":
+            F.FlashFFNv3Function.apply(x, wg, None, None, wu, None, None, wd, None, None)
+        elif function == "adapter":
+            F.FlashFFNv3AdapterFunction.apply(x, wg, None, None, None, None, wu, None, None, None,
+                                              None, wd, None, None, None, None)
+        else:
+            F.FlashFFNFunction.apply(x, wg, wu, wd)
+
+
+@pytest.mark.parametrize("shapes", [
+    ((64, 128), (192, 64)), ((64, 192), (128, 64)),
+    ((64, 128), (128, 64), (64, 128), (64, 64)), ((64, 128), (128, 64), (32, 64), (64, 64)),
+    ((64, 128), (128, 64), (64, 64), (64, 128))])
+def test_fp32_product_checks_every_extent(library, shapes):
+    ts = [torch.zeros(s) for s in shapes]
+    with pytest.raises(AssertionError):
+        G.mm_x3(ts[0], ts[1], G.Planes(), *ts[2:])
+    assert not library.calls
+
+
+def test_fp32_product_refuses_other_types(library):
+    a, b = torch.zeros(64, 128), torch.zeros(128, 64)
+    for u, v in ((a.bfloat16(), b), (a, b.bfloat16()), (a.double(), b.double())):
+        with pytest.raises(AssertionError):
+            G.mm_x3(u, v, G.Planes())
+    assert not library.calls
