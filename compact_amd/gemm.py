@@ -171,16 +171,22 @@ def _lora_args_whole(terms, n_q, r):
     return r, ldp, int(q_km), ldq, out, terms
 
 
-def _lora_args(terms, n_q, dims):
+def _lora_args(terms, n_q, dims, x):
     """(rank, ldp, q_kmajor, ldq, [(p, q, alpha) x 2], keep) for up to two
     terms (p [M, r], q the logical [r, N] factor, alpha) of a GEMM with the
-    (k, n) `dims` (lora_fusable); `keep` holds any
-    re-laid copies alive until the launch.  The kernels fetch P and K-major Q
-    in 16-byte chunks of 8 k, so a rank that is not a multiple of 8 is
+    (k, n) `dims` (lora_fusable) and rows and type of its left operand x; `keep`
+    holds any re-laid copies alive until the launch.  The kernels fetch P and
+    K-major Q in 16-byte chunks of 8 k, so a rank that is not a multiple of 8 is
     zero-padded to the next one (8, 16, 24 or 32): the padded k add exact zeros to
     each fp32 dot product."""
     terms = [t for t in terms if t is not None]
     assert 1 <= len(terms) <= 2
+    for pm, q, _ in terms:
+        assert pm.dtype == q.dtype == x.dtype, \
+            f"adapter factors of {pm.dtype} and {q.dtype} in a product of {x.dtype}"
+        assert pm.dim() == q.dim() == 2 and pm.shape[0] >= x.shape[0], \
+            f"adapter rows {tuple(pm.shape)} for {x.shape[0]} rows"
+    _require_device(*(t for pm, q, _ in terms for t in (pm, q)))
     r = terms[0][0].shape[1]
     fast = _lora_args_whole(terms, n_q, r)
     if fast is not None and lora_fusable(r, *dims):
@@ -731,7 +737,7 @@ def mm2(a, b, a2=None, b2=None, name: str = "gemm", lora=None) -> torch.Tensor:
             a, lda, ak = _layout_a(a)
             assert a2 is None, "adapter terms with a K-concatenated MN-major A"
         dims = ((K, N),) if a2 is None else ((K, N), (K2, N))
-        r, ldp, qk, ldq, t, keep = _lora_args(lora, N, dims)
+        r, ldp, qk, ldq, t, keep = _lora_args(lora, N, dims, a)
     half = dt == _lib.F16
     tiles, splits = ((128, 1) if (not half and (K % 64 or K2 % 64)) or N % 8 or not K
                      else tile_plan(M, N, (K + 63) // 64 + (K2 + 63) // 64, half))
@@ -834,7 +840,7 @@ def ffn_gate_up(x, w_gate, w_up, cache: int, group_size: int, want_h_mid: bool =
         # term 0 on the gate columns, term 1 on the up columns (absent: no-op)
         present = [t for t in (lora_gate, lora_up) if t is not None]
         r, ldp, qk, _, t, keep = _lora_args([(xa, bw.t(), s) for xa, bw, s in present], d,
-                                            ((hdim, d),))
+                                            ((hdim, d),), x)
         assert qk == 1, "the gate/up adapter B factors go K-major"
         if lora_gate is None:
             t = [(None, None, 0.0), t[0]]
@@ -894,7 +900,7 @@ def ffn_gate_up_outlier(x, w_gate, w_up, cache: int, group_size: int, slot_gate,
     if lora_gate is not None or lora_up is not None:
         present = [tt for tt in (lora_gate, lora_up) if tt is not None]
         rank, ldp, qk, _, t, keep = _lora_args([(xa, bw.t(), sc) for xa, bw, sc in present], d,
-                                               ((hdim, d),))
+                                               ((hdim, d),), x)
         assert qk == 1, "the gate/up adapter B factors go K-major"
         if lora_gate is None:
             t = [(None, None, 0.0), t[0]]
@@ -952,7 +958,7 @@ def ffn_down_dgrad(grad_y, w_down, cache: int, group_size: int, c_gate, s_gate, 
         if lora is not None:
             gyb, a_down, s = lora
             a_down = a_down.contiguous()
-            rank, ldp, qk, ldq, t, keep = _lora_args([(gyb, a_down, s)], d, ((hdim, d),))
+            rank, ldp, qk, ldq, t, keep = _lora_args([(gyb, a_down, s)], d, ((hdim, d),), grad_y)
             assert qk == 0 and ldq == d
             pp, qq, alpha = t[0]
         with _timed("ffn_down_dgrad"):
@@ -965,7 +971,7 @@ def ffn_down_dgrad(grad_y, w_down, cache: int, group_size: int, c_gate, s_gate, 
     elif lora is not None:
         gyb, a_down, s = lora
         a_down = a_down.contiguous()          # [r, inter] rows: the MN-major factor
-        r, ldp, qk, ldq, t, keep = _lora_args([(gyb, a_down, s)], d, ((hdim, d),))
+        r, ldp, qk, ldq, t, keep = _lora_args([(gyb, a_down, s)], d, ((hdim, d),), grad_y)
         assert qk == 0 and ldq == d
         with _timed("ffn_down_dgrad"):
             rc = _lib.api().cpt_ffn_down_dgrad_lora(

@@ -78,3 +78,49 @@ def test_fp32_product_refuses_other_types(library):
         with pytest.raises(AssertionError):
             G.mm_x3(u, v, G.Planes())
     assert not library.calls
+
+
+def _terms(n, d, r, dtype, rows=None):
+    """(P, B, alpha) of a projection's adapter term."""
+    return (torch.zeros(n if rows is None else rows, r, dtype=dtype),
+            torch.zeros(d, r, dtype=dtype), 2.0)
+
+
+@pytest.mark.parametrize("r", [4, 8])
+@pytest.mark.parametrize("product,factors", [(torch.bfloat16, torch.float16),
+                                             (torch.float16, torch.bfloat16),
+                                             (torch.bfloat16, torch.float32)])
+@pytest.mark.parametrize("call", ["mm2", "gate_up", "gate_up_outlier", "down_dgrad"])
+def test_adapter_factors_have_the_products_type(library, call, product, factors, r):
+    """A factor of another type would be read with the product's bits."""
+    n, h, d = 64, 128, 256
+    x, w = torch.zeros(n, h, dtype=product), torch.zeros(d, h, dtype=product)
+    p, b, s = _terms(n, d, r, factors)
+
+    def run():
+        if call == "mm2":
+            G.mm2(x, w.t(), lora=[(p, b.t(), s)])
+        elif call == "gate_up":
+            G.ffn_gate_up(x, w, w, _lib.CACHE_BF16, 64, lora_gate=(p, b, s))
+        elif call == "gate_up_outlier":
+            e = torch.empty
+            out = (e(n, d), e(n, d), e(n, d // 64), e(n, 8), e(n, d), e(n, d // 64), e(n, 8))
+            slot = torch.zeros(d, dtype=torch.int16)
+            G.ffn_gate_up_outlier(x, w, w, _lib.CACHE_INT8, 64, slot, slot, 8, out,
+                                  lora_gate=(p, b, s))
+        else:
+            hg = torch.zeros(n, d, dtype=product)
+            G.ffn_down_dgrad(x, w.t(), _lib.CACHE_BF16, 64, hg, None, hg, None, False,
+                             lora=(p, b.t().contiguous(), s))
+    with pytest.raises(AssertionError):
+        run()
+    assert not library.calls
+
+
+def test_adapter_rows_cover_the_products_rows(library):
+    x, w = torch.zeros(64, 128, dtype=torch.bfloat16), torch.zeros(256, 128, dtype=torch.bfloat16)
+    for r in (4, 8):
+        p, b, s = _terms(64, 256, r, torch.bfloat16, rows=63)
+        with pytest.raises(AssertionError):
+            G.mm2(x, w.t(), lora=[(p, b.t(), s)])
+    assert not library.calls
