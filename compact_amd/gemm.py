@@ -478,6 +478,10 @@ def skinny_dual_pair(x0: torch.Tensor, q0: torch.Tensor, p0: torch.Tensor, alpha
     their split sums in another (bit for bit the two calls' results): returns
     ([x0 q0^T | x1 q1^T] side by side [T, 2 R], alpha0 x0^T p0 [N, R],
     alpha1 x1^T p1 [N, R]), or None where the two do not share a layout."""
+    _require_device(x0, q0, p0, x1, q1, p1)
+    assert skinny_dual_ok(x0, q0, p0) and skinny_dual_ok(x1, q1, p1), "skinny_dual_pair operands"
+    assert x1.shape == x0.shape and q1.shape == q0.shape and x1.dtype == x0.dtype, \
+        f"tensors of two shapes or types: {tuple(x0.shape)} {x0.dtype}, {tuple(x1.shape)} {x1.dtype}"
     T, N = x0.shape
     R = q0.shape[0]
     q0, q_nr, ldq = _dual_q(q0)
@@ -486,7 +490,6 @@ def skinny_dual_pair(x0: torch.Tensor, q0: torch.Tensor, p0: torch.Tensor, alpha
             or not _row_major(x0) or not _row_major(x1) or x0.stride(0) < N
             or not _row_major(p0) or not _row_major(p1) or p0.stride(0) < R):
         return None
-    _require_device(x0, q0, p0, x1, q1, p1)
     splits = _dual_splits(T, N, max(x0.stride(0), p0.stride(0)))
     c = torch.empty((T, 2 * R), dtype=x0.dtype, device=x0.device)
     z0 = torch.empty((N, R), dtype=x0.dtype, device=x0.device)

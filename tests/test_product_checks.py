@@ -124,3 +124,27 @@ def test_adapter_rows_cover_the_products_rows(library):
         with pytest.raises(AssertionError):
             G.mm2(x, w.t(), lora=[(p, b.t(), s)])
     assert not library.calls
+
+
+@pytest.mark.parametrize("change", ["x1 rows", "x1 columns", "q1 rank", "q1 columns", "p1 rows",
+                                    "x1 type", "all of pair 1", "p0 rows", "odd rank"])
+def test_dual_pass_of_two_checks_shapes_and_types(library, change):
+    """The two tensors' strides may agree where their shapes or types do not."""
+    T, N, R, bf = 64, 512, 8, torch.bfloat16
+    base = torch.zeros(T, N, dtype=bf), torch.zeros(R, N, dtype=bf), torch.zeros(T, R, dtype=bf)
+    x0, q0, p0 = base
+    x1, q1, p1 = base
+    half = torch.float16
+    x1 = {"x1 rows": x0[:32], "x1 columns": x0[:, :256], "x1 type": x0.to(half)}.get(change, x1)
+    q1 = {"q1 rank": q0[:4], "q1 columns": q0[:, :256]}.get(change, q1)
+    p1 = p0[:32] if change == "p1 rows" else p1
+    p0 = p0[:32] if change == "p0 rows" else p0
+    if change == "all of pair 1":
+        x1, q1, p1 = (t.to(half) for t in base)
+    if change == "odd rank":
+        q0 = q1 = q0[:4]
+        p0 = p1 = torch.zeros(T, 4, dtype=bf)
+    with pytest.raises(AssertionError):
+        G.skinny_dual_pair(x0, q0, p0, 1.0, x1, q1, p1, 1.0)
+    assert not library.calls
+    assert G.skinny_dual_pair(*base, 1.0, *base, 1.0) is not None
