@@ -82,6 +82,14 @@ def _common_ld(x, x2, kmajor: int, is_b: bool):
     return _with_ld(x, ld, rows_dim), _with_ld(x2, ld, rows_dim), ld
 
 
+def _copied(t: torch.Tensor) -> torch.Tensor:
+    """t in contiguous rows from a 16-byte aligned base.  (contiguous() copies
+    nothing where the rows are whole already, whatever the base: a parameter
+    viewed out of a flat buffer.)"""
+    t = t.contiguous()
+    return t if t.data_ptr() % 16 == 0 else t.clone()
+
+
 def _check_bf16(*ts):
     for t in ts:
         assert t.dtype == torch.bfloat16, f"MFMA GEMM path is bf16-only, got {t.dtype}"
@@ -211,7 +219,7 @@ def _lora_args(terms, n_q, dims, x):
         _check_16(pm, q)
         assert pm.shape[1] == r and q.shape[0] == r and q.shape[1] == n_q
         if pm.stride(1) != 1 or pm.stride(0) % 8 or pm.data_ptr() % 16:
-            pm = pm.contiguous()
+            pm = _copied(pm)
         ps.append(pm)
         qs.append(q)
     ldp = ps[0].stride(0)
@@ -224,7 +232,7 @@ def _lora_args(terms, n_q, dims, x):
     elif all(q.stride(1) == 1 for q in qs) and len({q.stride(0) for q in qs}) == 1:
         q_kmajor, ldq = 0, qs[0].stride(0)
     else:
-        qs = [q.t().contiguous().t() for q in qs]
+        qs = [_copied(q.t()).t() for q in qs]
         q_kmajor, ldq = 1, r
     keep += ps + qs
     out = [(ps[i].data_ptr(), qs[i].data_ptr(), float(terms[i][2])) for i in range(len(terms))]
@@ -261,9 +269,9 @@ def skinny(a: torch.Tensor, q: torch.Tensor, alpha: float = 1.0,
     R = q.shape[0]
     assert q.shape[1] == K and R <= SKINNY_MAX_RANK
     if a.stride(1) != 1 or a.stride(0) % 8 or a.stride(0) < K or a.data_ptr() % 16:
-        a = a.contiguous()
+        a = _copied(a)
     if q.stride(1) != 1 or q.stride(0) % 8 or q.stride(0) < K or q.data_ptr() % 16:
-        q = q.contiguous()
+        q = _copied(q)
     if out is None and skinny_small_pays(M, K):
         return skinny_small(a, q, None, alpha, name)
     # K ranges for ~SKINNY_BLOCKS blocks of 128 rows (each range >= 256 of
@@ -316,7 +324,7 @@ def skinny_small(a: torch.Tensor, q0: torch.Tensor, q1: torch.Tensor | None = No
     def rows(t):
         ok = t.stride(1) == 1 and t.stride(0) % 8 == 0 and t.stride(0) >= K \
             and t.data_ptr() % 16 == 0
-        return t if ok else t.contiguous()
+        return t if ok else _copied(t)
     a, q0 = rows(a), rows(q0)
     r0, r1 = q0.shape[0], 0
     assert q0.shape[1] == K
@@ -349,9 +357,9 @@ def skinny_t(x: torch.Tensor, p: torch.Tensor, alpha: float = 1.0, trans: bool =
     R = p.shape[1]
     assert p.shape[0] == T and R <= SKINNY_MAX_RANK
     if not _row_major(x) or x.stride(0) < N:
-        x = x.contiguous()
+        x = _copied(x)
     if not _row_major(p) or p.stride(0) < R:
-        p = p.contiguous()
+        p = _copied(p)
     splits = skinny_t_splits(T, N)
     # each split reads its tokens (plus 128 of prefetch) within 32-bit offsets
     per = (_SPAN_BYTES // (2 * max(x.stride(0), p.stride(0))) - 129) // 64 * 64
@@ -420,7 +428,7 @@ def _dual_q(q: torch.Tensor):
         return q, 0, q.stride(0)
     if q.stride(0) == 1 and q.stride(1) >= R and q.data_ptr() % 16 == 0:
         return q, 1, q.stride(1)
-    q = q.contiguous()
+    q = _copied(q)
     return q, 0, q.stride(0)
 
 
@@ -448,10 +456,10 @@ def skinny_dual(x: torch.Tensor, q: torch.Tensor, p: torch.Tensor, alpha_c: floa
     T, N = x.shape
     R = q.shape[0]
     if not _row_major(x) or x.stride(0) < N:
-        x = x.contiguous()
+        x = _copied(x)
     q, q_nr, ldq = _dual_q(q)
     if not _row_major(p) or p.stride(0) < R:
-        p = p.contiguous()
+        p = _copied(p)
     splits = _dual_splits(T, N, max(x.stride(0), p.stride(0)))
     if out_c is None:
         c = torch.empty((T, R), dtype=x.dtype, device=x.device)

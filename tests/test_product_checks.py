@@ -148,3 +148,34 @@ def test_dual_pass_of_two_checks_shapes_and_types(library, change):
         G.skinny_dual_pair(x0, q0, p0, 1.0, x1, q1, p1, 1.0)
     assert not library.calls
     assert G.skinny_dual_pair(*base, 1.0, *base, 1.0) is not None
+
+
+def _off(t):
+    """t's values one element into a buffer of their own: whole rows, a base that
+    is not on 16 bytes."""
+    flat = torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)[1:]
+    return flat.view(t.shape).copy_(t)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_unaligned_factors_are_copied(library, dtype):
+    """The kernels read rank factors in 16-byte pieces; a factor viewed out of a
+    flat buffer at an odd offset goes in as an aligned copy of itself."""
+    x = torch.zeros(64, 512, dtype=dtype)
+    wide = torch.zeros(64, 8192, dtype=dtype)
+    q, p = torch.zeros(8, 512, dtype=dtype), torch.zeros(64, 8, dtype=dtype)
+    qo, po, xo = _off(q), _off(p), _off(x)
+    assert all(t.is_contiguous() and t.data_ptr() % 16 for t in (qo, po, xo))
+    G.skinny_small(xo, qo, qo)
+    G.skinny(_off(wide), _off(torch.zeros(8, 8192, dtype=dtype)))
+    G.skinny_t(xo, po)
+    G.skinny_dual(xo, qo, po)
+    args = {name: a for name, a in library.calls}
+    pointers = {"cpt_gemm16_skinny_small": (1, 3, 6), "cpt_gemm16_skinny": (1, 3),
+                "cpt_gemm16_skinny_t": (1, 3), "cpt_gemm16_skinny_dual": (1, 3, 6)}
+    for name, where in pointers.items():
+        assert all(args[name][i] % 16 == 0 for i in where), name
+    # an adapter term's P, and its B factor as rows of ranks
+    b = _off(torch.zeros(256, 8, dtype=dtype))
+    *_, terms, keep = G._lora_args([(po, b.t(), 1.0)], 256, ((512, 256),), x)
+    assert terms[0][0] % 16 == 0 and terms[0][1] % 16 == 0 and keep
