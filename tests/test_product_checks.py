@@ -179,3 +179,25 @@ def test_unaligned_factors_are_copied(library, dtype):
     b = _off(torch.zeros(256, 8, dtype=dtype))
     *_, terms, keep = G._lora_args([(po, b.t(), 1.0)], 256, ((512, 256),), x)
     assert terms[0][0] % 16 == 0 and terms[0][1] % 16 == 0 and keep
+
+
+@pytest.mark.parametrize("r", [1, 2, 8, 24])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("function", ["v3", "adapter"])
+def test_b_factors_stored_transposed(library, function, dtype, r):
+    """A B factor [d, r] that is the transposed view of [r, d] storage (for rank 1
+    a column whose other stride is d) goes into the fused products."""
+    n, h, d = 64, 128, 256
+    x = torch.zeros(n, h, dtype=dtype)
+    wg, wu, wd = (torch.zeros(s, dtype=dtype) for s in ((d, h), (d, h), (h, d)))
+    (ag, bg), (au, bu), (ad, bd) = ((torch.zeros(r, i, dtype=dtype, requires_grad=True),
+                                     torch.zeros(r, o, dtype=dtype).t().requires_grad_())
+                                    for o, i in ((d, h), (d, h), (h, d)))
+    assert bg.stride() == (1, d)
+    if function == "v3":
+        y = F.FlashFFNv3Function.apply(x, wg, ag, bg, wu, au, bu, wd, ad, bd, 2.0, 2.0, 2.0, "bf16")
+    else:
+        y = F.FlashFFNv3AdapterFunction.apply(x, wg, ag, bg, None, None, wu, au, bu, None, None, wd,
+                                              ad, bd, None, None, 2.0, 2.0, 2.0, "bf16")
+    y.backward(torch.zeros_like(y))
+    assert bg.grad.shape == (d, r)
