@@ -321,6 +321,7 @@ def _thin_backward(grad_h_gate, b_gate, xa_g, s_gate, grad_h_up, b_up, xa_u, s_u
     # one token reduction over x gives both A gradients below
     stack = (_stackable(b_gate.t() if b_gate is not None else None,
                         b_up.t() if b_up is not None else None)
+             and b_up.shape[1] % 8 == 0      # both halves' rows start on 16 bytes
              and (need_g or need_u) and grad_h_gate.shape[0] >= 256
              and (_mfma(grad_h_gate, b_gate, grad_h_up, b_up)
                   or (G.f16_fits(grad_h_gate, b_gate) and G.f16_fits(grad_h_up, b_up)))

@@ -201,3 +201,22 @@ def test_b_factors_stored_transposed(library, function, dtype, r):
                                               ad, bd, None, None, 2.0, 2.0, 2.0, "bf16")
     y.backward(torch.zeros_like(y))
     assert bg.grad.shape == (d, r)
+
+
+@pytest.mark.parametrize("ranks", [(8, 17), (16, 12), (24, 4), (8, 24)])
+@pytest.mark.parametrize("function", ["v3", "adapter"])
+def test_gate_and_up_of_two_ranks(library, function, ranks):
+    """Adapters of two ranks of which one is no multiple of 8: the backward's
+    dg B_g and du B_u stand side by side only where both halves' rows are aligned."""
+    n, h, d, bf = 300, 128, 512, torch.bfloat16
+    x = torch.zeros(n, h, dtype=bf, requires_grad=True)
+    wg, wu, wd = (torch.zeros(s, dtype=bf) for s in ((d, h), (d, h), (h, d)))
+    (ag, bg), (au, bu) = ((torch.zeros(r, h, dtype=bf, requires_grad=True),
+                           torch.zeros(r, d, dtype=bf).t().requires_grad_()) for r in ranks)
+    if function == "v3":
+        y = F.FlashFFNv3Function.apply(x, wg, ag, bg, wu, au, bu, wd, None, None, 2.0, 2.0, 0.0)
+    else:
+        y = F.FlashFFNv3AdapterFunction.apply(x, wg, ag, bg, None, None, wu, au, bu, None, None, wd,
+                                              None, None, None, None, 2.0, 2.0, 0.0)
+    y.backward(torch.zeros_like(y))
+    assert ag.grad.shape == (ranks[0], h) and bu.grad.shape == (d, ranks[1])
