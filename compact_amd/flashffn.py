@@ -288,13 +288,9 @@ def _gate_up_lora(x_2d, a_gate, b_gate, s_gate, a_up, b_up, s_up):
 
 
 def _gate_up_terms(a_gate, b_gate, s_gate, xa_g, a_up, b_up, s_up, xa_u):
-    """G.ffn_gate_up's keyword terms; a B factor goes in as rows of its ranks (a
-    single rank's column as rows of one, whatever stride its size-1 dimension
-    has: contiguous() would leave that stride)."""
+    """G.ffn_gate_up's keyword terms; a B factor goes in as rows of its ranks."""
     def rows(b):
-        if b.stride(1) == 1:
-            return b
-        return b.reshape(-1)[:, None] if b.shape[1] == 1 else b.contiguous()
+        return b if b.stride(1) == 1 else b.contiguous()
     return dict(lora_gate=None if a_gate is None else (xa_g, rows(b_gate), s_gate),
                 lora_up=None if a_up is None else (xa_u, rows(b_up), s_up))
 

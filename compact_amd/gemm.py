@@ -179,14 +179,15 @@ def _lora_args_whole(terms, n_q, r):
     return r, ldp, int(q_km), ldq, out, terms
 
 
-def _lora_args(terms, n_q, dims, x):
+def _lora_args(terms, n_q, dims, x, kmajor=None):
     """(rank, ldp, q_kmajor, ldq, [(p, q, alpha) x 2], keep) for up to two
     terms (p [M, r], q the logical [r, N] factor, alpha) of a GEMM with the
     (k, n) `dims` (lora_fusable) and rows and type of its left operand x; `keep`
     holds any re-laid copies alive until the launch.  The kernels fetch P and
     K-major Q in 16-byte chunks of 8 k, so a rank that is not a multiple of 8 is
     zero-padded to the next one (8, 16, 24 or 32): the padded k add exact zeros to
-    each fp32 dot product."""
+    each fp32 dot product.  kmajor: the layout of Q that the kernel takes, for a
+    single rank, whose strides fit both."""
     terms = [t for t in terms if t is not None]
     assert 1 <= len(terms) <= 2
     for pm, q, _ in terms:
@@ -208,7 +209,10 @@ def _lora_args(terms, n_q, dims, x):
         for pm, q, al in terms:
             # a factor given as [r, N] rows (an A weight) gains zero rows; one
             # stored [N, r] (a B weight, q its transposed view) zero columns
-            if q.stride(1) == 1 and q.stride(0) != 1:
+            rows = q.stride(1) == 1 and q.stride(0) != 1
+            if r == 1 and kmajor is not None:
+                rows = not kmajor
+            if rows:
                 q = pad(q, (0, 0, 0, rp - r))
             else:
                 q = pad(q.t(), (0, rp - r)).t()
@@ -851,7 +855,7 @@ def ffn_gate_up(x, w_gate, w_up, cache: int, group_size: int, want_h_mid: bool =
         # term 0 on the gate columns, term 1 on the up columns (absent: no-op)
         present = [t for t in (lora_gate, lora_up) if t is not None]
         r, ldp, qk, _, t, keep = _lora_args([(xa, bw.t(), s) for xa, bw, s in present], d,
-                                            ((hdim, d),), x)
+                                            ((hdim, d),), x, kmajor=True)
         assert qk == 1, "the gate/up adapter B factors go K-major"
         if lora_gate is None:
             t = [(None, None, 0.0), t[0]]
@@ -911,7 +915,7 @@ def ffn_gate_up_outlier(x, w_gate, w_up, cache: int, group_size: int, slot_gate,
     if lora_gate is not None or lora_up is not None:
         present = [tt for tt in (lora_gate, lora_up) if tt is not None]
         rank, ldp, qk, _, t, keep = _lora_args([(xa, bw.t(), sc) for xa, bw, sc in present], d,
-                                               ((hdim, d),), x)
+                                               ((hdim, d),), x, kmajor=True)
         assert qk == 1, "the gate/up adapter B factors go K-major"
         if lora_gate is None:
             t = [(None, None, 0.0), t[0]]
@@ -969,7 +973,8 @@ def ffn_down_dgrad(grad_y, w_down, cache: int, group_size: int, c_gate, s_gate, 
         if lora is not None:
             gyb, a_down, s = lora
             a_down = a_down.contiguous()
-            rank, ldp, qk, ldq, t, keep = _lora_args([(gyb, a_down, s)], d, ((hdim, d),), grad_y)
+            rank, ldp, qk, ldq, t, keep = _lora_args([(gyb, a_down, s)], d, ((hdim, d),),
+                                                     grad_y, kmajor=False)
             assert qk == 0 and ldq == d
             pp, qq, alpha = t[0]
         with _timed("ffn_down_dgrad"):
@@ -982,7 +987,8 @@ def ffn_down_dgrad(grad_y, w_down, cache: int, group_size: int, c_gate, s_gate, 
     elif lora is not None:
         gyb, a_down, s = lora
         a_down = a_down.contiguous()          # [r, inter] rows: the MN-major factor
-        r, ldp, qk, ldq, t, keep = _lora_args([(gyb, a_down, s)], d, ((hdim, d),), grad_y)
+        r, ldp, qk, ldq, t, keep = _lora_args([(gyb, a_down, s)], d, ((hdim, d),),
+                                              grad_y, kmajor=False)
         assert qk == 0 and ldq == d
         with _timed("ffn_down_dgrad"):
             rc = _lib.api().cpt_ffn_down_dgrad_lora(

@@ -220,3 +220,24 @@ def test_gate_and_up_of_two_ranks(library, function, ranks):
                                               None, None, None, None, 2.0, 2.0, 0.0)
     y.backward(torch.zeros_like(y))
     assert ag.grad.shape == (ranks[0], h) and bu.grad.shape == (d, ranks[1])
+
+
+@pytest.mark.parametrize("mode", ["bf16", "recompute"])
+@pytest.mark.parametrize("function", ["v3", "adapter"])
+@pytest.mark.parametrize("strides", [(1, 1), (256, 1), (7, 1)])
+def test_single_rank_down_factor_of_any_strides(library, function, mode, strides):
+    """A single-rank A_d [1, d] rides in the down dgrad's epilogue as a row, whatever
+    stride its size-1 dimension has (1 where it is a transposed column)."""
+    n, h, d, bf = 64, 128, 256, torch.bfloat16
+    x = torch.zeros(n, h, dtype=bf, requires_grad=True)
+    wg, wu, wd = (torch.zeros(s, dtype=bf) for s in ((d, h), (d, h), (h, d)))
+    ad = torch.zeros(d, dtype=bf).as_strided((1, d), strides).requires_grad_()
+    bd = torch.zeros(h, 1, dtype=bf, requires_grad=True)
+    if function == "v3":
+        y = F.FlashFFNv3Function.apply(x, wg, None, None, wu, None, None, wd, ad, bd, 0.0, 0.0, 2.0,
+                                       mode)
+    else:
+        y = F.FlashFFNv3AdapterFunction.apply(x, wg, None, None, None, None, wu, None, None, None,
+                                              None, wd, ad, bd, None, None, 0.0, 0.0, 2.0, mode)
+    y.backward(torch.zeros_like(y))
+    assert ad.grad.shape == (1, d)
