@@ -759,6 +759,12 @@ def _has(m, name: str) -> bool:
     return _attr(m, name, _MISSING) is not _MISSING
 
 
+def _own(m, name: str):
+    """m.name, its AttributeError included."""
+    v = _attr(m, name, _MISSING)
+    return getattr(m, name) if v is _MISSING else v
+
+
 def _holds_entries(proj: nn.Module, attr: str) -> bool:
     v = _attr(proj, attr)
     return v is not None and len(v) > 0
@@ -805,9 +811,9 @@ def _warn_dropout(family: str, drop: nn.Module):
 def _lora_factors(proj: nn.Module, family: str = "LoRA"):
     """(W, A, B, s) of a PEFT LoRA-style wrapper's active adapter."""
     name = _active_adapter(proj)
-    _warn_dropout(family, _attr(proj, "lora_dropout")[name])
-    return (_attr(proj.get_base_layer(), "weight"), _attr(_attr(proj, "lora_A")[name], "weight"),
-            _attr(_attr(proj, "lora_B")[name], "weight"), float(proj.scaling[name]))
+    _warn_dropout(family, _own(proj, "lora_dropout")[name])
+    return (_own(proj.get_base_layer(), "weight"), _own(_own(proj, "lora_A")[name], "weight"),
+            _own(_own(proj, "lora_B")[name], "weight"), float(proj.scaling[name]))
 
 
 def _v3_extract_proj(proj: nn.Module):

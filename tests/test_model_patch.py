@@ -139,3 +139,24 @@ def test_attribute_lookup_is_getattrs():
               nn.ModuleDict({"weight": nn.Linear(2, 2)}), object(), nn.BatchNorm1d(2)):
         for name in ("weight", "bias", "running_mean", "base_layer", "training"):
             assert _attr(m, name, "absent") is getattr(m, name, "absent")
+
+
+@pytest.mark.parametrize("missing", ["lora_A", "lora_B", "base_layer", "lora_dropout"])
+def test_factor_modules_without_their_weight_are_refused(missing):
+    """A factor module that keeps no `weight` (a wrapper around the Linear, say) is
+    an AttributeError: None would mean that the projection has no adapter."""
+    from compact_amd.flashffn import _v3_extract_proj, _v3_extract_proj_adapter
+    from compact_amd.model_patch import LoraLinear
+    proj = LoraLinear(nn.Linear(16, 8, bias=False), 4, 8.0)
+    wrapped = nn.Module()
+    if missing == "lora_dropout":
+        del proj.lora_dropout
+    elif missing == "base_layer":
+        wrapped.inner = proj.base_layer
+        proj.base_layer = wrapped
+    else:
+        wrapped.inner = getattr(proj, missing)["default"]
+        getattr(proj, missing)["default"] = wrapped
+    for extract in (_v3_extract_proj, lambda p: _v3_extract_proj_adapter(p, torch.float32)):
+        with pytest.raises(AttributeError):
+            extract(proj)
