@@ -504,6 +504,8 @@ class FlashFFNv3Function(torch.autograd.Function):
                 h_mid = K.silu_mul(h_gate, h_up)
 
         y, ha_d = _proj(h_mid, w_down, a_down, b_down, s_down, "gemm_fwd_down", planes)   # :1435-1439
+        if planes is not None:
+            planes.drop(h_mid)
 
         if not fused_quant:                                                # :1442-1451
             if quant and k_out > 0:
@@ -665,6 +667,8 @@ class FlashFFNv3Function(torch.autograd.Function):
                 grad_w_down = _mm(gy.t(), h_mid_hat, "gemm_wgrad_down", planes)
             if need_ad:
                 grad_a_down = _mm_scaled(gyB_d.t(), h_mid_hat, s_down, "gemm_grad_a_down", planes)
+            if planes is not None:
+                planes.drop(h_mid_hat)
             del h_mid_hat
         if need_bd and grad_b_down is None:
             grad_b_down = _mm_scaled(gy.t(), ha_d, s_down, "gemm_grad_b_down", planes)   # :1545
@@ -1036,6 +1040,8 @@ class FlashFFNv3AdapterFunction(torch.autograd.Function):
                 h_mid = K.silu_mul(h_gate, h_up)
 
         y, ha_d = _proj(h_mid, w_down, a_down, b_down, s_down, "gemm_fwd_down", planes)   # :1990-1994
+        if planes is not None:
+            planes.drop(h_mid)
         y = _scaled(y, m_down, nu_down, inplace=True)                              # :1996
 
         if not fused_quant:                                                         # :1998-2007
@@ -1195,6 +1201,8 @@ class FlashFFNv3AdapterFunction(torch.autograd.Function):
                         raw_d = _addmm(raw_d, ha_d, b_down.t(), s_down, "gemm_recompute_down_lora")
                 grad_m_down = K.col_dot_div(gy, raw_d, nu_down)
                 del raw_d
+            if planes is not None:
+                planes.drop(h_mid_hat)
             del h_mid_hat
         if need_bd and grad_b_down is None:
             grad_b_down = _mm_scaled(g_eff_y.t(), ha_d, s_down, "gemm_grad_b_down", planes)

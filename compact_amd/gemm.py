@@ -1104,34 +1104,57 @@ def mm_splitk(a: torch.Tensor, b: torch.Tensor, alpha: float = 1.0, splits: int 
 class Planes:
     """The bf16 planes of the fp32 operands of one forward or backward call.
 
-    Each operand is split once, however many of the call's products read it,
-    whatever view of it they take.  An instance lives for one call and holds its
-    operands, so no other tensor can take their memory meanwhile; an operand
-    must not be written between its products."""
+    An operand is split once for the products that follow each other on it,
+    whatever view of it they take.  Planes are 1.5 times their operand, so at most
+    KEEP_BYTES of them are held: the least recently used go first, and are made
+    again if a later product asks.  320 MiB is what the widest backward of 2048
+    tokens at 2048 x 5632 shares (grad_x's four operands and two before them); a
+    call of 8192 tokens would hold 1.3 GiB beside its own 0.7.  An entry holds its
+    operand, so no other tensor can take its memory meanwhile; an operand must not
+    be written between its products."""
 
+    KEEP_BYTES = 320 << 20
     MAX_FLAGS = 32
 
     def __init__(self):
         self._made = {}
+        self._bytes = 0
         self._flags = None
+        self._used = 0
 
     def of(self, t: torch.Tensor):
-        """(planes bf16 [3, rows, cols], flag int32 [1]) of row-major fp32 t."""
+        """(planes bf16 [3, rows, cols], flag int32 [1]) of row-major fp32 t.  The
+        caller keeps both until its product is launched."""
         key = (t.data_ptr(), t.shape, t.stride(0))
-        hit = self._made.get(key)
+        hit = self._made.pop(key, None)
         if hit is None:
-            if self._flags is None:
+            nbytes = 6 * t.numel()
+            while self._made and self._bytes + nbytes > self.KEEP_BYTES:
+                self._forget(next(iter(self._made)))
+            if self._flags is None or self._used == self.MAX_FLAGS:
                 self._flags = torch.zeros((self.MAX_FLAGS,), dtype=torch.int32, device=t.device)
-            i = len(self._made)
-            assert i < self.MAX_FLAGS
-            flag = self._flags[i:i + 1]
+                self._used = 0
+            flag = self._flags[self._used:self._used + 1]
+            self._used += 1
             planes = torch.empty((3,) + tuple(t.shape), dtype=torch.bfloat16, device=t.device)
             with _timed("split_f32"):
                 rc = _lib.api().cpt_split_f32(t.data_ptr(), t.stride(0), t.shape[0], t.shape[1],
                                               planes.data_ptr(), flag.data_ptr(), _stream(t))
             check(rc, "split_f32")
-            hit = self._made[key] = (planes, flag, t)
+            hit = (planes, flag, t)
+            self._bytes += nbytes
+        self._made[key] = hit
         return hit[0], hit[1]
+
+    def _forget(self, key):
+        self._bytes -= 6 * self._made.pop(key)[2].numel()
+
+    def drop(self, t: torch.Tensor) -> None:
+        """Forget t and every view of it: its last product is launched."""
+        base = t.untyped_storage().data_ptr()
+        for key in [k for k, e in self._made.items()
+                    if e[2].untyped_storage().data_ptr() == base]:
+            self._forget(key)
 
 
 def _x3_operand(t: torch.Tensor):
@@ -1204,9 +1227,41 @@ def mm_x3(a, b, planes: Planes, a2=None, b2=None, alpha: float = 1.0,
     assert a2 is None or (a2.shape[0] == M and tuple(b2.shape) == (a2.shape[1], N)), \
         f"second pair {tuple(a2.shape)} @ {tuple(b2.shape)} of an [{M}, {N}] product"
 
+    c = torch.empty((M, N), dtype=torch.float32, device=a.device)
+    pm, pn = _x3_panels(M, N, K if a2 is None else K + a2.shape[1], planes.KEEP_BYTES)
+    for m in range(0, M, pm):
+        for n in range(0, N, pn):
+            if pm >= M and pn >= N:
+                _x3_launch(c, a, b, a2, b2, planes, alpha, name)
+                break
+            row, col = slice(m, m + pm), slice(n, n + pn)
+            _x3_launch(c[row, col], a[row], b[:, col], None if a2 is None else a2[row],
+                       None if a2 is None else b2[:, col], planes, alpha, name)
+    return c
+
+
+def _x3_panels(m: int, n: int, k: int, limit: int) -> tuple[int, int]:
+    """(rows, columns) of the panels that an [m, n] product of k runs in, so that
+    the planes of one panel's operands stay within `limit` bytes (or are 256
+    wide): the wider side is halved first."""
+    pm, pn = m, n
+    while 6 * (pm + pn) * k > limit and max(pm, pn) > 256:
+        if pm >= pn:
+            pm = (pm // 2 + 255) // 256 * 256
+        else:
+            pn = (pn // 2 + 255) // 256 * 256
+    return pm, pn
+
+
+def _x3_launch(c, a, b, a2, b2, planes: Planes, alpha: float, name: str) -> None:
+    """One panel of mm_x3 into the view c."""
+    (M, K), N = a.shape, b.shape[1]
+    held = []
+
     def operand(t, left):
         s, own = _x3_operand(t)
         p, flag = planes.of(s)
+        held.append((p, flag))
         # [M][K] or [N][K] storage is K-major
         return p.data_ptr(), s.shape[0] * s.shape[1], s.shape[1], int(own == left), flag.data_ptr()
     pa, sa, lda, ak, fa = operand(a, True)
@@ -1218,25 +1273,24 @@ def mm_x3(a, b, planes: Planes, a2=None, b2=None, alpha: float = 1.0,
         pa2, sa2, lda2, ak2, fa2 = operand(a2, True)
         pb2, sb2, ldb2, bk2, fb2 = operand(b2, False)
         assert (lda2, ldb2, ak2, bk2) == (lda, ldb, ak, bk), "the pairs share one layout"
-    c = torch.empty((M, N), dtype=torch.float32, device=a.device)
     tiles, splits = x3_plan(M, N, 6 * ((K + 63) // 64 + (K2 + 63) // 64),
                             K % 64 == 0 and K2 % 64 == 0)
     ws = (torch.empty((splits * M * N,), dtype=torch.float32, device=a.device)
           if splits > 1 else None)
     st = _stream(a)
     L = _lib.api()
+    ldc = c.stride(0)
     with _timed(name):
         rc = L.cpt_gemm_f32x3(pa, sa, lda, ak, pb, sb, ldb, bk, pa2, sa2, pb2, sb2, K2, fa, fb,
-                              fa2, fb2, c.data_ptr(), N, M, N, K, float(alpha), tiles, splits,
+                              fa2, fb2, c.data_ptr(), ldc, M, N, K, float(alpha), tiles, splits,
                               None if ws is None else ws.data_ptr(), st)
         check(rc, name)
         for i, (u, v) in enumerate(((a, b), (a2, b2))[:1 if a2 is None else 2]):
             rc = L.cpt_gemm_any_if(fa, fb, fa2, fb2, _lib.F32, u.data_ptr(), u.stride(0),
                                    u.stride(1), v.data_ptr(), v.stride(0), v.stride(1),
-                                   c.data_ptr(), N, 1, M, N, u.shape[1], float(alpha),
+                                   c.data_ptr(), ldc, 1, M, N, u.shape[1], float(alpha),
                                    ANY_ADD if i else ANY_SCALE, st)
             check(rc, name)
-    return c
 
 
 # epilogues of the general-layout GEMM (cpt_gemm_any)

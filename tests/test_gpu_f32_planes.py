@@ -127,3 +127,58 @@ def test_192_column_tiles_equal_256(layout, m, n, k, ranges, monkeypatch):
         got.append((G.mm_x3(a, b, G.Planes()), G.mm_x3(a, b, G.Planes(), a2, b2)))
     assert all(torch.equal(u, v) for u, v in zip(*got))
     assert _errors(got[0][0], a, b)[1] < 2.0 ** -22
+
+
+@pytest.mark.parametrize("layout", ["nt", "nn", "tn", "tt"])
+@pytest.mark.parametrize("m,n,k", [(1000, 776, 512), (264, 2056, 320), (2304, 8, 640)])
+def test_panels_equal_the_whole_product(layout, m, n, k, monkeypatch):
+    """A product run in panels (its planes over the bound) has the bits of the whole
+    one where both take the same tiles, and a value outside the planes' range
+    sends its panels to the general-layout kernel."""
+    from compact_amd import gemm as G
+    monkeypatch.setattr(G, "x3_plan", lambda *_: (256, 1))
+    a, b = _operands(layout, m, n, k)
+    a2, b2 = _operands(layout, m, n, k, seed=5)
+    whole = G.mm_x3(a, b, G.Planes()), G.mm_x3(a, b, G.Planes(), a2, b2)
+    monkeypatch.setattr(G.Planes, "KEEP_BYTES", 1 << 20)
+    assert G._x3_panels(m, n, k, 1 << 20) != (m, n)
+    P = G.Planes()
+    assert torch.equal(whole[0], G.mm_x3(a, b, P))
+    assert torch.equal(whole[1], G.mm_x3(a, b, P, a2, b2))
+    a[m - 1, 3] = float("inf")
+    got, ref = G.mm_x3(a, b, G.Planes()), G.mm_any_kernel(a, b)
+    assert torch.equal(got[m - 1].view(torch.int32), ref[m - 1].view(torch.int32))
+    assert bool(got[:m - 1].isfinite().all())
+
+
+@pytest.mark.parametrize("train,mode", [("full", "int8"), ("full", "recompute"), ("none", "int8")])
+def test_peak_memory_of_a_step(train, mode, monkeypatch):
+    """An fp32 step holds at most Planes.KEEP_BYTES of planes and 64 MiB of split
+    partials (256 tiles) beside what it holds on the general-layout kernel."""
+    from compact_amd import flashffn as F
+    from compact_amd import gemm as G
+    n, h, d = 8192, 2048, 5632
+    x, gy = _rand(n, h, seed=1), _rand(n, h, seed=2)
+    ws = [_rand(*s, seed=3) * 0.02 for s in ((d, h), (d, h), (h, d))]
+    for t in [x] + ws:
+        t.requires_grad_(train == "full")
+
+    def step():
+        y = F.FlashFFNv3Function.apply(x, ws[0], None, None, ws[1], None, None, ws[2], None, None,
+                                       0.0, 0.0, 0.0, mode, 64)
+        return torch.autograd.grad(y, [x] + ws, gy) if train == "full" else y
+
+    def peak():
+        step()
+        torch.cuda.synchronize()
+        base = torch.cuda.memory_allocated()
+        torch.cuda.reset_peak_memory_stats()
+        out = step()
+        torch.cuda.synchronize()
+        del out
+        return torch.cuda.max_memory_allocated() - base
+    planes = peak()
+    monkeypatch.setattr(G, "x3_fits", lambda a, b: False)
+    general = peak()
+    print(f"{train} {mode}: {general / 2**20:.0f} MiB on the general kernel, {planes / 2**20:.0f}")
+    assert planes <= general + G.Planes.KEEP_BYTES + (64 << 20)

@@ -241,3 +241,53 @@ def test_single_rank_down_factor_of_any_strides(library, function, mode, strides
                                               None, wd, ad, bd, None, None, 0.0, 0.0, 2.0, mode)
     y.backward(torch.zeros_like(y))
     assert ad.grad.shape == (1, d)
+
+
+def _covered(calls, m, n, base):
+    """How often each output of an [m, n] fp32 product at `base` is written."""
+    seen = torch.zeros(m, n, dtype=torch.int32)
+    for name, a in calls:
+        if name == "cpt_gemm_f32x3":
+            at, ldc, rows, cols = (a[17] - base) // 4, a[18], a[19], a[20]
+            assert ldc == n
+            seen[at // n:at // n + rows, at % n:at % n + cols] += 1
+    return seen
+
+
+@pytest.mark.parametrize("left,right", [("nn", "nn"), ("tn", "tt")])
+@pytest.mark.parametrize("m,n,k", [(1000, 776, 512), (264, 2048, 320), (2304, 8, 640),
+                                   (256, 256, 4096)])
+def test_fp32_planes_stay_within_their_bound(library, monkeypatch, m, n, k, left, right):
+    """A product whose operands' planes exceed the bound runs in panels that write
+    every output once, and holds no more planes at a time than the bound (or one
+    256-wide panel of each operand)."""
+    limit = 1 << 20
+    monkeypatch.setattr(G.Planes, "KEEP_BYTES", limit)
+    a = torch.zeros(k, m).t() if left[0] == "t" else torch.zeros(m, k)
+    b = torch.zeros(n, k).t() if right[1] == "t" else torch.zeros(k, n)
+    P, held = G.Planes(), []
+    make = P.of
+    P.of = lambda t: (make(t), held.append(P._bytes))[0]
+    c = G.mm_x3(a, b, P)
+    assert bool((_covered(library.calls, m, n, c.data_ptr()) == 1).all())
+    assert max(held) <= max(limit, 6 * 512 * k)
+    assert P._bytes == sum(6 * e[2].numel() for e in P._made.values())
+    P.drop(a)
+    P.drop(b.t())
+    assert not P._made and P._bytes == 0
+
+
+def test_fp32_planes_of_two_products_are_shared(library):
+    """... and made again once others have pushed them out."""
+    x, w = torch.zeros(64, 128), torch.zeros(256, 128)
+    P = G.Planes()
+    G.mm_x3(x, w.t(), P)
+    G.mm_x3(x.t(), x, P)
+    splits = sum(name == "cpt_split_f32" for name, _ in library.calls)
+    assert splits == 2
+    P.KEEP_BYTES = 6 * 300 * 128
+    G.mm_x3(torch.zeros(128, 128), torch.zeros(128, 128), P)
+    assert P._bytes <= P.KEEP_BYTES
+    G.mm_x3(x, w.t(), P)
+    splits = sum(name == "cpt_split_f32" for name, _ in library.calls)
+    assert splits == 6
