@@ -213,7 +213,8 @@ def _mm_sum(a, b, a2, b2, name, planes=None):
     if _mfma(a, b, a2, b2) or (G.f16_fits(a, b) and G.f16_fits(a2, b2)):
         return G.mm2(a, b, a2, b2, name)
     if (a.dtype == torch.float32 and G.x3_fits(a, b) and G.x3_fits(a2, b2)
-            and a.stride() == a2.stride() and b.stride() == b2.stride()):
+            and a.stride() == a2.stride() and b.stride() == b2.stride()
+            and G.x3_pays(a.shape[0], b.shape[1], a.shape[1] + a2.shape[1])):
         return G.mm_x3(a, b, planes or G.Planes(), a2, b2, name=name)
     out = G.mm_any(a, b, name=name)
     return G.mm_any(a2, b2, 1.0, G.ANY_ADD, out=out, name=name)

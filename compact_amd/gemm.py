@@ -1189,6 +1189,24 @@ def x3_fits(a: torch.Tensor, b: torch.Tensor) -> bool:
     return K % 64 == 0 or (not oa[1] and ob[1])
 
 
+def x3_pays(m: int, n: int, k: int) -> bool:
+    """An fp32 product of k (both pairs' together) is faster on the planes than on
+    the general-layout kernel, whose time goes with k and its rounds of 128 x 128
+    tiles: below this its one launch costs less than two splits, the product and
+    the guarded general kernel.  Measured on MI355X, us general / planes with both
+    operands to split / with none:
+      64 x 704, k 256     32.3 / 42.4 / 22.1    kept general
+      64 x 704, k 320     38.9 / 42.6 / 22.7    kept general
+      64 x 704, k 448     52.0 / 42.9 / 22.3
+      2048 x 2048, k 256  35.0 / 51.9 / 44.5    kept general
+      2048 x 5632, k 64   29.5 / 37.7 / 24.0    kept general
+      2048 x 5632, k 128  45.6 / 40.8 / 29.9
+    and 1 token at 256 x 704, whole steps: forward 147 us general, 165 on the
+    planes; full fine-tune 400 and 444."""
+    tiles = ((m + 127) // 128) * ((n + 127) // 128)
+    return k * max(tiles, 256) >= 352 * 256
+
+
 def x3_plan(m: int, n: int, nk: int, whole: bool) -> tuple[int, int]:
     """(tile width, k ranges) of an fp32 product of nk k-tiles of plane pairs; 256
     x 256 and 256 x 192 tiles need whole k-tiles.  Times per k-tile with the chip
@@ -1304,9 +1322,10 @@ def mm_any(a: torch.Tensor, b: torch.Tensor, alpha: float = 1.0, mode: int = ANY
     """a [M, K] @ b [K, N] for float32 / float16 / bfloat16 operands of any
     strides, in the modes of mm_any_kernel: the products the bf16 engine does
     not take (config C1's float32, unaligned views, rank-1 factors).  fp32
-    operands that fit (x3_fits) go to the bf16 MFMAs, sharing the planes that
-    the caller's other products made."""
-    if mode != ANY_ADD and a.dtype == torch.float32 and x3_fits(a, b):
+    operands that fit (x3_fits) go to the bf16 MFMAs where that pays (x3_pays),
+    sharing the planes that the caller's other products made."""
+    if (mode != ANY_ADD and a.dtype == torch.float32 and x3_fits(a, b)
+            and x3_pays(a.shape[0], b.shape[1], a.shape[1])):
         return mm_x3(a, b, planes or Planes(), alpha=alpha if mode == ANY_SCALE else 1.0,
                      name=name)
     return mm_any_kernel(a, b, alpha, mode, out, name)

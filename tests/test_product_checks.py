@@ -33,13 +33,13 @@ def library(monkeypatch):
     return lib
 
 
-# weights (gate, up, down) that do not fit x [64, 256] or each other
+# weights (gate, up, down) that do not fit x [64, 512] or each other
 MISFITS = {
-    "wide_gate_up": ((128, 512), (128, 512), (256, 128)),
-    "narrow_gate_up": ((128, 192), (128, 192), (256, 128)),
-    "wide_up": ((128, 256), (128, 512), (256, 128)),
-    "wide_down": ((128, 256), (128, 256), (256, 192)),
-    "narrow_down": ((128, 256), (128, 256), (256, 64)),
+    "wide_gate_up": ((512, 1024), (512, 1024), (512, 512)),
+    "narrow_gate_up": ((512, 448), (512, 448), (512, 512)),
+    "wide_up": ((512, 512), (512, 1024), (512, 512)),
+    "wide_down": ((512, 512), (512, 512), (512, 576)),
+    "narrow_down": ((512, 512), (512, 512), (512, 448)),
 }
 
 
@@ -49,7 +49,7 @@ MISFITS = {
 def test_functions_refuse_weights_that_do_not_fit(library, function, misfit, dtype):
     """Whatever the type's route, a product whose inner dimensions differ is an
     AssertionError and never a launch over part (or past the end) of an operand."""
-    x = torch.zeros(64, 256, dtype=dtype)
+    x = torch.zeros(64, 512, dtype=dtype)
     wg, wu, wd = (torch.zeros(s, dtype=dtype, requires_grad=True) for s in MISFITS[misfit])
     with pytest.raises(AssertionError):
         if function == "v3":
@@ -291,3 +291,16 @@ def test_fp32_planes_of_two_products_are_shared(library):
     G.mm_x3(x, w.t(), P)
     splits = sum(name == "cpt_split_f32" for name, _ in library.calls)
     assert splits == 6
+
+
+@pytest.mark.parametrize("m,n,k,planes", [(1, 704, 256, False), (64, 704, 320, False),
+                                          (1, 704, 384, True), (2048, 2048, 256, False),
+                                          (2048, 5632, 64, False), (2048, 5632, 128, True),
+                                          (8, 2048, 64, False), (8, 2048, 2048, True)])
+def test_small_fp32_products_keep_the_general_kernel(library, m, n, k, planes):
+    """Where its one launch is faster than the splits and what follows them."""
+    G.mm_any(torch.zeros(m, k), torch.zeros(n, k).t())
+    G.mm_any(torch.zeros(m, k), torch.zeros(n, k).t(), 2.0, G.ANY_SCALE)
+    names = {name for name, _ in library.calls}
+    assert names == ({"cpt_split_f32", "cpt_gemm_f32x3", "cpt_gemm_any_if"} if planes
+                     else {"cpt_gemm_any"})
