@@ -158,6 +158,8 @@ __global__ __launch_bounds__(kBlock) void topk_abs_kernel(const St<DT>* __restri
 // place, and values and columns are staged in LDS and written in whole rows.
 // The histogram kernel's LDS atomics met on the few exponents of a row: 2048 x
 // 5632 bf16, k 1689: 51 us, here 26.
+constexpr int kCounterBytes = (2 + 8) * kWaves * 4;   // cnt and tot at 8 chunks
+
 template <int NC>
 __global__ __launch_bounds__(kBlock) void topk_abs16_kernel(const uint16_t* __restrict__ t,
                                                             int64_t d, int k,
@@ -168,6 +170,7 @@ __global__ __launch_bounds__(kBlock) void topk_abs16_kernel(const uint16_t* __re
   uint16_t* const si = sv + k;
   __shared__ int cnt[2][kWaves];
   __shared__ int tot[NC][kWaves];
+  static_assert(sizeof(cnt) + sizeof(tot) <= kCounterBytes, "static LDS");
   const int64_t row = blockIdx.x;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   uint4 w[NC];
@@ -288,9 +291,11 @@ int cpt_topk_abs(const void* t, int dtype, int64_t n, int64_t d, int64_t k, void
   if (!t || !values || !indices) return kErrShape;
   hipStream_t st = (hipStream_t)stream;
   const dim3 grid((unsigned)n);
-  // 16-bit rows that fit the registers (8 chunks of 2048) and whose entries fit
-  // 64 KiB of LDS
-  if (dtype != kF32 && d % 8 == 0 && aligned16(t) && d <= 8 * 2048) {
+  // 16-bit rows that fit the registers (8 chunks of 2048) and whose entries,
+  // beside the kernel's own counters, fit the 64 KiB of LDS that a launch may take
+  // without asking for more (k up to 16344)
+  if (dtype != kF32 && d % 8 == 0 && aligned16(t) && d <= 8 * 2048 &&
+      k * 4 + kCounterBytes <= 64 * 1024) {
     const auto kern = d <= 2 * 2048 ? topk_abs16_kernel<2>
                       : d <= 3 * 2048 ? topk_abs16_kernel<3>
                       : d <= 6 * 2048 ? topk_abs16_kernel<6>

@@ -137,3 +137,17 @@ def test_topk_register_rows_and_their_edges(d, dt):
         order = key.sort(dim=-1, descending=True, stable=True).indices[:, :k].sort(dim=-1).values
         assert torch.equal(i.long(), order)
         assert torch.equal(v.view(torch.int16), x.gather(1, order).view(torch.int16))
+
+
+@pytest.mark.parametrize("k", [16336, 16344, 16345, 16384])
+def test_topk_entries_at_the_lds_limit(k):
+    """The last k whose entries fit 64 KiB of LDS beside the register kernel's own
+    160 bytes, and the first that goes to the histogram kernel."""
+    from compact_amd import kernels as K
+    g = torch.Generator(device="cuda").manual_seed(k)
+    x = torch.randn(3, 16384, device="cuda", generator=g).to(torch.bfloat16)
+    v, i = K.topk_abs(x, k)
+    key = x.view(torch.int16).int() & 0x7FFF
+    order = key.sort(dim=-1, descending=True, stable=True).indices[:, :k].sort(dim=-1).values
+    assert torch.equal(i.long(), order)
+    assert torch.equal(v.view(torch.int16), x.gather(1, order).view(torch.int16))
