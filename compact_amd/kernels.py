@@ -505,8 +505,9 @@ def col_dot_div(a: torch.Tensor, b: torch.Tensor, den: torch.Tensor) -> torch.Te
     assert a.dtype == b.dtype == den.dtype, "col_dot_div: one dtype expected"
     a, b, den = a.contiguous(), b.contiguous(), den.contiguous()
     n, d = a.shape
-    # partials of at least 32 rows, at most 64 of them
-    rows = max(32, (n + 63) // 64)
+    # partials of 32 to 128 rows, 64 of them up to 8192 rows: an fp32 chain no longer
+    # than cpt_col_dot_div's (longer only where 65535 chunks, a grid's, run out)
+    rows = max(32, min(128, (n + 63) // 64), (n + 65534) // 65535)
     ws = torch.empty((max(1, (n + rows - 1) // rows), d), dtype=torch.float32, device=a.device)
     out = torch.empty((d,), dtype=a.dtype, device=a.device)
     with _timed("col_dot_div"):

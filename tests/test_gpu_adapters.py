@@ -312,3 +312,23 @@ def test_col_dot_div_row_chunks(n):
     ref, size = prod.sum(0) / den.double(), prod.abs().sum(0) / den.double()
     err = (K.col_dot_div(a, b, den).double() - ref).abs()
     assert bool((err <= 2.0 ** -8 * 1.01 * ref.abs() + (n + 2) * 2.0 ** -24 * size).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("n,d", [(8192, 72), (8193, 8), (20000, 24), (70000, 9)])
+def test_col_dot_div_of_many_rows(n, d, dtype):
+    """From 8192 rows on the partials are cpt_col_dot_div's of 128 rows, bit for bit:
+    no longer fp32 chain on narrow outputs of many rows."""
+    from compact_amd import _lib
+    from compact_amd import kernels as K
+    g = torch.Generator(device="cuda").manual_seed(n)
+    a, b = (torch.randn(n, d, device="cuda", generator=g).to(dtype) for _ in range(2))
+    den = torch.randn(d, device="cuda", generator=g).abs().add(0.5).to(dtype)
+    got = K.col_dot_div(a, b, den)
+    lib = _lib.lib()
+    ws = torch.empty(lib.cpt_col_dot_workspace_bytes(n, d) // 4, device="cuda")
+    ref = torch.empty_like(got)
+    _lib.check(lib.cpt_col_dot_div(a.data_ptr(), b.data_ptr(), den.data_ptr(), n, d,
+                                   _lib.F32 if dtype == torch.float32 else _lib.BF16, ws.data_ptr(),
+                                   ref.data_ptr(), torch.cuda.current_stream().cuda_stream), "ref")
+    assert torch.equal(got, ref)

@@ -304,3 +304,14 @@ def test_small_fp32_products_keep_the_general_kernel(library, m, n, k, planes):
     names = {name for name, _ in library.calls}
     assert names == ({"cpt_split_f32", "cpt_gemm_f32x3", "cpt_gemm_any_if"} if planes
                      else {"cpt_gemm_any"})
+
+
+@pytest.mark.parametrize("n,rows", [(0, 32), (1, 32), (2048, 32), (2049, 33), (8192, 128),
+                                    (8193, 128), (100000, 128), (8388480, 128), (8388481, 129)])
+def test_column_dot_chunks(library, n, rows):
+    """Rows of an fp32 partial: none above 128 while the grid has chunks left."""
+    t = torch.zeros(1, 8).expand(n, 8) if n < 1 << 20 else torch.zeros(n, 1, dtype=torch.bfloat16)
+    K.col_dot_div(t, t, torch.ones(t.shape[1], dtype=t.dtype))
+    (name, args), = library.calls
+    assert name == "cpt_col_dot_div_rows" and args[3] == n and args[5] == rows
+    assert -(-n // rows) <= 65535
