@@ -20,9 +20,9 @@
 //                 lgkmcnt(0)), barrier: stage kt % S is free, tile kt + 1 whole
 //   slots 16..31  sub-step 1 on F1, reading F0 of kt + 1; the first 4 loads of
 //                 tile kt + S into stage kt % S
-// Bound: with one block per CU (S = 4, 128 KiB) the k-tile costs 0.4 us, the
-// 32 KiB it loads at the latency of three tiles in flight, against 0.21 us of
-// MFMAs; a full grid reaches 1.07 PFLOP/s (2048 x 2048, k 5632: 44.0 us, where
+// Bound: with one block per CU (S = 4, 128 KiB) the k-tile costs 0.42 us (1 to
+// 128 blocks; 0.50 to 0.55 with 256), the 32 KiB it loads at the latency of three
+// tiles in flight, against 0.21 us of MFMAs; a full grid reaches 1.07 PFLOP/s (2048 x 2048, k 5632: 44.0 us, where
 // 64 tiles of 256 x 256 took 96.2).  S = 2 (64 KiB) lets two blocks share a CU:
 // the second block's MFMAs cover the first one's barrier, prologue and epilogue
 // (2048 x 4096, k 11008: 161.5 us against 202.7).

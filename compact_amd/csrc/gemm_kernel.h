@@ -1321,9 +1321,9 @@ int launch_nt16(const KArgs& A, hipStream_t st);
 // CACHE_BF16), which st16_reduce sums and finishes.
 template <int DT, bool AK, bool BK, int EPI, int CACHE, int LT, int S>
 int launch_st16(KArgs A, hipStream_t st);
-// Split products, and fp32 ones of bf16 planes (X3), on tiles of 256 x 32 NI
 // 256 x 192 tiles for a plain store, by the rounds of blocks (gemm16.hip)
 bool use_192(const KArgs& A, bool a_kmajor);
+// Split products, and fp32 ones of bf16 planes (X3), on tiles of 256 x 32 NI
 template <bool AK, bool BK, bool X3, int NI>
 int launch_nt16_f32(KArgs A, hipStream_t st);
 // Split sums, adapter terms (`terms` of A's) and epilogue of a split product:

@@ -1283,7 +1283,7 @@ def make_v3_adapter_forward(mlp: nn.Module, cache_mode: str = "int4", group_size
 
 def _gate_up(x_2d, w_gate, w_up, keep: bool):
     """(h_mid, h_gate | None, h_up | None): the fused dual GEMM + GLU on the
-    engine for bf16, the general-layout GEMMs + the GLU kernel otherwise."""
+    engine for bf16, _mm's products + the GLU kernel otherwise."""
     if _mfma(x_2d, w_gate, w_up) and x_2d.shape[0] > 0:
         h_mid, hg, hu, *_ = G.ffn_gate_up(x_2d, w_gate, w_up,
                                           _lib.CACHE_BF16 if keep else _lib.CACHE_NONE, 64)
@@ -1324,7 +1324,8 @@ class FlashFFNFunction(torch.autograd.Function):
           returns grad_x only.
     Device path: the fused dual GEMM + GLU forward and the fused dgrad GEMM +
     SwiGLU backward on the MFMA engine (bf16), the top-K select and scatter
-    kernels; the general-layout GEMMs + the GLU kernels for other dtypes."""
+    kernels; for fp16 and fp32 the products of _mm (16-bit tiles, bf16 planes made
+    for each product, or the general-layout GEMM) and the GLU kernels."""
 
     @staticmethod
     def forward(ctx, x, w_gate, w_up, w_down, k_fraction=0.3):

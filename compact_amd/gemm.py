@@ -476,8 +476,8 @@ def skinny_dual(x: torch.Tensor, q: torch.Tensor, p: torch.Tensor, alpha_c: floa
     ws = torch.empty((max(nbytes, 4) // 4,), dtype=torch.float32, device=x.device)
     with _timed(name):
         rc = _lib.api().cpt_gemm16_skinny_dual(
-            _DT16[x.dtype], x.data_ptr(), x.stride(0), q.data_ptr(), ldq, q_nr, p.data_ptr(), p.stride(0),
-            c.data_ptr(), c.stride(0), float(alpha_c), z.data_ptr(), z.stride(0), 0,
+            _DT16[x.dtype], x.data_ptr(), x.stride(0), q.data_ptr(), ldq, q_nr, p.data_ptr(),
+            p.stride(0), c.data_ptr(), c.stride(0), float(alpha_c), z.data_ptr(), z.stride(0), 0,
             float(alpha_z), T, N, R, splits, ws.data_ptr(), _stream(x))
     check(rc, name)
     return c, z
@@ -579,8 +579,9 @@ def small_tiles(m: int, n: int) -> bool:
 
 
 # Split products (cpt_gemm16): k-tiles per range at least, and k-tiles taken off
-# each block at least.  A lone block takes 0.4 us per k-tile; the first tiles'
-# latency is worth about 5, the partials and the second kernel about 20.
+# each block at least.  A block alone on its CU takes 0.42 us per k-tile (up to 128
+# of them, all that split_plan splits; 0.55 with 256, tile_plan's rate); the first
+# tiles' latency is worth about 5, the partials and the second kernel about 20.
 # Measured on MI355X, us unsplit / split (both with their launches):
 #   512 x 2048, k 5632   (64 tiles, 4 ranges)   39.6 / 24.0
 #   512 x 2048, k 11264  (64, 4)                81.3 / 35.8
@@ -610,8 +611,9 @@ def tile_plan(m: int, n: int, nk: int, half: bool = False) -> tuple[int, int]:
     split_plan has it, or, bf16 only, 256 x 256 tiles with k split to fill the
     CUs, whichever the measured rates make cheapest.
 
-    Rates on MI355X, us per k-tile: 0.55 for 128 x 128 tiles alone on a CU, 1.0
-    for two sharing it, 1.0 to 1.45 for a 256 x 256 tile as the chip fills up;
+    Rates on MI355X, us per k-tile: 0.55 for 128 x 128 tiles alone on a CU with
+    most CUs busy (240 of them, k 11264: 0.50 K-major, 0.52 MN-major B), 1.0 for two
+    sharing it, 1.0 to 1.45 for a 256 x 256 tile as the chip fills up;
     8 for a block's ends; a split adds 8 and 1.1 per million partials.  Measured,
     us unsplit (128 x 128 tiles) / split 256 x 256 ones:
       2048 x 4096, k 22016 (128 large tiles, 2 ranges)  382 / 277
@@ -619,7 +621,8 @@ def tile_plan(m: int, n: int, nk: int, half: bool = False) -> tuple[int, int]:
       3000 x 2048, k 11264 (96, 2)                      162 / 127
       1500 x 4096, k 11008 (96, 2)                      161 / 128
       1024 x 4096, k 11008 (64, 4)                       91 / 95     kept unsplit
-      4096 x 2048, k 5632  (128, 2)                      87 / 90     kept unsplit"""
+      4096 x 2048, k 5632  (128, 2)                      87 / 90     kept unsplit
+      1808 x 2048, k 11264 (64, 4)                       89 / 89, 92 / 90 kept unsplit"""
     t128 = ((m + 127) // 128) * ((n + 127) // 128)
     t256 = ((m + 255) // 256) * ((n + 255) // 256)
     if t128 == 0:
