@@ -155,19 +155,21 @@ def lora_fusable(rank: int, *dims) -> bool:
                                                 for k, n in dims))
 
 
-def _lora_args_whole(terms, n_q, r):
+def _lora_args_whole(terms, n_q, r, x):
     """_lora_args' result where the terms can be used as they are (a rank of
     whole 8-wide chunks, aligned rows, one layout for both), else None."""
     if r % 8:
         return None
     out = []
+    dt, m = x.dtype, x.shape[0]
     ldp = ldq = q_km = None
     for pm, q, al in terms:
         sp, sq = pm.stride(), q.stride()
         km = sq[0] == 1 and sq[1] == r
         if ((ldp is not None and (sp[0] != ldp or km != q_km or (not km and sq[0] != ldq)))
-                or sp[1] != 1 or sp[0] % 8 or pm.dtype not in _DT16 or q.dtype != pm.dtype
-                or pm.shape[1] != r or tuple(q.shape) != (r, n_q)):
+                or sp[1] != 1 or sp[0] % 8 or pm.dtype != dt or q.dtype != dt or not pm.is_cuda
+                or not q.is_cuda or pm.shape[0] < m or pm.shape[1] != r
+                or tuple(q.shape) != (r, n_q)):
             return None
         pp, qp = pm.data_ptr(), q.data_ptr()
         if pp % 16 or (qp % 16 if km else sq[1] != 1):
@@ -190,16 +192,16 @@ def _lora_args(terms, n_q, dims, x, kmajor=None):
     single rank, whose strides fit both."""
     terms = [t for t in terms if t is not None]
     assert 1 <= len(terms) <= 2
+    r = terms[0][0].shape[1]
+    fast = _lora_args_whole(terms, n_q, r, x)
+    if fast is not None and lora_fusable(r, *dims):
+        return fast
     for pm, q, _ in terms:
+        _require_device(pm, q)
         assert pm.dtype == q.dtype == x.dtype, \
             f"adapter factors of {pm.dtype} and {q.dtype} in a product of {x.dtype}"
         assert pm.dim() == q.dim() == 2 and pm.shape[0] >= x.shape[0], \
             f"adapter rows {tuple(pm.shape)} for {x.shape[0]} rows"
-    _require_device(*(t for pm, q, _ in terms for t in (pm, q)))
-    r = terms[0][0].shape[1]
-    fast = _lora_args_whole(terms, n_q, r)
-    if fast is not None and lora_fusable(r, *dims):
-        return fast
     assert lora_fusable(r, *dims), \
         f"adapter rank {r} not carried by a GEMM of (k, n) {tuple(dims)} (lora_fusable)"
     if r % 8:
