@@ -1111,12 +1111,15 @@ class Planes:
 
     An operand is split once for the products that follow each other on it,
     whatever view of it they take.  Planes are 1.5 times their operand, so at most
-    KEEP_BYTES of them are held: the least recently used go first, and are made
-    again if a later product asks.  320 MiB is what the widest backward of 2048
-    tokens at 2048 x 5632 shares (grad_x's four operands and two before them); a
-    call of 8192 tokens would hold 1.3 GiB beside its own 0.7.  An entry holds its
-    operand, so no other tensor can take its memory meanwhile; an operand must not
-    be written between its products."""
+    KEEP_BYTES of them are held, or as many bytes as the call's largest operand:
+    the least recently used go first, and are made again if a later product asks.
+    320 MiB is what the widest backward of 2048 tokens at 2048 x 5632 shares
+    (grad_x's four operands and two before them); held without a bound, a call of
+    8192 tokens peaks at 2059 MiB against 727 on the general-layout kernel and 1065
+    so, at 8.7 ms against 18.7 and 9.0.  With 320 MiB at 32768 tokens the weight
+    gradients' panels are narrow: 45.2 ms against 34.3 without a bound.  An entry
+    holds its operand, so no other tensor can take its memory meanwhile; an operand
+    must not be written between its products."""
 
     KEEP_BYTES = 320 << 20
     MAX_FLAGS = 32
@@ -1124,8 +1127,16 @@ class Planes:
     def __init__(self):
         self._made = {}
         self._bytes = 0
+        self._largest = 0
         self._flags = None
         self._used = 0
+
+    def bound(self, *operands) -> int:
+        """The bytes of planes held at a time, once the call has these operands."""
+        for t in operands:
+            if t is not None and 4 * t.numel() > self._largest:
+                self._largest = 4 * t.numel()
+        return max(self.KEEP_BYTES, self._largest)
 
     def of(self, t: torch.Tensor):
         """(planes bf16 [3, rows, cols], flag int32 [1]) of row-major fp32 t.  The
@@ -1134,7 +1145,7 @@ class Planes:
         hit = self._made.pop(key, None)
         if hit is None:
             nbytes = 6 * t.numel()
-            while self._made and self._bytes + nbytes > self.KEEP_BYTES:
+            while self._made and self._bytes + nbytes > self.bound():
                 self._forget(next(iter(self._made)))
             if self._flags is None or self._used == self.MAX_FLAGS:
                 self._flags = torch.zeros((self.MAX_FLAGS,), dtype=torch.int32, device=t.device)
@@ -1251,7 +1262,7 @@ def mm_x3(a, b, planes: Planes, a2=None, b2=None, alpha: float = 1.0,
         f"second pair {tuple(a2.shape)} @ {tuple(b2.shape)} of an [{M}, {N}] product"
 
     c = torch.empty((M, N), dtype=torch.float32, device=a.device)
-    pm, pn = _x3_panels(M, N, K if a2 is None else K + a2.shape[1], planes.KEEP_BYTES)
+    pm, pn = _x3_panels(M, N, K if a2 is None else K + a2.shape[1], planes.bound(a, b, a2, b2))
     for m in range(0, M, pm):
         for n in range(0, N, pn):
             if pm >= M and pn >= N:

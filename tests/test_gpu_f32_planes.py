@@ -141,6 +141,7 @@ def test_panels_equal_the_whole_product(layout, m, n, k, monkeypatch):
     a2, b2 = _operands(layout, m, n, k, seed=5)
     whole = G.mm_x3(a, b, G.Planes()), G.mm_x3(a, b, G.Planes(), a2, b2)
     monkeypatch.setattr(G.Planes, "KEEP_BYTES", 1 << 20)
+    monkeypatch.setattr(G.Planes, "bound", lambda self, *_: self.KEEP_BYTES)
     assert G._x3_panels(m, n, k, 1 << 20) != (m, n)
     P = G.Planes()
     assert torch.equal(whole[0], G.mm_x3(a, b, P))
