@@ -749,8 +749,9 @@ def _attr(m, name: str, default=None):
     if (isinstance(m, nn.Module) and name not in m.__dict__ and not hasattr(cls, name)
             and cls.__getattr__ is nn.Module.__getattr__
             and cls.__getattribute__ is object.__getattribute__):
+        tables = m.__dict__
         for table in ("_parameters", "_buffers", "_modules"):
-            t = m.__dict__.get(table)
+            t = tables.get(table)
             if t and name in t:
                 return t[name]
         return default
@@ -762,12 +763,6 @@ _MISSING = object()
 
 def _has(m, name: str) -> bool:
     return _attr(m, name, _MISSING) is not _MISSING
-
-
-def _own(m, name: str):
-    """m.name, its AttributeError included."""
-    v = _attr(m, name, _MISSING)
-    return getattr(m, name) if v is _MISSING else v
 
 
 def _holds_entries(proj: nn.Module, attr: str) -> bool:
@@ -816,9 +811,13 @@ def _warn_dropout(family: str, drop: nn.Module):
 def _lora_factors(proj: nn.Module, family: str = "LoRA"):
     """(W, A, B, s) of a PEFT LoRA-style wrapper's active adapter."""
     name = _active_adapter(proj)
-    _warn_dropout(family, _own(proj, "lora_dropout")[name])
-    return (_own(proj.get_base_layer(), "weight"), _own(_own(proj, "lora_A")[name], "weight"),
-            _own(_own(proj, "lora_B")[name], "weight"), float(proj.scaling[name]))
+    _warn_dropout(family, (_attr(proj, "lora_dropout") or proj.lora_dropout)[name])
+    base, la, lb = proj.get_base_layer(), _attr(proj, "lora_A")[name], _attr(proj, "lora_B")[name]
+    w, a, b = _attr(base, "weight"), _attr(la, "weight"), _attr(lb, "weight")
+    if w is None or a is None or b is None:
+        # a module that has no weight raises: None would mean no adapter
+        w, a, b = base.weight, la.weight, lb.weight
+    return w, a, b, float(proj.scaling[name])
 
 
 def _v3_extract_proj(proj: nn.Module):
