@@ -27,7 +27,7 @@ template int launch_nt16_f32<false, true, true, 6>(KArgs, hipStream_t);
 // (so no product or sum of the planes overflows where fp32's would not), or
 // below 2^-100 but not 0 (whose l would be subnormal or lost).  One such element
 // sends every product of its operand to the general-layout kernel, the splitting
-// paid for nothing: a full fine-tune step of 2048 tokens at 2048 x 5632 takes 2.37
+// paid for nothing: a full fine-tune step of 2048 tokens at 2048 x 5632 takes 2.31
 // ms, 4.36 with one in x and grad_y, 5.59 with one in every operand (5.25 without
 // planes at all).  HBM-bound: 4
 // bytes read and 6 written per element (2048 x 5632: 24 us, 4.8 TB/s).  rows of
